@@ -201,8 +201,8 @@ void solveSubspaceMatrix(const struct gridContext gc, const int l,
  *      stencil_optimization.h:5-15) ---------------------------------------- */
 DTYPE compute_volume(const struct gridContext gc, DTYPE *xPhys);
 float compute_change(DTYPE *x, DTYPE *xnew, const int nelem);
-/* OC bisection (gpu_definitions.c:127-157) on the device, three bisection
- * steps per pass over the elements; x_e sqrt(-dc_e / (dv_e lmid)) is formed
+/* OC bisection (gpu_definitions.c:127-157) on the device, 31 multipliers per
+ * pass over the elements; x_e sqrt(-dc_e / (dv_e lmid)) is formed
  * as x_e sqrt(-dc_e / dv_e) / sqrt(lmid), within a few ulp of the one-step
  * expression. */
 void update_solution(const DTYPE *x, DTYPE *xnew, const DTYPE *dv,
@@ -213,7 +213,7 @@ void update_solution(const DTYPE *x, DTYPE *xnew, const DTYPE *dv,
  * and dc must be device pointers or mapped host arrays (unmapped host arrays
  * are rejected, TOP3D_ERR_UNMAPPED, instead of being staged).  It calls no
  * hipMalloc/hipFree: the bisection state and the per-workgroup partial sums
- * live in a per-device static array of 8 + 15 * 1024 doubles (123 KB, the
+ * live in a per-device static array of 2 (8 + 31 * 256) doubles (127 KB, the
  * same for every nelem; nelem < 0 is rejected), held until the process
  * ends.  Calls on one GPU share that array, so calls that overlap on one GPU
  * (two host threads, or two streams) race; each call initialises the array

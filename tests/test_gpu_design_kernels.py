@@ -1,0 +1,76 @@
+"""GPU checks of the design-loop kernels at the sizes where they can go
+wrong: the OC bisection at its first, second and later passes over the
+multipliers, at ragged element counts and in place."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import top3d_amd
+
+pytestmark = pytest.mark.gpu
+
+
+def _p(t):
+    return ctypes.c_void_p(t.data_ptr())
+
+
+def oc_reference(x, dv, dc, gval):
+    """The bisection of the optimality-criteria update, one multiplier per
+    step, in double precision."""
+    l1, l2 = 0.0, 1e9
+    xnew = x
+    with np.errstate(divide="ignore", invalid="ignore"):
+        while (l2 - l1) / (l1 + l2) > 1e-6:
+            lmid = 0.5 * (l2 + l1)
+            t = x * np.sqrt(-dc / (dv * lmid))
+            xnew = np.fmax(0.0, np.fmax(x - 0.2, np.fmin(1.0, np.fmin(x + 0.2, t))))
+            if np.sum(dv * (xnew - x)) + gval > 0:
+                l1 = lmid
+            else:
+                l2 = lmid
+    return xnew
+
+
+# scale of the sensitivities: the root lies above 5e8 (no halving), within the
+# first 31 halvings of 1e9, within the second and within the third
+@pytest.mark.parametrize("scale", [1e9, 1.0, 1e-9, 1e-16])
+@pytest.mark.parametrize("n", [1, 1023, 1025, 262145, 524289 + 1024])
+def test_oc_update_matches_stepwise_bisection(n, scale):
+    print(f"[gpu oc] n {n} scale {scale}", flush=True)
+    rng = np.random.default_rng(n)
+    x = rng.uniform(0.05, 0.95, n)
+    dv = rng.uniform(0.5, 1.5, n)
+    dc = -scale * rng.uniform(0.5, 1.5, n)
+    gval = 0.01 * (1 if n % 2 else -1) * min(1.0, 0.5 * n * 0.05)
+    ref = oc_reference(x, dv, dc, gval)
+    d = [torch.from_numpy(a).cuda() for a in (x, dv, dc)]
+    got = torch.full((n,), -1.0, dtype=torch.float64, device="cuda")
+    lib = top3d_amd.library()
+    lib.top3d_set_stream(ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    lib.update_solution(_p(d[0]), _p(got), _p(d[1]), _p(d[2]), n, gval)
+    top3d_amd.check("update_solution")
+    # the same multiplier, visited by the same steps: x differs by the
+    # rounding of a sqrt(-dc/dv) / sqrt(lmid) (4 roundings of 2^-53)
+    assert np.abs(got.cpu().numpy() - ref).max() <= 8 * 2.0 ** -53
+
+
+def test_oc_update_in_place():
+    """xnew may be one of the inputs: the result of the update elsewhere."""
+    n = 300_001
+    rng = np.random.default_rng(11)
+    x, dv, dc = (torch.from_numpy(a).cuda() for a in (
+        rng.uniform(0.05, 0.95, n), rng.uniform(0.5, 1.5, n), -rng.uniform(0.5, 1.5, n)))
+    lib = top3d_amd.library()
+    lib.top3d_set_stream(ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    out = torch.empty_like(x)
+    torch.cuda.synchronize()
+    lib.update_solution(_p(x), _p(out), _p(dv), _p(dc), n, 0.01)
+    for k in range(3):
+        a = [x.clone(), dv.clone(), dc.clone()]
+        torch.cuda.synchronize()
+        lib.update_solution(_p(a[0]), _p(a[k]), _p(a[1]), _p(a[2]), n, 0.01)
+        top3d_amd.check("update_solution")
+        assert torch.equal(a[k], out)

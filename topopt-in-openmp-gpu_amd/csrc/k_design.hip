@@ -397,35 +397,32 @@ void launch_change(int64_t n, double *x, const double *xnew, double *partials, d
 
 // ---- optimality criteria (gpu_definitions.c:127-157) ----------------------
 // The bisection of gpu_definitions.c:127-157 evaluates one multiplier per
-// pass over the elements.  Here one pass evaluates the kOcDepth levels of the
-// bisection tree below the current interval (2^kOcDepth - 1 multipliers), and
-// a one-block kernel walks the tree with the sums, so the multipliers visited
-// are those of the step-by-step loop.  The element arrays are read once per
-// kOcDepth steps.  The candidate x_e sqrt(-dc_e / (dv_e lmid)) is formed as
-// x_e sqrt(-dc_e / dv_e) * (1 / sqrt(lmid)), one division and square root per
-// element instead of per multiplier (a few ulp from the one-step form).
-constexpr int kOcDepth = 3;
+// pass over the elements.  Here a pass evaluates kOcCand = 31 multipliers that
+// the loop would visit next, and the walk over their sums visits exactly the
+// multipliers of the step-by-step loop:
+//   l1 = 0 (no upward step yet): the 31 next halvings of l2, of which the
+//     walk takes all up to the first upward step, so that one or two passes
+//     replace the 30 to 60 steps from 1e9 down to the root's binade;
+//   l1 > 0: the five levels of the bisection tree below [l1, l2].
+// About 20 tree steps remain once l1 > 0, so an update takes 5 or 6 passes.
+// (x_e sqrt(-dc_e / (dv_e lmid)) is formed as x_e sqrt(-dc_e / dv_e) times
+// 1 / sqrt(lmid): one division and square root per element and pass.)
+//
+// A pass reads 24 bytes per element and spends 4 FP64 instructions per
+// multiplier and element; at 31 multipliers the instructions bound it (35 us
+// at 256x128x128, 18 of them the reads').  An update of that grid takes 6
+// passes, 0.24 ms with the final write, against 0.66 ms for the 20 passes of 7
+// multipliers (20.6 us each, and a one-workgroup walk of 6.6 us after each)
+// that it replaced.  Fewer multipliers per pass come out even: a pass costs
+// about 20 us more than 0.5 us per multiplier.  The walk over a pass's sums is done redundantly by every
+// workgroup of the next kernel (kOcCand x kOcBlocks partial sums, 63 KB from
+// the L2) instead of by a one-workgroup kernel in between.
+constexpr int kOcDepth = 5;
 constexpr int kOcCand = (1 << kOcDepth) - 1;
-constexpr int kOcChunk = 24;  // passes between host checks (72 bisection steps)
-static_assert(kOcScratchDoubles >= 8 + kOcCand * kPartials, "OC scratch size");
-
-// Multipliers of the tree below [l1, l2], in heap order: node n has the
-// lower half as child 2n+1 and the upper half as child 2n+2.
-__device__ __forceinline__ void oc_tree(double l1, double l2, double (&mid)[kOcCand]) {
-  double lo[kOcCand], hi[kOcCand];
-  lo[0] = l1;
-  hi[0] = l2;
-#pragma unroll
-  for (int n = 0; n < kOcCand; n++) {
-    mid[n] = 0.5 * (hi[n] + lo[n]);
-    if (2 * n + 2 < kOcCand) {
-      lo[2 * n + 1] = lo[n];
-      hi[2 * n + 1] = mid[n];
-      lo[2 * n + 2] = mid[n];
-      hi[2 * n + 2] = hi[n];
-    }
-  }
-}
+constexpr int kOcBS = 1024;     // threads: 16 waves, one workgroup per CU
+constexpr int kOcBlocks = 256;
+constexpr int kOcPasses = 6;    // passes between host checks
+static_assert(kOcScratchDoubles >= 2 * (8 + kOcCand * kOcBlocks), "OC scratch size");
 
 // xnew_e for a multiplier with rl = 1 / sqrt(lmid), a = x_e sqrt(-dc_e / dv_e):
 // move limit 0.2, bounds [0, 1].
@@ -434,122 +431,212 @@ __device__ __forceinline__ double oc_x(double xi, double a, double rl) {
   return fmax(0.0, fmax(xi - move, fmin(1.0, fmin(xi + move, a * rl))));
 }
 
-// state: [0] l1, [1] l2, [3] converged flag, [4] gval, [5] last multiplier,
-// [6] steps taken.  partials: kOcCand rows of gridDim.x block sums.
-__global__ __launch_bounds__(kBS) void k_oc_pass(int64_t n, const double *__restrict__ x,
-                                                 const double *__restrict__ dv,
-                                                 const double *__restrict__ dc,
-                                                 const double *__restrict__ state,
-                                                 double *__restrict__ partials) {
-  if (state[3] != 0.0) return;
-  double rl[kOcCand];
-  oc_tree(state[0], state[1], rl);
-  double s[kOcCand];
-#pragma unroll
-  for (int c = 0; c < kOcCand; c++) {
-    rl[c] = 1.0 / sqrt(rl[c]);
-    s[c] = 0.0;
+// The bisection state.  pending: the partial sums of the candidates of
+// [l1, l2] are waiting to be walked.
+struct OcState {
+  double l1, l2, done, gval, lmid, steps, pending, unused;
+};
+
+// Candidates of [l1, l2]: for l1 = 0 candidate c is l2 halved c + 1 times;
+// else heap order, node n with the lower half as child 2n+1 and the upper
+// half as child 2n+2 (the path from the root is spelt by the bits of n + 1).
+__device__ __forceinline__ double oc_candidate(double l1, double l2, int c) {
+  if (l1 == 0.0) {
+    double mid = 0.5 * (l2 + l1);
+    for (int q = 0; q < c; q++) mid = 0.5 * (mid + l1);
+    return mid;
   }
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double xi = x[i], dvi = dv[i];
-    const double a = xi * sqrt(-dc[i] / dvi);
-#pragma unroll
-    for (int c = 0; c < kOcCand; c++) s[c] += dvi * (oc_x(xi, a, rl[c]) - xi);
+  double lo = l1, hi = l2, mid = 0.5 * (hi + lo);
+  const int depth = 31 - __clz(c + 1);
+  for (int d = depth - 1; d >= 0; d--) {
+    if (((c + 1) >> d) & 1) lo = mid; else hi = mid;
+    mid = 0.5 * (hi + lo);
   }
-#pragma unroll
-  for (int c = 0; c < kOcCand; c++) {
-    const double t = blk_sum(s[c]);
-    if (threadIdx.x == 0) partials[(int64_t)c * gridDim.x + blockIdx.x] = t;
-  }
+  return mid;
 }
 
-// One workgroup of kOcCand wavefronts, wave c summing multiplier c's
-// partials; then up to kOcDepth bisection steps down the tree, stopping where
-// the interval has converged.
-__global__ __launch_bounds__(64 * kOcCand) void k_oc_walk(const double *__restrict__ partials,
-                                                          int np, double *__restrict__ state) {
-  if (state[3] != 0.0) return;
-  __shared__ double S[kOcCand];
-  const int c = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  double s = 0;
-  for (int i = lane; i < np; i += 64) s += partials[c * np + i];
+// The state after walking the pending sums (np partial sums per candidate),
+// in LDS for every thread; S: kOcCand doubles of LDS.
+__device__ __forceinline__ OcState oc_walk(const OcState *__restrict__ in,
+                                           const double *__restrict__ partials, int np,
+                                           double *S, OcState *st) {
+  const OcState old = *in;
+  if (old.done == 0.0 && old.pending != 0.0) {
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int c = w; c < kOcCand; c += kOcBS / 64) {
+      double s = 0.0;
+      for (int i = lane; i < np; i += 64) s += partials[c * np + i];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if (lane == 0) S[c] = s;
+      for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+      if (lane == 0) S[c] = s;
+    }
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    double l1 = state[0], l2 = state[1];
-    int node = 0;
-    for (int d = 0; d < kOcDepth; d++) {
-      const double lmid = 0.5 * (l2 + l1);
-      state[5] = lmid;
-      state[6] += 1.0;
-      if (S[node] + state[4] > 0) {
-        l1 = lmid;
-        node = 2 * node + 2;
-      } else {
-        l2 = lmid;
-        node = 2 * node + 1;
-      }
-      if (!((l2 - l1) / (l1 + l2) > 1e-6)) {
-        state[3] = 1.0;
-        break;
+    OcState n = old;
+    if (old.done == 0.0 && old.pending != 0.0) {
+      const bool spine = old.l1 == 0.0;
+      n.pending = 0.0;
+      int node = 0;
+      for (int d = 0; d < (spine ? kOcCand : kOcDepth); d++) {
+        const double lmid = 0.5 * (n.l2 + n.l1);
+        const bool up = S[node] + n.gval > 0;
+        n.lmid = lmid;
+        n.steps += 1.0;
+        if (up) n.l1 = lmid; else n.l2 = lmid;
+        node = spine ? node + 1 : 2 * node + (up ? 2 : 1);
+        if (spine && !up && n.l2 > 0.0) continue;  // l1 = 0: the ratio is 1
+        if (!((n.l2 - n.l1) / (n.l1 + n.l2) > 1e-6)) {
+          n.done = 1.0;
+          break;
+        }
+        if (spine && up) break;
       }
     }
-    state[0] = l1;
-    state[1] = l2;
+    *st = n;
+  }
+  __syncthreads();
+  return *st;
+}
+
+// One pass: walks the sums of the previous one, then leaves the partial sums
+// of the new candidates.  state, partials: the two buffers of each, of which
+// [cur] is read and [cur ^ 1] written (every workgroup reads the old ones).
+// first: the state is [0, 1e9] with this gval.  A: where xnew overlaps none of
+// the inputs, the first pass leaves x_e sqrt(-dc_e / dv_e) in xnew for the
+// passes after it (57 of their 181 instructions per element), which the
+// final write replaces.
+template <bool FIRST, bool A>
+__global__ __launch_bounds__(kOcBS) void k_oc_pass(int64_t n, const double *x, const double *dv,
+                                                   const double *dc, double *xnew,
+                                                   double gval, OcState *state,
+                                                   double *partials, int cur) {
+  __shared__ double S[kOcCand + 1];
+  __shared__ OcState sst;
+  __shared__ double red[kOcBS / 64][kOcCand + 1];
+  const int t = threadIdx.x, np = gridDim.x;
+  OcState st;
+  if (FIRST) {
+    st = OcState{0.0, 1e9, 0.0, gval, 0.0, 0.0, 0.0, 0.0};
+  } else {
+    st = oc_walk(state + cur, partials + cur * kOcCand * kOcBlocks, np, S, &sst);
+  }
+  if (st.done == 0.0) st.pending = 1.0;
+  if (blockIdx.x == 0 && t == 0) state[cur ^ 1] = st;
+  if (st.done != 0.0) return;  // (uniform)
+  __syncthreads();
+  if (t < kOcCand) S[t] = 1.0 / sqrt(oc_candidate(st.l1, st.l2, t));
+  __syncthreads();
+  double rl[kOcCand], s[kOcCand + 1];
+#pragma unroll
+  for (int c = 0; c < kOcCand; c++) {
+    // one value for the workgroup: kept in scalar registers
+    const uint64_t b = __double_as_longlong(S[c]);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+    rl[c] = __longlong_as_double(((uint64_t)hi << 32) | lo);
+    s[c] = 0.0;
+  }
+  s[kOcCand] = 0.0;
+  const double move = 0.2;
+  const int64_t stride = (int64_t)gridDim.x * kOcBS;
+  // two elements per step; past the end element i again, with weight 0
+  for (int64_t i = (int64_t)blockIdx.x * kOcBS + t; i < n; i += 2 * stride) {
+    double xe[2], ve[2], ae[2];
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const int64_t j = e == 0 || i + stride < n ? i + e * stride : i;
+      xe[e] = x[j];
+      ve[e] = dv[j];
+      ae[e] = A && !FIRST ? xnew[j] : dc[j];
+    }
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const bool in = e == 0 || i + stride < n;
+      const double a = A && !FIRST ? ae[e] : xe[e] * sqrt(-ae[e] / ve[e]);
+      if (A && FIRST && in) xnew[i + e * stride] = a;
+      const double w = in ? ve[e] : 0.0;
+      const double hi = fmin(1.0, xe[e] + move), lo = fmax(0.0, xe[e] - move);
+      // slot kOcCand: the sum of dv x that every candidate's sum leaves out
+#pragma unroll
+      for (int c = 0; c < kOcCand; c++) s[c] = fma(w, fmax(lo, fmin(hi, a * rl[c])), s[c]);
+      s[kOcCand] = fma(w, xe[e], s[kOcCand]);
+    }
+  }
+  // Wave sums of the 32 values by halving: at each step a lane keeps half of
+  // its values and adds its partner's copies of them (32 exchanges instead of
+  // 6 per value); lane l ends with the sum of value brev5(l & 31), over its
+  // half of the wave, and the last exchange adds the other half.
+  const int lane = t & 63;
+#pragma unroll
+  for (int h = 16; h > 0; h >>= 1) {
+    const int bit = 16 / h;  // lane bits 1, 2, 4, 8, 16
+    const bool upper = (lane & bit) != 0;
+#pragma unroll
+    for (int c = 0; c < h; c++) {
+      const double give = upper ? s[c] : s[c + h], keep = upper ? s[c + h] : s[c];
+      s[c] = keep + __shfl_xor(give, bit, 64);
+    }
+  }
+  s[0] += __shfl_xor(s[0], 32, 64);
+  if (lane < 32) red[t >> 6][__brev((unsigned)lane) >> 27] = s[0];
+  __syncthreads();
+  if (t < kOcCand) {
+    double v = 0.0;
+    for (int w = 0; w < kOcBS / 64; w++) v += red[w][t] - red[w][kOcCand];
+    partials[((cur ^ 1) * kOcCand) * kOcBlocks + (int64_t)t * np + blockIdx.x] = v;
   }
 }
 
-// xnew for the last multiplier the walk visited.
-__global__ __launch_bounds__(kBS) void k_oc_write(int64_t n, const double *__restrict__ x,
-                                                  double *__restrict__ xnew,
-                                                  const double *__restrict__ dv,
-                                                  const double *__restrict__ dc,
-                                                  const double *__restrict__ state) {
-  const double rl = 1.0 / sqrt(state[5]);
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
+// xnew for the last multiplier the walk visited; the state for the host.
+__global__ __launch_bounds__(kOcBS) void k_oc_write(int64_t n, const double *x, double *xnew,
+                                                    const double *dv, const double *dc,
+                                                    OcState *state, const double *partials,
+                                                    int cur) {
+  __shared__ double S[kOcCand + 1];
+  __shared__ OcState sst;
+  const OcState st =
+      oc_walk(state + cur, partials + cur * kOcCand * kOcBlocks, gridDim.x, S, &sst);
+  if (blockIdx.x == 0 && threadIdx.x == 0) state[cur ^ 1] = st;
+  const double rl = 1.0 / sqrt(st.lmid);
+  for (int64_t i = (int64_t)blockIdx.x * kOcBS + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * kOcBS) {
     const double xi = x[i];
     xnew[i] = oc_x(xi, xi * sqrt(-dc[i] / dv[i]), rl);
   }
 }
 
-// the bisection state of one OC update: [l1, l2] = [0, 1e9], not converged
-__global__ void k_oc_init(double gval, double *__restrict__ state) {
-  if (threadIdx.x < 8) {
-    const double init[8] = {0.0, 1e9, 0.0, 0.0, gval, 0.0, 0.0, 0.0};
-    state[threadIdx.x] = init[threadIdx.x];
-  }
-}
-
-// Runs the bisection, checking on the host every kOcChunk passes (passes
+// Runs the bisection, checking on the host every kOcPasses passes (passes
 // after convergence return at once).  xnew is written after each chunk for
 // the last multiplier, so a converged chunk needs no further launch.
-// scratch (kOcScratchDoubles doubles of device memory) is initialised here:
-// its previous contents do not matter.  Returns the number of bisection
-// steps or -1.
+// scratch (kOcScratchDoubles doubles of device memory): its previous contents
+// do not matter.  Returns the number of bisection steps or -1.
 int oc_update(const double *x, double *xnew, const double *dv, const double *dc,
               int64_t nelem, double gval, double *scratch) {
-  double *state = scratch;          // 8 doubles
-  double *partials = scratch + 8;   // kOcCand * kPartials doubles
-  hipLaunchKernelGGL(k_oc_init, dim3(1), dim3(64), 0, stream(), gval, state);
-  if (!T3D_HIP(hipGetLastError())) return -1;
-  double h[8];
-  for (int it = 0; it < 4096; it += kOcChunk * kOcDepth) {
-    for (int q = 0; q < kOcChunk; q++) {
-      hipLaunchKernelGGL(k_oc_pass, dim3(kPartials), dim3(kBS), 0, stream(), nelem, x, dv, dc,
-                         state, partials);
-      hipLaunchKernelGGL(k_oc_walk, dim3(1), dim3(64 * kOcCand), 0, stream(), partials,
-                         kPartials, state);
+  OcState *state = (OcState *)scratch;  // 2 of 8 doubles
+  double *partials = scratch + 16;      // 2 x kOcCand x kOcBlocks
+  const dim3 grid((unsigned)std::max<int64_t>(
+      1, std::min<int64_t>(kOcBlocks, (nelem + kOcBS - 1) / kOcBS)));
+  int cur = 0;
+  OcState h{};
+  auto apart = [&](const double *p) { return p + nelem <= xnew || xnew + nelem <= p; };
+  // the first chunk only: the write after it replaces what a pass left there
+  bool a = apart(x) && apart(dv) && apart(dc);
+  for (int pass = 0; h.steps < 4096.0; a = false) {
+    for (int q = 0; q < kOcPasses; q++, pass++, cur ^= 1) {
+      auto *k = pass == 0 ? (a ? k_oc_pass<true, true> : k_oc_pass<true, false>)
+                          : (a ? k_oc_pass<false, true> : k_oc_pass<false, false>);
+      hipLaunchKernelGGL(k, grid, dim3(kOcBS), 0, stream(), nelem, x, dv, dc, xnew, gval, state,
+                         partials, cur);
     }
-    hipLaunchKernelGGL(k_oc_write, dim3(kPartials), dim3(kBS), 0, stream(), nelem, x, xnew, dv,
-                       dc, state);
-    if (!T3D_HIP(hipMemcpyAsync(h, state, sizeof(h), hipMemcpyDeviceToHost, stream())) ||
+    hipLaunchKernelGGL(k_oc_write, grid, dim3(kOcBS), 0, stream(), nelem, x, xnew, dv, dc, state,
+                       partials, cur);
+    cur ^= 1;
+    if (!T3D_HIP(hipGetLastError()) ||
+        !T3D_HIP(hipMemcpyAsync(&h, state + cur, sizeof(h), hipMemcpyDeviceToHost, stream())) ||
         !T3D_HIP(hipStreamSynchronize(stream())))
       return -1;
-    if (h[3] != 0.0) return (int)h[6];
+    if (h.done != 0.0) return (int)h.steps;
   }
   set_error(TOP3D_ERR_NO_CONVERGE, "update_solution: OC bisection did not converge in 4096 steps");
   return -1;
