@@ -381,6 +381,17 @@ int top3d_compliance_backward(const struct gpuGrid *gpu_gc, double rmin,
                               const double *xPhys_dev, const double *U_dev,
                               double grad_c, double *grad_x_dev);
 
+/* The density filter out = (H in) / Hs (transpose = 0) or its transpose
+ * out = H (in / Hs) between two device (or mapped) element arrays, in != out;
+ * the halo elements of out keep their values, become zero or take those of
+ * in.  applyDensityFilter and applyDensityFilterGradient without their staging
+ * and, for the latter, without the copy back into its in-place argument.     */
+#define TOP3D_HALO_KEEP 0
+#define TOP3D_HALO_ZERO 1
+#define TOP3D_HALO_COPY 2
+int top3d_density_filter(const struct gridContext *gc, double rmin, int transpose, int halo,
+                         const double *in, double *out);
+
 /* Times `reps` back-to-back launches of one hot kernel on the buffers of the
  * last solve (HIP events on the library stream).  `which`:
  *   0 fine damped-Jacobi sweep, FP32 (mixed V-cycle)

@@ -1,12 +1,14 @@
 """GPU checks of the design-loop kernels at the sizes where they can go
 wrong: the OC bisection at its first, second and later passes over the
-multipliers, at ragged element counts and in place."""
+multipliers and at ragged element counts, the density filter's tiles at the
+edges of tiles and at grids narrower than the window."""
 import ctypes
 
 import numpy as np
 import pytest
 import torch
 
+import pyoracle
 import top3d_amd
 
 pytestmark = pytest.mark.gpu
@@ -55,6 +57,47 @@ def test_oc_update_matches_stepwise_bisection(n, scale):
     # the same multiplier, visited by the same steps: x differs by the
     # rounding of a sqrt(-dc/dv) / sqrt(lmid) (4 roundings of 2^-53)
     assert np.abs(got.cpu().numpy() - ref).max() <= 8 * 2.0 ** -53
+
+
+@pytest.mark.parametrize("shape", [(8, 4, 4), (36, 12, 20), (16, 32, 8), (12, 36, 44)])
+@pytest.mark.parametrize("rmin", [0.7, 1.0, 1.5, 2.0, 2.9, 3.5, 4.5, 6.0, 7.0, 7.5])
+def test_filter_tiles(shape, rmin):
+    print(f"[gpu filter] {shape} rmin {rmin}", flush=True)
+    nelx, nely, nelz = shape
+    g, o = top3d_amd.Grid(nelx, nely, nelz, 3), pyoracle.Grid(nelx, nely, nelz, 3)
+    rng = np.random.default_rng(3)
+    inter = g.interior_elements()
+    x = g.density(rng.uniform(0.1, 1.0, inter.size))
+    v = g.density(rng.uniform(-1.0, 1.0, inter.size))
+    halo = np.ones(g.nelem, bool)
+    halo[inter] = False
+    v[torch.from_numpy(halo).cuda()] = 7.0  # read by nothing, kept in the result
+    r = np.arange(-8, 9)
+    d = np.sqrt(r[:, None, None] ** 2 + r[None, :, None] ** 2 + r[None, None, :] ** 2)
+    taps = int((d < rmin).sum())
+    tol = (2 * taps + 4) * 2.0 ** -53  # each sum in an order of its own, a division
+    y = g.filter(rmin, x).cpu().numpy()
+    ref = o.filter(rmin, x.cpu().numpy())
+    assert np.abs(y[inter] - ref[inter]).max() <= tol * np.abs(ref[inter]).max()
+    assert not y[halo].any()
+    w = g.filter_grad(rmin, v).cpu().numpy()
+    vr = v.cpu().numpy()
+    ref = o.filter_grad(rmin, vr.copy())
+    size = o.filter_grad(rmin, np.abs(vr))  # the sums' absolute terms
+    assert (np.abs(w - ref)[inter] <= tol * size[inter]).all()
+    assert (w[halo] == 7.0).all()
+    # a NaN reaches the elements within the radius only (the tiles apply no
+    # zero weight; beyond radius 7 the loop over the whole window runs)
+    c = (nelx // 2 + 1, nelz // 2 + 1, nely // 2 + 1)
+    x[(c[0] * (nelz + 2) + c[1]) * (nely + 2) + c[2]] = float("nan")
+    i, k, j = np.meshgrid(*(np.arange(1, m + 1) for m in (nelx, nelz, nely)), indexing="ij")
+    near = np.sqrt((i - c[0]) ** 2 + (k - c[1]) ** 2 + (j - c[2]) ** 2).ravel() < rmin
+    bad = np.isnan(g.filter(rmin, x).cpu().numpy())[inter]
+    assert bad[near].all()
+    if rmin <= 7.0:
+        assert not bad[~near].any()
+    g.close()
+    o.close()
 
 
 def test_oc_update_in_place():

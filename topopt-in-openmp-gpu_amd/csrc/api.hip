@@ -13,7 +13,7 @@ namespace t3d {
 
 enum { kApplyMode = 0, kJacobiMode = 1, kResidualMode = 2 };
 enum { kSlotE64 = 0, kSlotE32 = 1, kSlotTmp = 2, kSlotRed = 3, kSlotKe = 4, kSlotS = 5,
-       kSlotVec = 6, kSlotAux = 7 };
+       kSlotVec = 6 };
 
 static double *young64(DevGrid &g, const double *dx) {
   double *E = (double *)g.work(kSlotE64, sizeof(double) * g.nelem);
@@ -722,7 +722,7 @@ void applyDensityFilter(const struct gridContext gc, const DTYPE rmin, const DTY
   if (!vr.open(rho, sizeof(double) * g->nelem, true, false) ||
       !vo.open(out, sizeof(double) * g->nelem, true, true))
     return;
-  launch_filter(*g, rmin, (const double *)vr.dev, (double *)vo.dev);
+  launch_filter(*g, rmin, (const double *)vr.dev, (double *)vo.dev, 0);
   sync_ok();
   vo.close();
   vr.close();
@@ -735,14 +735,29 @@ void applyDensityFilterGradient(const struct gridContext gc, const DTYPE rmin, D
   DevView vv;
   if (!vv.open(v, sizeof(double) * g->nelem, true, true)) return;
   double *tmp = (double *)g->work(kSlotTmp, sizeof(double) * g->nelem);
-  double *tmp2 = (double *)g->work(kSlotAux, sizeof(double) * g->nelem);
-  launch_filter_grad(*g, rmin, (const double *)vv.dev, tmp, tmp2);
-  // interior elements take the filtered value; the halo of v is untouched
-  hipLaunchKernelGGL(k_copy_interior_elems, dim3((g->nelem + 255) / 256), dim3(256), 0, stream(),
-                     g->nelem, g->nelx, g->nely, g->nelz, g->ewy, g->ewz, tmp2,
-                     (double *)vv.dev);
+  if (tmp && launch_filter_grad(*g, rmin, (const double *)vv.dev, tmp, 0))
+    // interior elements take the filtered value; the halo of v is untouched
+    hipLaunchKernelGGL(k_copy_interior_elems, dim3((g->nelem + 255) / 256), dim3(256), 0,
+                       stream(), g->nelem, g->nelx, g->nely, g->nelz, g->ewy, g->ewz, tmp,
+                       (double *)vv.dev);
   sync_ok();
   vv.close();
+}
+
+int top3d_density_filter(const struct gridContext *gc, double rmin, int transpose, int halo,
+                         const double *in, double *out) {
+  DevGrid *g = dev_grid(gc);
+  if (!g) return top3d_last_error();
+  const double *di = (const double *)dptr(in, "top3d_density_filter in");
+  double *dout = (double *)dptr(out, "top3d_density_filter out");
+  if (!di || !dout || di == dout || halo < TOP3D_HALO_KEEP || halo > TOP3D_HALO_COPY) {
+    if (di && dout) set_error(TOP3D_ERR_ARG, "top3d_density_filter: in == out, or halo=%d", halo);
+    return top3d_last_error();
+  }
+  bool ok = true;
+  if (transpose) ok = launch_filter_grad(*g, rmin, di, dout, halo);
+  else launch_filter(*g, rmin, di, dout, halo);
+  return sync_ok() && ok ? TOP3D_OK : top3d_last_error();
 }
 
 // gpu_definitions.c:159-195: map every array the design loop uses
@@ -796,9 +811,7 @@ int top3d_compliance_backward(const struct gpuGrid *gpu_gc, double rmin,
   hipLaunchKernelGGL(k_scale, dim3((g->nelem + 255) / 256), dim3(256), 0, stream(), g->nelem,
                      grad_c, dc);
   if (rmin > 0) {
-    double *tmp = (double *)g->work(kSlotTmp, sizeof(double) * g->nelem);
-    launch_fill<double>(g->nelem, grad_x_dev, 0.0);
-    launch_filter_grad(*g, rmin, dc, tmp, grad_x_dev);
+    if (!launch_filter_grad(*g, rmin, dc, grad_x_dev, 1)) return top3d_last_error();
   } else {
     hipMemcpyAsync(grad_x_dev, dc, sizeof(double) * g->nelem, hipMemcpyDeviceToDevice, stream());
   }

@@ -201,154 +201,358 @@ __global__ __launch_bounds__(kBS) void k_filter(int nelx, int nely, int nelz, in
   if (MODE == 2) out[e1] = acc;
 }
 
-// The non-zero weights of the window, in the loop order of the kernel above
-// (i2, then k2, then j2 ascending).  The window's zero weights add nothing to
-// either sum, so leaving them out keeps both sums bit for bit; the weights use
-// the same expression as the loop (rmin 2.5: 81 of 216 terms).  The list is
-// padded to the kernel's unrolled length with zero weights at offset 0, which
-// add +0 to both sums.
-constexpr int kFilterMaxTaps = 240;
-struct FilterTaps {
-  int8_t di[kFilterMaxTaps], dk[kFilterMaxTaps], dj[kFilterMaxTaps];
-  double w[kFilterMaxTaps];
+// Radii up to 7: tiles in LDS.  The window's non-zero weights are those of
+// the offsets with |d| < rmin, so |di|, |dk|, |dj| <= R = ceil(rmin) - 1, and
+// a weight depends on the squared distance only (the expression above).  The
+// elements outside the grid are staged as zeros; a weight that is zero is
+// never applied.
+constexpr int kFilterMaxR = 6;
+constexpr int kFTK = 8, kFTJ = 32;  // tile in z and y, one thread per column
+// what the filter does with the elements outside the grid
+enum { kHaloKeep = 0, kHaloZero = 1, kHaloCopy = 2 };
+
+// The workgroups at the grid's faces also write the halo elements beside
+// their elements [i0, i1] x kFTK x kFTJ.
+__device__ __forceinline__ void filter_write_halo(int i0, int i1, int k0, int j0, int nelx,
+                                                  int nely, int nelz, int few, int fez, int halo,
+                                                  const double *__restrict__ in,
+                                                  double *__restrict__ out) {
+  const int il = i0 == 1 ? 0 : i0, ih = i1 >= nelx ? nelx + 1 : i1;
+  const int kl = k0 == 1 ? 0 : k0, kh = k0 + kFTK > nelz ? nelz + 1 : k0 + kFTK - 1;
+  const int jl = j0 == 1 ? 0 : j0, jh = j0 + kFTJ > nely ? nely + 1 : j0 + kFTJ - 1;
+  if (!(il == 0 || ih > nelx || kl == 0 || kh > nelz || jl == 0 || jh > nely)) return;
+  const int nj = jh - jl + 1, nk = kh - kl + 1, ni = ih - il + 1;
+  for (int q = threadIdx.x; q < ni * nk * nj; q += kFTK * kFTJ) {
+    const int jj = jl + q % nj, kk = kl + (q / nj) % nk, ii = il + q / (nj * nk);
+    if (ii >= 1 && ii <= nelx && kk >= 1 && kk <= nelz && jj >= 1 && jj <= nely) continue;
+    const int64_t e = ((int64_t)ii * fez + kk) * few + jj;
+    out[e] = halo == kHaloCopy ? in[e] : 0.0;
+  }
+}
+
+// R = 1 (rmin <= 2, weights w0..w3 at squared distance 0..3).  A workgroup
+// marches along x over ni element planes of its 32 x 8 columns, with the next
+// plane's loads in flight and one barrier per plane.  Per plane a thread sums
+// its 9 neighbours by in-plane distance,
+//   A0 the element, A1 the 4 beside it, A2 the 4 corners,
+// and an element's sum takes those of three planes,
+//   w0 A0 + w1 (A1 + A0- + A0+) + w2 (A2 + A1- + A1+) + w3 (A2- + A2+).
+// The sum of the weights Hs follows from the same counts of elements inside
+// the grid (C1 of 4, C2 of 4, n of 2 planes).
+// TR = false: out = (H in) / Hs; TR = true: out = H (in / Hs).
+// Bound by the step of each plane (wait, barrier, nine LDS reads) rather than
+// by its 16 bytes per element: 29 us (filter) and 30 us (transpose) at
+// 256x128x128, where one thread per element with its window's loads and
+// range checks took 43 us, and 20 us for the division and 41 us for the sums
+// of the transpose, with a fill and two copies around them.
+template <bool TR>
+__global__ __launch_bounds__(kFTJ *kFTK) void k_filter_march(
+    int nelx, int nely, int nelz, int few, int fez, int ni, double w0, double w1, double w2,
+    double w3, const double *__restrict__ in, double *__restrict__ out, int halo) {
+  constexpr int LJ = kFTJ + 2, LK = kFTK + 2, NS = LJ * LK, NT = kFTJ * kFTK;
+  __shared__ double tile[2][NS];
+  const int t = threadIdx.x;
+  const int j0 = 1 + kFTJ * blockIdx.x, k0 = 1 + kFTK * blockIdx.y, i0 = 1 + ni * blockIdx.z;
+  const int i1 = min(i0 + ni - 1, nelx);
+  // Hs = base + n * slope at a column, n of the planes beside it in the grid
+  auto column = [&](int k, int j, double &base, double &slope) {
+    const double cj = (j > 1) + (j < nely), ck = (k > 1) + (k < nelz);
+    const double c1 = cj + ck, c2 = cj * ck;
+    base = w0 + (w1 * c1 + w2 * c2);
+    slope = w1 + (w2 * c1 + w3 * c2);
+  };
+  auto planes = [&](int i) { return (double)((i > 1) + (i < nelx)); };
+  // the one or two elements of a plane that this thread stages
+  bool ok[2];
+  int64_t off[2];
+  double sb[2], ss[2], v[2];
+#pragma unroll
+  for (int e = 0; e < 2; e++) {
+    const int q = t + e * NT;
+    const int j = j0 - 1 + q % LJ, k = k0 - 1 + q / LJ;
+    ok[e] = q < NS && k >= 1 && k <= nelz && j >= 1 && j <= nely;
+    off[e] = ok[e] ? (int64_t)k * few + j : 0;
+    if (TR) column(k, j, sb[e], ss[e]);
+  }
+  const int64_t plane = (int64_t)fez * few;
+  auto load = [&](int i) {  // (planes 0 and nelx + 1 exist, and count as zero)
+#pragma unroll
+    for (int e = 0; e < 2; e++) v[e] = in[i * plane + off[e]];
+  };
+  const int tj = t % kFTJ, tk = t / kFTJ, j = j0 + tj, k = k0 + tk;
+  const bool own = j <= nely && k <= nelz;
+  double base, slope;
+  column(k, j, base, slope);
+  double am[3] = {0, 0, 0}, a0[3] = {0, 0, 0}, ap[3];
+  load(i0 - 1);
+  for (int p = i0 - 1; p <= i1 + 1; p++) {
+    double *buf = tile[p & 1];
+    const bool pin = p >= 1 && p <= nelx;
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      double x = ok[e] && pin ? v[e] : 0.0;
+      if (TR) x /= ss[e] * planes(p) + sb[e];
+      if (t + e * NT < NS) buf[t + e * NT] = x;
+    }
+    load(min(p + 1, i1 + 1));
+    __syncthreads();
+    const double *c = buf + (tk + 1) * LJ + tj + 1;
+    ap[0] = c[0];
+    ap[1] = (c[-1] + c[1]) + (c[-LJ] + c[LJ]);
+    ap[2] = (c[-LJ - 1] + c[-LJ + 1]) + (c[LJ - 1] + c[LJ + 1]);
+    const int i = p - 1;
+    if (own && i >= i0 && i <= i1) {
+      double acc = w0 * a0[0];
+      if (w1 != 0.0) acc += w1 * (a0[1] + (am[0] + ap[0]));
+      if (w2 != 0.0) acc += w2 * (a0[2] + (am[1] + ap[1]));
+      if (w3 != 0.0) acc += w3 * (am[2] + ap[2]);
+      out[i * plane + (int64_t)k * few + j] = TR ? acc : acc / (slope * planes(i) + base);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      am[q] = a0[q];
+      a0[q] = ap[q];
+    }
+  }
+  if (halo != kHaloKeep)
+    filter_write_halo(i0, i1, k0, j0, nelx, nely, nelz, few, fez, halo, in, out);
+}
+
+// R >= 2.  A workgroup stages its kFTI x 8 x 32 elements (x, z, y) and R more
+// on every side, and each thread sums the kFTI elements of one column along
+// x.  The offsets (dk, dj) of one in-plane distance m share their weights, so
+// their columns are added first (one LDS read and one addition per value) and
+// the weights are applied once per m, to a column whose half length is the
+// largest |di| with a weight.  The LDS reads bound it (rmin 3.5: 86 per
+// element for 179 weights).  At 168x72x104, rmin 3.5: 54 us (filter) and 60
+// us (transpose); a list of taps with the address arithmetic and the range
+// check per tap took 1.05 ms, and 0.67 + 1.03 ms.
+constexpr int kFTI = 8;
+struct FilterClasses {
+  double w2[3 * kFilterMaxR * kFilterMaxR + 1];  // weight at squared distance
+  int16_t first[2 * kFilterMaxR * kFilterMaxR + 2];  // offsets of class n: first[n]..first[n+1]
+  int8_t m[2 * kFilterMaxR * kFilterMaxR + 1], h[2 * kFilterMaxR * kFilterMaxR + 1];
+  int8_t dk[(2 * kFilterMaxR + 1) * (2 * kFilterMaxR + 1)];
+  int8_t dj[(2 * kFilterMaxR + 1) * (2 * kFilterMaxR + 1)];
+  int count;
 };
 
-static int filter_taps(double rmin, FilterTaps &t) {
-  const int cr = (int)std::ceil(rmin);
-  int n = 0;
-  for (int di = -(cr - 1); di <= cr; di++)
-    for (int dk = -(cr - 1); dk <= cr; dk++)
-      for (int dj = -(cr - 1); dj <= cr; dj++) {
-        const double w = std::fmax(0.0, rmin - std::sqrt((double)(di * di + dj * dj + dk * dk)));
-        if (w == 0.0) continue;
-        if (n == kFilterMaxTaps) return -1;
-        t.di[n] = (int8_t)di;
-        t.dk[n] = (int8_t)dk;
-        t.dj[n] = (int8_t)dj;
-        t.w[n++] = w;
-      }
-  for (int q = n; q < kFilterMaxTaps; q++) {
-    t.di[q] = t.dk[q] = t.dj[q] = 0;
-    t.w[q] = 0.0;
-  }
-  return n;
+// The sum of the weights Hs depends only on how the window is clipped, per
+// axis one of 2R + 1 classes of positions: the class of position p in 1..nel
+// and a position of class c.
+__device__ __forceinline__ int filter_class(int p, int nel, int R) {
+  if (nel <= 2 * R + 1 || p - 1 < R) return p - 1;
+  return nel - p < R ? 2 * R - (nel - p) : R;
+}
+__device__ __forceinline__ int filter_class_pos(int c, int nel, int R) {
+  return (nel <= 2 * R + 1 || c <= R) ? c + 1 : nel - (2 * R - c);
 }
 
-template <int MODE, int NT>
-__global__ __launch_bounds__(kBS) void k_filter_taps(int nelx, int nely, int nelz, int few,
-                                                     int fez, const FilterTaps taps,
-                                                     const double *__restrict__ in,
-                                                     double *__restrict__ out) {
-  const uint32_t ne = (uint32_t)nelx * nely * nelz;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ne) return;
-  const uint32_t ty = t / (uint32_t)nely, tz = ty / (uint32_t)nelz;
-  const int j1 = (int)(t - ty * nely) + 1, k1 = (int)(ty - tz * nelz) + 1, i1 = (int)tz + 1;
-  const int64_t e1 = ((int64_t)i1 * fez + k1) * few + j1;
-  double acc = 0.0, ws = 0.0;
-  // branch-free: a tap outside the grid reads the element itself with weight
-  // +0, so every load of the window can be in flight at once
-#pragma unroll
-  for (int q = 0; q < NT; q++) {
-    const int i2 = i1 + taps.di[q], k2 = k1 + taps.dk[q], j2 = j1 + taps.dj[q];
-    const bool in_grid = i2 >= 1 && i2 <= nelx && k2 >= 1 && k2 <= nelz && j2 >= 1 && j2 <= nely;
-    const double w = in_grid ? taps.w[q] : 0.0;
-    const int64_t off = in_grid ? ((int64_t)taps.di[q] * fez + taps.dk[q]) * few + taps.dj[q] : 0;
-    if (MODE != 1) acc += w * in[e1 + off];
-    ws += w;
+// Hs of every class triple, one wavefront each
+__global__ __launch_bounds__(64) void k_filter_sums(int R, int nelx, int nely, int nelz,
+                                                    const FilterClasses W,
+                                                    double *__restrict__ hs) {
+  const int nc = 2 * R + 1, q = blockIdx.x;
+  const int j1 = filter_class_pos(q % nc, nely, R), k1 = filter_class_pos((q / nc) % nc, nelz, R),
+            i1 = filter_class_pos(q / (nc * nc), nelx, R);
+  double ws = 0.0;
+  for (int e = threadIdx.x; e < nc * nc * nc; e += 64) {
+    const int dj = e % nc - R, dk = (e / nc) % nc - R, di = e / (nc * nc) - R;
+    const bool in_grid = i1 + di >= 1 && i1 + di <= nelx && k1 + dk >= 1 && k1 + dk <= nelz &&
+                         j1 + dj >= 1 && j1 + dj <= nely;
+    if (in_grid) ws += W.w2[di * di + dk * dk + dj * dj];
   }
-  if (MODE == 0) out[e1] = acc / ws;
-  if (MODE == 1) out[e1] = in[e1] / ws;
-  if (MODE == 2) out[e1] = acc;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) ws += __shfl_down(ws, off, 64);
+  // (a class beyond a narrow grid has no element)
+  if (threadIdx.x == 0) hs[q] = i1 <= nelx && k1 <= nelz && j1 <= nely ? ws : 1.0;
 }
 
-// Radius at most 2 (window offsets -1..2 per axis): the offsets with
-// di^2 + dk^2 + dj^2 <= D2MAX are compile-time constants, the weight depends
-// only on that squared distance (w2[d2], same expression as the loop), and
-// the per-axis range checks are formed once per element.
-template <int MODE, int D2MAX>
-__global__ __launch_bounds__(kBS) void k_filter_r2(int nelx, int nely, int nelz, int few,
-                                                   int fez, double w0, double w1, double w2,
-                                                   double w3, const double *__restrict__ in,
-                                                   double *__restrict__ out) {
-  const uint32_t ne = (uint32_t)nelx * nely * nelz;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ne) return;
-  const uint32_t ty = t / (uint32_t)nely, tz = ty / (uint32_t)nelz;
-  const int j1 = (int)(t - ty * nely) + 1, k1 = (int)(ty - tz * nelz) + 1, i1 = (int)tz + 1;
-  const int64_t e1 = ((int64_t)i1 * fez + k1) * few + j1;
-  const int64_t plane = (int64_t)fez * few;
-  const double wd[4] = {w0, w1, w2, w3};
-  bool oi[4], ok[4], oj[4];  // offset d = index - 1 inside the grid
+// the offsets of one class, half length H
+template <int H, int LD, int LJ>
+__device__ __forceinline__ void filter_class_columns(const double *base, const FilterClasses &W,
+                                                     int n, double (&acc)[kFTI]) {
+  double w[H + 1], u[kFTI + 2 * H];
+  const int m = W.m[n], q1 = W.first[n + 1];
 #pragma unroll
-  for (int d = 0; d < 4; d++) {
-    oi[d] = i1 + d - 1 >= 1 && i1 + d - 1 <= nelx;
-    ok[d] = k1 + d - 1 >= 1 && k1 + d - 1 <= nelz;
-    oj[d] = j1 + d - 1 >= 1 && j1 + d - 1 <= nely;
+  for (int d = 0; d <= H; d++) w[d] = W.w2[m + d * d];
+#pragma unroll
+  for (int p = 0; p < kFTI + 2 * H; p++) u[p] = 0.0;
+#pragma unroll 2
+  for (int q = W.first[n]; q < q1; q++) {
+    const double *col = base + W.dk[q] * LJ + W.dj[q];
+#pragma unroll
+    for (int p = 0; p < kFTI + 2 * H; p++) u[p] += col[(p - H) * LD];
   }
-  double acc = 0.0, ws = 0.0;
 #pragma unroll
-  for (int di = -1; di <= 2; di++)
+  for (int p = 0; p < kFTI + 2 * H; p++)
 #pragma unroll
-    for (int dk = -1; dk <= 2; dk++)
+    for (int o = 0; o < kFTI; o++) {
+      const int d = p - H > o ? p - H - o : o - (p - H);
+      if (d <= H) acc[o] += w[d] * u[p];
+    }
+}
+
+// TR as in k_filter_march
+template <bool TR, int R>
+__global__ __launch_bounds__(kFTJ *kFTK) void k_filter_tile(
+    int nelx, int nely, int nelz, int few, int fez, const FilterClasses W,
+    const double *__restrict__ hs, const double *__restrict__ in, double *__restrict__ out,
+    int halo) {
+  constexpr int LI = kFTI + 2 * R, LK = kFTK + 2 * R, LJ = kFTJ + 2 * R;
+  constexpr int NT = kFTJ * kFTK, NC = 2 * R + 1, LD = LK * LJ;
+  __shared__ double tile[LI * LK * LJ];
+  const int t = threadIdx.x;
+  const int j0 = 1 + kFTJ * blockIdx.x, k0 = 1 + kFTK * blockIdx.y, i0 = 1 + kFTI * blockIdx.z;
+  auto hsum = [&](int i, int k, int j) {
+    return hs[(filter_class(i, nelx, R) * NC + filter_class(k, nelz, R)) * NC +
+              filter_class(j, nely, R)];
+  };
+#pragma unroll 4
+  for (int q = t; q < LI * LK * LJ; q += NT) {
+    const int j = j0 - R + q % LJ, k = k0 - R + (q / LJ) % LK, i = i0 - R + q / LD;
+    double v = 0.0;
+    if (i >= 1 && i <= nelx && k >= 1 && k <= nelz && j >= 1 && j <= nely) {
+      v = in[((int64_t)i * fez + k) * few + j];
+      if (TR) v /= hsum(i, k, j);
+    }
+    tile[q] = v;
+  }
+  __syncthreads();
+  const int tj = t % kFTJ, tk = t / kFTJ;
+  double acc[kFTI];
 #pragma unroll
-      for (int dj = -1; dj <= 2; dj++) {
-        const int d2 = di * di + dk * dk + dj * dj;
-        if (d2 > D2MAX) continue;
-        const bool in_grid = oi[di + 1] && ok[dk + 1] && oj[dj + 1];
-        const double w = in_grid ? wd[d2] : 0.0;
-        if (MODE != 1) acc += w * in[in_grid ? e1 + di * plane + dk * few + dj : e1];
-        ws += w;
-      }
-  if (MODE == 0) out[e1] = acc / ws;
-  if (MODE == 1) out[e1] = in[e1] / ws;
-  if (MODE == 2) out[e1] = acc;
+  for (int o = 0; o < kFTI; o++) acc[o] = 0.0;
+  const double *base = tile + (R * LK + tk + R) * LJ + tj + R;
+#pragma unroll 1
+  for (int n = 0; n < W.count; n++) {
+    const int h = W.h[n];
+    if (h == 0) filter_class_columns<0, LD, LJ>(base, W, n, acc);
+    if (h == 1) filter_class_columns<1, LD, LJ>(base, W, n, acc);
+    if (h == 2) filter_class_columns<2, LD, LJ>(base, W, n, acc);
+    if constexpr (R >= 3)
+      if (h == 3) filter_class_columns<3, LD, LJ>(base, W, n, acc);
+    if constexpr (R >= 4)
+      if (h == 4) filter_class_columns<4, LD, LJ>(base, W, n, acc);
+    if constexpr (R >= 5)
+      if (h == 5) filter_class_columns<5, LD, LJ>(base, W, n, acc);
+    if constexpr (R >= 6)
+      if (h == 6) filter_class_columns<6, LD, LJ>(base, W, n, acc);
+  }
+  const int j = j0 + tj, k = k0 + tk;
+  if (j <= nely && k <= nelz) {
+#pragma unroll
+    for (int o = 0; o < kFTI; o++) {
+      const int i = i0 + o;
+      if (i <= nelx)
+        out[((int64_t)i * fez + k) * few + j] = TR ? acc[o] : acc[o] / hsum(i, k, j);
+    }
+  }
+  if (halo != kHaloKeep)
+    filter_write_halo(i0, i0 + kFTI - 1, k0, j0, nelx, nely, nelz, few, fez, halo, in, out);
+}
+
+template <bool TR, int R>
+static void filter_tile(const DevGrid &g, const FilterClasses &W, const double *hs,
+                        const double *in, double *out, int halo) {
+  const Level &L = g.lv[0];
+  const dim3 grid((L.nely + kFTJ - 1) / kFTJ, (L.nelz + kFTK - 1) / kFTK,
+                  (L.nelx + kFTI - 1) / kFTI);
+  hipLaunchKernelGGL((k_filter_tile<TR, R>), grid, dim3(kFTJ * kFTK), 0, stream(), L.nelx,
+                     L.nely, L.nelz, g.ewy, g.ewz, W, hs, in, out, halo);
+}
+
+static FilterClasses filter_classes(double rmin, int R) {
+  FilterClasses W{};
+  for (int d2 = 0; d2 <= 3 * R * R; d2++) W.w2[d2] = std::fmax(0.0, rmin - std::sqrt((double)d2));
+  int q = 0;
+  for (int m = 0; m <= 2 * R * R; m++) {
+    int h = -1;
+    while (h < R && W.w2[m + (h + 1) * (h + 1)] > 0.0) h++;
+    if (h < 0) continue;
+    const int q0 = q;
+    for (int dk = -R; dk <= R; dk++)
+      for (int dj = -R; dj <= R; dj++)
+        if (dk * dk + dj * dj == m) {
+          W.dk[q] = (int8_t)dk;
+          W.dj[q++] = (int8_t)dj;
+        }
+    if (q == q0) continue;
+    W.m[W.count] = (int8_t)m;
+    W.h[W.count] = (int8_t)h;
+    W.first[W.count++] = (int16_t)q0;
+  }
+  W.first[W.count] = (int16_t)q;
+  return W;
+}
+
+// false where the loop over the window runs: no weight at all (rmin <= 0), a
+// tile beyond the LDS (rmin > 7), or a grid beyond the launch limits.
+template <bool TR>
+static bool filter_tiles(DevGrid &g, double rmin, const double *in, double *out, int halo) {
+  const Level &L = g.lv[0];
+  if (!(rmin > 0.0) || rmin > kFilterMaxR + 1 || L.nelz > kFTK * 65535 || L.nelx > 65535)
+    return false;
+  const int R = std::max(1, (int)std::ceil(rmin) - 1);
+  if (R == 1) {
+    double w[4];
+    for (int d2 = 0; d2 < 4; d2++) w[d2] = std::fmax(0.0, rmin - std::sqrt((double)d2));
+    const int nty = (L.nely + kFTJ - 1) / kFTJ, ntz = (L.nelz + kFTK - 1) / kFTK;
+    // planes per workgroup: four workgroups per CU, between 2 and 32 planes
+    // (each march stages two planes more than it writes)
+    const int ni = (int)std::max<int64_t>(
+        2, std::min<int64_t>(32, (int64_t)nty * ntz * L.nelx / 1024));
+    hipLaunchKernelGGL((k_filter_march<TR>), dim3(nty, ntz, (L.nelx + ni - 1) / ni),
+                       dim3(kFTJ * kFTK), 0, stream(), L.nelx, L.nely, L.nelz, g.ewy, g.ewz, ni,
+                       w[0], w[1], w[2], w[3], in, out, halo);
+    return true;
+  }
+  const FilterClasses W = filter_classes(rmin, R);
+  const int nc = 2 * R + 1, n = nc * nc * nc;
+  double *hs = (double *)g.work(kSlotFilterSums, sizeof(double) * n);
+  if (!hs) return true;  // (the error is recorded)
+  hipLaunchKernelGGL(k_filter_sums, dim3(n), dim3(64), 0, stream(), R, L.nelx, L.nely, L.nelz, W,
+                     hs);
+  switch (R) {
+    case 2: filter_tile<TR, 2>(g, W, hs, in, out, halo); break;
+    case 3: filter_tile<TR, 3>(g, W, hs, in, out, halo); break;
+    case 4: filter_tile<TR, 4>(g, W, hs, in, out, halo); break;
+    case 5: filter_tile<TR, 5>(g, W, hs, in, out, halo); break;
+    default: filter_tile<TR, 6>(g, W, hs, in, out, halo); break;
+  }
+  return true;
 }
 
 template <int MODE>
-static void filter_pass(const DevGrid &g, double rmin, const double *in, double *out) {
+static void filter_window(const DevGrid &g, double rmin, const double *in, double *out) {
   const Level &L = g.lv[0];
-  const int64_t ne = L.elements();
-  const dim3 grid((ne + kBS - 1) / kBS);
-  if (ne < (int64_t)INT32_MAX && rmin > 0.0 && rmin <= 2.0) {
-    double w[4];
-    int d2max = -1;
-    for (int d2 = 0; d2 < 4; d2++) {
-      w[d2] = std::fmax(0.0, rmin - std::sqrt((double)d2));
-      if (w[d2] != 0.0) d2max = d2;
-    }
-#define T3D_FILTER_R2(D)                                                                    \
-  hipLaunchKernelGGL((k_filter_r2<MODE, D>), grid, dim3(kBS), 0, stream(), L.nelx, L.nely, \
-                     L.nelz, g.ewy, g.ewz, w[0], w[1], w[2], w[3], in, out)
-    if (d2max == 0) T3D_FILTER_R2(0);
-    if (d2max == 1) T3D_FILTER_R2(1);
-    if (d2max == 2) T3D_FILTER_R2(2);
-    if (d2max == 3) T3D_FILTER_R2(3);
-#undef T3D_FILTER_R2
-    return;
-  }
-  FilterTaps taps;
-  const int n = ne < (int64_t)INT32_MAX ? filter_taps(rmin, taps) : -1;
-#define T3D_FILTER_TAPS(NT)                                                                  \
-  hipLaunchKernelGGL((k_filter_taps<MODE, NT>), grid, dim3(kBS), 0, stream(), L.nelx, L.nely, \
-                     L.nelz, g.ewy, g.ewz, taps, in, out)
-  if (n >= 0 && n <= 64) T3D_FILTER_TAPS(64);
-  else if (n >= 0) T3D_FILTER_TAPS(kFilterMaxTaps);
-  else
-    hipLaunchKernelGGL((k_filter<MODE>), grid, dim3(kBS), 0, stream(), L.nelx, L.nely, L.nelz,
-                       g.ewy, g.ewz, rmin, (int)std::ceil(rmin), in, out);
-#undef T3D_FILTER_TAPS
+  const dim3 grid((L.elements() + kBS - 1) / kBS);
+  hipLaunchKernelGGL((k_filter<MODE>), grid, dim3(kBS), 0, stream(), L.nelx, L.nely, L.nelz,
+                     g.ewy, g.ewz, rmin, (int)std::ceil(rmin), in, out);
 }
 
-void launch_filter(const DevGrid &g, double rmin, const double *rho, double *out) {
-  filter_pass<0>(g, rmin, rho, out);
+// the halo elements of out before a window pass that leaves them
+static void filter_halo(const DevGrid &g, const double *in, double *out, int halo) {
+  if (halo == kHaloZero) launch_fill<double>(g.nelem, out, 0.0);
+  if (halo == kHaloCopy)
+    hipMemcpyAsync(out, in, sizeof(double) * g.nelem, hipMemcpyDeviceToDevice, stream());
 }
 
-void launch_filter_grad(const DevGrid &g, double rmin, const double *v, double *tmp,
-                        double *out) {
+void launch_filter(DevGrid &g, double rmin, const double *rho, double *out, int halo) {
+  if (filter_tiles<false>(g, rmin, rho, out, halo)) return;
+  filter_halo(g, rho, out, halo);
+  filter_window<0>(g, rmin, rho, out);
+}
+
+bool launch_filter_grad(DevGrid &g, double rmin, const double *v, double *out, int halo) {
+  if (filter_tiles<true>(g, rmin, v, out, halo)) return true;
+  double *tmp = (double *)g.work(kSlotFilterTmp, sizeof(double) * g.nelem);
+  if (!tmp) return false;
   launch_fill<double>(g.nelem, tmp, 0.0);
-  filter_pass<1>(g, rmin, v, tmp);
-  filter_pass<2>(g, rmin, tmp, out);
+  filter_window<1>(g, rmin, v, tmp);
+  filter_halo(g, v, out, halo);
+  filter_window<2>(g, rmin, tmp, out);
+  return true;
 }
 
 // ---- volume (gpu_definitions.c:94-110) ------------------------------------

@@ -78,7 +78,7 @@ struct DevGrid {
   // element's nodal values (valid if wh0)
   bool wh0 = false;
   double M0[8][3][3] = {};
-  static constexpr int kScratchSlots = 9;
+  static constexpr int kScratchSlots = 11;
   void *scratch[kScratchSlots] = {};   // lazily allocated work arrays of the API
   size_t scratch_bytes[kScratchSlots] = {};
   LevelArgs args(int l) const;
@@ -128,6 +128,9 @@ int64_t level1_moduli_count(const DevGrid &g);
 // DevGrid::work slot of the transformed moduli formed by launch_level1
 // when the caller passes none
 constexpr int kSlotLevel1Moduli = 8;
+// the density filter's sums of weights, and its intermediate array at radii
+// beyond the tiles
+constexpr int kSlotFilterSums = 9, kSlotFilterTmp = 10;
 bool tile_level1_available();  // the level-1 element matrices have the mirror structure
 bool tile_fine_diag_available();  // the fine tile sweep can form its diagonal from E
 // launch_fine mode 3 forms the diagonal from E (no invD read)
@@ -303,10 +306,10 @@ void launch_copy_fixed(const DevGrid &g, int l, const double *in, double *out);
 // design-loop kernels
 void launch_sensitivity(const DevGrid &g, const double *x, const double *u,
                         double *dc, double *partials, double *c);
-void launch_filter(const DevGrid &g, double rmin, const double *rho,
-                   double *out);
-void launch_filter_grad(const DevGrid &g, double rmin, const double *v,
-                        double *tmp, double *out);
+// density filter and its transpose on the real elements; the halo elements
+// of out keep their values (0), become zero (1) or those of the input (2)
+void launch_filter(DevGrid &g, double rmin, const double *rho, double *out, int halo);
+bool launch_filter_grad(DevGrid &g, double rmin, const double *v, double *out, int halo);
 void launch_volume(const DevGrid &g, const double *x, double *partials,
                    double *result);
 void launch_change(int64_t n, double *x, const double *xnew, double *partials,

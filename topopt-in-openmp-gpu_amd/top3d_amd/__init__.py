@@ -26,6 +26,7 @@ c_int, c_double, c_float, c_void_p, c_u64 = (ctypes.c_int, ctypes.c_double, ctyp
 TOP3D_FP64, TOP3D_MIXED = 0, 1
 TOP3D_BC_REFERENCE, TOP3D_BC_SYMMETRIC = 0, 1
 TOP3D_SUPPORT_STRIPS, TOP3D_SUPPORT_FACE = 0, 1
+HALO_ZERO, HALO_COPY = 1, 2
 SUPPORTS = {"strips": TOP3D_SUPPORT_STRIPS, "face": TOP3D_SUPPORT_FACE}
 ERRORS = {0: "ok", 1: "hip", 2: "argument", 3: "unmapped", 4: "not SPD", 5: "no convergence",
           6: "non-finite"}
@@ -166,6 +167,7 @@ SIGNATURES = {
     "top3d_solver_stats": (None, [P, P]),
     "top3d_compliance_forward": (c_int, [P, P, c_int, c_double, P, P, P, P]),
     "top3d_compliance_backward": (c_int, [P, c_double, P, P, c_double, P]),
+    "top3d_density_filter": (c_int, [P, c_double, c_int, c_int, P, P]),
     "top3d_dense_spd_inverse": (c_int, [P, c_int, c_int]),
     "top3d_time_kernel": (c_int, [P, c_int, c_int, P, P]),
     "top3d_memory_info": (c_int, [P, c_int]),
@@ -405,17 +407,34 @@ class Grid:
         check("getComplianceAndSensetivity_halo")
         return c.value, dc
 
+    def _filter(self, rmin, v, transpose, halo):
+        if (v.dtype != self.torch.float64 or not v.is_cuda or not v.is_contiguous()
+                or v.numel() != self.nelem):
+            return None
+        out = self.torch.empty_like(v)
+        if self.lib.top3d_density_filter(ctypes.byref(self.gc), rmin, transpose, halo, _ptr(v),
+                                         _ptr(out)):
+            check("top3d_density_filter")
+        return out
+
     def filter(self, rmin, rho):
-        out = self.torch.zeros_like(rho)
-        self.lib.applyDensityFilter(self.gc, rmin, _ptr(rho), _ptr(out))
-        check("applyDensityFilter")
+        """applyDensityFilter; the halo elements of the result are zero."""
+        out = self._filter(rmin, rho, 0, HALO_ZERO)
+        if out is None:  # other layouts and types as the C entry point takes them
+            out = self.torch.zeros_like(rho)
+            self.lib.applyDensityFilter(self.gc, rmin, _ptr(rho), _ptr(out))
+            check("applyDensityFilter")
         return out
 
     def filter_grad(self, rmin, v):
-        v = v.clone()
-        self.lib.applyDensityFilterGradient(self.gc, rmin, _ptr(v))
-        check("applyDensityFilterGradient")
-        return v
+        """applyDensityFilterGradient on a copy of v, whose halo elements the
+        result keeps."""
+        out = self._filter(rmin, v, 1, HALO_COPY)
+        if out is None:
+            out = v.clone()
+            self.lib.applyDensityFilterGradient(self.gc, rmin, _ptr(out))
+            check("applyDensityFilterGradient")
+        return out
 
     def volume(self, xphys):
         v = self.lib.compute_volume(self.gc, _ptr(xphys))
@@ -578,11 +597,14 @@ def _filter_fn():
         @staticmethod
         def backward(ctx, gout):
             grid = ctx.grid
-            g = torch.zeros_like(gout)
-            idx = grid._interior_index()
-            g[idx] = gout[idx]
-            out = torch.zeros_like(gout)
-            out[idx] = grid.filter_grad(ctx.rmin, g)[idx]
+            # the filter reads and writes the real elements; zero halo
+            out = grid._filter(ctx.rmin, gout, 1, HALO_ZERO)
+            if out is None:
+                g = torch.zeros_like(gout)
+                idx = grid._interior_index()
+                g[idx] = gout[idx]
+                out = torch.zeros_like(gout)
+                out[idx] = grid.filter_grad(ctx.rmin, g)[idx]
             return out, None, None
 
     return _DensityFilter
