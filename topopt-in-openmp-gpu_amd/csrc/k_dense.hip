@@ -37,61 +37,25 @@ __device__ inline double4_t mfma4(double a, double b, double4_t c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// acc += X Y^T on the wave's 32x32 quadrant (rows qr.., cols qc..) of a
-// 64x64 product; X, Y are 64x64 tiles in LDS with row stride kLd.
-__device__ inline void mm_nt_tile(const double *X, const double *Y, int qr, int qc, int lane,
-                                  double4_t acc[2][2]) {
-  const int li = lane & 15, lk = lane >> 4;
-  for (int k = 0; k < kNB; k += 4) {
-    double av[2], bv[2];
-#pragma unroll
-    for (int x = 0; x < 2; x++) av[x] = X[(qr + 16 * x + li) * kLd + k + lk];
-#pragma unroll
-    for (int y = 0; y < 2; y++) bv[y] = Y[(qc + 16 * y + li) * kLd + k + lk];
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-      for (int y = 0; y < 2; y++) acc[x][y] = mfma4(av[x], bv[y], acc[x][y]);
-  }
-}
-
-__device__ inline void zero_acc(double4_t acc[2][2]) {
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++) acc[x][y] = double4_t{0.0, 0.0, 0.0, 0.0};
-}
-
-// Store the wave's quadrant of an accumulator into a 64x64 LDS tile.
-__device__ inline void store_acc(double *X, const double4_t acc[2][2], int qr, int qc, int lane) {
-  const int li = lane & 15, lk = lane >> 4;
-#pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) X[(qr + 16 * x + lk + 4 * v) * kLd + qc + 16 * y + li] = acc[x][y][v];
-}
-
 // ---------------------------------------------------------------------------
 // Cholesky and inverse of one 64x64 SPD tile in LDS, 256 threads (4 waves),
-// blocked by 16: per diagonal block kb
-//   (a) wave 0, lanes 0..15 (one row each; each pivot column broadcast
-//       through LDS): the 16x16 Cholesky L_D (reciprocal square roots
-//       refined by Newton steps) and its inverse X_D by forward substitution;
-//   (b) the panel below: P <- P X_D^T on MFMA;
-//   (c) the trailing lower triangle: C -= P P^T as 16x16 MFMA tiles;
-// then the off-diagonal 16x16 blocks of the inverse by distance on MFMA.
-// In: T (lower triangle; rows/cols beyond the matrix padded with identity).
-// Out: T = L (zeros above the diagonal), X = L^{-1}.  A non-positive pivot
-// sets *info (and is replaced by 1 so that the factorization finishes).
-// Value of v in lane `lane` (a wave-uniform index), for every lane.
-__device__ inline double readlane_d(double v, int lane) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
+// blocked by 16.  The 64 pivots are a serial chain, and a wave alone on its
+// SIMD issues one FP64 instruction in about 8 cycles, so the chain costs the
+// instructions of one wave.  Wave 0 does nothing else: it holds a 64x16 panel
+// in registers, the diagonal block's rows in each of its four rows of 16
+// lanes (so that pivot and multipliers are broadcast by DPP) and beside them
+// the rows below.  Per panel the 16 columns of the next panel are then updated
+// on MFMA by all waves, and the rest of the trailing triangle, and the
+// inverses of the finished diagonal blocks, by waves 1-3 while wave 0 factors
+// the next panel.  The off-diagonal 16x16 blocks of the inverse follow on
+// MFMA.  A tile takes 24,000 cycles (10 us), 19,000 of them the four panels;
+// with the 16x16 diagonal blocks factored on their own, each pivot column sent
+// through LDS, and panel, trailing triangle and inverses between barriers, it
+// took about twice that (a launch of one task 33 us against 23).
+// In: T (lower triangle, as 16x16 blocks; rows/cols beyond the matrix padded
+// with identity), X = 0.  Out: T = L (above the diagonal undefined),
+// X = L^{-1}.  A non-positive pivot sets *info (and is replaced by 1 so that
+// the factorization finishes).
 
 // 1/sqrt(x) for x > 0: the hardware estimate and two Newton steps
 // y <- y + y (1 - x y^2) / 2
@@ -105,149 +69,277 @@ __device__ inline double rsqrt_refined(double x) {
   return y;
 }
 
-__device__ __forceinline__ void factor_tile(double *T, double *X, int *info) {
-  __shared__ double col[16];  // the current pivot column of a 16x16 block
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const int li = lane & 15, lk = lane >> 4;
-  for (int e = t; e < kNB * kNB; e += 256) X[(e >> 6) * kLd + (e & 63)] = 0.0;
-  __syncthreads();
-  for (int kb = 0; kb < 4; kb++) {
-    const int d0 = 16 * kb;
-    if (t < 16) {  // (a): one row per lane
-      const int r = t;
-      // the row's entries right of the diagonal are updated as well and
-      // dropped when the row is stored: a lane only ever reads the column
-      // values of lanes below the current pivot, which are exact
-      double v[16], inv[16];
-#pragma unroll
-      for (int c = 0; c < 16; c++) v[c] = T[(d0 + r) * kLd + d0 + c];
-#pragma unroll
-      for (int j = 0; j < 16; j++) {
-        double piv = readlane_d(v[j], j);
-        if (!(piv > 0.0)) {
-          if (r == 0) info[0] = 1;
-          piv = 1.0;
-        }
-        const double ij = rsqrt_refined(piv);
-        inv[j] = ij;  // 1 / L_jj
-        const double lrj = (r == j) ? piv * ij : v[j] * ij;
-        v[j] = lrj;
-        if (j < 15) {
-          // column j to every lane through LDS (the wave's LDS accesses
-          // complete in order: each read sees this write, and the next
-          // pivot's write follows these reads)
-          col[r] = lrj;
-#pragma unroll
-          for (int c = j + 1; c < 16; c++) v[c] -= lrj * col[c];
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < 16; c++) T[(d0 + r) * kLd + d0 + c] = (c <= r) ? v[c] : 0.0;
-      // column r of X_D = L_D^{-1}: forward substitution with the rows of
-      // L_D read back from LDS (the same address for every lane), two
-      // partial sums to halve the dependent chain
-      double x[16];
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        double a0 = (i == r) ? 1.0 : 0.0, a1 = 0.0;
-#pragma unroll
-        for (int m = 0; m < i; m += 2) {
-          a0 -= T[(d0 + i) * kLd + d0 + m] * x[m];
-          if (m + 1 < i) a1 -= T[(d0 + i) * kLd + d0 + m + 1] * x[m + 1];
-        }
-        x[i] = (a0 + a1) * inv[i];
-        X[(d0 + i) * kLd + d0 + r] = x[i];
-      }
-    }
-    __syncthreads();
-    const int npan = kNB - d0 - 16;  // panel rows below the diagonal block
-    if (npan > 0) {
-      // (b) P[p][c] <- sum_m P[p][m] X_D[c][m], one 16-row block per wave
-      const int p0 = d0 + 16 + 16 * w;
-      double4_t pacc = {0.0, 0.0, 0.0, 0.0};
-      if (16 * w < npan) {
-#pragma unroll
-        for (int k = 0; k < 16; k += 4)
-          pacc = mfma4(T[(p0 + li) * kLd + d0 + k + lk], X[(d0 + li) * kLd + d0 + k + lk], pacc);
-      }
-      __syncthreads();
-      if (16 * w < npan) {
-#pragma unroll
-        for (int v = 0; v < 4; v++) T[(p0 + lk + 4 * v) * kLd + d0 + li] = pacc[v];
-      }
-      __syncthreads();
-      // (c) trailing tiles (ti, tj), kb < tj <= ti < 4, round-robin over waves
-      const int nt = 3 - kb, ntiles = nt * (nt + 1) / 2;
-      for (int q = w; q < ntiles; q += 4) {
-        int ti = 0, tj = 0, cnt = 0;
-        for (int a = 0; a < nt; a++)
-          for (int b2 = 0; b2 <= a; b2++) {
-            if (cnt == q) {
-              ti = kb + 1 + a;
-              tj = kb + 1 + b2;
-            }
-            cnt++;
-          }
-        double4_t acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int k = 0; k < 16; k += 4)
-          acc = mfma4(T[(16 * ti + li) * kLd + d0 + k + lk], T[(16 * tj + li) * kLd + d0 + k + lk],
-                      acc);
-#pragma unroll
-        for (int v = 0; v < 4; v++) T[(16 * ti + lk + 4 * v) * kLd + 16 * tj + li] -= acc[v];
-      }
-      __syncthreads();
-    }
+// FP64 instructions with one operand from another lane of the row of 16 lanes
+// (DPP row_newbcast), which saves the two v_readlane per broadcast value.
+// s_nop 1: a VGPR may be read through DPP two wait states after it was
+// written.
+template <int N>
+__device__ __forceinline__ double row_bcast(double x) {  // lane N's x
+  double r;
+  asm("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+      : "=v"(r)
+      : "v"(x), "n"(N));
+  return r;
+}
+// a[c] -= (lane c's x) m, c = C..15
+template <int C>
+__device__ __forceinline__ void row_update(double (&a)[16], double x, double m) {
+  if constexpr (C + 3 < 16) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f64_dpp %0, %4, -%5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %1, %4, -%5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %2, %4, -%5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %3, %4, -%5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+        : "+v"(a[C]), "+v"(a[C + 1]), "+v"(a[C + 2]), "+v"(a[C + 3])
+        : "v"(x), "v"(m), "n"(C), "n"(C + 1), "n"(C + 2), "n"(C + 3));
+    row_update<C + 4>(a, x, m);
+  } else if constexpr (C < 16) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+        : "+v"(a[C])
+        : "v"(x), "v"(m), "n"(C));
+    row_update<C + 1>(a, x, m);
   }
-  for (int e = t; e < kNB * kNB; e += 256) {
-    const int r = e >> 6, c = e & 63;
-    if (c > r) T[r * kLd + c] = 0.0;
-  }
-  __syncthreads();
-  // off-diagonal blocks of the inverse by distance d, one block per wave:
-  //   Y = sum_{K=J}^{I-1} L_IK X_KJ,  X_IJ = -X_II Y
-  // (the accumulator of Y is the B operand of the second product as is:
-  // register v of lane l holds Y[l/16 + 4v][l%16], the B element of k-step v)
-  for (int d = 1; d < 4; d++) {
-    if (w < 4 - d) {
-      const int J = w, I = d + w;
-      double4_t y = {0.0, 0.0, 0.0, 0.0};
-      for (int K = J; K < I; K++)
-#pragma unroll
-        for (int k = 0; k < 16; k += 4)
-          y = mfma4(T[(16 * I + li) * kLd + 16 * K + k + lk], X[(16 * K + k + lk) * kLd + 16 * J + li],
-                    y);
-      double4_t o = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int v = 0; v < 4; v++)
-        o = mfma4(X[(16 * I + li) * kLd + 16 * I + 4 * v + lk], y[v], o);
-#pragma unroll
-      for (int v = 0; v < 4; v++) X[(16 * I + lk + 4 * v) * kLd + 16 * J + li] = -o[v];
+}
+// x[q] -= (lane M's x[q]) m
+template <int M>
+__device__ __forceinline__ void row_eliminate(double (&x)[4], double m) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %0, -%4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %1, -%4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %2, %2, -%4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %3, %3, -%4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+      : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3])
+      : "v"(m), "n"(M));
+}
+
+// Pivot J of a panel and those after it: u the diagonal block's rows (the
+// same in each row of 16 lanes), v the lane's row below it, ij[j] = 1 / L_jj.
+template <int J, bool V>
+__device__ __forceinline__ void panel_pivots(double (&u)[16], double (&v)[16], double (&ij)[16],
+                                             bool &bad) {
+  if constexpr (J < 16) {
+    double piv = row_bcast<J>(u[J]);
+    const bool ok = piv > 0.0;
+    bad = bad || !ok;
+    piv = ok ? piv : 1.0;
+    ij[J] = rsqrt_refined(piv);
+    u[J] *= ij[J];
+    row_update<J + 1>(u, u[J], u[J]);
+    if constexpr (V) {
+      v[J] *= ij[J];
+      row_update<J + 1>(v, u[J], v[J]);
     }
-    __syncthreads();
+    panel_pivots<J + 1, V>(u, v, ij, bad);
   }
 }
 
-// Write the factored diagonal tile (blk, blk): L to Lf, L^{-1} to Dinv.
-__device__ inline void store_diag(const double *T, const double *X, double *__restrict__ Lf,
-                                  double *__restrict__ Dinv, int np, int blk) {
-  const int64_t k0 = (int64_t)blk * kNB;
-  for (int e = threadIdx.x; e < kNB * kNB; e += 256) {
-    const int r = e >> 6, c = e & 63;
-    Lf[(k0 + r) * np + k0 + c] = T[r * kLd + c];
-    Dinv[(int64_t)blk * kNB * kNB + e] = X[r * kLd + c];
+// Elimination step M of the inverse of a 16x16 factor: u its rows, ij the
+// reciprocals of its diagonal, x four columns of the inverse (times its
+// row's diagonal), r the lane's row.
+template <int M>
+__device__ __forceinline__ void inverse_steps(const double (&u)[16], const double (&ij)[16],
+                                              double (&x)[4], int r) {
+  if constexpr (M < 15) {
+    row_eliminate<M>(x, r > M ? u[M] * ij[M] : 0.0);
+    inverse_steps<M + 1>(u, ij, x, r);
   }
+}
+
+// X block b = inverse of the diagonal block b of L, by one wave: lane l has
+// row l % 16 and the columns 4 (l / 16) + q of the inverse.
+__device__ __forceinline__ void invert_block(double *X, int b, const double (&u)[16],
+                                             const double (&ij)[16], int lane) {
+  const int r = lane & 15, g = lane >> 4;
+  double x[4], s = 0.0;
+#pragma unroll
+  for (int q = 0; q < 4; q++) x[q] = r == 4 * g + q ? 1.0 : 0.0;
+  inverse_steps<0>(u, ij, x, r);
+#pragma unroll
+  for (int i = 0; i < 16; i++) s = r == i ? ij[i] : s;
+#pragma unroll
+  for (int q = 0; q < 4; q++) X[(16 * b + r) * kLd + 16 * b + 4 * g + q] = x[q] * s;
+}
+
+// Columns [16 kb, 16 kb + 16) of the factor by one wave: u the diagonal
+// block, v the rows below (lane l: row l % 16 of the blocks kb and
+// kb + 1 + l / 16); LAST: the last block, whose inverse follows at once.
+template <bool LAST>
+__device__ __forceinline__ void factor_panel(double *T, double *X, double *inv, int kb, int lane,
+                                             int *info) {
+  const int r = lane & 15, g = lane >> 4, d0 = 16 * kb;
+  const int vrow = 16 * min(kb + 1 + g, 3) + r;
+  double u[16], v[16], ij[16];
+  bool bad = false;
+#pragma unroll
+  for (int c = 0; c < 16; c++) {
+    u[c] = T[(d0 + r) * kLd + d0 + c];
+    v[c] = LAST ? 0.0 : T[vrow * kLd + d0 + c];
+  }
+  panel_pivots<0, !LAST>(u, v, ij, bad);
+  if (bad && lane == 0) info[0] = 1;
+  if constexpr (LAST) {
+    invert_block(X, kb, u, ij, lane);
+  } else {
+    if (g == 0) {
+#pragma unroll
+      for (int c = 0; c < 16; c++) {
+        T[(d0 + r) * kLd + d0 + c] = u[c];
+        inv[d0 + c] = ij[c];  // (16 lanes write the same value)
+      }
+    }
+    if (kb + 1 + g < 4) {
+#pragma unroll
+      for (int c = 0; c < 16; c++) T[vrow * kLd + d0 + c] = v[c];
+    }
+  }
+}
+
+// the inverse of a diagonal block from the factor in LDS
+__device__ __forceinline__ void invert_block_lds(const double *T, double *X, const double *inv,
+                                                 int b, int lane) {
+  double u[16], ij[16];
+#pragma unroll
+  for (int c = 0; c < 16; c++) {
+    u[c] = T[(16 * b + (lane & 15)) * kLd + 16 * b + c];
+    ij[c] = inv[16 * b + c];
+  }
+  invert_block(X, b, u, ij, lane);
+}
+
+// Block (ti, tj) of the trailing triangle minus the product of the panel
+// columns [d0, d0 + 16) of its rows and columns.
+__device__ __forceinline__ void trail_block(double *T, int ti, int tj, int d0, int lane) {
+  const int li = lane & 15, lk = lane >> 4;
+  double *C = T + (16 * ti + lk) * kLd + 16 * tj + li;
+  double4_t acc;
+#pragma unroll
+  for (int v = 0; v < 4; v++) acc[v] = C[4 * v * kLd];
+#pragma unroll
+  for (int k = 0; k < 16; k += 4)
+    acc = mfma4(-T[(16 * ti + li) * kLd + d0 + k + lk], T[(16 * tj + li) * kLd + d0 + k + lk], acc);
+#pragma unroll
+  for (int v = 0; v < 4; v++) C[4 * v * kLd] = acc[v];
+}
+
+// y += L_IK X_KJ (16x16 blocks)
+__device__ __forceinline__ void inv_term(const double *T, const double *X, int I, int K, int J,
+                                         int lane, double4_t &y) {
+  const int li = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int k = 0; k < 16; k += 4)
+    y = mfma4(T[(16 * I + li) * kLd + 16 * K + k + lk], X[(16 * K + k + lk) * kLd + 16 * J + li],
+              y);
+}
+// X_IJ = -X_II y (the accumulator of y is the B operand as it is: register v
+// of lane l holds y[l/16 + 4v][l%16], the B element of k-step v)
+__device__ __forceinline__ void inv_block(double *X, int I, int J, int lane, const double4_t &y) {
+  const int li = lane & 15, lk = lane >> 4;
+  double4_t o = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int v = 0; v < 4; v++) o = mfma4(-X[(16 * I + li) * kLd + 16 * I + 4 * v + lk], y[v], o);
+#pragma unroll
+  for (int v = 0; v < 4; v++) X[(16 * I + lk + 4 * v) * kLd + 16 * J + li] = o[v];
+}
+
+// inv: 64 doubles of LDS.  T and X are complete (barrier) on entry and exit.
+__device__ __forceinline__ void factor_tile(double *T, double *X, double *inv, int *info) {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const double4_t zero = {0.0, 0.0, 0.0, 0.0};
+  double4_t y30 = zero;
+#pragma unroll 1
+  for (int kb = 0; kb < 4; kb++) {
+    const int d0 = 16 * kb;
+    if (w == 0) {
+      if (kb < 3) factor_panel<false>(T, X, inv, kb, lane, info);
+      else factor_panel<true>(T, X, inv, kb, lane, info);
+    } else if (kb > 0) {
+      // what the panel before left: its blocks (ti, tj), kb < tj <= ti, and
+      // the inverse of its diagonal block
+      if (kb == 1) trail_block(T, w == 1 ? 2 : 3, w == 3 ? 3 : 2, d0 - 16, lane);
+      if (kb == 2 && w == 1) trail_block(T, 3, 3, d0 - 16, lane);
+      if (w == 3) invert_block_lds(T, X, inv, kb - 1, lane);
+      if (kb == 3 && w == 1) {
+        double4_t y = zero;
+        inv_term(T, X, 1, 0, 0, lane, y);
+        inv_block(X, 1, 0, lane, y);
+      }
+      if (kb == 3 && w == 2) inv_term(T, X, 3, 0, 0, lane, y30);
+    }
+    __syncthreads();
+    if (kb < 3) {  // the next panel's columns
+      if (w < 3 - kb) trail_block(T, kb + 1 + w, kb + 1, d0, lane);
+      __syncthreads();
+    }
+  }
+  // the rest of X: X_10 and the diagonal blocks are there
+  double4_t y = zero;
+  if (w == 0) {
+    inv_term(T, X, 2, 1, 1, lane, y);
+    inv_block(X, 2, 1, lane, y);
+  } else if (w == 1) {
+    inv_term(T, X, 2, 0, 0, lane, y);
+    inv_term(T, X, 2, 1, 0, lane, y);
+    inv_block(X, 2, 0, lane, y);
+  } else if (w == 2) {
+    inv_term(T, X, 3, 1, 0, lane, y30);
+  } else {
+    inv_term(T, X, 3, 2, 2, lane, y);
+    inv_block(X, 3, 2, lane, y);
+  }
+  __syncthreads();
+  if (w == 1) {
+    y = zero;
+    inv_term(T, X, 3, 1, 1, lane, y);
+    inv_term(T, X, 3, 2, 1, lane, y);
+    inv_block(X, 3, 1, lane, y);
+  } else if (w == 2) {
+    inv_term(T, X, 3, 2, 0, lane, y30);
+    inv_block(X, 3, 0, lane, y30);
+  }
+  __syncthreads();
+}
+
+// Q = P D^T in place on the wave's 16 rows of a 64x64 tile P in LDS, D lower
+// triangular (the columns of block cb need k < 16 (cb + 1) only: 40 MFMA
+// instead of 64); Q also goes to the tile at `out` (row stride np) if given.
+// A wave reads and writes its own rows only.
+__device__ __forceinline__ void panel_product(double *P, const double *D, int w, int lane,
+                                              double *__restrict__ out, int np) {
+  const int li = lane & 15, lk = lane >> 4;
+  double4_t acc[4];
+#pragma unroll
+  for (int cb = 0; cb < 4; cb++) acc[cb] = double4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < kNB; k += 4) {
+    const double av = P[(16 * w + li) * kLd + k + lk];
+#pragma unroll
+    for (int cb = k / 16; cb < 4; cb++)
+      acc[cb] = mfma4(av, D[(16 * cb + li) * kLd + k + lk], acc[cb]);
+  }
+#pragma unroll
+  for (int cb = 0; cb < 4; cb++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int r = 16 * w + lk + 4 * v, c = 16 * cb + li;
+      P[r * kLd + c] = acc[cb][v];
+      if (out) out[(int64_t)r * np + c] = acc[cb][v];
+    }
 }
 
 // One task of an elimination step (one workgroup): the trailing tile (I, J),
 // I >= J, receives the updates of the tile columns K[0..nsrc) eliminated in
 // this step,
 //   C_IJ = A_IJ - sum_K Q_IK Q_JK^T,   Q_XK = A_XK L_KK^{-T}
-// (each workgroup forms the two panel tiles it needs on MFMA).  The task of a
-// diagonal tile (I, I) also writes L_IK = Q_IK.  With kTaskFactor the tile is
-// complete after this update and is factored in LDS right away (Cholesky,
-// then the inverse of the 64x64 factor); nsrc = 0 factors A_II as it is.
+// (each workgroup forms the two panel tiles it needs on MFMA).  C is loaded
+// into the accumulators: a 32x32 quadrant per wave, or for a diagonal tile,
+// of which only the 16x16 blocks on and below the diagonal are used, 2 or 3
+// of those blocks.  The task of a diagonal tile (I, I) also writes
+// L_IK = Q_IK.  With kTaskFactor the tile is complete after this update and
+// is factored in LDS right away (Cholesky, then the inverse of the 64x64
+// factor, which goes to Dinv); nsrc = 0 factors A_II as it is.
 // Matrices are np x np row-major, np a multiple of 64.
+// Latency bound: a launch takes as long as its longest chain of loads,
+// products and one factorization.
 __global__ __launch_bounds__(256) void k_chol_task(double *__restrict__ A, double *__restrict__ Lf,
                                                    double *__restrict__ Dinv, int np,
                                                    const CholTask *__restrict__ tasks,
@@ -255,87 +347,105 @@ __global__ __launch_bounds__(256) void k_chol_task(double *__restrict__ A, doubl
   __shared__ double PI[kNB * kLd];
   __shared__ double PJ[kNB * kLd];
   __shared__ double DV[kNB * kLd];
-  __shared__ double CT[kNB * kLd];
+  __shared__ double inv[kNB];
   const CholTask tk = tasks[blockIdx.x];
-  const int tid = threadIdx.x;
-  const bool diag = tk.I == tk.J;
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const bool diag = tk.I == tk.J, fac = (tk.flags & kTaskFactor) != 0;
   const int64_t gi = (int64_t)tk.I * kNB, gj = (int64_t)tk.J * kNB;
-  if (tk.nsrc == 0) {
-    double rv[16];
+  double *Cg = A + gi * np + gj;
+  // the wave's blocks of the target: of a diagonal tile (row, column) blocks
+  // (0,0) (3,3) | (1,0) (1,1) | (2,0) (2,1) (2,2) | (3,0) (3,1) (3,2), else
+  // the quadrant's four
+  int rb[4], cb[4];
+  const int nb = diag ? (w < 2 ? 2 : 3) : 4;
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int e = tid + 256 * q;
-      rv[q] = A[(gi + (e >> 6)) * np + gi + (e & 63)];
-    }
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int e = tid + 256 * q;
-      DV[(e >> 6) * kLd + (e & 63)] = rv[q];
-    }
-  } else {
-    const int w = tid >> 6, lane = tid & 63;
-    const int qr = (w >> 1) * 32, qc = (w & 1) * 32;
-    double4_t cacc[2][2];
-    zero_acc(cacc);
-    for (int s = 0; s < tk.nsrc; s++) {
-      const int64_t gk = (int64_t)tk.K[s] * kNB;
-      // stage A_IK, A_JK, L_KK^{-1} (and C_IJ with the first source); all
-      // loads of a thread are issued before its LDS stores
-      double ri[16], rj[16], rd[16], rc[16];
-#pragma unroll
-      for (int q = 0; q < 16; q++) {
-        const int e = tid + 256 * q, r = e >> 6, c = e & 63;
-        ri[q] = A[(gi + r) * np + gk + c];
-        rj[q] = diag ? 0.0 : A[(gj + r) * np + gk + c];
-        rd[q] = Dinv[(int64_t)tk.K[s] * kNB * kNB + e];
-        rc[q] = s == 0 ? A[(gi + r) * np + gj + c] : 0.0;
-      }
-      __syncthreads();  // the previous source's products are done with the tiles
-#pragma unroll
-      for (int q = 0; q < 16; q++) {
-        const int e = tid + 256 * q, o = (e >> 6) * kLd + (e & 63);
-        PI[o] = ri[q];
-        if (!diag) PJ[o] = rj[q];
-        DV[o] = rd[q];
-        if (s == 0) CT[o] = rc[q];
-      }
-      __syncthreads();
-      double4_t qi[2][2], qj[2][2];
-      zero_acc(qi);
-      zero_acc(qj);
-      mm_nt_tile(PI, DV, qr, qc, lane, qi);  // Q_I = A_IK L_KK^{-T}
-      if (!diag) mm_nt_tile(PJ, DV, qr, qc, lane, qj);
-      __syncthreads();
-      store_acc(PI, qi, qr, qc, lane);
-      if (!diag) store_acc(PJ, qj, qr, qc, lane);
-      __syncthreads();
-      if (diag) {
-#pragma unroll 4
-        for (int e = tid; e < kNB * kNB; e += 256) {
-          const int r = e >> 6, c = e & 63;
-          Lf[(gi + r) * np + gk + c] = PI[r * kLd + c];
-        }
-      }
-      mm_nt_tile(PI, diag ? PI : PJ, qr, qc, lane, cacc);  // += Q_I Q_J^T
-    }
-    const bool fac = (tk.flags & kTaskFactor) != 0;
-    const int li = lane & 15, lk = lane >> 4;
-#pragma unroll
-    for (int x = 0; x < 2; x++)
-#pragma unroll
-      for (int y = 0; y < 2; y++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int r = qr + 16 * x + lk + 4 * v, c = qc + 16 * y + li;
-          const double a = CT[r * kLd + c] - cacc[x][y][v];
-          if (fac) DV[r * kLd + c] = a;
-          else A[(gi + r) * np + gj + c] = a;
-        }
-    if (!fac) return;
+  for (int b = 0; b < 4; b++) {
+    rb[b] = diag ? (w == 0 ? 3 * (b & 1) : w) : (w & 2) + (b >> 1);
+    cb[b] = diag ? (w == 0 ? 3 * (b & 1) : b) : 2 * (w & 1) + (b & 1);
   }
+  if (fac) {
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const int e = tid + 256 * q;
+      PJ[(e >> 6) * kLd + (e & 63)] = 0.0;
+    }
+  }
+  double4_t acc[4];
+#pragma unroll
+  for (int b = 0; b < 4; b++)
+    if (b < nb) {
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        acc[b][v] = Cg[(int64_t)(16 * rb[b] + lk + 4 * v) * np + 16 * cb[b] + li];
+    }
+  for (int s = 0; s < tk.nsrc; s++) {
+    const int64_t gk = (int64_t)tk.K[s] * kNB;
+    // stage A_IK, A_JK and L_KK^{-1}; all loads of a thread are issued before
+    // its LDS stores
+    double ri[16], rj[16], rd[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const int e = tid + 256 * q, r = e >> 6, c = e & 63;
+      ri[q] = A[(gi + r) * np + gk + c];
+      rj[q] = diag ? 0.0 : A[(gj + r) * np + gk + c];
+      rd[q] = Dinv[(int64_t)tk.K[s] * kNB * kNB + e];
+    }
+    __syncthreads();  // the previous source's products are done with the tiles
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const int e = tid + 256 * q, o = (e >> 6) * kLd + (e & 63);
+      PI[o] = ri[q];
+      if (!diag) PJ[o] = rj[q];
+      DV[o] = rd[q];
+    }
+    __syncthreads();
+    // Q_I = A_IK L_KK^{-T}
+    panel_product(PI, DV, w, lane, diag ? Lf + gi * np + gk : nullptr, np);
+    if (!diag) panel_product(PJ, DV, w, lane, nullptr, np);
+    __syncthreads();
+    const double *Y = diag ? PI : PJ;
+    if (diag) {
+#pragma unroll 4
+      for (int k = 0; k < kNB; k += 4)
+#pragma unroll
+        for (int b = 0; b < 3; b++)
+          if (b < nb)
+            acc[b] = mfma4(-PI[(16 * rb[b] + li) * kLd + k + lk],
+                           Y[(16 * cb[b] + li) * kLd + k + lk], acc[b]);
+    } else {
+#pragma unroll 4
+      for (int k = 0; k < kNB; k += 4) {
+        double av[2], bv[2];
+#pragma unroll
+        for (int x = 0; x < 2; x++) {
+          av[x] = -PI[(16 * rb[2 * x] + li) * kLd + k + lk];
+          bv[x] = Y[(16 * cb[x] + li) * kLd + k + lk];
+        }
+#pragma unroll
+        for (int b = 0; b < 4; b++) acc[b] = mfma4(av[b >> 1], bv[b & 1], acc[b]);
+      }
+    }
+  }
+  if (fac) __syncthreads();  // L_KK^{-1} is done with, X is cleared
+#pragma unroll
+  for (int b = 0; b < 4; b++)
+    if (b < nb) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int r = 16 * rb[b] + lk + 4 * v, c = 16 * cb[b] + li;
+        if (fac) DV[r * kLd + c] = acc[b][v];
+        else Cg[(int64_t)r * np + c] = acc[b][v];
+      }
+    }
+  if (!fac) return;
   __syncthreads();
-  factor_tile(DV, PJ, info);
-  store_diag(DV, PJ, Lf, Dinv, np, tk.I);
+  factor_tile(DV, PJ, inv, info);
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    const int e = tid + 256 * q;
+    Dinv[(int64_t)tk.I * kNB * kNB + e] = PJ[(e >> 6) * kLd + (e & 63)];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -474,7 +584,10 @@ __global__ __launch_bounds__(256) void k_gemm_wtw(const double *__restrict__ WT,
   const int li = lane & 15, lk = lane >> 4;
   const int qr = (w >> 1) * 32, qc = (w & 1) * 32;
   double4_t acc[2][2];
-  zero_acc(acc);
+#pragma unroll
+  for (int x = 0; x < 2; x++)
+#pragma unroll
+    for (int y = 0; y < 2; y++) acc[x][y] = double4_t{0.0, 0.0, 0.0, 0.0};
   for (int m0 = std::max(i0, j0); m0 < n; m0 += 16) {
     for (int e = tid; e < kNB * 16; e += 256) {
       const int r = e >> 4, k = e & 15;
