@@ -183,6 +183,20 @@ bool build_coarse_schedule(int n, int bw, int planes, CoarseSchedule &out) {
     out.colinfo[2 * J] = r0;
     out.colinfo[2 * J + 1] = (int)out.rows.size() / 4 - r0;
   }
+  out.list_stride = nblk + 1;
+  out.wlist.assign((size_t)nblk * out.list_stride, -1);
+  out.wtlist.assign((size_t)nblk * out.list_stride, -1);
+  for (int J = 0; J < nblk; J++) out.wlist[(size_t)J * out.list_stride] = 0;
+  for (int J = 0; J < nblk; J++) {
+    int *col = &out.wtlist[(size_t)J * out.list_stride];
+    col[0] = 0;
+    for (int q = -1; q < out.colinfo[2 * J + 1]; q++) {
+      const int I = q < 0 ? J : out.rows[4 * (out.colinfo[2 * J] + q)];
+      col[++col[0]] = I;
+      int *row = &out.wlist[(size_t)I * out.list_stride];
+      row[++row[0]] = J;
+    }
+  }
   return true;
 }
 

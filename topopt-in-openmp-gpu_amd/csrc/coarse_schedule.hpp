@@ -30,6 +30,11 @@ struct CoarseSchedule {
   // colinfo[2J]; row r is (I, klist offset, klist count, 0) at rows[4r..];
   // klist holds the K < I of the column's earlier rows with L_IK != 0
   std::vector<int> colinfo, rows, klist;
+  // the tiles of each tile row of W, and of W^T, that can be non-zero:
+  // list_stride entries per tile row, the count, then the tile columns in
+  // ascending order, then -1
+  int list_stride = 0;
+  std::vector<int> wlist, wtlist;
   std::string error;
 };
 

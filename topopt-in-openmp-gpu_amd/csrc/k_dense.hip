@@ -27,6 +27,7 @@ namespace t3d {
 constexpr int kNB = kTile;      // tile size
 constexpr int kLd = kNB + 1;    // LDS row stride of a 64x64 tile
 constexpr int kStrip = 16;      // columns per workgroup of the W = L^{-1} kernel
+constexpr int kTriBatch = 64;   // tiles per batch of loads of the triangular products
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
@@ -668,13 +669,17 @@ bool CoarseFactor::allocate(int n_, int bw_, bool f32, int planes) {
   dcolinfo = (int2 *)dalloc(sizeof(int) * cs.colinfo.size());
   drows = (int4 *)dalloc(sizeof(int) * std::max<size_t>(4, cs.rows.size()));
   dklist = (int *)dalloc(sizeof(int) * std::max<size_t>(1, cs.klist.size()));
+  // (the products read up to kTriBatch entries past a row's list)
+  list_stride = cs.list_stride;
+  dwlist = (int *)dalloc(sizeof(int) * (cs.wlist.size() + kTriBatch));
+  dwtlist = (int *)dalloc(sizeof(int) * (cs.wtlist.size() + kTriBatch));
   if (f32) {
     W32 = (float *)dalloc(sizeof(float) * nn);
     WT32 = (float *)dalloc(sizeof(float) * nn);
     cw32 = (float *)dalloc(sizeof(float) * 2 * (size_t)np);
   }
   if (!(A && L && W && WT && Dinv && info && cw64 && pos && ipos && dtasks && dcolinfo &&
-        drows && dklist && dztiles && (!f32 || (W32 && WT32 && cw32))))
+        drows && dklist && dztiles && dwlist && dwtlist && (!f32 || (W32 && WT32 && cw32))))
     return false;
   launch_first = cs.launch_first;
   launch_count = cs.launch_count;
@@ -688,6 +693,8 @@ bool CoarseFactor::allocate(int n_, int bw_, bool f32, int planes) {
          up(dcolinfo, cs.colinfo.data(), sizeof(int) * cs.colinfo.size()) &&
          up(drows, cs.rows.data(), sizeof(int) * cs.rows.size()) &&
          up(dklist, cs.klist.data(), sizeof(int) * cs.klist.size()) &&
+         up(dwlist, cs.wlist.data(), sizeof(int) * cs.wlist.size()) &&
+         up(dwtlist, cs.wtlist.data(), sizeof(int) * cs.wtlist.size()) &&
          T3D_HIP(hipStreamSynchronize(s));
 }
 
@@ -756,10 +763,10 @@ void CoarseFactor::factor_async(bool f32out) {
 }
 
 // ---------------------------------------------------------------------------
-// Coarsest solve z = W^T (W r) in the factor's storage order: gather the
-// interior DOFs to their storage positions, lower-triangular GEMV,
-// upper-triangular GEMV scattered back to the halo layout (the halo of z
-// stays zero).  One workgroup per row, FP64 accumulation.
+// Coarsest solve z = W^T (W r) in the factor's storage order: lower-triangular
+// GEMV, upper-triangular GEMV scattered back to the halo layout (the halo of z
+// stays zero).  The V-cycle's restriction writes r in storage order; the
+// gather is for other callers.
 template <typename T>
 __global__ void k_gather_interior(int nx, int ny, int nz, int wy, int wz,
                                   const int *__restrict__ pos, const T *__restrict__ in,
@@ -772,47 +779,92 @@ __global__ void k_gather_interior(int nx, int ny, int nz, int wy, int wz,
   out[pos[d]] = in[3 * (((int64_t)(i + 1) * wz + (k + 1)) * wy + (j + 1)) + d % 3];
 }
 
-// One 256-thread workgroup per row: the row (up to n values) is read by all
-// four waves at once, FP64 partial sums, fixed-order block reduction.
-__device__ __forceinline__ double row_block_sum(double s) {
-  __shared__ double sm[4];
+// Two rows of M x per workgroup of 4 waves, FP64 accumulation, over the tiles
+// of the rows' tile row that can be non-zero (41% of the triangle at coarse
+// 16x8x8): the tile columns come from a list, whose entries all threads load
+// at once, and 16 or 32 lanes read a tile's row of M (16 bytes each), so that
+// a row takes one wait for the list and one for its loads.  The product is
+// bound by those waits.
+// s[0], s[1]: the rows' sums, valid in thread 0.
+template <typename T>
+__device__ __forceinline__ void tri_rows(const T *__restrict__ M, int64_t np, int row0,
+                                         const int *__restrict__ list, const T *__restrict__ x,
+                                         double (&s)[2]) {
+  constexpr int V = 16 / sizeof(T), kLanes = kNB / V;  // values per load, lanes per tile
+  constexpr int kTiles = 256 / kLanes;                 // tiles per load of the workgroup
+  constexpr int kU = sizeof(T) == 4 ? 4 : 5;           // loads per batch
+  static_assert(kU * kTiles <= kTriBatch, "list padding");
+  typedef T vec __attribute__((ext_vector_type(V)));
+  const int t = threadIdx.x, off = V * (t % kLanes), tile = t / kLanes;
+  const T *a0 = M + (int64_t)row0 * np, *a1 = a0 + np;
+  const int cnt = list[0];
+  s[0] = s[1] = 0.0;
+  for (int b = 0; b < cnt; b += kU * kTiles) {  // (uniform)
+    int c[kU];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = s;
+    for (int u = 0; u < kU; u++) c[u] = list[1 + b + u * kTiles + tile];
+    vec v0[kU], v1[kU], xv[kU];
+#pragma unroll
+    for (int u = 0; u < kU; u++) {
+      const bool in = b + u * kTiles + tile < cnt;
+      const int col = in ? kNB * c[u] + off : off;
+      v0[u] = *reinterpret_cast<const vec *>(a0 + col);
+      v1[u] = *reinterpret_cast<const vec *>(a1 + col);
+      xv[u] = *reinterpret_cast<const vec *>(x + col);
+      c[u] = in;
+    }
+#pragma unroll
+    for (int u = 0; u < kU; u++)
+#pragma unroll
+      for (int e = 0; e < V; e++) {
+        const double xe = (double)xv[u][e];
+        s[0] += c[u] ? (double)v0[u][e] * xe : 0.0;
+        s[1] += c[u] ? (double)v1[u][e] * xe : 0.0;
+      }
+  }
+  __shared__ double sm[4][2];
+#pragma unroll
+  for (int r = 0; r < 2; r++) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) s[r] += __shfl_down(s[r], d, 64);
+    if ((t & 63) == 0) sm[t >> 6][r] = s[r];
+  }
   __syncthreads();
-  return (sm[0] + sm[1]) + (sm[2] + sm[3]);  // meaningful in thread 0
+#pragma unroll
+  for (int r = 0; r < 2; r++) s[r] = (sm[0][r] + sm[1][r]) + (sm[2][r] + sm[3][r]);
 }
 
+// (the tile rows with the longest lists come last in storage order, and first
+// in the grid)
 template <typename T>
-__global__ __launch_bounds__(256) void k_trmv_lower(const T *__restrict__ Wm, int n,
+__global__ __launch_bounds__(256) void k_trmv_lower(const T *__restrict__ Wm, int np,
+                                                    const int *__restrict__ lists, int stride,
                                                     const T *__restrict__ x, T *__restrict__ y) {
-  const int row = blockIdx.x;
-  const T *a = Wm + (int64_t)row * n;
-  double s = 0.0;
-  // (unrolled so that several loads are in flight; the sum order is unchanged)
-#pragma unroll 8
-  for (int c = threadIdx.x; c <= row; c += 256) s += (double)a[c] * (double)x[c];
-  s = row_block_sum(s);
-  if (threadIdx.x == 0) y[row] = (T)s;
+  const int row0 = np - 2 - 2 * (int)blockIdx.x;
+  double s[2];
+  tri_rows(Wm, np, row0, lists + (row0 / kNB) * stride, x, s);
+  if (threadIdx.x == 0) {
+    y[row0] = (T)s[0];
+    y[row0 + 1] = (T)s[1];
+  }
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_trmv_upper_scatter(int nx, int ny, int nz, int wy, int wz,
+__global__ __launch_bounds__(256) void k_trmv_upper_scatter(int ny, int nz, int wy, int wz,
                                                             const int *__restrict__ ipos,
-                                                            const T *__restrict__ WTm, int n,
-                                                            const T *__restrict__ y,
+                                                            const T *__restrict__ WTm, int np,
+                                                            const int *__restrict__ lists,
+                                                            int stride, const T *__restrict__ y,
                                                             T *__restrict__ out) {
-  const int row = blockIdx.x;
-  const T *a = WTm + (int64_t)row * n;
-  double s = 0.0;
-#pragma unroll 8
-  for (int c = row + threadIdx.x; c < n; c += 256) s += (double)a[c] * (double)y[c];
-  s = row_block_sum(s);
-  const int d = ipos[row];
-  if (threadIdx.x == 0 && d >= 0) {
-    const int64_t p = d / 3;
-    const int j = (int)(p % ny), k = (int)((p / ny) % nz), i = (int)(p / ((int64_t)ny * nz));
-    out[3 * (((int64_t)(i + 1) * wz + (k + 1)) * wy + (j + 1)) + d % 3] = (T)s;
+  const int row0 = 2 * blockIdx.x;
+  const int d = ipos[row0 + (threadIdx.x & 1)];
+  double s[2];
+  tri_rows(WTm, np, row0, lists + (row0 / kNB) * stride, y, s);
+  if (threadIdx.x < 2 && d >= 0) {
+    const int p = d / 3;
+    const int j = p % ny, k = (p / ny) % nz, i = p / (ny * nz);
+    out[3 * (((int64_t)(i + 1) * wz + (k + 1)) * wy + (j + 1)) + d % 3] =
+        (T)(threadIdx.x ? s[1] : s[0]);
   }
 }
 
@@ -820,14 +872,15 @@ template <typename T>
 void launch_coarse_apply(const DevGrid &g, int l, const CoarseFactor &cf, const T *in, T *out) {
   const Level &L = g.lv[l];
   const int n = cf.n, np = cf.np;
-  const T *Wm = cf.w<T>(), *WTm = cf.wt<T>();
   T *x = cf.cw<T>(), *y = x + np;  // padding entries of x stay zero
   const int bs = 256;
-  hipLaunchKernelGGL((k_gather_interior<T>), dim3((n + bs - 1) / bs), dim3(bs), 0, stream(),
-                     L.nx, L.ny, L.nz, L.wy, L.wz, cf.pos, in, x);
-  hipLaunchKernelGGL((k_trmv_lower<T>), dim3(np), dim3(256), 0, stream(), Wm, np, x, y);
-  hipLaunchKernelGGL((k_trmv_upper_scatter<T>), dim3(np), dim3(256), 0, stream(), L.nx,
-                     L.ny, L.nz, L.wy, L.wz, cf.ipos, WTm, np, y, out);
+  if (in)
+    hipLaunchKernelGGL((k_gather_interior<T>), dim3((n + bs - 1) / bs), dim3(bs), 0, stream(),
+                       L.nx, L.ny, L.nz, L.wy, L.wz, cf.pos, in, x);
+  hipLaunchKernelGGL((k_trmv_lower<T>), dim3(np / 2), dim3(256), 0, stream(), cf.w<T>(), np,
+                     cf.dwlist, cf.list_stride, x, y);
+  hipLaunchKernelGGL((k_trmv_upper_scatter<T>), dim3(np / 2), dim3(256), 0, stream(), L.ny, L.nz,
+                     L.wy, L.wz, cf.ipos, cf.wt<T>(), np, cf.dwtlist, cf.list_stride, y, out);
 }
 
 template void launch_coarse_apply<double>(const DevGrid &, int, const CoarseFactor &,

@@ -588,18 +588,30 @@ void launch_jacobi_zero(const DevGrid &g, int l, const TB *b, const T *invD, T o
 template <typename T>
 __global__ void k_restrict(int cnx, int cny, int cnz, int cwy, int cwz, int fwy, int fwz,
                            const T *__restrict__ fine, T *__restrict__ coarse,
-                           const T *__restrict__ invDc, T omega, T *__restrict__ zc) {
+                           const T *__restrict__ invDc, T omega, T *__restrict__ zc,
+                           const int *__restrict__ pos, T *__restrict__ xs) {
   // one thread per interior coarse node; only those are written
   // (stencil_methods.c:629-686).  With zc, also the coarse level's first
   // pre-smoothing sweep from zero, zc = omega invDc rc (as k_jacobi_zero; the
-  // other nodes of zc stay zero)
+  // other nodes of zc stay zero).  With xs, also the coarse vector in the
+  // storage order pos of the coarsest level's factor
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (int64_t)cnx * cny * cnz) return;
   const int j = (int)(t % cny) + 1, k = (int)((t / cny) % cnz) + 1,
             i = (int)(t / ((int64_t)cny * cnz)) + 1;
   const int64_t cn = ((int64_t)i * cwz + k) * cwy + j;
   const int fi = 2 * i - 1, fj = 2 * j - 1, fk = 2 * k - 1;
-  T acc[3] = {0, 0, 0};
+  T acc[3] = {0, 0, 0}, dc[3] = {0, 0, 0};
+  int ps[3] = {0, 0, 0};
+  // (loaded with the fine values, not after them)
+  if (zc) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) dc[c] = invDc[3 * cn + c];
+  }
+  if (xs) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) ps[c] = pos[3 * t + c];
+  }
 #pragma unroll
   for (int dx = -1; dx <= 1; dx++)
 #pragma unroll
@@ -617,17 +629,22 @@ __global__ void k_restrict(int cnx, int cny, int cnz, int cwy, int cwz, int fwy,
   coarse[3 * cn + 2] = acc[2];
   if (zc) {
 #pragma unroll
-    for (int c = 0; c < 3; c++) zc[3 * cn + c] = omega * invDc[3 * cn + c] * (acc[c] - T(0));
+    for (int c = 0; c < 3; c++) zc[3 * cn + c] = omega * dc[c] * (acc[c] - T(0));
+  }
+  if (xs) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) xs[ps[c]] = acc[c];
   }
 }
 
 template <typename T>
 void launch_restrict(const DevGrid &g, int l, const T *fine, T *coarse, const T *invDc,
-                     T omega, T *zc) {
+                     T omega, T *zc, const CoarseFactor *cf) {
   const Level &C = g.lv[l + 1], &F = g.lv[l];
   const int64_t nth = C.interior_nodes();
   hipLaunchKernelGGL((k_restrict<T>), dim3((nth + 255) / 256), dim3(256), 0, stream(), C.nx,
-                     C.ny, C.nz, C.wy, C.wz, F.wy, F.wz, fine, coarse, invDc, omega, zc);
+                     C.ny, C.nz, C.wy, C.wz, F.wy, F.wz, fine, coarse, invDc, omega, zc,
+                     cf ? cf->pos : nullptr, cf ? cf->cw<T>() : nullptr);
 }
 
 // Trilinear prolongation level l+1 -> l (stencil_methods.c:521-590);
@@ -838,7 +855,8 @@ void launch_invdiag_stencil(const DevGrid &g, int l, const double *S, T *invD) {
   template void launch_stencil_half<T>(const DevGrid &, int, int, const T *, const T *,  \
                                        T *, const T *, const T *, T);                    \
   template void launch_invdiag_half<T>(const DevGrid &, int, const double *, T *);       \
-  template void launch_restrict<T>(const DevGrid &, int, const T *, T *, const T *, T, T *); \
+  template void launch_restrict<T>(const DevGrid &, int, const T *, T *, const T *, T, T *, \
+                                   const CoarseFactor *);                                \
   template void launch_prolong_add<T>(const DevGrid &, int, const T *, T *);             \
   template void launch_prolong<T>(const DevGrid &, int, const T *, T *);                 \
   template void launch_invdiag_mf<T>(const DevGrid &, int, const double *, T *);         \

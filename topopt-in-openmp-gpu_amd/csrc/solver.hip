@@ -314,9 +314,9 @@ void SolverState::vcycle(int l, bool zero_done) {
   T *other = (zc == z_) ? t_ : z_;
   op<T>(l, 2, zc, d_, r_);  // d = r - K z
   if (nl == l + 2) {
-    launch_restrict<T>(*g, l, d_, vec<T>(l + 1, kR));
+    launch_restrict<T>(*g, l, d_, vec<T>(l + 1, kR), nullptr, T(0), nullptr, &coarse);
     join_coarse();
-    launch_coarse_apply<T>(*g, l + 1, coarse, vec<T>(l + 1, kR), vec<T>(l + 1, kZ));
+    launch_coarse_apply<T>(*g, l + 1, coarse, nullptr, vec<T>(l + 1, kZ));
   } else {
     // the restriction also writes level l+1's first sweep from zero into the
     // buffer smooth_from_zero starts in; level l+1's inverse diagonal is

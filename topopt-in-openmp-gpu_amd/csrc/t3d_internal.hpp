@@ -160,9 +160,12 @@ bool launch_fine_jacobi_zero(const DevGrid &g, const TB *b, const T *E, T omega,
 template <typename TB, typename T>
 void launch_jacobi_zero(const DevGrid &g, int l, const TB *b, const T *invD,
                         T omega, T *out);
+// zc: also the coarse level's first sweep from zero; cf: also the coarse
+// vector in that factor's storage order (cf->cw)
 template <typename T>
 void launch_restrict(const DevGrid &g, int l, const T *fine, T *coarse,
-                     const T *invDc = nullptr, T omega = T(0), T *zc = nullptr);
+                     const T *invDc = nullptr, T omega = T(0), T *zc = nullptr,
+                     const struct CoarseFactor *cf = nullptr);
 template <typename T>
 void launch_prolong_add(const DevGrid &g, int l, const T *coarse, T *fine);
 template <typename T>
@@ -229,6 +232,8 @@ struct CoarseFactor {
   int2 *dcolinfo = nullptr;
   int4 *drows = nullptr;
   int *dklist = nullptr;
+  int list_stride = 0;  // non-zero tiles per tile row of W and W^T (CoarseSchedule)
+  int *dwlist = nullptr, *dwtlist = nullptr;
   // the tiles I * nblk + J the factorization reads (targets and sources of
   // its tasks): the only part of A that assembly has to clear
   int *dztiles = nullptr;
@@ -254,7 +259,8 @@ struct CoarseFactor {
     if constexpr (sizeof(T) == 8) return (T *)cw64; else return (T *)cw32;
   }
 };
-// out (level-l halo layout) = A^{-1} in (interior DOFs)
+// out (level-l halo layout) = A^{-1} in (interior DOFs); in = nullptr: the
+// right-hand side is in the factor's storage order already (launch_restrict)
 template <typename T>
 void launch_coarse_apply(const DevGrid &g, int l, const CoarseFactor &cf, const T *in, T *out);
 
