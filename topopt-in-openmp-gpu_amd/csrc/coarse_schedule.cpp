@@ -35,7 +35,8 @@ std::vector<Step> band_steps(int nblk, int bw) {
 // every other plane of the remaining chain (an independent set), which
 // couples their neighbours, and repeat; about log2(planes) levels of tp
 // tile columns each.  slot[p] = position of plane p in the elimination order.
-std::vector<Step> plane_steps(int planes, int tp, std::vector<int> &slot) {
+std::vector<Step> plane_steps(int planes, int tp, std::vector<int> &slot,
+                              std::vector<int> &tile_level) {
   std::vector<std::vector<int>> levels;
   std::vector<int> rem(planes);
   for (int p = 0; p < planes; p++) rem[p] = p;
@@ -47,8 +48,11 @@ std::vector<Step> plane_steps(int planes, int tp, std::vector<int> &slot) {
   }
   slot.assign(planes, 0);
   int next = 0;
-  for (const auto &lev : levels)
-    for (int p : lev) slot[p] = next++;
+  for (size_t v = 0; v < levels.size(); v++)
+    for (int p : levels[v]) {
+      slot[p] = next++;
+      tile_level.insert(tile_level.end(), tp, (int)v);
+    }
   // symbolic elimination on the plane graph
   std::vector<std::vector<int>> adj(planes);
   for (int p = 0; p + 1 < planes; p++) {
@@ -95,12 +99,13 @@ bool build_coarse_schedule(int n, int bw, int planes, CoarseSchedule &out) {
   if (planes > 1 && n % planes == 0) {
     const int pm = n / planes, tp = (pm + kTile - 1) / kTile;
     std::vector<int> slot;
-    steps = plane_steps(planes, tp, slot);
+    steps = plane_steps(planes, tp, slot, out.tile_level);
     out.np = planes * tp * kTile;
     for (int d = 0; d < n; d++) out.pos[d] = slot[d / pm] * tp * kTile + d % pm;
   } else {
     out.np = (n + kTile - 1) / kTile * kTile;
     steps = band_steps(out.np / kTile, std::max(0, bw));
+    out.tile_level.assign(out.np / kTile, 0);
     for (int d = 0; d < n; d++) out.pos[d] = d;
   }
   const int nblk = out.nblk = out.np / kTile;
@@ -163,9 +168,16 @@ bool build_coarse_schedule(int n, int bw, int planes, CoarseSchedule &out) {
       out.launch_count.push_back((int)tasks.size() - first);
     }
   }
+  // (launch t factors step t's tiles: a launch is left out only after the
+  // last step, which has no panel)
+  out.nlevels = out.tile_level.back() + 1;
+  out.level_launch.assign(out.nlevels, 0);
+  for (size_t t = 0; t < steps.size(); t++)
+    out.level_launch[out.tile_level[steps[t].src[0].first]] = (int)t;
   // non-zero tile rows of each column of W = L^{-1}: forward reach through
   // the tiles of L
   out.colinfo.assign(2 * nblk, 0);
+  out.lcolinfo.assign(2 * (size_t)out.nlevels * nblk, 0);
   for (int J = 0; J < nblk; J++) {
     std::vector<char> in(nblk, 0);
     in[J] = 1;
@@ -176,7 +188,12 @@ bool build_coarse_schedule(int n, int bw, int planes, CoarseSchedule &out) {
         if (in[K]) ks.push_back(K);
       if (ks.empty()) continue;
       std::sort(ks.begin(), ks.end());
-      out.rows.insert(out.rows.end(), {I, (int)out.klist.size(), (int)ks.size(), 0});
+      const int lower = (int)std::count_if(ks.begin(), ks.end(), [&](int K) {
+        return out.tile_level[K] < out.tile_level[I];
+      });
+      int *lc = &out.lcolinfo[2 * ((size_t)out.tile_level[I] * nblk + J)];
+      if (lc[1]++ == 0) lc[0] = (int)out.rows.size() / 4;
+      out.rows.insert(out.rows.end(), {I, (int)out.klist.size(), (int)ks.size(), lower});
       out.klist.insert(out.klist.end(), ks.begin(), ks.end());
       in[I] = 1;
     }

@@ -27,9 +27,18 @@ struct CoarseSchedule {
   std::vector<CholTask> tasks;         // all launches, concatenated
   std::vector<int> launch_first, launch_count;
   // W = L^{-1}: tile column J has colinfo[2J+1] rows starting at row
-  // colinfo[2J]; row r is (I, klist offset, klist count, 0) at rows[4r..];
-  // klist holds the K < I of the column's earlier rows with L_IK != 0
+  // colinfo[2J]; row r is (I, klist offset, klist count, klist entries of a
+  // lower level than I) at rows[4r..]; klist holds the K < I of the column's
+  // earlier rows with L_IK != 0, in ascending order
   std::vector<int> colinfo, rows, klist;
+  // Levels of the elimination (the levels of the dissection; one for a
+  // band): after launch level_launch[v] the diagonal tiles of level v are
+  // factored and its rows of L written as far as the level's own columns,
+  // after the next one (if any) all rows of L in its columns.  Tile column J
+  // has lcolinfo[2 (v nblk + J) + 1] rows of W in level v, from row
+  // lcolinfo[2 (v nblk + J)].
+  int nlevels = 0;
+  std::vector<int> tile_level, level_launch, lcolinfo;
   // the tiles of each tile row of W, and of W^T, that can be non-zero:
   // list_stride entries per tile row, the count, then the tile columns in
   // ascending order, then -1

@@ -14,9 +14,9 @@
 //      (v_mfma_f64_16x16x4f64) and applies C_IJ -= sum_K Q_IK Q_JK^T; the
 //      workgroup of a diagonal tile eliminated next factors it in LDS right
 //      after its update (Cholesky, then the inverse of the 64x64 factor);
-//   2. W = L^{-1} (lower triangle, zero outside the reach of each column),
-//      one workgroup per 16-column strip visiting only the tile rows where
-//      its column of W is non-zero; W^T is written alongside.
+//   2. W = L^{-1} (lower triangle, zero outside the reach of each column) by
+//      16-column strips and levels of the dissection, beside the Cholesky
+//      launches of the next level; W^T is written alongside.
 // A V-cycle applies A^{-1} = P^T W^T W P as two triangular GEMVs.
 #include <algorithm>
 
@@ -450,123 +450,137 @@ __global__ __launch_bounds__(256) void k_chol_task(double *__restrict__ A, doubl
 }
 
 // ---------------------------------------------------------------------------
-// W = L^{-1}, WT = W^T by 16-column strips.  The strip [16s, 16s+16) of tile
-// column J starts with W_JJ = L_JJ^{-1} and visits the tile rows where column
-// J of W is non-zero, in increasing order:
+// W = L^{-1}, WT = W^T by 16-column strips, level by level of the elimination
+// so that only the last level's rows remain when the factorization ends.  A
+// strip [16s, 16s+16) of tile column J has W_JJ = L_JJ^{-1} and, in the tile
+// rows I of the reach of J,
 //   W_I = -L_II^{-1} sum_{K in ks(I)} L_IK W_K,
-// ks(I) the strip's earlier rows with L_IK != 0 (row and K lists from the
-// elimination schedule).  Two groups of 4 waves take alternate K of a row,
-// each with its own double-buffered LDS stage for the L_IK tiles (the next
-// tile in flight during the current product); their 64x16 partial sums meet
-// in LDS.  W_K is read back from W (written by this workgroup
-// before a barrier).  W is always written; WT, W32 and WT32 (FP32 copies)
-// when given.
-constexpr int kLinvGroups = 2;
-
-__global__ __launch_bounds__(256 * kLinvGroups) void k_linv_seq(
-    const double *__restrict__ Lf, const double *__restrict__ Dinv, int np,
-    const int2 *__restrict__ colinfo, const int4 *__restrict__ rows,
-    const int *__restrict__ klist, double *__restrict__ W, double *__restrict__ WT,
-    float *__restrict__ W32, float *__restrict__ WT32) {
-  __shared__ double Bx[kLinvGroups][kNB * 17];
-  __shared__ double Lt[kLinvGroups][2 * kNB * kLd];
-  const int tid = threadIdx.x, grp = tid >> 8, gtid = tid & 255;
-  const int w = gtid >> 6, lane = tid & 63;
-  const int li = lane & 15, lk = lane >> 4;
-  const int c0 = blockIdx.x * kStrip;
-  const int J = c0 / kNB, cofs = c0 - J * kNB;
-  const int gc = c0 + li;
-  for (int e = tid; e < kNB * kStrip; e += 256 * kLinvGroups) {
-    const int r = e >> 4, j = e & 15;
-    const double v = Dinv[(int64_t)J * kNB * kNB + r * kNB + cofs + j];
-    const int64_t gr = (int64_t)J * kNB + r;
-    W[gr * np + c0 + j] = v;
-    if (WT) WT[(int64_t)(c0 + j) * np + gr] = v;
-    if (W32) {
-      W32[gr * np + c0 + j] = (float)v;
-      WT32[(int64_t)(c0 + j) * np + gr] = (float)v;
-    }
+// ks(I) the strip's earlier rows with L_IK != 0 (lists from the elimination
+// schedule).  k_linv_sums leaves the terms of the lower levels in W_I, one
+// workgroup per row and strip; k_linv_rows adds those of the row's own level
+// (at most the tiles of a plane; all of them for a band), row by row, and
+// multiplies by L_II^{-1}.  (One launch after the factorization that walked
+// all rows of a strip took 270 us at coarse 16x8x8.)  W is always written;
+// WT, W32 and WT32 (FP32 copies) when given.
+//
+// acc += L_IK W_K for the wave's 16 rows (row block rb) of the strip: lane l
+// feeds k = 16 (l/16) + q of MFMA step q, so that its part of L_IK is a run of
+// 128 bytes; the next term's loads are issued before this one's products.
+struct LinvTerm {
+  double a[16], b[16];
+};
+__device__ __forceinline__ void linv_load(const double *__restrict__ Lf, const double *W, int np,
+                                          int I, int K, int rb, int gc, LinvTerm &t) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const double2 *pa = reinterpret_cast<const double2 *>(
+      Lf + ((int64_t)I * kNB + 16 * rb + li) * np + (int64_t)K * kNB + 16 * lk);
+  const double *pb = W + ((int64_t)K * kNB + 16 * lk) * np + gc;
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const double2 v = pa[q];
+    t.a[2 * q] = v.x;
+    t.a[2 * q + 1] = v.y;
   }
-  auto load_tile = [&](int I, int K, double (&reg)[16]) {
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int e = gtid + 256 * q;
-      reg[q] = Lf[((int64_t)I * kNB + (e >> 6)) * np + (int64_t)K * kNB + (e & 63)];
+  for (int q = 0; q < 16; q++) t.b[q] = pb[(int64_t)q * np];
+}
+__device__ __forceinline__ void linv_product(const LinvTerm &t, double4_t &acc0, double4_t &acc1) {
+#pragma unroll
+  for (int q = 0; q < 16; q += 2) {
+    acc0 = mfma4(t.a[q], t.b[q], acc0);
+    acc1 = mfma4(t.a[q + 1], t.b[q + 1], acc1);
+  }
+}
+// the terms ks[t0], ks[t0 + dt], ... below ks[t1]
+__device__ __forceinline__ double4_t linv_terms(const double *__restrict__ Lf, const double *W,
+                                                int np, int I, const int *__restrict__ ks, int t0,
+                                                int t1, int dt, int rb, int gc) {
+  double4_t acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
+  LinvTerm cur, nxt;
+  if (t0 < t1) linv_load(Lf, W, np, I, ks[t0], rb, gc, cur);
+  for (int t = t0; t < t1; t += dt) {
+    if (t + dt < t1) linv_load(Lf, W, np, I, ks[t + dt], rb, gc, nxt);
+    linv_product(cur, acc0, acc1);
+    cur = nxt;
+  }
+  return acc0 + acc1;
+}
+
+// blockIdx.x: strip, blockIdx.y: its row within the level
+__global__ __launch_bounds__(256) void k_linv_sums(const double *__restrict__ Lf, int np,
+                                                   const int2 *__restrict__ colinfo,
+                                                   const int4 *__restrict__ rows,
+                                                   const int *__restrict__ klist, double *W) {
+  const int c0 = blockIdx.x * kStrip;
+  const int2 ci = colinfo[c0 / kNB];
+  if ((int)blockIdx.y >= ci.y) return;
+  const int4 rw = rows[ci.x + blockIdx.y];
+  if (rw.w == 0) return;
+  const int rb = threadIdx.x >> 6, lane = threadIdx.x & 63, gc = c0 + (lane & 15);
+  const double4_t acc = linv_terms(Lf, W, np, rw.x, klist + rw.y, 0, rw.w, 1, rb, gc);
+#pragma unroll
+  for (int v = 0; v < 4; v++)
+    W[((int64_t)rw.x * kNB + 16 * rb + (lane >> 4) + 4 * v) * np + gc] = acc[v];
+}
+
+constexpr int kLinvGroups = 2;  // groups of 4 waves, which take alternate terms
+
+__global__ __launch_bounds__(256 * kLinvGroups) void k_linv_rows(
+    const double *__restrict__ Lf, const double *__restrict__ Dinv, int np,
+    const int2 *__restrict__ colinfo, const int *__restrict__ tile_level, int level,
+    const int4 *__restrict__ rows, const int *__restrict__ klist, double *W,
+    double *__restrict__ WT, float *__restrict__ W32, float *__restrict__ WT32) {
+  __shared__ double Bx[kLinvGroups][kNB * 17];
+  const int tid = threadIdx.x, grp = tid >> 8, rb = (tid >> 6) & 3, lane = tid & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const int c0 = blockIdx.x * kStrip, J = c0 / kNB, cofs = c0 - J * kNB;
+  const int gc = c0 + li;
+  auto put = [&](int64_t gr, int c, double v) {
+    W[gr * np + c] = v;
+    if (WT) WT[(int64_t)c * np + gr] = v;
+    if (W32) {
+      W32[gr * np + c] = (float)v;
+      WT32[(int64_t)c * np + gr] = (float)v;
     }
   };
-  auto store_tile = [&](double *dst, const double (&reg)[16]) {
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int e = gtid + 256 * q;
-      dst[(e >> 6) * kLd + (e & 63)] = reg[q];
+  if (tile_level[J] == level) {
+    for (int e = tid; e < kNB * kStrip; e += 256 * kLinvGroups) {
+      const int r = e >> 4, j = e & 15;
+      put((int64_t)J * kNB + r, c0 + j, Dinv[(int64_t)J * kNB * kNB + r * kNB + cofs + j]);
     }
-  };
-  // this lane's B elements of W_K: rows k + lk (k = 0, 4, .., 60), column gc
-  auto load_b = [&](int K, double (&breg)[16]) {
-    const double *wk = W + (int64_t)K * kNB * np + gc;
-#pragma unroll
-    for (int q = 0; q < 16; q++) breg[q] = wk[(int64_t)(4 * q + lk) * np];
-  };
-  double *Lg = Lt[grp];
-  __syncthreads();
+    __syncthreads();
+  }
   const int2 ci = colinfo[J];
   for (int q = 0; q < ci.y; q++) {
-    const int4 rw = rows[ci.x + q];  // (I, offset into klist, count, -)
-    const int I = rw.x, nk = rw.z;
-    double dreg[16];  // group 0: rows 16w.. of L_II^{-1}, columns k < 16(w+1)
+    const int4 rw = rows[ci.x + q];
+    const int I = rw.x;
+    double dreg[16];  // group 0: rows 16 rb.. of L_II^{-1}, columns k < 16 (rb + 1)
+    double4_t sum = {0.0, 0.0, 0.0, 0.0};
     if (grp == 0) {
       const double *D = Dinv + (int64_t)I * kNB * kNB;
 #pragma unroll
       for (int t = 0; t < 16; t++)
-        dreg[t] = (4 * t < 16 * (w + 1)) ? D[(16 * w + li) * kNB + 4 * t + lk] : 0.0;
-    }
-    double treg[16], bcur[16];
-    if (grp < nk) {  // this group's first K: t = grp
-      load_tile(I, klist[rw.y + grp], treg);
-      store_tile(Lg, treg);
-    }
-    __syncthreads();
-    double4_t acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
-    const int iters = (nk + kLinvGroups - 1) / kLinvGroups;
-    for (int it = 0; it < iters; it++) {
-      const int t = kLinvGroups * it + grp;  // this group's K-term
-      const bool has = t < nk, more = t + kLinvGroups < nk;
-      const double *cur = Lg + (size_t)(it & 1) * kNB * kLd;
-      double *nxt = Lg + (size_t)((it & 1) ^ 1) * kNB * kLd;
-      if (more) load_tile(I, klist[rw.y + t + kLinvGroups], treg);  // in flight meanwhile
-      if (has) {
-        load_b(klist[rw.y + t], bcur);
+        dreg[t] = (4 * t < 16 * (rb + 1)) ? D[(16 * rb + li) * kNB + 4 * t + lk] : 0.0;
+      if (rw.w > 0) {
 #pragma unroll
-        for (int qq = 0; qq < 16; qq += 2) {
-          acc0 = mfma4(cur[(16 * w + li) * kLd + 4 * qq + lk], bcur[qq], acc0);
-          acc1 = mfma4(cur[(16 * w + li) * kLd + 4 * qq + 4 + lk], bcur[qq + 1], acc1);
-        }
+        for (int v = 0; v < 4; v++)
+          sum[v] = W[((int64_t)I * kNB + 16 * rb + lk + 4 * v) * np + gc];
       }
-      if (more) store_tile(nxt, treg);
-      __syncthreads();
     }
+    sum += linv_terms(Lf, W, np, I, klist + rw.y, rw.w + grp, rw.z, kLinvGroups, rb, gc);
 #pragma unroll
-    for (int v = 0; v < 4; v++) Bx[grp][(16 * w + lk + 4 * v) * 17 + li] = acc0[v] + acc1[v];
+    for (int v = 0; v < 4; v++) Bx[grp][(16 * rb + lk + 4 * v) * 17 + li] = sum[v];
     __syncthreads();
     if (grp == 0) {
       double4_t o = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int t = 0; t < 16; t++)
-        if (4 * t < 16 * (w + 1))
+        if (4 * t < 16 * (rb + 1))
           o = mfma4(dreg[t], Bx[0][(4 * t + lk) * 17 + li] + Bx[1][(4 * t + lk) * 17 + li], o);
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int64_t gr = (int64_t)I * kNB + 16 * w + lk + 4 * v;
-        const double val = -o[v];
-        W[gr * np + gc] = val;
-        if (WT) WT[(int64_t)gc * np + gr] = val;
-        if (W32) {
-          W32[gr * np + gc] = (float)val;
-          WT32[(int64_t)gc * np + gr] = (float)val;
-        }
-      }
+      for (int v = 0; v < 4; v++) put((int64_t)I * kNB + 16 * rb + lk + 4 * v, gc, -o[v]);
     }
-    __syncthreads();
+    __syncthreads();  // W_I is there for the next row, Bx for its sums
   }
 }
 
@@ -666,7 +680,10 @@ bool CoarseFactor::allocate(int n_, int bw_, bool f32, int planes) {
   dztiles = (int *)dalloc(sizeof(int) * std::max<size_t>(1, zt.size()));
   ntask = (int)cs.tasks.size();
   dtasks = (CholTask *)dalloc(sizeof(CholTask) * std::max<size_t>(1, cs.tasks.size()));
-  dcolinfo = (int2 *)dalloc(sizeof(int) * cs.colinfo.size());
+  dcolinfo = (int2 *)dalloc(sizeof(int) * cs.lcolinfo.size());
+  dlevel = (int *)dalloc(sizeof(int) * cs.tile_level.size());
+  for (hipEvent_t &e : ev_level)
+    if (!T3D_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming))) return false;
   drows = (int4 *)dalloc(sizeof(int) * std::max<size_t>(4, cs.rows.size()));
   dklist = (int *)dalloc(sizeof(int) * std::max<size_t>(1, cs.klist.size()));
   // (the products read up to kTriBatch entries past a row's list)
@@ -679,10 +696,15 @@ bool CoarseFactor::allocate(int n_, int bw_, bool f32, int planes) {
     cw32 = (float *)dalloc(sizeof(float) * 2 * (size_t)np);
   }
   if (!(A && L && W && WT && Dinv && info && cw64 && pos && ipos && dtasks && dcolinfo &&
-        drows && dklist && dztiles && dwlist && dwtlist && (!f32 || (W32 && WT32 && cw32))))
+        drows && dklist && dztiles && dwlist && dwtlist && dlevel && (!f32 || (W32 && WT32 && cw32))))
     return false;
   launch_first = cs.launch_first;
   launch_count = cs.launch_count;
+  level_launch = cs.level_launch;
+  level_rows.assign(cs.nlevels, 0);
+  for (int v = 0; v < cs.nlevels; v++)
+    for (int J = 0; J < nblk; J++)
+      level_rows[v] = std::max(level_rows[v], cs.lcolinfo[2 * ((size_t)v * nblk + J) + 1]);
   hipStream_t s = stream();
   auto up = [&](void *dst, const void *src, size_t bytes) {
     return bytes == 0 || T3D_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
@@ -690,9 +712,10 @@ bool CoarseFactor::allocate(int n_, int bw_, bool f32, int planes) {
   return up(pos, cs.pos.data(), sizeof(int) * n) && up(ipos, hipos.data(), sizeof(int) * np) &&
          up(dztiles, zt.data(), sizeof(int) * zt.size()) &&
          up(dtasks, cs.tasks.data(), sizeof(CholTask) * cs.tasks.size()) &&
-         up(dcolinfo, cs.colinfo.data(), sizeof(int) * cs.colinfo.size()) &&
          up(drows, cs.rows.data(), sizeof(int) * cs.rows.size()) &&
          up(dklist, cs.klist.data(), sizeof(int) * cs.klist.size()) &&
+         up(dcolinfo, cs.lcolinfo.data(), sizeof(int) * cs.lcolinfo.size()) &&
+         up(dlevel, cs.tile_level.data(), sizeof(int) * cs.tile_level.size()) &&
          up(dwlist, cs.wlist.data(), sizeof(int) * cs.wlist.size()) &&
          up(dwtlist, cs.wtlist.data(), sizeof(int) * cs.wtlist.size()) &&
          T3D_HIP(hipStreamSynchronize(s));
@@ -749,17 +772,44 @@ int CoarseFactor::check_info() {
   return TOP3D_OK;
 }
 
-void CoarseFactor::factor_async(bool f32out) {
+void CoarseFactor::factor_async(bool f32out, hipStream_t with_w) {
   hipStream_t s = stream();
   if (!T3D_HIP(hipMemsetAsync(info, 0, sizeof(int), s))) return;
-  for (size_t q = 0; q < launch_first.size(); q++)
+  const bool f32 = f32out && W32;  // FP32 W, W^T for the mixed V-cycle, else FP64 W^T
+  const int nlev = (int)level_launch.size(), nlaunch = (int)launch_first.size();
+  hipStream_t sw = with_w ? with_w : s;
+  auto rows_of = [&](int v) {  // level v's rows of W
+    hipLaunchKernelGGL(k_linv_rows, dim3(np / kStrip), dim3(256 * kLinvGroups), 0, sw, L, Dinv, np,
+                       dcolinfo + (size_t)v * nblk, dlevel, v, drows, dklist, W,
+                       f32 ? nullptr : WT, f32 ? W32 : nullptr, f32 ? WT32 : nullptr);
+  };
+  auto sums_of = [&](int v) {  // and their terms of the lower levels
+    if (level_rows[v] > 0)
+      hipLaunchKernelGGL(k_linv_sums, dim3(np / kStrip, level_rows[v]), dim3(256), 0, sw, L, np,
+                         dcolinfo + (size_t)v * nblk, drows, dklist, W);
+  };
+  // With a stream of its own, level v's rows of W follow the launch after the
+  // level's last one (which completes L in its columns for the sums of the
+  // levels above), and the last level's rows the last launch.
+  int v = 0;
+  for (int q = 0; q < nlaunch; q++) {
     hipLaunchKernelGGL(k_chol_task, dim3(launch_count[q]), dim3(256), 0, s, A, L, Dinv, np,
                        dtasks + launch_first[q], info);
-  const bool f32 = f32out && W32;  // FP32 W, W^T for the mixed V-cycle, else FP64 W^T
-  hipLaunchKernelGGL(k_linv_seq, dim3(np / kStrip), dim3(256 * kLinvGroups), 0, s, L, Dinv, np,
-                     dcolinfo,
-                     drows, dklist, W, f32 ? nullptr : WT, f32 ? W32 : nullptr,
-                     f32 ? WT32 : nullptr);
+    if (with_w && v + 1 < nlev && q == level_launch[v] + 1) {
+      hipEventRecord(ev_level[v & 1], s);
+      hipStreamWaitEvent(sw, ev_level[v & 1], 0);
+      rows_of(v);
+      sums_of(++v);
+    }
+  }
+  if (with_w) {
+    hipEventRecord(ev_level[v & 1], s);
+    hipStreamWaitEvent(sw, ev_level[v & 1], 0);
+  }
+  for (; v < nlev; v++) {
+    rows_of(v);
+    if (v + 1 < nlev) sums_of(v + 1);
+  }
 }
 
 // ---------------------------------------------------------------------------

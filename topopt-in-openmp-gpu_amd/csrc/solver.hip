@@ -84,6 +84,7 @@ bool SolverState::allocate(DevGrid *grid, int nlev) {
   if (!T3D_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming))) return false;
   if (!T3D_HIP(hipStreamCreateWithFlags(&aux, hipStreamNonBlocking)) ||
       !T3D_HIP(hipStreamCreateWithFlags(&aux2, hipStreamNonBlocking)) ||
+      !T3D_HIP(hipStreamCreateWithFlags(&aux3, hipStreamNonBlocking)) ||
       !T3D_HIP(hipEventCreateWithFlags(&ev_base, hipEventDisableTiming)) ||
       !T3D_HIP(hipEventCreateWithFlags(&ev_stencil, hipEventDisableTiming)) ||
       !T3D_HIP(hipEventCreateWithFlags(&ev_coarse, hipEventDisableTiming)) ||
@@ -99,6 +100,7 @@ void SolverState::release() {
   hipStreamSynchronize(stream());
   if (aux) hipStreamSynchronize(aux);
   if (aux2) hipStreamSynchronize(aux2);
+  if (aux3) hipStreamSynchronize(aux3);
   auto f = [](void *ptr) { dfree(ptr); };
   for (int l = 0; l < nl; l++) {
     f(invD64[l]);
@@ -126,7 +128,8 @@ void SolverState::release() {
   }
   if (aux) hipStreamDestroy(aux);
   if (aux2) hipStreamDestroy(aux2);
-  aux = aux2 = nullptr;
+  if (aux3) hipStreamDestroy(aux3);
+  aux = aux2 = aux3 = nullptr;
   for (hipEvent_t e : sw_ev) hipEventDestroy(e);
   sw_ev.clear();
   magic = 0;
@@ -186,8 +189,10 @@ bool SolverState::setup_aux() {
       }
     }
     launch_stencil_to_dense(*g, nl - 1, S64[nl - 1], coarse);
-    coarse.factor_async(mixed);
-    if (!T3D_HIP(hipEventRecord(ev_coarse, aux))) return false;
+    // the rows of W on `aux3` beside the factorization; the last of them
+    // follow it, so that their end is the factor's
+    coarse.factor_async(mixed, aux3);
+    if (!T3D_HIP(hipEventRecord(ev_coarse, aux3))) return false;
     // the fine inverse diagonal is not read by the fine sweeps when they form
     // it from E; it is still filled in for callers of the SolverDataBuffer
     if (fine_sweep_forms_diagonal() && !launch_fine_invdiag(*g, E64, invD64[0]))
@@ -376,6 +381,7 @@ int SolverState::solve(const double *x, const double *b, double *u, double tol, 
   if (!setup_aux()) {
     hipStreamSynchronize(aux);
     hipStreamSynchronize(aux2);
+    hipStreamSynchronize(aux3);
     hipStreamSynchronize(stream());
     wait_stencil = wait_coarse = false;
     stats.status = top3d_last_error();

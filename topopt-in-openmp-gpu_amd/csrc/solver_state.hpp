@@ -57,7 +57,8 @@ struct SolverState {
   // The element matrices of the assembled levels and the coarse factor run
   // on `aux`; the smoother levels' stencils run on `aux2` as their element
   // matrices become ready (ev_ke[l]), off the coarse factor's path.
-  hipStream_t aux = nullptr, aux2 = nullptr;
+  // aux3 builds W = L^{-1} of the coarse factor level by level.
+  hipStream_t aux = nullptr, aux2 = nullptr, aux3 = nullptr;
   hipEvent_t ev_base = nullptr, ev_stencil = nullptr, ev_coarse = nullptr, ev_done = nullptr;
   hipEvent_t ev_done2 = nullptr;
   hipEvent_t ev_ke[kMaxLevels] = {};

@@ -229,7 +229,11 @@ struct CoarseFactor {
   CholTask *dtasks = nullptr;
   int ntask = 0;
   std::vector<int> launch_first, launch_count;
-  int2 *dcolinfo = nullptr;
+  std::vector<int> level_launch;  // last launch of each level (CoarseSchedule)
+  std::vector<int> level_rows;    // most rows of W of a column in each level
+  hipEvent_t ev_level[2] = {};
+  int2 *dcolinfo = nullptr;       // rows of W per level and tile column
+  int *dlevel = nullptr;          // level of each tile column
   int4 *drows = nullptr;
   int *dklist = nullptr;
   int list_stride = 0;  // non-zero tiles per tile row of W and W^T (CoarseSchedule)
@@ -247,7 +251,9 @@ struct CoarseFactor {
   // TOP3D_OK or TOP3D_ERR_NOT_SPD / TOP3D_ERR_HIP; f32out: W32 and WT32 for
   // the FP32 apply instead of the FP64 WT
   int factor(bool f32out = false);
-  void factor_async(bool f32out);  // the same work, queued without waiting
+  // the same work, queued without waiting; with_w: a stream for the rows of
+  // W, which run beside the factorization (the caller waits for both)
+  void factor_async(bool f32out, hipStream_t with_w = nullptr);
   int check_info();                // after factor_async has completed
   template <typename T> const T *w() const {
     if constexpr (sizeof(T) == 8) return (const T *)W; else return (const T *)W32;
