@@ -6,17 +6,19 @@
 //   u^[q][c] = sum_p (-1)^{q.p} u[p][c]      (p, q in {0,1}^3, bit 0 = x),
 // KE becomes 8 independent 3x3 blocks: block s couples the components c with
 // q = s ^ (1 << c).  Blocks 1, 2, 4 contain a rigid translation (zero row and
-// column) and blocks 3, 5, 6 split into a 2x2 and a 1x1, so one element
-// product costs 72 + 45 + 21 + 72 operations (transform, blocks, modulus,
-// inverse transform) instead of 576 multiply-adds.  The host derives the
+// column) and blocks 3, 5, 6 split into a 2x2 and a 1x1; with the symmetries of
+// the isotropic cube (Blocks) one element product costs 72 + 33 + 8 + 72
+// operations (transform, blocks, modulus, inverse transform) instead of 576
+// multiply-adds.  The host derives the
 // blocks from KE_0 and checks the zero pattern (hadamard_blocks()).
 //
-// Tiling.  A workgroup owns a tile of TY x TZ element columns in (y, z),
-// one thread per column, and marches along x over NX node planes.  Per
-// x-step each thread computes its element in the current slab, adds the
-// pending x+ face of the previous slab to the x- face of this one, keeps the
-// corner it owns (node (j+1, k+1)) and hands the other three corners to their
-// owners through LDS (9 values, one barrier).  Tiles overlap by one element
+// Tiling.  A workgroup owns a tile of TY x TZ element columns in (y, z) and
+// marches along x over NX node planes, a thread per column on level 1, a thread
+// per node of the columns on the fine level.  Per x-step each thread computes
+// its element in the current slab, adds the pending x+ face of the previous
+// slab to the x- face of this one, keeps the corner it owns (node (j+1, k+1) of
+// element (j, k)) and hands the other three corners to their owners through LDS
+// (9 values, one barrier).  Tiles overlap by one element
 // in every direction, so every owned node of a tile interior is complete
 // without atomics and the result is deterministic.
 #include <climits>
@@ -88,9 +90,20 @@ bool hadamard_blocks(const double *KE, double M[8][3][3]) {
   return true;
 }
 
+// The blocks' values: KE of the isotropic cube is the same under the exchange
+// of any two axes, which leaves 8 of the 45 non-zeros, and sigma = (1, -1, 1),
+// the reference's direction of y, carries all their signs.  With x the inputs
+// of block s (fine_blocks() checks every entry of the 8 matrices):
+//   s = 0, 7: (a - b) I + b sigma sigma^T          (d0, b0; d7, b7)
+//   s = one axis k: p on the diagonal, q sigma_c sigma_d off it, for the two
+//     other components c and d; zero for k         (p1, q1)
+//   s = two axes c, d: r (1, sigma_c sigma_d)^T (1, sigma_c sigma_d) for
+//     these; t for the third                       (r2, t2)
+// Held in scalar registers throughout the march; with all 45 the kernels
+// loaded most of them again at every slab.
 template <typename T>
 struct Blocks {
-  T m[8][3][3];
+  T d0, b0, p1, q1, r2, t2, d7, b7;
   // 1 / KE[3a+c][3a+c]: the diagonal of KE is the same for all 8 nodes, so
   // the assembled diagonal at a node is KE[c][c] times the sum of the moduli
   // of its elements
@@ -138,26 +151,32 @@ __device__ __forceinline__ void face_iwht(const T (&G)[4][3], T (&y)[2][2][3]) {
 template <typename T>
 __device__ __forceinline__ void element_core(const Blocks<T> &B, T E, const T (&h)[8][3],
                                              T (&g)[8][3]) {
-  // block products, modulus, zero pattern of the reflection blocks
+  // (the modulus times the 8 values: fewer products than with the 21 outputs)
+  constexpr int sg[3] = {1, -1, 1};
 #pragma unroll
-  for (int s = 0; s < 8; s++) {
-    T x[3];
+  for (int s = 0; s < 8; s += 7) {
+    const T d = E * (s ? B.d7 : B.d0), b = E * (s ? B.b7 : B.b0);
+    const T x0 = h[s ^ 1][0], x1 = h[s ^ 2][1], x2 = h[s ^ 4][2];
+    const T w = b * ((x0 + x2) - x1);
+    g[s ^ 1][0] = d * x0 + w;
+    g[s ^ 2][1] = d * x1 - w;
+    g[s ^ 4][2] = d * x2 + w;
+  }
+  const T p = E * B.p1, q = E * B.q1, r = E * B.r2, t = E * B.t2;
 #pragma unroll
-    for (int c = 0; c < 3; c++) x[c] = h[s ^ (1 << c)][c];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      T acc = 0;
-#pragma unroll
-      for (int d = 0; d < 3; d++) {
-        const bool one_bit = s != 0 && (s & (s - 1)) == 0;
-        const bool two_bit = s != 0 && s != 7 && !one_bit;
-        bool zero = false;
-        if (one_bit) zero = (s == (1 << c)) || (s == (1 << d));
-        if (two_bit) zero = (c != d) && (!((s >> c) & 1) || !((s >> d) & 1));
-        if (!zero) acc += B.m[s][c][d] * x[d];
-      }
-      g[s ^ (1 << c)][c] = E * acc;
-    }
+  for (int k = 0; k < 3; k++) {
+    const int c = k == 0 ? 1 : 0, d = k == 2 ? 1 : 2;  // the other two
+    const bool neg = sg[c] * sg[d] < 0;
+    const int s1 = 1 << k, s2 = 7 ^ s1;
+    const T xc = h[s1 ^ (1 << c)][c], xd = h[s1 ^ (1 << d)][d];
+    g[0][k] = 0;
+    g[s1 ^ (1 << c)][c] = neg ? p * xc - q * xd : p * xc + q * xd;
+    g[s1 ^ (1 << d)][d] = neg ? p * xd - q * xc : p * xd + q * xc;
+    const T yc = h[s2 ^ (1 << c)][c], yd = h[s2 ^ (1 << d)][d];
+    const T w = r * (neg ? yc - yd : yc + yd);
+    g[s2 ^ (1 << c)][c] = w;
+    g[s2 ^ (1 << d)][d] = neg ? -w : w;
+    g[7][k] = t * h[7][k];
   }
 }
 
@@ -367,8 +386,33 @@ struct TileArgs {
   int few, fez;          // fine element strides
   int TY, TZ, NX;        // tile: element columns in y and z, node planes in x
   int nty;               // tiles along y
-  uint32_t out_bytes;    // size of the output vector (below 2^32 - 32)
+  int stream_out;        // store the output past the caches
+  uint32_t out_bytes;    // size of the level's vectors (below 2^32 - 32)
+  uint32_t e_bytes;      // size of the moduli (below 2^32)
 };
+
+// The tile of a workgroup of the (slabs, tiles) grid.  The device deals
+// workgroups to its 8 XCDs, each with an L2 of its own, in turn: every XCD
+// takes an eighth of the tiles in the order y, z, slab, so that the tiles whose
+// edges overlap march together behind one L2.  (Dealt by the plain index that
+// was so only where the number of slabs is a multiple of 8: an FP32 sweep of
+// 88 tiles in 17 slabs took 55.1 us so, 38.4 us in this order.)
+struct TilePos {
+  int by, bz, slab, dot;  // dot: place of the workgroup's partial sum
+};
+
+__device__ __forceinline__ TilePos tile_pos(const TileArgs &a) {
+  const uint32_t ntx = gridDim.x, yz = gridDim.y, n = ntx * yz;
+  const uint32_t id = blockIdx.y * ntx + blockIdx.x, xcd = id & 7;
+  const uint32_t t = xcd * (n >> 3) + min(xcd, n & 7) + (id >> 3);
+  const uint32_t slab = t / yz, tile = t - slab * yz;
+  TilePos p;
+  p.bz = (int)(tile / (uint32_t)a.nty);
+  p.by = (int)(tile - p.bz * a.nty);
+  p.slab = (int)slab;
+  p.dot = (int)(tile * ntx + slab);
+  return p;
+}
 
 // p[idx] with the byte offset formed in 32 bits, so that the load or store
 // takes the uniform base in scalar registers and a 32-bit offset (no 64-bit
@@ -392,53 +436,79 @@ __device__ __forceinline__ T recip(T x) {
 }
 
 // Stores the 3 components of a node through a buffer resource of the output
-// vector: an offset at or beyond its size (the resource's record count)
-// writes nothing, which the hardware guarantees for out-of-range buffer
-// stores, so that every lane can issue the store without a branch.
+// vector, at per-thread byte offset `off` and uniform byte offset `base`: an
+// offset at or beyond its size (the resource's record count) writes nothing,
+// which the hardware guarantees for out-of-range buffer stores, so that every
+// lane can issue the store without a branch.  kNt: past the caches.
+constexpr int kCached = 0, kNt = 2;
+template <int AUX = kCached>
 __device__ __forceinline__ void store_node(__amdgpu_buffer_rsrc_t r, uint32_t off,
-                                           const float (&o)[3]) {
+                                           const float (&o)[3], uint32_t base = 0) {
   typedef uint32_t u3 __attribute__((ext_vector_type(3)));
   const u3 v = {__float_as_uint(o[0]), __float_as_uint(o[1]), __float_as_uint(o[2])};
-  __builtin_amdgcn_raw_buffer_store_b96(v, r, (int)off, 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b96(v, r, (int)off, (int)base, AUX);
 }
+template <int AUX = kCached>
 __device__ __forceinline__ void store_node(__amdgpu_buffer_rsrc_t r, uint32_t off,
-                                           const double (&o)[3]) {
+                                           const double (&o)[3], uint32_t base = 0) {
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   typedef uint32_t u2 __attribute__((ext_vector_type(2)));
   const uint64_t b0 = __double_as_longlong(o[0]), b1 = __double_as_longlong(o[1]),
                  b2 = __double_as_longlong(o[2]);
   const u4 lo = {(uint32_t)b0, (uint32_t)(b0 >> 32), (uint32_t)b1, (uint32_t)(b1 >> 32)};
   const u2 hi = {(uint32_t)b2, (uint32_t)(b2 >> 32)};
-  __builtin_amdgcn_raw_buffer_store_b128(lo, r, (int)off, 0, 0);
-  __builtin_amdgcn_raw_buffer_store_b64(hi, r, (int)(off + 16u), 0, 0);
+  __builtin_amdgcn_raw_buffer_store_b128(lo, r, (int)off, (int)base, AUX);
+  __builtin_amdgcn_raw_buffer_store_b64(hi, r, (int)(off + 16u), (int)base, AUX);
 }
 
-// LVL 0: fine level, one modulus per element; LVL 1: level 1, eight fine
-// moduli per element.  MODE: apply / Jacobi sweep / residual.
-// fixplane[i] != 0 if a node of plane i has a fixed DOF; planes without one
-// skip the per-node mask.  PIPE: the loads of a step are issued a step ahead
-// (below); else at the step's head, where the step waits for them.
-template <typename T, int LVL, int MODE, bool BCSYM, bool PIPE>
-__device__ __forceinline__ void tile_sweep_body(
-    TileArgs a, std::conditional_t<LVL == 0, Blocks<T>, K1Vals<T>> B, const T *__restrict__ E,
-    const T *__restrict__ in, T *__restrict__ out, const T *__restrict__ b,
-    const T *__restrict__ invD, T omega, const uint8_t *__restrict__ fix,
-    const int *__restrict__ fixplane, double *__restrict__ dotp) {
-  static_assert(LVL == 0 || MODE != kModeJacobiDiag, "level 1 reads its inverse diagonal");
-  constexpr bool kDiag = MODE == kModeJacobiDiag;
-  // LDS values per thread and buffer: 9, or 10 with the modulus, padded to
-  // an odd stride so that 64 consecutive threads hit distinct banks
-  constexpr int XS = kDiag ? 11 : 9;
+// Loads through a buffer resource: per-thread byte offset `off`, uniform byte
+// offset `base` (no address arithmetic per access)
+template <typename T>
+__device__ __forceinline__ T load1(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t base) {
+  if constexpr (sizeof(T) == 4)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)base, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, (int)base, 0));
+}
+template <typename T>
+__device__ __forceinline__ void load3(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t base,
+                                      T (&v)[3]) {
+  if constexpr (sizeof(T) == 4) {
+    const auto q = __builtin_amdgcn_raw_buffer_load_b96(r, (int)off, (int)base, 0);
+#pragma unroll
+    for (int c = 0; c < 3; c++) v[c] = __uint_as_float(q[c]);
+  } else {
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const d2 q = __builtin_bit_cast(
+        d2, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)base, 0));
+    v[0] = q[0];
+    v[1] = q[1];
+    v[2] = load1<T>(r, off + 16u, base);
+  }
+}
+
+// Level 1, eight fine moduli per element.  MODE: apply / Jacobi sweep /
+// residual.  fixplane[i] != 0 if a node of plane i has a fixed DOF; planes
+// without one skip the per-node mask.
+template <typename T, int MODE, bool BCSYM>
+__device__ __forceinline__ void level1_sweep_body(
+    TileArgs a, K1Vals<T> B, const T *__restrict__ E, const T *__restrict__ in,
+    T *__restrict__ out, const T *__restrict__ b, const T *__restrict__ invD, T omega,
+    const uint8_t *__restrict__ fix, const int *__restrict__ fixplane) {
+  // LDS values per thread and buffer, an odd stride so that 64 consecutive
+  // threads hit distinct banks
+  constexpr int XS = 9;
   extern __shared__ unsigned char smem_raw[];
   T *xch = reinterpret_cast<T *>(smem_raw);  // [2][nthreads][XS]
   const int nthr = a.TY * a.TZ;
   const int t = threadIdx.x;
   const bool active = t < nthr;
   const int ty = t % a.TY, tz = t / a.TY;
-  const int by = blockIdx.y % a.nty, bz = blockIdx.y / a.nty;
+  const TilePos w = tile_pos(a);
+  const int by = w.by, bz = w.bz;
   const int j = by * (a.TY - 1) + ty;  // element column (halo index)
   const int k = bz * (a.TZ - 1) + tz;
-  const int i0 = 1 + blockIdx.x * a.NX;
+  const int i0 = 1 + w.slab * a.NX;
   const int i1 = min(i0 + a.NX - 1, a.nelx + 1);  // last output plane
   // the element exists in memory (0..nel+1) and may carry a non-zero modulus
   const bool elem_ok = active && j <= a.nely && k <= a.nelz;
@@ -453,16 +523,12 @@ __device__ __forceinline__ void tile_sweep_body(
   // Threads whose element column lies outside the grid read the halo node
   // (0, 0) of each plane and the halo element (i, 0, 0) instead, both in
   // bounds; that element's modulus is 0, so their products are 0 and no
-  // branch guards the loads.  (Level 1: E holds the transformed moduli of
+  // branch guards the loads.  (E holds the transformed moduli of
   // k_level1_moduli, 8 per element slot, with strides few, fez of its own.)
   const uint32_t n00c = elem_ok ? n00 : 0u;
   const uint32_t e00c = elem_ok ? (uint32_t)k * a.few + j : 0u;
   const uint32_t noff[2][2] = {{0u, (uint32_t)a.wy}, {1u, (uint32_t)a.wy + 1u}};  // [py][pz]
   const uint32_t nown = (uint32_t)(k + 1) * a.wy + (uint32_t)(j + 1);  // owned node in a plane
-  // with dotp: partial sum of in . out (apply) or b . out (Jacobi sweeps)
-  double dacc = 0.0;
-  // kDiag: moduli of the 4 elements of the previous slab at the owned node
-  T es_prev = 0;
 
   // raw values of the face of node plane i (zero outside the grid)
   auto fetch_face = [&](int i, T (&v)[2][2][3]) {
@@ -502,18 +568,15 @@ __device__ __forceinline__ void tile_sweep_body(
 #pragma unroll
     for (int c = 0; c < 3; c++) pendT[f][c] = 0;
 
-  // PIPE: every load is issued a step ahead of its use, so that its latency
+  // Every load but the slab's moduli is issued a step ahead of its use, so that its latency
   // hides behind a step of element work; per step, in issue order:
-  //   head: wait for the raw face of plane i+1 and the slab's modulus (issued
-  //         at the last step's head), then issue those of the next step;
+  //   head: wait for the raw face of plane i+1 (issued at the last step's
+  //         head), then issue that of the next step;
   //   end:  the owned node's output of plane i, then the loads of the owned
   //         node's operands for step i+1 (b, invD, mask), issued after this
   //         step's operands have been used so that one set is live at a time.
   // Every path through a step issues the same memory operations, so the
   // waits leave the younger ones in flight (the memory counter is in order).
-  // This pays where the element work per load is large (FP64, level 1); the
-  // FP32 fine level, whose waves are bound by their VALU issue, runs faster
-  // without the copies and the scheduling barrier it takes.
   struct NodeIn {  // the owned node's b, invD and fixed-DOF mask
     T bb[3], di[3];
     uint8_t m;
@@ -537,17 +600,11 @@ __device__ __forceinline__ void tile_sweep_body(
     }
     sv.m = fixplane[i] != 0 ? fix[nd] : uint8_t(0);
   };
-  // (the march visits slabs i <= nelx + 1)
-  auto load_modulus = [&](int i) -> T {
-    if constexpr (LVL == 0) return *at32(E, (uint32_t)i * a.fez * a.few + e00c);
-    return T(0);
-  };
   // the output vector as a buffer resource (stride 0, size in bytes); the
   // offset out_bytes addresses nothing
   const __amdgpu_buffer_rsrc_t orsrc =
       __builtin_amdgcn_make_buffer_rsrc(out, (short)0, (int)a.out_bytes, 0x00020000);
   NodeIn nv{};
-  T Ecur = 0;
   // u0: the owned node (j+1, k+1) of plane i, node (1, 1) of this thread's
   // face of plane i; u1: that of plane i+1 (unmasked even when BCSYM masks
   // the faces)
@@ -558,35 +615,22 @@ __device__ __forceinline__ void tile_sweep_body(
   auto step = [&](int i, const T (&Fc)[4][3], T (&Fn)[4][3]) {
     const bool emit = i >= i0;  // uniform
     const uint32_t d0 = 3u * ((uint32_t)i * sx + nown);
-    T Ee = 0;
-    if constexpr (PIPE) {
-      // The values of the face and the modulus are copied into registers of
-      // their own here, where they have been waited for: the loads issued
-      // below then land in the registers they leave (an empty asm with a
-      // "+v" operand fixes the transformed face here).
+    // The values of the face are copied into registers of their own here,
+    // where they have been waited for: the loads issued below then land in
+    // the registers they leave (an empty asm with a "+v" operand fixes the
+    // transformed face here).
 #pragma unroll
-      for (int c = 0; c < 3; c++) u1[c] = copy_here(vq[1][1][c]);
-      mask_face(i + 1, vq);
-      face_wht<T>(vq, Fn);
+    for (int c = 0; c < 3; c++) u1[c] = copy_here(vq[1][1][c]);
+    mask_face(i + 1, vq);
+    face_wht<T>(vq, Fn);
 #pragma unroll
-      for (int f = 0; f < 4; f++)
+    for (int f = 0; f < 4; f++)
 #pragma unroll
-        for (int c = 0; c < 3; c++) asm volatile("" : "+v"(Fn[f][c]));
-      if constexpr (LVL == 0) Ee = copy_here(Ecur);
-      // nothing moves across
-      __builtin_amdgcn_sched_barrier(0);
-      // (unconditional, the last step repeats its plane and slab)
-      Ecur = load_modulus(min(i + 1, i1));
-      fetch_face(min(i + 2, i1 + 1), vq);
-    } else {
-      fetch_face(i + 1, vq);
-      Ee = load_modulus(i);
-      load_node(i, nv);
-#pragma unroll
-      for (int c = 0; c < 3; c++) u1[c] = vq[1][1][c];
-      mask_face(i + 1, vq);
-      face_wht<T>(vq, Fn);
-    }
+      for (int c = 0; c < 3; c++) asm volatile("" : "+v"(Fn[f][c]));
+    // nothing moves across
+    __builtin_amdgcn_sched_barrier(0);
+    // (unconditional, the last step repeats its plane)
+    fetch_face(min(i + 2, i1 + 1), vq);
     T h[8][3];
 #pragma unroll
     for (int f = 0; f < 4; f++)
@@ -595,48 +639,34 @@ __device__ __forceinline__ void tile_sweep_body(
         h[2 * f][c] = Fc[f][c] + Fn[f][c];
         h[2 * f + 1][c] = Fc[f][c] - Fn[f][c];
       }
-    // g[0][c] (the element's rigid translations) is zero at both levels and
-    // is never formed or read below
+    // g[0][c] (the element's rigid translations) is zero and is never formed
+    // or read below
     T g[8][3];
-    if constexpr (LVL == 0) {
-      element_core<T>(B, Ee, h, g);
-      if constexpr (kDiag) {
-        if (i < i0 && own_ok) {  // first slab: the neighbours' moduli from memory
-          const uint32_t eb = ((uint32_t)i * a.fez + k) * a.few + j;
-          T es = Ee;
-          if (!last_y) es += *at32(E, eb + 1);
-          if (!last_z) es += *at32(E, eb + a.few);
-          if (!last_y && !last_z) es += *at32(E, eb + a.few + 1);
-          es_prev = es;
-        }
+    // Ehat: the per-element 8-point transform of the element's fine moduli,
+    // formed once per set of moduli (k_level1_moduli); zero for halo
+    // elements, which threads outside the grid read
+    T Eh[8];
+    const uint32_t eh = 8u * ((uint32_t)i * (uint32_t)(a.fez * a.few) + e00c);
+    if constexpr (sizeof(T) == 4) {
+      typedef float f4 __attribute__((ext_vector_type(4)));
+      const f4 *pe = reinterpret_cast<const f4 *>(at32(E, eh));
+      const f4 lo = pe[0], hi = pe[1];
+#pragma unroll
+      for (int o = 0; o < 4; o++) {
+        Eh[o] = lo[o];
+        Eh[o + 4] = hi[o];
       }
     } else {
-      // Ehat: the per-element 8-point transform of the element's fine moduli,
-      // formed once per set of moduli (k_level1_moduli); zero for halo
-      // elements, which threads outside the grid read
-      T Eh[8];
-      const uint32_t eh = 8u * ((uint32_t)i * (uint32_t)(a.fez * a.few) + e00c);
-      if constexpr (sizeof(T) == 4) {
-        typedef float f4 __attribute__((ext_vector_type(4)));
-        const f4 *pe = reinterpret_cast<const f4 *>(at32(E, eh));
-        const f4 lo = pe[0], hi = pe[1];
+      typedef double d2 __attribute__((ext_vector_type(2)));
+      const d2 *pe = reinterpret_cast<const d2 *>(at32(E, eh));
 #pragma unroll
-        for (int o = 0; o < 4; o++) {
-          Eh[o] = lo[o];
-          Eh[o + 4] = hi[o];
-        }
-      } else {
-        typedef double d2 __attribute__((ext_vector_type(2)));
-        const d2 *pe = reinterpret_cast<const d2 *>(at32(E, eh));
-#pragma unroll
-        for (int o = 0; o < 4; o++) {
-          const d2 v = pe[o];
-          Eh[2 * o] = v[0];
-          Eh[2 * o + 1] = v[1];
-        }
+      for (int o = 0; o < 4; o++) {
+        const d2 v = pe[o];
+        Eh[2 * o] = v[0];
+        Eh[2 * o + 1] = v[1];
       }
-      element_core_l1<T>(B, Eh, h, g);
     }
+    element_core_l1<T>(B, Eh, h, g);
     T o[3] = {0, 0, 0};
     const T *bb = nv.bb, *di = nv.di;
     const uint8_t m = nv.m;
@@ -663,34 +693,21 @@ __device__ __forceinline__ void tile_sweep_body(
           buf[3 + c] = tot[1][0][c];           // node (j+1, k)  -> thread (ty, tz-1)
           buf[6 + c] = tot[0][0][c];           // node (j, k)    -> thread (ty-1, tz-1)
         }
-        if constexpr (kDiag) buf[9] = Ee;
       }
       lds_barrier();
       if (own_ok) {
         T kin[3] = {tot[1][1][0], tot[1][1][1], tot[1][1][2]};
-        T es = Ee;  // kDiag: moduli of this slab's 4 elements at the node
         if (!last_y) {
 #pragma unroll
           for (int c = 0; c < 3; c++) kin[c] += buf[XS + c];
-          if constexpr (kDiag) es += buf[XS + 9];
         }
         if (!last_z) {
 #pragma unroll
           for (int c = 0; c < 3; c++) kin[c] += buf[XS * a.TY + 3 + c];
-          if constexpr (kDiag) es += buf[XS * a.TY + 9];
         }
         if (!last_y && !last_z) {
 #pragma unroll
           for (int c = 0; c < 3; c++) kin[c] += buf[XS * (a.TY + 1) + 6 + c];
-          if constexpr (kDiag) es += buf[XS * (a.TY + 1) + 9];
-        }
-        T dd[3] = {di[0], di[1], di[2]};
-        if constexpr (kDiag) {
-          // diagonal KE[c][c] (es_prev + es); identity rows at fixed DOFs
-          const T rs = recip<T>(es_prev + es);
-          es_prev = es;
-#pragma unroll
-          for (int c = 0; c < 3; c++) dd[c] = ((m >> c) & 1) ? T(1) : rs * B.ikd[c];
         }
 #pragma unroll
         for (int c = 0; c < 3; c++) {
@@ -699,10 +716,8 @@ __device__ __forceinline__ void tile_sweep_body(
           if ((m >> c) & 1) kv = uc;  // identity row
           if (MODE == kModeApply) {
             o[c] = kv;
-            if (dotp) dacc += (double)uc * (double)o[c];
-          } else if (MODE == kModeJacobi || kDiag) {
-            o[c] = uc + omega * dd[c] * (bb[c] - kv);
-            if (dotp) dacc += (double)bb[c] * (double)o[c];
+          } else if (MODE == kModeJacobi) {
+            o[c] = uc + omega * di[c] * (bb[c] - kv);
           } else {
             o[c] = bb[c] - kv;
           }
@@ -713,7 +728,7 @@ __device__ __forceinline__ void tile_sweep_body(
     // step's wait for its face leaves it in flight): the owned node of an
     // emitted plane, else nothing
     store_node(orsrc, emit && own_ok ? d0 * (uint32_t)sizeof(T) : a.out_bytes, o);
-    if constexpr (PIPE) load_node(min(i + 1, i1), nv);
+    load_node(min(i + 1, i1), nv);
 #pragma unroll
     for (int c = 0; c < 3; c++) pendT[0][c] = -g[1][c];
 #pragma unroll
@@ -729,15 +744,12 @@ __device__ __forceinline__ void tile_sweep_body(
   for (int c = 0; c < 3; c++) u0[c] = vq[1][1][c];
   mask_face(i0 - 1, vq);
   face_wht<T>(vq, Fa);
-  if constexpr (PIPE) {
-    // the loads a step's head and end would have issued before the first
-    // step (the store writes nothing; the first step emits no plane and
-    // leaves the node operands unused)
-    Ecur = load_modulus(i0 - 1);
-    fetch_face(i0, vq);
-    store_node(orsrc, a.out_bytes, u0);
-    load_node(i0 - 1, nv);
-  }
+  // the loads a step's head and end would have issued before the first step
+  // (the store writes nothing; the first step emits no plane and leaves the
+  // node operands unused)
+  fetch_face(i0, vq);
+  store_node(orsrc, a.out_bytes, u0);
+  load_node(i0 - 1, nv);
   for (int i = i0 - 1; i <= i1; i++) {
     step(i, Fa, Fb);
 #pragma unroll
@@ -747,6 +759,285 @@ __device__ __forceinline__ void tile_sweep_body(
 #pragma unroll
     for (int c = 0; c < 3; c++) u0[c] = u1[c];
   }
+}
+
+// Keeps a value that a loop loads again from being loaded inside the loop only
+// (the compiler would merge the loads before the loop with those in it and
+// issue them where they are used).
+template <typename T>
+__device__ __forceinline__ void pin(T &x) {
+  asm volatile("" : "+v"(x));
+}
+
+// The fine level.  A workgroup has a thread per node of its (TY + 1) x (TZ + 1)
+// node tile, up to 255 nodes in 4 waves; each loads its own node of the plane
+// and hands it on through LDS with the exchange of the element's corners, under
+// the same barrier, and works on the element whose upper corner (j, k) is its
+// node (none for the tile's lower edges).  Every LDS array is [value][thread],
+// so that a wave's access is contiguous but for the three face nodes of other
+// rows.  Every load is issued a step before its value is used, as on level 1;
+// every lane forms its node's row, and the store decides by its offset.
+//
+// What bounds it: the arithmetic in FP32 (about 230 instructions per element,
+// of 4 cycles each, and 170 MB per sweep at 257x129x129 nodes: 34.5 us), the
+// memory in FP64 (341 MB, more than the memory-side cache holds).  Before,
+// with a thread per element that loaded the four nodes of its face through the
+// first-level cache, all 45 values of the blocks and masks at every node: 40.0
+// us and, FP64, 101 us per sweep and 72.5 us per apply, now 77.3 and 59.5.
+constexpr int kMarchThreads = 256;
+
+// LDS values per thread: two buffers of the exchange (9 corners, in the
+// diagonal-forming sweep the modulus too) and of the plane's 3 components
+constexpr int march_lds_values(bool diag) { return 2 * ((diag ? 10 : 9) + 3); }
+
+template <typename T, int MODE, bool BCSYM>
+__device__ __forceinline__ void fine_march_body(
+    TileArgs a, Blocks<T> B, const T *__restrict__ E, const T *__restrict__ in,
+    T *__restrict__ out, const T *__restrict__ b, const T *__restrict__ invD, T omega,
+    const uint8_t *__restrict__ fix, const int *__restrict__ fixplane,
+    double *__restrict__ dotp) {
+  constexpr bool kDiag = MODE == kModeJacobiDiag;
+  constexpr int N = kMarchThreads, XV = kDiag ? 10 : 9;
+  extern __shared__ unsigned char smem_raw[];
+  T *xch = reinterpret_cast<T *>(smem_raw);  // [2][XV][N]; slot N-1: zeros
+  T *nodes = xch + 2 * XV * N;               // [2][3][N]
+  const int t = threadIdx.x, nrow = a.TY + 1;
+  const bool active = t < nrow * (a.TZ + 1);
+  const int ty = t % nrow, tz = t / nrow;
+  const TilePos w = tile_pos(a);
+  const int j = w.by * (a.TY - 1) + ty, k = w.bz * (a.TZ - 1) + tz;  // the node's column
+  const int i0 = 1 + w.slab * a.NX;
+  const int i1 = min(i0 + a.NX - 1, a.nelx + 1);  // last output plane
+  const bool elem_ok = active && ty > 0 && tz > 0 && j - 1 <= a.nely && k - 1 <= a.nelz;
+  const bool last_y = (ty == a.TY), last_z = (tz == a.TZ);
+  const bool own_ok = elem_ok && (!last_y || j == a.nely + 1) && (!last_z || k == a.nelz + 1);
+  // bytes of a plane of each array
+  const uint32_t sx = (uint32_t)a.wy * (uint32_t)a.wz, sv = 3u * sx * (uint32_t)sizeof(T);
+  const uint32_t se = (uint32_t)a.fez * (uint32_t)a.few * (uint32_t)sizeof(T);
+  // nodes beyond the level's arrays read node 0 of the plane
+  const uint32_t node =
+      active && j < a.wy && k < a.wz ? (uint32_t)k * a.wy + (uint32_t)j : 0u;
+  const uint32_t vnode = 3u * (uint32_t)sizeof(T) * node;
+  const uint32_t vout = own_ok ? vnode : a.out_bytes;  // (a store there writes nothing)
+  const uint32_t velem =
+      elem_ok ? (uint32_t)sizeof(T) * ((uint32_t)(k - 1) * a.few + (uint32_t)(j - 1)) : 0u;
+  // node (j - 1, k - 1) of the face
+  const int f00 = max(t - nrow - 1, 0), f01 = f00 + nrow;
+  // the neighbours' corners: zeros beyond the tile's last element
+  const int n01 = last_y ? N - 1 : t + 1;
+  const int n10 = last_z ? N - 1 : t + nrow;
+  const int n11 = last_y || last_z ? N - 1 : t + nrow + 1;
+  double dacc = 0.0;
+  T es_prev = 0;
+  auto rsrc = [](const void *p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes,
+                                             0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t rin = rsrc(in, a.out_bytes), re = rsrc(E, a.e_bytes);
+  const __amdgpu_buffer_rsrc_t rfix = rsrc(fix, a.out_bytes / (3u * (uint32_t)sizeof(T)));
+  const __amdgpu_buffer_rsrc_t rb = rsrc(MODE == kModeApply ? in : b, a.out_bytes);
+  const __amdgpu_buffer_rsrc_t rd = rsrc(MODE == kModeJacobi ? invD : in, a.out_bytes);
+  // the planes from plane fbase on with a fixed DOF
+  int fbase = i0 - 1;
+  auto fixed_planes = [&]() {
+    return __ballot(fixplane[min(fbase + (int)__lane_id(), a.nelx + 2)] != 0);
+  };
+  uint64_t fbits = fixed_planes();
+  // operands in flight: the node to hand on, the slab's modulus, the owned
+  // node's b, invD and fixed-DOF mask
+  struct Operands {
+    T p[3], e, bb[3], di[3];
+    uint32_t m;
+    bool fixed;  // a fixed DOF in the plane (uniform)
+  } s{};
+  auto load_plane = [&](int i, T (&p)[3]) {  // (the march reads planes up to i1 + 1)
+    load3<T>(rin, vnode, (uint32_t)min(i, i1 + 1) * sv, p);
+  };
+  auto load_modulus = [&](int i) { return load1<T>(re, velem, (uint32_t)min(i, i1) * se); };
+  auto load_node = [&](int i_) {
+    const int i = min(i_, i1);
+    if (MODE != kModeApply) load3<T>(rb, vnode, (uint32_t)i * sv, s.bb);
+    if (MODE == kModeJacobi) load3<T>(rd, vnode, (uint32_t)i * sv, s.di);
+    if (i - fbase >= 64) {
+      fbase = i;
+      fbits = fixed_planes();
+    }
+    // (no branch: the merged value would be waited for here)
+    s.fixed = (fbits >> (i - fbase)) & 1;
+    s.m = __builtin_amdgcn_raw_buffer_load_b8(rfix, (int)(s.fixed ? node : 0u),
+                                              (int)((uint32_t)i * sx), 0);
+  };
+  // plane i into LDS buffer P; u: the values; BCSYM: the fixed DOFs are
+  // handed on, and read back, as zeros
+  auto put_plane = [&](int i, int P, const T (&p)[3], T (&u)[3]) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) u[c] = copy_here(p[c]);
+    if (BCSYM && fixplane[min(i, i1 + 1)] != 0) {
+      const uint8_t m = fix[(uint32_t)min(i, i1 + 1) * sx + node];
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        if ((m >> c) & 1) u[c] = 0;
+    }
+    T *nb = nodes + P * 3 * N + t;
+#pragma unroll
+    for (int c = 0; c < 3; c++) nb[c * N] = u[c];
+  };
+  // transformed face of the plane in LDS buffer P, whose node (j, k) holds u
+  auto get_face = [&](int P, T (&F)[4][3], const T (&u)[3]) {
+    const T *nb = nodes + P * 3 * N;
+    T v[2][2][3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      v[0][0][c] = nb[c * N + f00];
+      v[1][0][c] = nb[c * N + f00 + 1];
+      v[0][1][c] = nb[c * N + f01];
+      v[1][1][c] = u[c];
+    }
+    face_wht<T>(v, F);
+  };
+
+  T pendT[4][3];
+#pragma unroll
+  for (int f = 0; f < 4; f++)
+#pragma unroll
+    for (int c = 0; c < 3; c++) pendT[f][c] = 0;
+
+  // element slab i, the (P + 1)th or (P + 3)th, ... of the march: Fc the
+  // transformed face of plane i, Fn that of plane i+1; u0, u1, u2 the node's
+  // values of planes i, i+1 and i+2
+  auto step = [&](int i, auto par, const T (&Fc)[4][3], T (&Fn)[4][3], const T (&u0)[3],
+                  const T (&u1)[3], T (&u2)[3]) {
+    constexpr int P = decltype(par)::value;
+    const bool emit = i >= i0;  // uniform
+    const T Ee = copy_here(s.e);
+    s.e = load_modulus(i + 1);
+    get_face(1 - P, Fn, u1);
+    T hh[8][3];
+#pragma unroll
+    for (int f = 0; f < 4; f++)
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        hh[2 * f][c] = Fc[f][c] + Fn[f][c];
+        hh[2 * f + 1][c] = Fc[f][c] - Fn[f][c];
+      }
+    T g[8][3];
+    element_core<T>(B, Ee, hh, g);
+    T totT[4][3], tot[2][2][3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) totT[0][c] = g[1][c] + pendT[0][c];
+#pragma unroll
+    for (int f = 1; f < 4; f++)
+#pragma unroll
+      for (int c = 0; c < 3; c++) totT[f][c] = (g[2 * f][c] + g[2 * f + 1][c]) + pendT[f][c];
+#pragma unroll
+    for (int c = 0; c < 3; c++) pendT[0][c] = -g[1][c];
+#pragma unroll
+    for (int f = 1; f < 4; f++)
+#pragma unroll
+      for (int c = 0; c < 3; c++) pendT[f][c] = g[2 * f][c] - g[2 * f + 1][c];
+    face_iwht<T>(totT, tot);
+    T *buf = xch + P * XV * N;
+    if (active) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        buf[c * N + t] = tot[0][1][c];        // node (j-1, k)    -> its thread
+        buf[(3 + c) * N + t] = tot[1][0][c];  // node (j, k-1)
+        buf[(6 + c) * N + t] = tot[0][0][c];  // node (j-1, k-1)
+      }
+      if constexpr (kDiag) buf[9 * N + t] = Ee;
+    }
+    put_plane(i + 2, P, s.p, u2);
+    load_plane(i + 3, s.p);
+    lds_barrier();
+    // the owned node's row, in every lane: stored where own_ok and emit
+    T kin[3] = {tot[1][1][0], tot[1][1][1], tot[1][1][2]}, o[3], uo[3], dd[3];
+#pragma unroll
+    for (int c = 0; c < 3; c++) kin[c] += buf[c * N + n01];
+#pragma unroll
+    for (int c = 0; c < 3; c++) kin[c] += buf[(3 + c) * N + n10];
+#pragma unroll
+    for (int c = 0; c < 3; c++) kin[c] += buf[(6 + c) * N + n11];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      uo[c] = u0[c];
+      dd[c] = s.di[c];
+    }
+    if constexpr (kDiag) {  // the moduli of the two slabs' 4 elements each at the node
+      const T es = ((Ee + buf[9 * N + n01]) + buf[9 * N + n10]) + buf[9 * N + n11];
+      const T rs = recip<T>(es_prev + es);
+      es_prev = es;
+#pragma unroll
+      for (int c = 0; c < 3; c++) dd[c] = rs * B.ikd[c];
+    }
+    uint32_t m = s.m;
+    pin(m);  // (used in the branch only, its copies for the next step would wait for the load)
+    if (s.fixed) {
+      if (BCSYM && m != 0) {  // u0 holds zeros there
+        const T *pu = at32(in, 3u * ((uint32_t)i * sx + node));
+#pragma unroll
+        for (int c = 0; c < 3; c++) uo[c] = pu[c];
+      }
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        if ((m >> c) & 1) {  // identity row
+          kin[c] = uo[c];
+          if constexpr (kDiag) dd[c] = T(1);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      if (MODE == kModeApply) o[c] = kin[c];
+      else if (MODE == kModeJacobi || kDiag) o[c] = uo[c] + omega * dd[c] * (s.bb[c] - kin[c]);
+      else o[c] = s.bb[c] - kin[c];
+    }
+    if (MODE != kModeResidual && dotp) {
+      double d = dacc;
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        d += (double)(MODE == kModeApply ? uo[c] : s.bb[c]) * (double)o[c];
+      dacc = emit && own_ok ? d : dacc;
+    }
+    // (an empty resource where the plane is another workgroup's)
+    const __amdgpu_buffer_rsrc_t ro = rsrc(out, emit ? a.out_bytes : 0u);
+    if (a.stream_out) store_node<kNt>(ro, vout, o, (uint32_t)i * sv);
+    else store_node(ro, vout, o, (uint32_t)i * sv);
+    load_node(i + 1);
+  };
+
+  // planes i0-1 and i0 straight to LDS
+  T ua[3], ub[3], uc[3], pa[3], pb[3], Fa[4][3], Fb[4][3];
+  load_plane(i0 - 1, pa);
+  load_plane(i0, pb);
+  load_plane(i0 + 1, s.p);
+  s.e = load_modulus(i0 - 1);
+  load_node(i0 - 1);
+  if (t < 2 * XV) xch[t * N + N - 1] = 0;
+  put_plane(i0 - 1, 0, pa, ua);
+  put_plane(i0, 1, pb, ub);
+  __syncthreads();
+  get_face(0, Fa, ua);
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    pin(s.p[c]);
+    if (MODE != kModeApply) pin(s.bb[c]);
+    if (MODE == kModeJacobi) pin(s.di[c]);
+  }
+  pin(s.e);
+  __syncthreads();  // plane i0-1 is read: its buffer takes plane i0+1
+  // two slabs per turn, so that faces, LDS buffers and node values change
+  // places without copies
+  for (int i = i0 - 1;;) {
+    step(i, std::integral_constant<int, 0>{}, Fa, Fb, ua, ub, uc);
+    if (++i > i1) break;
+    step(i, std::integral_constant<int, 1>{}, Fb, Fa, ub, uc, ua);
+    if (++i > i1) break;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const T uz = uc[c];
+      ub[c] = ua[c];
+      ua[c] = uz;
+    }
+  }
   if (MODE != kModeResidual && dotp) {  // one partial per workgroup, fixed order
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) dacc += __shfl_down(dacc, off, 64);
@@ -755,37 +1046,29 @@ __device__ __forceinline__ void tile_sweep_body(
     if ((t & 63) == 0) red[t >> 6] = dacc;
     __syncthreads();
     if (t == 0) {
-      double s = 0.0;
-      for (int w = 0; w < (int)(blockDim.x >> 6); w++) s += red[w];
-      dotp[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = s;
+      double sum = 0.0;
+      for (int v = 0; v < (int)(blockDim.x >> 6); v++) sum += red[v];
+      dotp[w.dot] = sum;
     }
   }
 }
 
-// Waves per SIMD the register allocation must allow: FP64 fine level 3
-// (three 4-wave workgroups of 17 x 12 columns per CU, at most 168 VGPRs);
-// otherwise what the launch bounds already imply (one workgroup per CU).
-template <typename T, int LVL, int MODE, bool BCSYM>
-__global__ __launch_bounds__(sizeof(T) == 4 ? 1024 : 512)
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : LVL == 0 ? 3 : 2))) void k_tile_sweep(
-    TileArgs a, std::conditional_t<LVL == 0, Blocks<T>, K1Vals<T>> B, const T *__restrict__ E,
-    const T *__restrict__ in, T *__restrict__ out, const T *__restrict__ b,
-    const T *__restrict__ invD, T omega, const uint8_t *__restrict__ fix,
-    const int *__restrict__ fixplane, double *__restrict__ dotp) {
-  tile_sweep_body<T, LVL, MODE, BCSYM, true>(a, B, E, in, out, b, invD, omega, fix, fixplane,
-                                             dotp);
+template <typename T, int MODE, bool BCSYM>
+__global__ __launch_bounds__(kMarchThreads)
+    __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 3))) void k_fine_march(
+    TileArgs a, Blocks<T> B, const T *__restrict__ E, const T *__restrict__ in,
+    T *__restrict__ out, const T *__restrict__ b, const T *__restrict__ invD, T omega,
+    const uint8_t *__restrict__ fix, const int *__restrict__ fixplane,
+    double *__restrict__ dotp) {
+  fine_march_body<T, MODE, BCSYM>(a, B, E, in, out, b, invD, omega, fix, fixplane, dotp);
 }
 
-// fine level in FP32: workgroups of up to 1024 threads; two 9-wave
-// workgroups of 33 x 17 columns share a CU
-template <int MODE, bool BCSYM>
-__global__ __launch_bounds__(1024) void k_tile_sweep_f32(
-    TileArgs a, Blocks<float> B, const float *__restrict__ E, const float *__restrict__ in,
-    float *__restrict__ out, const float *__restrict__ b, const float *__restrict__ invD,
-    float omega, const uint8_t *__restrict__ fix, const int *__restrict__ fixplane,
-    double *__restrict__ dotp) {
-  tile_sweep_body<float, 0, MODE, BCSYM, false>(a, B, E, in, out, b, invD, omega, fix, fixplane,
-                                                dotp);
+template <typename T, int MODE, bool BCSYM>
+__global__ __launch_bounds__(sizeof(T) == 4 ? 1024 : 512) void k_level1_sweep(
+    TileArgs a, K1Vals<T> B, const T *__restrict__ E, const T *__restrict__ in,
+    T *__restrict__ out, const T *__restrict__ b, const T *__restrict__ invD, T omega,
+    const uint8_t *__restrict__ fix, const int *__restrict__ fixplane) {
+  level1_sweep_body<T, MODE, BCSYM>(a, B, E, in, out, b, invD, omega, fix, fixplane);
 }
 
 // ---------------------------------------------------------------------------
@@ -800,6 +1083,30 @@ struct HostCoef {
 };
 static HostCoef g_coef;
 
+// The 8 values of the blocks; false if an entry of M is not what they give.
+static bool fine_blocks(const double M[8][3][3], Blocks<double> &B, Blocks<float> &F) {
+  const double a0 = M[0][0][0], b0 = M[0][0][2], p = M[1][1][1], q = M[2][0][2];
+  const double r = M[3][0][0], t = M[3][2][2], a7 = M[7][0][0], b7 = M[7][0][2];
+  const int sg[3] = {1, -1, 1};
+  for (int s = 0; s < 8; s++)
+    for (int c = 0; c < 3; c++)
+      for (int d = 0; d < 3; d++) {
+        const bool in_c = (s >> c) & 1, in_d = (s >> d) & 1;
+        const int bits = __builtin_popcount(s);
+        double v = 0.0;  // |entry|
+        if (bits == 0) v = c == d ? a0 : b0;
+        if (bits == 3) v = c == d ? a7 : b7;
+        if (bits == 1 && !in_c && !in_d) v = c == d ? p : q;
+        if (bits == 2 && in_c && in_d) v = r;
+        if (bits == 2 && c == d && !in_c) v = t;
+        if (std::fabs(M[s][c][d] - sg[c] * sg[d] * v) > 1e-12 * a0) return false;
+      }
+  B.d0 = a0 - b0, B.b0 = b0, B.p1 = p, B.q1 = q, B.r2 = r, B.t2 = t, B.d7 = a7 - b7, B.b7 = b7;
+  F.d0 = (float)B.d0, F.b0 = (float)B.b0, F.p1 = (float)p, F.q1 = (float)q;
+  F.r2 = (float)r, F.t2 = (float)t, F.d7 = (float)B.d7, F.b7 = (float)b7;
+  return true;
+}
+
 static void init_coef() {
   if (g_coef.done) return;
   g_coef.done = true;
@@ -808,13 +1115,7 @@ static void init_coef() {
   element_matrices(0.3, 1, KE1.data());
   double M[8][3][3];
   g_coef.ok0 = hadamard_blocks(KE.data(), M);
-  if (g_coef.ok0)
-    for (int s = 0; s < 8; s++)
-      for (int c = 0; c < 3; c++)
-        for (int d = 0; d < 3; d++) {
-          g_coef.b64.m[s][c][d] = M[s][c][d];
-          g_coef.b32.m[s][c][d] = (float)M[s][c][d];
-        }
+  if (g_coef.ok0) g_coef.ok0 = fine_blocks(M, g_coef.b64, g_coef.b32);
   if (g_coef.ok0) {
     g_coef.diag0 = true;
     for (int c = 0; c < 3; c++) {
@@ -858,72 +1159,65 @@ bool tile_fine_diag_available() {
   return g_coef.ok0 && g_coef.diag0;
 }
 
+template <typename T>
+static Blocks<T> fine_values() {
+  if constexpr (sizeof(T) == 8) return g_coef.b64;
+  else return g_coef.b32;
+}
+
 struct TileShape {
   int TY, TZ, NX, nty, ntz, ntx;
 };
 
-// Tile of TY x TZ element columns marching over NX node planes.  LDS holds
-// two exchange buffers of 9 or 10 values per thread (under 80 KiB).  Tuning
-// override: TOP3D_TILE_L<level>=TY,TZ,NX (NX = 0: from the occupancy).
-//
-// Shapes measured on MI355X at 256x128x128 (fine) / 128x64x64 (level 1):
-// for the FP32 fine level 33 x 17 (561 threads in 9 waves, two workgroups
-// per CU, 32 tiles of 32 x 16 owned node columns) ran 42.8 us in the
-// V-cycle against 44.9 us for 65 x 11 (12 waves), 44.0 us for 44 x 17,
-// 47.3 us for 65 x 7, 47.7 us for 33 x 23 and 55.3 us for 65 x 12 (one
-// workgroup per CU); for the FP64 fine level 17 x 12 (4 waves) ran the
-// outer CG's apply in 73.6 us (repeated on one buffer) against 75.8 us
-// for 65 x 7, 81-112 us for 33 x 7/12/15, 25 x 20, 45 x 11 and 17 x 24;
-// for level 1 (128x64x64) 65 x 7 with the x-march length below ran 15.5 us
-// in FP32 and 23.6 us in FP64 (repeated on one buffer set; 20.6 and 33.7 us
-// with the memory-side cache flushed) against 15.8 / 27.1 us for 65 x 11
-// (NX 4, FP32) and 65 x 6 (NX 8, FP64), and 15.8-19.3 / 24.3-30.5 us for
-// 65 x 3/5/6/11, 33 x 6/9/11/12/15/21 and 17 x 12/23.
-// The x-march length
-// follows from the number of workgroups the device holds at once (`slots`):
-// a launch that overflows them by a few
-// workgroups pays a whole extra round, so NX is chosen to minimise
-// rounds x (NX + 3), the per-workgroup cost in slab steps.
-static TileShape tile_shape(const Level &L, int lvl, int elem_bytes, int &nx_fixed) {
-  TileShape s{};
-  // LDS values per thread: 2 buffers of 9 (11 on the fine level, whose
-  // diagonal-forming sweep also exchanges a modulus; padded to an odd stride)
-  const int lds_threads = 80 * 1024 / ((lvl == 0 ? 22 : 18) * elem_bytes);
-  // launch bounds: 1024 threads in FP32, 512 in FP64
-  const int max_threads = std::min(elem_bytes == 4 ? 1024 : 512, lds_threads);
-  struct Rule {
-    int ycap, tz, nx;
-  };
-  static constexpr Rule kRules[2][2] = {{{17, 12, 0}, {33, 17, 0}},  // level 0: f64, f32
-                                        {{65, 7, 0}, {65, 7, 0}}};   // level 1
-  const Rule r = kRules[lvl == 0 ? 0 : 1][elem_bytes == 4 ? 1 : 0];
-  s.TY = std::max(2, std::min(L.nely + 1, r.ycap));
-  s.TZ = std::max(2, std::min({L.nelz + 1, r.tz, max_threads / s.TY}));
-  nx_fixed = r.nx;
-  const char *env = std::getenv(lvl == 0 ? (elem_bytes == 8 ? "TOP3D_TILE_L0_F64" : "TOP3D_TILE_L0")
-                                          : "TOP3D_TILE_L1");
-  int oy = 0, oz = 0, ox = 0;
-  if (env && std::sscanf(env, "%d,%d,%d", &oy, &oz, &ox) == 3 && oy >= 2 && oz >= 2 && ox >= 0 &&
-      oy * oz <= max_threads) {
-    s.TY = std::min(oy, std::max(2, L.nely + 1));
-    s.TZ = std::min(oz, std::max(2, L.nelz + 1));
-    nx_fixed = ox;
-  }
+// tiles of up to ty x tz element columns
+static void set_tiles(TileShape &s, const Level &L, int ty, int tz) {
+  s.TY = std::max(2, std::min(L.nely + 1, ty));
+  s.TZ = std::max(2, std::min(L.nelz + 1, tz));
   // a tile owns TY-1 node rows, plus the last row of the grid (its upper
   // neighbour element is halo)
   auto tiles = [](int nodes, int T) { return nodes <= T ? 1 : (nodes - T + T - 2) / (T - 1) + 1; };
   s.nty = tiles(L.ny, s.TY);
   s.ntz = tiles(L.nz, s.TZ);
+}
+
+// Level 1: tile of TY x TZ element columns marching over NX node planes.  LDS
+// holds two exchange buffers of 9 values per thread (under 80 KiB).  Tuning
+// override: TOP3D_TILE_L1=TY,TZ,NX (NX = 0: from the occupancy).
+//
+// Shapes measured on MI355X at 128x64x64: 65 x 7 with the x-march length below
+// ran 15.5 us in FP32 and 23.6 us in FP64 (repeated on one buffer set; 20.6 and
+// 33.7 us with the memory-side cache flushed) against 15.8 / 27.1 us for
+// 65 x 11 (NX 4, FP32) and 65 x 6 (NX 8, FP64), and 15.8-19.3 / 24.3-30.5 us
+// for 65 x 3/5/6/11, 33 x 6/9/11/12/15/21 and 17 x 12/23.
+static TileShape level1_shape(const Level &L, int elem_bytes, int &nx_fixed) {
+  TileShape s{};
+  const int lds_threads = 80 * 1024 / (18 * elem_bytes);
+  // launch bounds: 1024 threads in FP32, 512 in FP64
+  const int max_threads = std::min(elem_bytes == 4 ? 1024 : 512, lds_threads);
+  set_tiles(s, L, 65, std::min(7, max_threads / std::max(2, std::min(L.nely + 1, 65))));
+  nx_fixed = 0;
+  const char *env = std::getenv("TOP3D_TILE_L1");
+  int oy = 0, oz = 0, ox = 0;
+  if (env && std::sscanf(env, "%d,%d,%d", &oy, &oz, &ox) == 3 && oy >= 2 && oz >= 2 && ox >= 0 &&
+      oy * oz <= max_threads) {
+    set_tiles(s, L, oy, oz);
+    nx_fixed = ox;
+  }
   return s;
 }
 
-static void tile_x(TileShape &s, const Level &L, int nx_fixed, int64_t slots) {
+// The x-march length follows from the number of workgroups the device holds at
+// once (`slots`): a launch that overflows them by a few workgroups pays a whole
+// extra round, so NX is chosen to minimise rounds x (NX + 3), the per-workgroup
+// cost in slab steps.  Sets
+// the march length of a shape and the launch's cost in slab steps
+static int64_t tile_x(TileShape &s, const Level &L, int nx_fixed, int64_t slots) {
   const int64_t yz = (int64_t)s.nty * s.ntz;
+  int64_t best_cost = INT64_MAX;
   if (nx_fixed > 0) {
     s.NX = std::min(nx_fixed, L.nx);
   } else {
     int best = L.nx;
-    int64_t best_cost = INT64_MAX;
     for (int k = 1; k <= 8; k++) {
       const int64_t ntx = std::max<int64_t>(1, std::min<int64_t>(L.nx, k * slots / yz));
       const int nx = (int)((L.nx + ntx - 1) / ntx);
@@ -937,6 +1231,41 @@ static void tile_x(TileShape &s, const Level &L, int nx_fixed, int64_t slots) {
     s.NX = best;
   }
   s.ntx = (L.nx + s.NX - 1) / s.NX;
+  return best_cost;
+}
+
+// The fine level's shape (k_fine_march): (TY + 1) x (TZ + 1) nodes within the
+// workgroup's threads, one of which holds the zeros.  At 257x129x129 nodes, in
+// FP64, 23 x 9 columns ran a sweep in 81.6 us, 24 x 9 in 83.8 us, 20 x 11 in
+// 85.5 us, 17 x 12 in 84.4 us, 17 x 13 in 87.9 us, 22 x 10, whose 97 tiles
+// leave 7 slabs instead of 8, in 93.1 us, 15 x 15 and 26 x 8 likewise in 104
+// us and 9 x 23, short rows, in 93.5 us; in FP32 17 x 13 in 35.2-36.7, 20 x 11
+// in 34.4-35.6, 23 x 9 in 37.6 and 22 x 10 in 39.7 us: rows of 17 to 23 columns
+// with the cheapest launch, the longest among equals.  Tuning override:
+// TOP3D_TILE_L0 (FP32), TOP3D_TILE_L0_F64=TY,TZ,NX (NX = 0: the march length
+// from the occupancy).
+static TileShape march_shape(const Level &L, int64_t slots, bool f64, int &nx_fixed) {
+  constexpr int kNodes = kMarchThreads - 1;
+  TileShape best{};
+  int64_t best_cost = INT64_MAX;
+  nx_fixed = 0;
+  for (int ty = 17; ty <= 23; ty++) {
+    TileShape s{};
+    set_tiles(s, L, ty, kNodes / (std::min(ty, std::max(2, L.nely + 1)) + 1) - 1);
+    const int64_t cost = tile_x(s, L, 0, slots);
+    if (cost <= best_cost) {
+      best_cost = cost;
+      best = s;
+    }
+  }
+  const char *env = std::getenv(f64 ? "TOP3D_TILE_L0_F64" : "TOP3D_TILE_L0");
+  int oy = 0, oz = 0, ox = 0;
+  if (env && std::sscanf(env, "%d,%d,%d", &oy, &oz, &ox) == 3 && oy >= 2 && oz >= 2 && ox >= 0 &&
+      oy <= kNodes && oz <= kNodes && (oy + 1) * (oz + 1) <= kNodes) {
+    set_tiles(best, L, oy, oz);
+    nx_fixed = ox;
+  }
+  return best;
 }
 
 // workgroups of `nthr` threads and `shm` bytes of LDS one CU holds at once.
@@ -969,117 +1298,150 @@ static int device_cus() {
   return ncu[dev];
 }
 
-template <typename T, int LVL>
-static int launch_tile(const DevGrid &g, int mode, const T *E, const T *in, T *out, const T *b,
-                       const T *invD, T omega, int bcsym, double *dotp = nullptr,
-                       int dot_cap = 0) {
-  init_coef();
-  if (!(LVL == 0 ? g_coef.ok0 : g_coef.ok1)) {
+// checks that a level's offsets fit in 32 bits (the output's byte size also
+// bounds the store offset that writes nothing, plus 16) and fills the
+// kernels' arguments
+template <typename T>
+static bool tile_args(const Level &L, int64_t nmod, bool available, TileArgs &a) {
+  if (!available) {
     set_error(TOP3D_ERR_ARG, "element matrix lacks the reflection structure");
-    return 0;
+    return false;
   }
-  const Level &L = g.lv[LVL];
-  const int64_t nmod = LVL == 0 ? g.nelem : level1_moduli_count(g);
-  // (the output's byte size also bounds the store offset that writes
-  // nothing, plus 16, in 32 bits)
   if ((int64_t)sizeof(T) * 3 * L.nodes() >= (int64_t(1) << 32) - 32 ||
       (int64_t)sizeof(T) * nmod >= (int64_t(1) << 32)) {
     set_error(TOP3D_ERR_ARG, "grid too large for 32-bit offsets (%lld nodes)",
               (long long)L.nodes());
-    return 0;
+    return false;
   }
-  // the diagonal from the moduli needs the fine level and a KE whose
-  // diagonal is one value per component
-  if (mode == kModeJacobiDiag && !(LVL == 0 && g_coef.diag0)) mode = kModeJacobi;
-  const bool diag = mode == kModeJacobiDiag;
-  int nx_fixed = 0;
-  TileShape s = tile_shape(L, LVL, (int)sizeof(T), nx_fixed);
-  const int nthr = s.TY * s.TZ;
-  const int bs = (nthr + 63) / 64 * 64;
-  const size_t shm = sizeof(T) * 2 * (diag ? 11 : 9) * (size_t)nthr;
-  // per instantiation, [0] sweeps reading invD, [1] forming the diagonal
-  static int cached_nthr[2] = {-1, -1}, cached_slots[2] = {1, 1};
-  constexpr bool kF32Fine = sizeof(T) == 4 && LVL == 0;
-  if (cached_nthr[diag] != nthr) {
-    const void *kfn;
-    // the FP32 fine level sizes every mode's x-march for two workgroups per
-    // CU, the diagonal-forming sweep's occupancy (a third, which the
-    // residual's registers and LDS would allow, shortened the march: 43.1
-    // against 38.5 us per residual at 256x128x128)
-    if constexpr (kF32Fine)
-      kfn = (const void *)k_tile_sweep_f32<kModeJacobiDiag, false>;
-    else if constexpr (LVL == 0)
-      kfn = diag ? (const void *)k_tile_sweep<T, LVL, kModeJacobiDiag, false>
-                 : (const void *)k_tile_sweep<T, LVL, kModeJacobi, false>;
-    else
-      kfn = (const void *)k_tile_sweep<T, LVL, kModeJacobi, false>;
-    cached_slots[diag] =
-        wg_per_cu(kfn, bs, kF32Fine ? sizeof(T) * 2 * 11 * (size_t)nthr : shm);
-    cached_nthr[diag] = nthr;
-  }
-  tile_x(s, L, nx_fixed, (int64_t)cached_slots[diag] * device_cus());
-  TileArgs a;
   a.nelx = L.nelx;
   a.nely = L.nely;
   a.nelz = L.nelz;
   a.wy = L.wy;
   a.wz = L.wz;
-  a.few = LVL == 0 ? g.ewy : L.nely + 1;  // level 1: the slots of k_level1_moduli
-  a.fez = LVL == 0 ? g.ewz : L.nelz + 1;
+  a.out_bytes = (uint32_t)(sizeof(T) * 3 * L.nodes());
+  a.e_bytes = (uint32_t)(sizeof(T) * nmod);
+  a.stream_out = 0;
+  return true;
+}
+
+static void tile_args_shape(const TileShape &s, TileArgs &a) {
   a.TY = s.TY;
   a.TZ = s.TZ;
   a.NX = s.NX;
   a.nty = s.nty;
-  a.out_bytes = (uint32_t)(sizeof(T) * 3 * L.nodes());
-  dim3 grid(s.ntx, s.nty * s.ntz);
+}
+
+template <typename T>
+static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out, const T *b,
+                       const T *invD, T omega, int bcsym, double *dotp = nullptr,
+                       int dot_cap = 0) {
+  init_coef();
+  const Level &L = g.lv[0];
+  TileArgs a;
+  if (!tile_args<T>(L, g.nelem, g_coef.ok0, a)) return 0;
+  a.few = g.ewy;
+  a.fez = g.ewz;
+  // the diagonal from the moduli needs a KE whose diagonal is one value per
+  // component
+  if (mode == kModeJacobiDiag && !g_coef.diag0) mode = kModeJacobi;
+  const bool diag = mode == kModeJacobiDiag;
+  const size_t shm = sizeof(T) * march_lds_values(diag) * (size_t)kMarchThreads;
+  // workgroups per CU, [0] sweeps reading invD, [1] forming the diagonal
+  static int per_cu[2] = {0, 0};
+  if (!per_cu[diag])
+    per_cu[diag] = wg_per_cu(diag ? (const void *)k_fine_march<T, kModeJacobiDiag, false>
+                                  : (const void *)k_fine_march<T, kModeJacobi, false>,
+                             kMarchThreads, shm);
+  const int64_t slots = (int64_t)per_cu[diag] * device_cus();
+  int nx_fixed = 0;
+  TileShape s = march_shape(L, slots, sizeof(T) == 8, nx_fixed);
+  tile_x(s, L, nx_fixed, slots);
+  tile_args_shape(s, a);
+  // Past the caches where the sweep's vectors and moduli exceed the memory-side
+  // cache (256 MB): the output would push out what the next workgroups read
+  // (256x128x128 in FP64, 341 MB: 77.3 against 84.1 us per sweep; below, where
+  // the next sweep reads it from that cache, the same store costs: FP32, 171
+  // MB, 42.7 against 34.5 us).
+  const int64_t vectors = mode == kModeApply ? 2 : mode == kModeJacobi ? 4 : 3;
+  a.stream_out = vectors * a.out_bytes + a.e_bytes > (int64_t(256) << 20);
+  const dim3 grid(s.ntx, s.nty * s.ntz);
+  const int bs = ((s.TY + 1) * (s.TZ + 1) + 63) / 64 * 64;
   const int nwg = s.ntx * s.nty * s.ntz;
   if (dotp && nwg > dot_cap) dotp = nullptr;
-  std::conditional_t<LVL == 0, Blocks<T>, K1Vals<T>> B;
-  if constexpr (LVL == 0) {
-    if constexpr (sizeof(T) == 8) B = g_coef.b64; else B = g_coef.b32;
-  } else {
-    if constexpr (sizeof(T) == 8) B = g_coef.k64; else B = g_coef.k32;
-  }
-#define T3D_LAUNCH(M, S)                                                                      \
-  do {                                                                                       \
-    if constexpr (kF32Fine)                                                                  \
-      hipLaunchKernelGGL((k_tile_sweep_f32<M, S>), grid, dim3(bs), shm, stream(), a, B, E,   \
-                         in, out, b, invD, omega, g.fixmask[LVL], g.fixplane[LVL], dotp);    \
-    else                                                                                     \
-      hipLaunchKernelGGL((k_tile_sweep<T, LVL, M, S>), grid, dim3(bs), shm, stream(), a, B, \
-                         E, in, out, b, invD, omega, g.fixmask[LVL], g.fixplane[LVL], dotp); \
-  } while (0)
+  const auto B = fine_values<T>();
+#define T3D_LAUNCH(M, S)                                                                  \
+  hipLaunchKernelGGL((k_fine_march<T, M, S>), grid, dim3(bs), shm, stream(), a, B, E, in, \
+                     out, b, invD, omega, g.fixmask[0], g.fixplane[0], dotp)
   if (bcsym) {
     if (mode == kModeApply) T3D_LAUNCH(kModeApply, true);
     else if (mode == kModeJacobi) T3D_LAUNCH(kModeJacobi, true);
     else if (mode == kModeResidual) T3D_LAUNCH(kModeResidual, true);
-    else if constexpr (LVL == 0) T3D_LAUNCH(kModeJacobiDiag, true);
+    else T3D_LAUNCH(kModeJacobiDiag, true);
   } else {
     if (mode == kModeApply) T3D_LAUNCH(kModeApply, false);
     else if (mode == kModeJacobi) T3D_LAUNCH(kModeJacobi, false);
     else if (mode == kModeResidual) T3D_LAUNCH(kModeResidual, false);
-    else if constexpr (LVL == 0) T3D_LAUNCH(kModeJacobiDiag, false);
+    else T3D_LAUNCH(kModeJacobiDiag, false);
   }
 #undef T3D_LAUNCH
   return dotp ? nwg : 0;
 }
 
 template <typename T>
+static void run_level1(const DevGrid &g, int mode, const T *Eh, const T *in, T *out,
+                          const T *b, const T *invD, T omega, int bcsym) {
+  init_coef();
+  const Level &L = g.lv[1];
+  TileArgs a;
+  if (!tile_args<T>(L, level1_moduli_count(g), g_coef.ok1, a)) return;
+  a.few = L.nely + 1;  // the slots of k_level1_moduli
+  a.fez = L.nelz + 1;
+  if (mode == kModeJacobiDiag) mode = kModeJacobi;
+  int nx_fixed = 0;
+  TileShape s = level1_shape(L, (int)sizeof(T), nx_fixed);
+  const int nthr = s.TY * s.TZ, bs = (nthr + 63) / 64 * 64;
+  const size_t shm = sizeof(T) * 2 * 9 * (size_t)nthr;
+  static int cached_nthr = -1, cached_per_cu = 1;
+  if (cached_nthr != nthr) {
+    cached_per_cu = wg_per_cu((const void *)k_level1_sweep<T, kModeJacobi, false>, bs, shm);
+    cached_nthr = nthr;
+  }
+  tile_x(s, L, nx_fixed, (int64_t)cached_per_cu * device_cus());
+  tile_args_shape(s, a);
+  const dim3 grid(s.ntx, s.nty * s.ntz);
+  K1Vals<T> B;
+  if constexpr (sizeof(T) == 8) B = g_coef.k64; else B = g_coef.k32;
+#define T3D_LAUNCH(M, S)                                                                    \
+  hipLaunchKernelGGL((k_level1_sweep<T, M, S>), grid, dim3(bs), shm, stream(), a, B, Eh, in, \
+                     out, b, invD, omega, g.fixmask[1], g.fixplane[1])
+  if (bcsym) {
+    if (mode == kModeApply) T3D_LAUNCH(kModeApply, true);
+    else if (mode == kModeJacobi) T3D_LAUNCH(kModeJacobi, true);
+    else T3D_LAUNCH(kModeResidual, true);
+  } else {
+    if (mode == kModeApply) T3D_LAUNCH(kModeApply, false);
+    else if (mode == kModeJacobi) T3D_LAUNCH(kModeJacobi, false);
+    else T3D_LAUNCH(kModeResidual, false);
+  }
+#undef T3D_LAUNCH
+}
+
+template <typename T>
 void launch_fine_tile(const DevGrid &g, int mode, const T *E, const T *in, T *out,
                       const T *b, const T *invD, T omega, int bcsym) {
-  launch_tile<T, 0>(g, mode, E, in, out, b, invD, omega, bcsym);
+  run_fine<T>(g, mode, E, in, out, b, invD, omega, bcsym);
 }
 
 int launch_fine_apply_dot(const DevGrid &g, const double *E, const double *p, double *q,
                           int bcsym, double *partials, int cap) {
-  return launch_tile<double, 0>(g, kModeApply, E, p, q, nullptr, nullptr, 0.0, bcsym, partials,
+  return run_fine<double>(g, kModeApply, E, p, q, nullptr, nullptr, 0.0, bcsym, partials,
                                 cap);
 }
 
 template <typename T>
 int launch_fine_tile_sweep_dot(const DevGrid &g, const T *E, const T *in, T *out, const T *b,
                                const T *invD, T omega, int bcsym, double *partials, int cap) {
-  return launch_tile<T, 0>(g, kModeJacobiDiag, E, in, out, b, invD, omega, bcsym, partials, cap);
+  return run_fine<T>(g, kModeJacobiDiag, E, in, out, b, invD, omega, bcsym, partials, cap);
 }
 template int launch_fine_tile_sweep_dot<float>(const DevGrid &, const float *, const float *,
                                                float *, const float *, const float *, float, int,
@@ -1091,7 +1453,7 @@ template int launch_fine_tile_sweep_dot<double>(const DevGrid &, const double *,
 template <typename T>
 void launch_level1_tile(const DevGrid &g, int mode, const T *Eh, const T *in, T *out,
                         const T *b, const T *invD, T omega, int bcsym) {
-  launch_tile<T, 1>(g, mode, Eh, in, out, b, invD, omega, bcsym);
+  run_level1<T>(g, mode, Eh, in, out, b, invD, omega, bcsym);
 }
 
 // Per level-1 element slot (i, k, j), i in 0..nelx+1, k in 0..nelz, j in
@@ -1196,8 +1558,7 @@ template <typename TB, typename T>
 bool launch_fine_jacobi_zero(const DevGrid &g, const TB *b, const T *E, T omega, T *out) {
   if (!tile_fine_diag_available()) return false;
   const Level &L = g.lv[0];
-  Blocks<T> B;
-  if constexpr (sizeof(T) == 8) B = g_coef.b64; else B = g_coef.b32;
+  const Blocks<T> B = fine_values<T>();
   dim3 bs(256), gs((L.wy * L.wz + 255) / 256, L.wx);
   hipLaunchKernelGGL((k_jacobi_zero_fine<TB, T>), gs, bs, 0, stream(), L.nx, L.ny, L.nz, L.wy,
                      L.wz, g.ewy, g.ewz, b, E, g.fixmask[0], B, omega, out);
