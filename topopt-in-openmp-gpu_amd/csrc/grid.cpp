@@ -243,6 +243,7 @@ void release_dev_grid(const struct gridContext *gc) {
     dfree(g->KEf[i]);
   }
   dfree(g->KE2);
+  dfree(g->KE2b);
   dfree(g->KE3);
   for (int l = 0; l < kMaxLevels; l++) dfree(g->KEdiag[l]);
   for (int i = 0; i < DevGrid::kScratchSlots; i++) dfree(g->scratch[i]);
@@ -324,6 +325,19 @@ static DevGrid *build_dev_grid(struct gridContext *gc, int nl) {
     g->KE2 = (double *)dalloc(sizeof(double) * cnt);
     T3D_HIP(hipMemcpyAsync(g->KE2, gc->precomputedKE[2], sizeof(double) * cnt,
                            hipMemcpyHostToDevice, stream()));
+    T3D_HIP(hipStreamSynchronize(stream()));
+  }
+  if (nl >= 4) {  // KE_2 as node-pair blocks for the level-2 smoother's stencil
+    std::vector<double> kb(64 * (size_t)kKeBlocks, 0.0);
+    for (int f = 0; f < 64; f++)
+      for (int a = 0; a < 8; a++)
+        for (int b = a; b < 8; b++)
+          for (int q = 0; q < 9; q++)
+            kb[(size_t)kKeBlocks * f + 9 * ke_block(a, b) + q] =
+                gc->precomputedKE[2][576 * f + 24 * (3 * a + q / 3) + 3 * b + q % 3];
+    g->KE2b = (double *)dalloc(sizeof(double) * kb.size());
+    T3D_HIP(hipMemcpyAsync(g->KE2b, kb.data(), sizeof(double) * kb.size(), hipMemcpyHostToDevice,
+                           stream()));
     T3D_HIP(hipStreamSynchronize(stream()));
   }
   if (nl >= 4) {  // level-3 sub-cell matrices: level-3 element matrices as one GEMM

@@ -117,20 +117,29 @@ __global__ __launch_bounds__(576) void k_galerkin(
 // Level-2 element matrices as one GEMM on FP64 MFMA:
 //   Ke2[e][q] = sum_{f<64} E[fine(e, f)] KE_2[f][q],  q < 576,
 // with f = 16 ii + 4 kk + jj the reference's sub-cell index
-// (local_matrix.c:283).  A workgroup owns 128 level-2 elements: their 64
-// moduli are gathered into LDS, and each wave sweeps 9 of the 36 16-column
-// tiles of KE_2, holding the tile's 64x16 slice in registers while it runs
-// over the 8 16-element row tiles (v_mfma_f64_16x16x4f64, K = 64).
-constexpr int kL2Rows = 128;
-
+// (local_matrix.c:283).  A workgroup owns kRows level-2 elements: their 64
+// moduli are gathered into LDS, and each wave sweeps every 4th of the
+// workgroup's 16-column tiles of KE_2 (36 over gridDim.y), holding the tile's
+// 64x16 slice in registers while it runs over the 16-element row tiles
+// (v_mfma_f64_16x16x4f64, K = 64).
+// Few elements leave the device idle: 16 rows per workgroup and the columns
+// over 9 or 3 workgroups took 8 us for 1024 elements and 25-28 us for 8192,
+// against 71 and 80 us with 128 rows and all columns, and 39 us for 1024 with
+// 64 rows.  From 32768 elements on the gather of the moduli, repeated by each
+// column group, and the output's bandwidth decide: 64 rows and all columns
+// took 1.0-1.2 ms for 524288 elements (2.4 GB) against 1.2-1.8 ms with 128
+// rows, 1.5-1.8 with 16 and 3 groups.
+// kCols: 576, or the kKeBlocks values of the node-pair blocks (58% of the
+// products and of the output).
+template <int kRows, int kCols>
 __global__ __launch_bounds__(256) void k_elem_level2_mfma(
     int nelx, int nely, int nelz, int few, int fez, const double *__restrict__ KE2,
     const double *__restrict__ E, double *__restrict__ Ke2) {
-  __shared__ double As[kL2Rows][65];
+  __shared__ double As[kRows][65];
   const int64_t nel = (int64_t)nelx * nely * nelz;
-  const int64_t e0 = (int64_t)blockIdx.x * kL2Rows;
+  const int64_t e0 = (int64_t)blockIdx.x * kRows;
   const int tid = threadIdx.x;
-  for (int q = tid; q < kL2Rows * 64; q += 256) {
+  for (int q = tid; q < kRows * 64; q += 256) {
     const int r = q >> 6, f = q & 63;
     const int64_t e = e0 + r;
     double v = 0.0;
@@ -145,12 +154,13 @@ __global__ __launch_bounds__(256) void k_elem_level2_mfma(
   __syncthreads();
   const int w = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
   typedef double double4_v __attribute__((ext_vector_type(4)));
-  for (int nt = w; nt < 36; nt += 4) {
+  const int ntile = kCols / 16 / gridDim.y, nt1 = (blockIdx.y + 1) * ntile;
+  for (int nt = blockIdx.y * ntile + w; nt < nt1; nt += 4) {
     double bfrag[16];
 #pragma unroll
-    for (int k = 0; k < 16; k++) bfrag[k] = KE2[(4 * k + lk) * 576 + 16 * nt + li];
+    for (int k = 0; k < 16; k++) bfrag[k] = KE2[(4 * k + lk) * kCols + 16 * nt + li];
 #pragma unroll 2
-    for (int mt = 0; mt < kL2Rows / 16; mt++) {
+    for (int mt = 0; mt < kRows / 16; mt++) {
       double4_v acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int k = 0; k < 16; k++)
@@ -159,18 +169,37 @@ __global__ __launch_bounds__(256) void k_elem_level2_mfma(
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int64_t e = e0 + 16 * mt + lk + 4 * v;
-        if (e < nel) Ke2[e * 576 + 16 * nt + li] = acc[v];
+        if (e < nel) Ke2[e * kCols + 16 * nt + li] = acc[v];
       }
     }
   }
+}
+
+template <int kCols>
+static void run_elem_level2(const DevGrid &g, const double *KE, const double *E, double *Ke) {
+  const Level &L = g.lv[2];
+  const int64_t nel = L.elements();
+  constexpr int kMany = kCols == 576 ? 9 : 7;  // column groups (of the 36 or 21 tiles)
+  if (nel < 32768)
+    hipLaunchKernelGGL((k_elem_level2_mfma<16, kCols>),
+                       dim3((nel + 15) / 16, nel <= 4096 ? kMany : 3), dim3(256), 0, stream(),
+                       L.nelx, L.nely, L.nelz, g.ewy, g.ewz, KE, E, Ke);
+  else
+    hipLaunchKernelGGL((k_elem_level2_mfma<64, kCols>), dim3((nel + 63) / 64), dim3(256), 0,
+                       stream(), L.nelx, L.nely, L.nelz, g.ewy, g.ewz, KE, E, Ke);
+}
+
+bool launch_elem_level2_blocks(const DevGrid &g, const double *E, double *Ke2b) {
+  if (!g.KE2b) return false;
+  run_elem_level2<kKeBlocks>(g, g.KE2b, E, Ke2b);
+  return true;
 }
 
 void launch_elem_level2(const DevGrid &g, const double *E, double *Ke2) {
   const Level &L = g.lv[2];
   const int64_t nel = L.elements();
   if (g.KE2) {
-    hipLaunchKernelGGL(k_elem_level2_mfma, dim3((nel + kL2Rows - 1) / kL2Rows), dim3(256), 0,
-                       stream(), L.nelx, L.nely, L.nelz, g.ewy, g.ewz, g.KE2, E, Ke2);
+    run_elem_level2<576>(g, g.KE2, E, Ke2);
     return;
   }
   hipLaunchKernelGGL((k_galerkin<0>), dim3(nel), dim3(576), 0, stream(), L.nelx,
@@ -255,22 +284,14 @@ void launch_elem_galerkin(const DevGrid &g, int l, const double *Kchild, double 
 // S[(nb*9 + r*3 + c) * nint + n]; symmetric elimination of fixed DOFs.
 // bc_symmetric = 0 keeps the columns of fixed DOFs and only replaces fixed
 // rows by identity rows (the matrix-free convention, stencil_methods.c:515-518).
-// S32: an FP32 copy written alongside when given.
-// HALF: the symmetric half layout of a matrix with symmetric elimination
-// (kHalfPlanes planes): the 13 neighbours nb = 14..26 as full 3x3 blocks at
-// planes (nb-14)*9 + 3r + c, the centre's upper triangle r <= c at planes
-// 117 + half_centre_index(r, c); one thread per stored neighbour.
 constexpr int kNsNodes = 32;
 
-template <bool HALF>
 __global__ __launch_bounds__(27 * kNsNodes) void k_node_stencil(
     int nelx, int nely, int nelz, int wy, int wz, const double *__restrict__ Ke,
-    const uint8_t *__restrict__ fix, double *__restrict__ S, float *__restrict__ S32,
-    int bc_symmetric) {
-  constexpr int kPlanes = HALF ? kHalfPlanes : 243;
-  __shared__ double tile[kPlanes * kNsNodes];
+    const uint8_t *__restrict__ fix, double *__restrict__ S, int bc_symmetric) {
+  __shared__ double tile[243 * kNsNodes];
   const int64_t nx = nelx + 1, ny = nely + 1, nz = nelz + 1, nint = nx * ny * nz;
-  const int nb = HALF ? 13 + threadIdx.x : threadIdx.x;
+  const int nb = threadIdx.x;
   const int64_t n0 = (int64_t)blockIdx.x * kNsNodes;
   const int64_t n = n0 + threadIdx.y;
   const int nloc = (int)min((int64_t)kNsNodes, nint - n0);
@@ -302,43 +323,134 @@ __global__ __launch_bounds__(27 * kNsNodes) void k_node_stencil(
           if (fr || fc) v[3 * r + c] = (nb == 13 && r == c) ? 1.0 : 0.0;
         }
     }
-    if (!HALF) {
 #pragma unroll
-      for (int q = 0; q < 9; q++) tile[(nb * 9 + q) * kNsNodes + threadIdx.y] = v[q];
-    } else if (nb > 13) {
-#pragma unroll
-      for (int q = 0; q < 9; q++) tile[((nb - 14) * 9 + q) * kNsNodes + threadIdx.y] = v[q];
-    } else {
-#pragma unroll
-      for (int r = 0; r < 3; r++)
-#pragma unroll
-        for (int c = r; c < 3; c++)
-          tile[(117 + half_centre_index(r, c)) * kNsNodes + threadIdx.y] = v[3 * r + c];
-    }
+    for (int q = 0; q < 9; q++) tile[(nb * 9 + q) * kNsNodes + threadIdx.y] = v[q];
   }
   __syncthreads();
   const int tid = threadIdx.y * blockDim.x + threadIdx.x;
-  for (int e = tid; e < kPlanes * kNsNodes; e += blockDim.x * kNsNodes) {
+  for (int e = tid; e < 243 * kNsNodes; e += blockDim.x * kNsNodes) {
     const int q = e / kNsNodes, nn = e % kNsNodes;
-    if (nn < nloc) {
-      const double val = tile[e];
-      S[(int64_t)q * nint + n0 + nn] = val;
-      if (S32) S32[(int64_t)q * nint + n0 + nn] = (float)val;
-    }
+    if (nn < nloc) S[(int64_t)q * nint + n0 + nn] = tile[e];
   }
 }
 
 void launch_node_stencil(const DevGrid &g, int l, const double *Ke, double *S,
-                         int bc_symmetric, float *S32, bool half) {
+                         int bc_symmetric) {
   const Level &L = g.lv[l];
   const int64_t nint = L.interior_nodes();
-  const dim3 grid((unsigned)((nint + kNsNodes - 1) / kNsNodes));
-  if (half)
-    hipLaunchKernelGGL((k_node_stencil<true>), grid, dim3(14, kNsNodes), 0, stream(), L.nelx,
-                       L.nely, L.nelz, L.wy, L.wz, Ke, g.fixmask[l], S, S32, 1);
+  hipLaunchKernelGGL(k_node_stencil, dim3((unsigned)((nint + kNsNodes - 1) / kNsNodes)),
+                     dim3(27, kNsNodes), 0, stream(), L.nelx, L.nely, L.nelz, L.wy, L.wz, Ke,
+                     g.fixmask[l], S, bc_symmetric);
+}
+
+// The symmetric half layout of a matrix with symmetric elimination
+// (kHalfPlanes planes): the 13 neighbours nb = 14..26 as full 3x3 blocks at
+// planes (nb-14)*9 + 3r + c, the centre's upper triangle r <= c at planes
+// 117 + half_centre_index(r, c); with S32 the FP32 form of the V-cycle, and of
+// S the centre's diagonal, which the inverse diagonal is formed from.
+// A node's 14 blocks are sums over 1 to 8 of its elements, 36 element blocks in
+// all, each element block in the sum of one node.  A workgroup has a thread
+// per element block of its 16 nodes: all of them are loaded at once, meet in
+// LDS, and are summed in the order of the elements and written, 16 nodes to a
+// plane.  Bound by the loads, 72 bytes each from a line of its own (level 2 of
+// 512x256x256: 1.4 GB of blocks, XX us; a thread per neighbour, which loaded one
+// element after the other, 24 bytes at a time, and wrote S in FP64 too, 2260).
+constexpr int kHsNodes = 16, kHsItems = 36;
+// first item of neighbour nb = 13 (the node itself) .. 26, 27: their number
+__device__ __forceinline__ int half_first(int nb) {
+  constexpr uint8_t kFirst[15] = {0, 8, 12, 14, 18, 20, 21, 23, 24, 26, 30, 32, 33, 35, 36};
+  return kFirst[nb - 13];
+}
+
+template <bool BLOCKS>
+__global__ __launch_bounds__(kHsNodes *kHsItems) void k_node_stencil_half(
+    int nelx, int nely, int nelz, int wy, int wz, const double *__restrict__ Ke,
+    const uint8_t *__restrict__ fix, double *__restrict__ S, float *__restrict__ S32,
+    uint32_t nblk) {
+  __shared__ double item[kHsItems * 9 * kHsNodes];  // [item][3 r + c][node]
+  __shared__ uint8_t mask[14 * kHsNodes];           // fixed DOFs of neighbour nb - 13
+  // contiguous eighths of the nodes to the XCDs: a plane's line is written by
+  // workgroups of one
+  const uint32_t xcd = blockIdx.x & 7u;
+  const uint32_t blk = xcd * (nblk >> 3) + min(xcd, nblk & 7u) + (blockIdx.x >> 3);
+  const int nx = nelx + 1, ny = nely + 1, nz = nelz + 1;
+  const int64_t nint = (int64_t)nx * ny * nz, n0 = (int64_t)blk * kHsNodes;
+  const int nloc = (int)min((int64_t)kHsNodes, nint - n0);
+  const int nn = threadIdx.x, it = threadIdx.y;
+  {
+    int nb = 13;
+    while (it >= half_first(nb + 1)) nb++;
+    const int64_t n = min(n0 + nn, nint - 1);
+    const int j = (int)(n % ny), k = (int)((n / ny) % nz), i = (int)(n / ((int64_t)ny * nz));
+    const int dx = nb / 9 - 1, dz = (nb / 3) % 3 - 1, dy = nb % 3 - 1;
+    // the item's element: offset -1 or 0 per direction; free where the
+    // neighbour's offset is 0
+    int t = it - half_first(nb), d[3] = {dx, dy, dz}, ofs[3];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      const bool free = d[q] == 0;
+      ofs[q] = (free ? (t & 1) : d[q] > 0) ? 0 : -1;
+      if (free) t >>= 1;
+    }
+    const int ie = i + ofs[0], je = j + ofs[1], ke = k + ofs[2];
+    const bool in = ie >= 0 && ie < nelx && je >= 0 && je < nely && ke >= 0 && ke < nelz;
+    const int a = cn_of(-ofs[0], -ofs[1], -ofs[2]);
+    const int b = cn_of(dx - ofs[0], dy - ofs[1], dz - ofs[2]);
+    const int64_t e = in ? ((int64_t)ie * nelz + ke) * nely + je : 0;
+    double v[9];
+    if constexpr (BLOCKS) {
+      const double *K = Ke + kKeBlocks * e + 9 * ke_block(min(a, b), max(a, b));
+#pragma unroll
+      for (int q = 0; q < 9; q++) v[q] = K[q];
+    } else {
+      const double *K = Ke + 576 * e + 72 * a + 3 * b;
+#pragma unroll
+      for (int q = 0; q < 9; q++) v[q] = K[24 * (q / 3) + q % 3];
+    }
+    const bool tr = BLOCKS && a > b;  // block (b, a) transposed
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        item[(it * 9 + 3 * r + c) * kHsNodes + nn] = in ? (tr ? v[3 * c + r] : v[3 * r + c]) : 0.0;
+    if (it == half_first(nb))  // (neighbours beyond the grid are nodes of the halo)
+      mask[(nb - 13) * kHsNodes + nn] =
+          fix[((int64_t)(i + dx + 1) * wz + (k + dz + 1)) * wy + (j + dy + 1)];
+  }
+  __syncthreads();
+  for (int o = threadIdx.y * kHsNodes + threadIdx.x; o < kHalfPlanes * kHsNodes;
+       o += kHsNodes * kHsItems) {
+    const int q = o / kHsNodes, m = o % kHsNodes;
+    if (m >= nloc) continue;
+    int nb = 13, r, c;
+    if (q < 117) {
+      nb = 14 + q / 9;
+      r = (q % 9) / 3, c = q % 3;
+    } else {  // upper triangle of the centre, row by row
+      r = q < 120 ? 0 : q < 122 ? 1 : 2;
+      c = q - (r == 0 ? 117 : r == 1 ? 119 : 120);
+    }
+    double v = 0.0;
+    for (int f = half_first(nb); f < half_first(nb + 1); f++)
+      v += item[(f * 9 + 3 * r + c) * kHsNodes + m];
+    const bool diag = nb == 13 && r == c;
+    if (((mask[m] >> r) | (mask[(nb - 13) * kHsNodes + m] >> c)) & 1) v = diag ? 1.0 : 0.0;
+    if (!S32 || diag) S[(int64_t)q * nint + n0 + m] = v;
+    if (S32) S32[(int64_t)q * nint + n0 + m] = (float)v;
+  }
+}
+
+void launch_node_stencil_half(const DevGrid &g, int l, const double *Ke, double *S, float *S32,
+                              bool blocks) {
+  const Level &L = g.lv[l];
+  const uint32_t nblk = (uint32_t)((L.interior_nodes() + kHsNodes - 1) / kHsNodes);
+  const dim3 bs(kHsNodes, kHsItems);
+  if (blocks)
+    hipLaunchKernelGGL(k_node_stencil_half<true>, dim3(nblk), bs, 0, stream(), L.nelx, L.nely,
+                       L.nelz, L.wy, L.wz, Ke, g.fixmask[l], S, S32, nblk);
   else
-    hipLaunchKernelGGL((k_node_stencil<false>), grid, dim3(27, kNsNodes), 0, stream(), L.nelx,
-                       L.nely, L.nelz, L.wy, L.wz, Ke, g.fixmask[l], S, S32, bc_symmetric);
+    hipLaunchKernelGGL(k_node_stencil_half<false>, dim3(nblk), bs, 0, stream(), L.nelx, L.nely,
+                       L.nelz, L.wy, L.wz, Ke, g.fixmask[l], S, S32, nblk);
 }
 
 // the assembled coarsest level into the coarse factor's np x np storage

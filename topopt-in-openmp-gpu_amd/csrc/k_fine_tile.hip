@@ -770,7 +770,7 @@ __device__ __forceinline__ void pin(T &x) {
 }
 
 // The fine level.  A workgroup has a thread per node of its (TY + 1) x (TZ + 1)
-// node tile, up to 255 nodes in 4 waves; each loads its own node of the plane
+// node tile, up to 255 nodes in FP64 and 511 in FP32; each loads its own node of the plane
 // and hands it on through LDS with the exchange of the element's corners, under
 // the same barrier, and works on the element whose upper corner (j, k) is its
 // node (none for the tile's lower edges).  Every LDS array is [value][thread],
@@ -779,12 +779,19 @@ __device__ __forceinline__ void pin(T &x) {
 // every lane forms its node's row, and the store decides by its offset.
 //
 // What bounds it: the arithmetic in FP32 (about 230 instructions per element,
-// of 4 cycles each, and 170 MB per sweep at 257x129x129 nodes: 34.5 us), the
+// of 4 cycles each, and 170 MB per sweep at 257x129x129 nodes: 33-35 us), the
 // memory in FP64 (341 MB, more than the memory-side cache holds).  Before,
 // with a thread per element that loaded the four nodes of its face through the
 // first-level cache, all 45 values of the blocks and masks at every node: 40.0
-// us and, FP64, 101 us per sweep and 72.5 us per apply, now 77.3 and 59.5.
-constexpr int kMarchThreads = 256;
+// us and, FP64, 101 us per sweep and 72.5 us per apply, now 79 and 55-60.  At
+// 513x257x257 nodes FP32 317-326 -> 293-298 us, FP64 770 -> 661 and 636 -> 489.
+// (FP32 in workgroups of 4 waves: 34.6 and 356 us.)
+// threads of a workgroup: two of 8 waves (FP32, 88 registers) or three of 4
+// waves (FP64, 168 registers) share a CU
+template <typename T>
+constexpr int march_threads() {
+  return sizeof(T) == 4 ? 512 : 256;
+}
 
 // LDS values per thread: two buffers of the exchange (9 corners, in the
 // diagonal-forming sweep the modulus too) and of the plane's 3 components
@@ -795,9 +802,9 @@ __device__ __forceinline__ void fine_march_body(
     TileArgs a, Blocks<T> B, const T *__restrict__ E, const T *__restrict__ in,
     T *__restrict__ out, const T *__restrict__ b, const T *__restrict__ invD, T omega,
     const uint8_t *__restrict__ fix, const int *__restrict__ fixplane,
-    double *__restrict__ dotp) {
+    double *__restrict__ dotp, float *__restrict__ out32) {
   constexpr bool kDiag = MODE == kModeJacobiDiag;
-  constexpr int N = kMarchThreads, XV = kDiag ? 10 : 9;
+  constexpr int N = march_threads<T>(), XV = kDiag ? 10 : 9;
   extern __shared__ unsigned char smem_raw[];
   T *xch = reinterpret_cast<T *>(smem_raw);  // [2][XV][N]; slot N-1: zeros
   T *nodes = xch + 2 * XV * N;               // [2][3][N]
@@ -1001,6 +1008,10 @@ __device__ __forceinline__ void fine_march_body(
     const __amdgpu_buffer_rsrc_t ro = rsrc(out, emit ? a.out_bytes : 0u);
     if (a.stream_out) store_node<kNt>(ro, vout, o, (uint32_t)i * sv);
     else store_node(ro, vout, o, (uint32_t)i * sv);
+    if (MODE == kModeResidual && sizeof(T) == 8 && out32) {  // the FP32 copy too
+      const float o32[3] = {(float)o[0], (float)o[1], (float)o[2]};
+      store_node(rsrc(out32, emit ? a.out_bytes / 2 : 0u), vout / 2, o32, (uint32_t)i * sv / 2);
+    }
     load_node(i + 1);
   };
 
@@ -1054,13 +1065,14 @@ __device__ __forceinline__ void fine_march_body(
 }
 
 template <typename T, int MODE, bool BCSYM>
-__global__ __launch_bounds__(kMarchThreads)
-    __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 3))) void k_fine_march(
+__global__ __launch_bounds__(march_threads<T>())
+    __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 3))) void k_fine_march(
     TileArgs a, Blocks<T> B, const T *__restrict__ E, const T *__restrict__ in,
     T *__restrict__ out, const T *__restrict__ b, const T *__restrict__ invD, T omega,
     const uint8_t *__restrict__ fix, const int *__restrict__ fixplane,
-    double *__restrict__ dotp) {
-  fine_march_body<T, MODE, BCSYM>(a, B, E, in, out, b, invD, omega, fix, fixplane, dotp);
+    double *__restrict__ dotp, float *__restrict__ out32) {
+  fine_march_body<T, MODE, BCSYM>(a, B, E, in, out, b, invD, omega, fix, fixplane, dotp,
+                                  out32);
 }
 
 template <typename T, int MODE, bool BCSYM>
@@ -1239,17 +1251,18 @@ static int64_t tile_x(TileShape &s, const Level &L, int nx_fixed, int64_t slots)
 // FP64, 23 x 9 columns ran a sweep in 81.6 us, 24 x 9 in 83.8 us, 20 x 11 in
 // 85.5 us, 17 x 12 in 84.4 us, 17 x 13 in 87.9 us, 22 x 10, whose 97 tiles
 // leave 7 slabs instead of 8, in 93.1 us, 15 x 15 and 26 x 8 likewise in 104
-// us and 9 x 23, short rows, in 93.5 us; in FP32 17 x 13 in 35.2-36.7, 20 x 11
-// in 34.4-35.6, 23 x 9 in 37.6 and 22 x 10 in 39.7 us: rows of 17 to 23 columns
-// with the cheapest launch, the longest among equals.  Tuning override:
+// us and 9 x 23, short rows, in 93.5 us; in FP32 33 x 14 in 32.7, 23 x 20 in
+// 33.7, 20 x 23 in 34.2, 45 x 10 in 34.3, 26 x 17 and 38 x 12, which cost a slab
+// more, in 36.7 and 37.6 us: rows of 17 to 23 columns, 35 in FP32, with the
+// cheapest launch, the longest among equals.  Tuning override:
 // TOP3D_TILE_L0 (FP32), TOP3D_TILE_L0_F64=TY,TZ,NX (NX = 0: the march length
 // from the occupancy).
 static TileShape march_shape(const Level &L, int64_t slots, bool f64, int &nx_fixed) {
-  constexpr int kNodes = kMarchThreads - 1;
+  const int kNodes = (f64 ? march_threads<double>() : march_threads<float>()) - 1;
   TileShape best{};
   int64_t best_cost = INT64_MAX;
   nx_fixed = 0;
-  for (int ty = 17; ty <= 23; ty++) {
+  for (int ty = 17; ty <= (f64 ? 23 : 35); ty++) {
     TileShape s{};
     set_tiles(s, L, ty, kNodes / (std::min(ty, std::max(2, L.nely + 1)) + 1) - 1);
     const int64_t cost = tile_x(s, L, 0, slots);
@@ -1334,7 +1347,7 @@ static void tile_args_shape(const TileShape &s, TileArgs &a) {
 template <typename T>
 static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out, const T *b,
                        const T *invD, T omega, int bcsym, double *dotp = nullptr,
-                       int dot_cap = 0) {
+                       int dot_cap = 0, float *out32 = nullptr) {
   init_coef();
   const Level &L = g.lv[0];
   TileArgs a;
@@ -1345,25 +1358,30 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
   // component
   if (mode == kModeJacobiDiag && !g_coef.diag0) mode = kModeJacobi;
   const bool diag = mode == kModeJacobiDiag;
-  const size_t shm = sizeof(T) * march_lds_values(diag) * (size_t)kMarchThreads;
+  const size_t shm = sizeof(T) * march_lds_values(diag) * (size_t)march_threads<T>();
   // workgroups per CU, [0] sweeps reading invD, [1] forming the diagonal
   static int per_cu[2] = {0, 0};
   if (!per_cu[diag])
     per_cu[diag] = wg_per_cu(diag ? (const void *)k_fine_march<T, kModeJacobiDiag, false>
                                   : (const void *)k_fine_march<T, kModeJacobi, false>,
-                             kMarchThreads, shm);
+                             march_threads<T>(), shm);
   const int64_t slots = (int64_t)per_cu[diag] * device_cus();
   int nx_fixed = 0;
   TileShape s = march_shape(L, slots, sizeof(T) == 8, nx_fixed);
   tile_x(s, L, nx_fixed, slots);
   tile_args_shape(s, a);
-  // Past the caches where the sweep's vectors and moduli exceed the memory-side
-  // cache (256 MB): the output would push out what the next workgroups read
-  // (256x128x128 in FP64, 341 MB: 77.3 against 84.1 us per sweep; below, where
-  // the next sweep reads it from that cache, the same store costs: FP32, 171
-  // MB, 42.7 against 34.5 us).
-  const int64_t vectors = mode == kModeApply ? 2 : mode == kModeJacobi ? 4 : 3;
-  a.stream_out = vectors * a.out_bytes + a.e_bytes > (int64_t(256) << 20);
+  // Past the caches where the launch reads no more than the memory-side cache
+  // holds (256 MB) and with its output exceeds it: the output would push out
+  // what the next launch reads again.  FP64, repeated: sweep of 256x128x128 (238
+  // MB read, 341 in all) 79.5 against 84 us, apply of 320x128x128 (171 and 297
+  // MB) 65 against 78; where the reads do not fit the store is slower, 113
+  // against 110 us per sweep of 320x128x128 (297 and 424 MB), 218 against 200
+  // per apply of 384x192x192 (465 and 807), as where all fits, 42.7 against 34.5
+  // us per FP32 sweep of 256x128x128 (171 MB in all).
+  const int64_t cache = int64_t(256) << 20;
+  const int64_t reads =
+      (mode == kModeApply ? 1 : mode == kModeJacobi ? 3 : 2) * (int64_t)a.out_bytes + a.e_bytes;
+  a.stream_out = reads <= cache && reads + a.out_bytes > cache;
   const dim3 grid(s.ntx, s.nty * s.ntz);
   const int bs = ((s.TY + 1) * (s.TZ + 1) + 63) / 64 * 64;
   const int nwg = s.ntx * s.nty * s.ntz;
@@ -1371,7 +1389,7 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
   const auto B = fine_values<T>();
 #define T3D_LAUNCH(M, S)                                                                  \
   hipLaunchKernelGGL((k_fine_march<T, M, S>), grid, dim3(bs), shm, stream(), a, B, E, in, \
-                     out, b, invD, omega, g.fixmask[0], g.fixplane[0], dotp)
+                     out, b, invD, omega, g.fixmask[0], g.fixplane[0], dotp, out32)
   if (bcsym) {
     if (mode == kModeApply) T3D_LAUNCH(kModeApply, true);
     else if (mode == kModeJacobi) T3D_LAUNCH(kModeJacobi, true);
@@ -1430,6 +1448,12 @@ template <typename T>
 void launch_fine_tile(const DevGrid &g, int mode, const T *E, const T *in, T *out,
                       const T *b, const T *invD, T omega, int bcsym) {
   run_fine<T>(g, mode, E, in, out, b, invD, omega, bcsym);
+}
+
+// r = b - K u and its FP32 copy when r32 is given
+void launch_fine_tile_residual(const DevGrid &g, const double *E, const double *u, double *r,
+                               float *r32, const double *b, int bcsym) {
+  run_fine<double>(g, kModeResidual, E, u, r, b, nullptr, 0.0, bcsym, nullptr, 0, r32);
 }
 
 int launch_fine_apply_dot(const DevGrid &g, const double *E, const double *p, double *q,

@@ -42,7 +42,8 @@ __device__ __forceinline__ T finish(int mode, T kin, T in, T b, T invD, T omega,
 template <typename T, typename TX>
 __global__ void k_young(int nelx, int nely, int nelz, int few, int fez,
                         int64_t nelem, double E0, double Emin,
-                        const TX *__restrict__ x, T *__restrict__ E) {
+                        const TX *__restrict__ x, T *__restrict__ E,
+                        float *__restrict__ E32) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= nelem) return;
   const int j = (int)(e % few);
@@ -55,21 +56,22 @@ __global__ void k_young(int nelx, int nely, int nelz, int few, int fez,
     v = (T)(Emin + (double)x3 * (E0 - Emin));
   }
   E[e] = v;
+  if (E32) E32[e] = (float)v;
 }
 
 template <typename T>
-void launch_young(const DevGrid &g, const double *x, T *E) {
+void launch_young(const DevGrid &g, const double *x, T *E, float *E32) {
   const int bs = 256;
   const int64_t nb = (g.nelem + bs - 1) / bs;
   hipLaunchKernelGGL((k_young<T, double>), dim3(nb), dim3(bs), 0, stream(), g.nelx,
-                     g.nely, g.nelz, g.ewy, g.ewz, g.nelem, g.E0, g.Emin, x, E);
+                     g.nely, g.nelz, g.ewy, g.ewz, g.nelem, g.E0, g.Emin, x, E, E32);
 }
 template <typename T>
 void launch_young_float_input(const DevGrid &g, const float *x, T *E) {
   const int bs = 256;
   const int64_t nb = (g.nelem + bs - 1) / bs;
   hipLaunchKernelGGL((k_young<T, float>), dim3(nb), dim3(bs), 0, stream(), g.nelx,
-                     g.nely, g.nelz, g.ewy, g.ewz, g.nelem, g.E0, g.Emin, x, E);
+                     g.nely, g.nelz, g.ewy, g.ewz, g.nelem, g.E0, g.Emin, x, E, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -183,6 +185,16 @@ void launch_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
   else
     hipLaunchKernelGGL((k_fine<T, kResidual>), gs, bs, 0, stream(), a, KE, E, in, out,
                        b, invD, omega, g.fixmask[0], bcsym);
+}
+
+void launch_fine_residual(const DevGrid &g, const double *E, const double *u, double *r,
+                          float *r32, const double *b, int bcsym) {
+  if (!use_node_kernel()) {
+    launch_fine_tile_residual(g, E, u, r, r32, b, bcsym);
+    return;
+  }
+  launch_fine<double>(g, kResidual, E, u, r, b, nullptr, 0.0, bcsym);
+  if (r32) launch_convert<float, double>(g.lv[0].ndof, r, r32);
 }
 
 // A fine Jacobi sweep that also writes per-workgroup partial sums of b . out
@@ -842,7 +854,7 @@ void launch_invdiag_stencil(const DevGrid &g, int l, const double *S, T *invD) {
 // ---------------------------------------------------------------------------
 // explicit instantiations
 #define T3D_INST(T)                                                                      \
-  template void launch_young<T>(const DevGrid &, const double *, T *);                   \
+  template void launch_young<T>(const DevGrid &, const double *, T *, float *);          \
   template void launch_young_float_input<T>(const DevGrid &, const float *, T *);        \
   template void launch_fine<T>(const DevGrid &, int, const T *, const T *, T *,          \
                                const T *, const T *, T, int);                            \

@@ -139,10 +139,9 @@ void SolverState::release() {
 // per-solve set-up (stencil_solvers.c:283-302): the fine levels on the
 // library stream
 bool SolverState::setup_main(const double *x) {
-  launch_young<double>(*g, x, E64);
+  launch_young<double>(*g, x, E64, mixed ? E32 : nullptr);
   // the second stream needs only E64
   if (!T3D_HIP(hipEventRecord(ev_base, stream()))) return false;
-  if (mixed) launch_convert<float, double>(g->nelem, E64, E32);
   eh1_set = false;
   if (nl >= 2 && Eh1 && tile_level1_available()) {
     if (mixed) launch_level1_moduli<float>(*g, E32, (float *)Eh1);
@@ -184,7 +183,7 @@ bool SolverState::setup_aux() {
         if (!T3D_HIP(hipEventRecord(ev_ke[l], aux))) return false;
       } else {
         // the coarsest level: the full stencil for its dense assembly
-        launch_node_stencil(*g, l, Ke[l], S64[l], 1, nullptr, false);
+        launch_node_stencil(*g, l, Ke[l], S64[l], 1);
         launch_invdiag_stencil<double>(*g, l, S64[l], invD64[l]);
       }
     }
@@ -193,23 +192,30 @@ bool SolverState::setup_aux() {
     // follow it, so that their end is the factor's
     coarse.factor_async(mixed, aux3);
     if (!T3D_HIP(hipEventRecord(ev_coarse, aux3))) return false;
+  }
+  {
     // the fine inverse diagonal is not read by the fine sweeps when they form
-    // it from E; it is still filled in for callers of the SolverDataBuffer
+    // it from E; it is still filled in for callers of the SolverDataBuffer,
+    // after the last rows of W (beside them it delayed the first coarse solve)
+    StreamScope on_aux3(aux3);
     if (fine_sweep_forms_diagonal() && !launch_fine_invdiag(*g, E64, invD64[0]))
       launch_invdiag_mf<double>(*g, 0, E64, invD64[0]);
-    if (!T3D_HIP(hipEventRecord(ev_done, aux))) return false;
+    if (!T3D_HIP(hipEventRecord(ev_done, aux3))) return false;
   }
   {
     StreamScope on_aux2(aux2);
+    bool blocks2 = false;  // the level-2 matrices as node-pair blocks
     if (direct3) {
       if (!T3D_HIP(hipStreamWaitEvent(aux2, ev_base, 0))) return false;
-      launch_elem_level2(*g, E64, Ke[2]);
+      blocks2 = launch_elem_level2_blocks(*g, E64, Ke[2]);
+      if (!blocks2) launch_elem_level2(*g, E64, Ke[2]);
     }
     // smoother levels: the symmetric half layout (and its FP32 copy for the
     // mixed V-cycle)
     for (int l = 2; l < nl - 1; l++) {
       if (!(direct3 && l == 2) && !T3D_HIP(hipStreamWaitEvent(aux2, ev_ke[l], 0))) return false;
-      launch_node_stencil(*g, l, Ke[l], S64[l], 1, mixed ? S32[l] : nullptr, true);
+      launch_node_stencil_half(*g, l, Ke[l], S64[l], mixed ? S32[l] : nullptr,
+                               l == 2 && blocks2);
       launch_invdiag_half<double>(*g, l, S64[l], invD64[l]);
       if (mixed) launch_convert<float, double>(g->lv[l].ndof, invD64[l], invD32[l]);
     }
@@ -368,15 +374,13 @@ int SolverState::solve(const double *x, const double *b, double *u, double tol, 
   const auto t0 = clk::now();
   stats = Top3dSolveStats{};
   const int64_t n0 = g->lv[0].ndof;
-  hipMemcpyAsync(z, u, sizeof(double) * n0, hipMemcpyDeviceToDevice, stream());
   if (!setup_main(x)) {
     stats.status = top3d_last_error();
     return stats.status;
   }
-  launch_fine<double>(*g, 2, E64, z, r, b, nullptr, 0.0, bcsym);  // r = b - K z
+  launch_fine_residual(*g, E64, u, r, mixed ? v32[0][kR] : nullptr, b, bcsym);  // r = b - K u
   hscal[4] = 0.0;
   launch_dot<double>(b, b, n0, partials, scal + 4, hscal_dev + 4);  // b.b, also into hscal[4]
-  if (mixed) launch_convert<float, double>(n0, r, v32[0][kR]);
   // the coarse set-up is queued while the library stream computes r
   if (!setup_aux()) {
     hipStreamSynchronize(aux);
@@ -405,17 +409,17 @@ int SolverState::solve(const double *x, const double *b, double *u, double tol, 
     int nrz = rz_parts;
     if (mixed) {
       if (nrz == 0) launch_dot_rz<float>(v32[0][kR], v32[0][kZ], n0, part_rz);
-      launch_pupdate_fused<float>(n0, part_rz, nrz ? nrz : kPartRZ, scal, p, v32[0][kZ],
+      launch_pupdate_fused<float>(n0, part_rz, nrz ? nrz : kPartRR, scal, p, v32[0][kZ],
                                   iter == 0, u);
     } else {
       if (nrz == 0) launch_dot_rz<double>(r, z, n0, part_rz);
-      launch_pupdate_fused<double>(n0, part_rz, nrz ? nrz : kPartRZ, scal, p, z, iter == 0, u);
+      launch_pupdate_fused<double>(n0, part_rz, nrz ? nrz : kPartRR, scal, p, z, iter == 0, u);
     }
     // q = K p with the partial sums of p.q
     int npq = launch_fine_apply_dot(*g, E64, p, q, bcsym, part_pq, kPartPQ);
     if (npq == 0) {
       launch_dot_rz<double>(p, q, n0, part_pq);
-      npq = kPartRZ;
+      npq = kPartRR;
     }
     // r -= alpha q (and its FP32 copy), r.r (also into hscal[3]); u += alpha p
     // follows with the next p update

@@ -44,7 +44,7 @@ struct SolverState {
   int ncoarse = 0, bandwidth = 0;
   CoarseFactor coarse;
   // device scalars, reduction partials, pinned host copy
-  static constexpr int kPartRZ = 1024, kPartPQ = 1 << 16, kPartRR = 1024;
+  static constexpr int kPartRZ = 1 << 16, kPartPQ = 1 << 16, kPartRR = 1024;
   double *scal = nullptr, *partials = nullptr, *hscal = nullptr;
   double *cgpart = nullptr;  // partial sums of r.z, p.q, r.r
   double *hscal_dev = nullptr;  // device address of hscal

@@ -72,6 +72,7 @@ struct DevGrid {
   double *KE[2] = {};                  // device KE_0 (576), KE_1 (8*576)
   float *KEf[2] = {};
   double *KE2 = nullptr;               // device KE_2 (64*576), nl >= 3
+  double *KE2b = nullptr;              // its node-pair blocks a <= b (64*kKeBlocks), nl >= 4
   double *KE3 = nullptr;               // device KE_3 (512*576), nl >= 4
   double *KEdiag[kMaxLevels] = {};     // diagonals of the level-l sub-cell matrices (24 each)
   // 3x3 blocks of KE_0 in the per-component Walsh-Hadamard basis of the
@@ -102,7 +103,7 @@ void dfree(void *p);
 // ---------------------------------------------------------------------------
 // Kernel launchers.  T is double or float; all run on stream().
 template <typename T>
-void launch_young(const DevGrid &g, const double *x, T *E);
+void launch_young(const DevGrid &g, const double *x, T *E, float *E32 = nullptr);
 template <typename T>
 void launch_young_float_input(const DevGrid &g, const float *x, T *E);
 
@@ -178,6 +179,13 @@ void launch_invdiag_stencil(const DevGrid &g, int l, const double *S, T *invD);
 
 // coarse element matrices and stencils (FP64)
 void launch_elem_level2(const DevGrid &g, const double *E, double *Ke2);
+// An element matrix as its 36 3x3 blocks of the node pairs a <= b, block
+// ke_block(a, b) row-major, padded to whole 16-column tiles
+constexpr int kKeBlocks = 336;
+__host__ __device__ constexpr int ke_block(int a, int b) { return 8 * a - a * (a - 1) / 2 + b - a; }
+// the level-2 matrices in that form, kKeBlocks values per element; false if
+// the grid has no table for it
+bool launch_elem_level2_blocks(const DevGrid &g, const double *E, double *Ke2b);
 // Level-3 element matrices Ke3[e] = sum over the element's 512 fine elements
 // f of E_f KE_3[f], as a library FP64 GEMM on the moduli gathered into Eg
 // (level-3 elements x 512); false if it cannot run (no KE_3, library error).
@@ -193,7 +201,11 @@ __host__ __device__ constexpr int half_centre_index(int r, int c) {
   return r == 0 ? c : (r == 1 ? 2 + c : 5);  // (0,0..2) -> 0..2, (1,1..2) -> 3..4, (2,2) -> 5
 }
 void launch_node_stencil(const DevGrid &g, int l, const double *Ke, double *S,
-                         int bc_symmetric, float *S32 = nullptr, bool half = false);
+                         int bc_symmetric);
+// the half layout with symmetric elimination: into S, or, given S32, into S32
+// and of S the centre's diagonal planes only; blocks: Ke as kKeBlocks values
+void launch_node_stencil_half(const DevGrid &g, int l, const double *Ke, double *S, float *S32,
+                              bool blocks);
 // smoother sweep with a half-layout stencil (interior nodes only, as
 // launch_stencil_rows)
 template <typename T>
@@ -302,6 +314,11 @@ void launch_axpy_fused(int64_t n, const double *pq_part, int npart, double *scal
 // count (0 if `cap` is too small)
 // fine Jacobi sweep (diagonal from the moduli) with per-workgroup partial
 // sums of b . out; returns their count (0: none written)
+void launch_fine_tile_residual(const DevGrid &g, const double *E, const double *u, double *r,
+                               float *r32, const double *b, int bcsym);
+// r = b - K u and its FP32 copy when r32 is given
+void launch_fine_residual(const DevGrid &g, const double *E, const double *u, double *r,
+                          float *r32, const double *b, int bcsym);
 template <typename T>
 int launch_fine_tile_sweep_dot(const DevGrid &g, const T *E, const T *in, T *out, const T *b,
                                const T *invD, T omega, int bcsym, double *partials, int cap);
