@@ -349,77 +349,76 @@ void launch_node_stencil(const DevGrid &g, int l, const double *Ke, double *S,
 // 117 + half_centre_index(r, c); with S32 the FP32 form of the V-cycle, and of
 // S the centre's diagonal, which the inverse diagonal is formed from.
 // A node's 14 blocks are sums over 1 to 8 of its elements, 36 element blocks in
-// all, each element block in the sum of one node.  A workgroup has a thread
-// per element block of its 16 nodes: all of them are loaded at once, meet in
-// LDS, and are summed in the order of the elements and written, 16 nodes to a
-// plane.  Bound by the loads, 72 bytes each from a line of its own (level 2 of
-// 512x256x256: 1.4 GB of blocks, XX us; a thread per neighbour, which loaded one
-// element after the other, 24 bytes at a time, and wrote S in FP64 too, 2260).
-constexpr int kHsNodes = 16, kHsItems = 36;
-// first item of neighbour nb = 13 (the node itself) .. 26, 27: their number
-__device__ __forceinline__ int half_first(int nb) {
-  constexpr uint8_t kFirst[15] = {0, 8, 12, 14, 18, 20, 21, 23, 24, 26, 30, 32, 33, 35, 36};
-  return kFirst[nb - 13];
-}
+// all, each element block in the sum of one node: that of its first node in the
+// order x, z, y, which is the neighbours' order too.  With the element's nodes
+// numbered in that order the blocks of a node in one element are a run, so that
+// consecutive threads load consecutive values; they meet in LDS, are summed in
+// the order of the elements and written, 16 nodes to a plane.  Bound by memory
+// (level 2 of 512x256x256, 1.4 GB of blocks and 0.3 GB of stencil, beside the
+// first fine sweeps: 1.3-1.7 ms; a thread per element block took 2.9 ms, with
+// every load in a line of its own, and a thread per neighbour, which loaded one
+// element after the other, 24 bytes at a time, and wrote S in FP64 too, 2.3-2.8).
+constexpr int kHsNodes = 16, kHsThreads = 512;
+constexpr int kHsValues = 9 * 36, kHsLd = kHsValues + 1;
+// x, z, y order of the node at (x, y, z) of an element
+__host__ __device__ constexpr int ke_rank(int x, int y, int z) { return 4 * x + 2 * z + y; }
 
 template <bool BLOCKS>
-__global__ __launch_bounds__(kHsNodes *kHsItems) void k_node_stencil_half(
+__global__ __launch_bounds__(kHsThreads) void k_node_stencil_half(
     int nelx, int nely, int nelz, int wy, int wz, const double *__restrict__ Ke,
     const uint8_t *__restrict__ fix, double *__restrict__ S, float *__restrict__ S32,
     uint32_t nblk) {
-  __shared__ double item[kHsItems * 9 * kHsNodes];  // [item][3 r + c][node]
-  __shared__ uint8_t mask[14 * kHsNodes];           // fixed DOFs of neighbour nb - 13
+  __shared__ double val[kHsNodes * kHsLd];  // [node][ke_block(rank, .) of its element]
+  __shared__ int elem[kHsNodes * 8];        // [node][its rank in the element]; -1: none
+  __shared__ uint8_t mask[14 * kHsNodes];   // fixed DOFs of neighbour nb - 13
   // contiguous eighths of the nodes to the XCDs: a plane's line is written by
   // workgroups of one
   const uint32_t xcd = blockIdx.x & 7u;
   const uint32_t blk = xcd * (nblk >> 3) + min(xcd, nblk & 7u) + (blockIdx.x >> 3);
-  const int nx = nelx + 1, ny = nely + 1, nz = nelz + 1;
-  const int64_t nint = (int64_t)nx * ny * nz, n0 = (int64_t)blk * kHsNodes;
-  const int nloc = (int)min((int64_t)kHsNodes, nint - n0);
-  const int nn = threadIdx.x, it = threadIdx.y;
+  const uint32_t nx = nelx + 1, ny = nely + 1, nz = nelz + 1, nint = nx * ny * nz;
+  const uint32_t n0 = blk * kHsNodes;
+  const int nloc = (int)min((uint32_t)kHsNodes, nint - n0);
+  const int tid = threadIdx.x;
   {
-    int nb = 13;
-    while (it >= half_first(nb + 1)) nb++;
-    const int64_t n = min(n0 + nn, nint - 1);
-    const int j = (int)(n % ny), k = (int)((n / ny) % nz), i = (int)(n / ((int64_t)ny * nz));
-    const int dx = nb / 9 - 1, dz = (nb / 3) % 3 - 1, dy = nb % 3 - 1;
-    // the item's element: offset -1 or 0 per direction; free where the
-    // neighbour's offset is 0
-    int t = it - half_first(nb), d[3] = {dx, dy, dz}, ofs[3];
-#pragma unroll
-    for (int q = 0; q < 3; q++) {
-      const bool free = d[q] == 0;
-      ofs[q] = (free ? (t & 1) : d[q] > 0) ? 0 : -1;
-      if (free) t >>= 1;
-    }
-    const int ie = i + ofs[0], je = j + ofs[1], ke = k + ofs[2];
-    const bool in = ie >= 0 && ie < nelx && je >= 0 && je < nely && ke >= 0 && ke < nelz;
-    const int a = cn_of(-ofs[0], -ofs[1], -ofs[2]);
-    const int b = cn_of(dx - ofs[0], dy - ofs[1], dz - ofs[2]);
-    const int64_t e = in ? ((int64_t)ie * nelz + ke) * nely + je : 0;
-    double v[9];
-    if constexpr (BLOCKS) {
-      const double *K = Ke + kKeBlocks * e + 9 * ke_block(min(a, b), max(a, b));
-#pragma unroll
-      for (int q = 0; q < 9; q++) v[q] = K[q];
-    } else {
-      const double *K = Ke + 576 * e + 72 * a + 3 * b;
-#pragma unroll
-      for (int q = 0; q < 9; q++) v[q] = K[24 * (q / 3) + q % 3];
-    }
-    const bool tr = BLOCKS && a > b;  // block (b, a) transposed
-#pragma unroll
-    for (int r = 0; r < 3; r++)
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-        item[(it * 9 + 3 * r + c) * kHsNodes + nn] = in ? (tr ? v[3 * c + r] : v[3 * r + c]) : 0.0;
-    if (it == half_first(nb))  // (neighbours beyond the grid are nodes of the halo)
+    const int nn = tid & (kHsNodes - 1), it = tid / kHsNodes;
+    const uint32_t n = min(n0 + nn, nint - 1);
+    const int j = (int)(n % ny), k = (int)(n / ny % nz), i = (int)(n / (ny * nz));
+    if (it < 8) {
+      const int ie = i - (it >> 2), ke = k - ((it >> 1) & 1), je = j - (it & 1);
+      const bool in = ie >= 0 && ie < nelx && je >= 0 && je < nely && ke >= 0 && ke < nelz;
+      elem[nn * 8 + it] = in ? (ie * nelz + ke) * nely + je : -1;
+    } else if (it < 8 + 14) {  // (neighbours beyond the grid are nodes of the halo)
+      const int nb = 13 + it - 8, dx = nb / 9 - 1, dz = (nb / 3) % 3 - 1, dy = nb % 3 - 1;
       mask[(nb - 13) * kHsNodes + nn] =
           fix[((int64_t)(i + dx + 1) * wz + (k + dz + 1)) * wy + (j + dy + 1)];
+    }
   }
   __syncthreads();
-  for (int o = threadIdx.y * kHsNodes + threadIdx.x; o < kHalfPlanes * kHsNodes;
-       o += kHsNodes * kHsItems) {
+#pragma unroll
+  for (int t = 0; t < (kHsNodes * kHsValues + kHsThreads - 1) / kHsThreads; t++) {
+    const int o = tid + kHsThreads * t, nn = o / kHsValues, q = o - nn * kHsValues;
+    if (nn < kHsNodes) {
+      const int bq = q / 9;
+      int ra = 0;  // the run that holds block bq
+#pragma unroll
+      for (int r = 1; r < 8; r++) ra += bq >= ke_block(r, r);
+      const int e = elem[nn * 8 + ra];
+      double v = 0.0;
+      if (e >= 0) {
+        if constexpr (BLOCKS) {
+          v = Ke[(int64_t)kKeBlocks * e + q];
+        } else {
+          const int rb = bq - ke_block(ra, ra) + ra;
+          const int a = cn_of(ra >> 2, ra & 1, (ra >> 1) & 1);
+          const int b = cn_of(rb >> 2, rb & 1, (rb >> 1) & 1);
+          v = Ke[576 * (int64_t)e + 24 * (3 * a + q % 9 / 3) + 3 * b + q % 3];
+        }
+      }
+      val[nn * kHsLd + q] = v;
+    }
+  }
+  __syncthreads();
+  for (int o = tid; o < kHalfPlanes * kHsNodes; o += kHsThreads) {
     const int q = o / kHsNodes, m = o % kHsNodes;
     if (m >= nloc) continue;
     int nb = 13, r, c;
@@ -430,9 +429,15 @@ __global__ __launch_bounds__(kHsNodes *kHsItems) void k_node_stencil_half(
       r = q < 120 ? 0 : q < 122 ? 1 : 2;
       c = q - (r == 0 ? 117 : r == 1 ? 119 : 120);
     }
+    const int dx = nb / 9 - 1, dz = (nb / 3) % 3 - 1, dy = nb % 3 - 1;
     double v = 0.0;
-    for (int f = half_first(nb); f < half_first(nb + 1); f++)
-      v += item[(f * 9 + 3 * r + c) * kHsNodes + m];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {  // the node at (x, y, z) of the element, (7 - e)'s bits
+      const int x = 1 - (e & 1), y = 1 - (e >> 1 & 1), z = 1 - (e >> 2);
+      const int x2 = x + dx, y2 = y + dy, z2 = z + dz;
+      if (((x2 | y2 | z2) & ~1) == 0)  // the neighbour is a node of it
+        v += val[m * kHsLd + 9 * ke_block(ke_rank(x, y, z), ke_rank(x2, y2, z2)) + 3 * r + c];
+    }
     const bool diag = nb == 13 && r == c;
     if (((mask[m] >> r) | (mask[(nb - 13) * kHsNodes + m] >> c)) & 1) v = diag ? 1.0 : 0.0;
     if (!S32 || diag) S[(int64_t)q * nint + n0 + m] = v;
@@ -444,7 +449,7 @@ void launch_node_stencil_half(const DevGrid &g, int l, const double *Ke, double 
                               bool blocks) {
   const Level &L = g.lv[l];
   const uint32_t nblk = (uint32_t)((L.interior_nodes() + kHsNodes - 1) / kHsNodes);
-  const dim3 bs(kHsNodes, kHsItems);
+  const dim3 bs(kHsThreads);
   if (blocks)
     hipLaunchKernelGGL(k_node_stencil_half<true>, dim3(nblk), bs, 0, stream(), L.nelx, L.nely,
                        L.nelz, L.wy, L.wz, Ke, g.fixmask[l], S, S32, nblk);

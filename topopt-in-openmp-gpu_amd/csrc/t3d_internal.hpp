@@ -179,8 +179,9 @@ void launch_invdiag_stencil(const DevGrid &g, int l, const double *S, T *invD);
 
 // coarse element matrices and stencils (FP64)
 void launch_elem_level2(const DevGrid &g, const double *E, double *Ke2);
-// An element matrix as its 36 3x3 blocks of the node pairs a <= b, block
-// ke_block(a, b) row-major, padded to whole 16-column tiles
+// An element matrix as its 36 3x3 blocks of the node pairs a <= b, the nodes
+// numbered x, z, y (y fastest): block ke_block(a, b) row-major, rows of a,
+// padded to whole 16-column tiles
 constexpr int kKeBlocks = 336;
 __host__ __device__ constexpr int ke_block(int a, int b) { return 8 * a - a * (a - 1) / 2 + b - a; }
 // the level-2 matrices in that form, kKeBlocks values per element; false if
