@@ -48,6 +48,7 @@ bool SolverState::allocate(DevGrid *grid, int nlev) {
   z = alloc_t<double>(n0);
   E64 = alloc_t<double>(g->nelem);
   E32 = alloc_t<float>(g->nelem);
+  rs0 = alloc_t<double>(g->lv[0].nodes());
   if (nl >= 2) Eh1 = alloc_t<double>(level1_moduli_count(*g));
   for (int l = 0; l < nl; l++) {
     const int64_t nd = g->lv[l].ndof;
@@ -115,7 +116,7 @@ void SolverState::release() {
     f(S64[l]);
     f(S32[l]);
   }
-  f(r); f(p); f(q); f(z); f(E64); f(E32); f(Eh1); f(Eg3);
+  f(r); f(p); f(q); f(z); f(E64); f(E32); f(rs0); f(Eh1); f(Eg3);
   coarse.release();
   f(scal); f(partials); f(cgpart);
   if (hscal) hipHostFree(hscal);
@@ -152,6 +153,8 @@ bool SolverState::setup_main(const double *x) {
   // the fine Jacobi sweeps form their diagonal from E when they can
   const bool fdiag = fine_sweep_forms_diagonal();
   if (!fdiag) launch_invdiag_mf<double>(*g, 0, E64, invD64[0]);
+  else if (mixed) launch_recip_moduli<float>(*g, E32, (float *)rs0);
+  else launch_recip_moduli<double>(*g, E64, (double *)rs0);
   launch_invdiag_mf<double>(*g, 1, E64, invD64[1]);
   if (mixed)
     for (int l = fdiag ? 1 : 0; l < 2; l++)
@@ -283,15 +286,19 @@ template <typename T>
 T *SolverState::smooth_from_zero(int l, const T *b, T *zb, T *tb, bool zero_done) {
   T *cur = (nswp % 2 == 1) ? zb : tb;
   T *oth = (cur == zb) ? tb : zb;
-  if (zero_done)
-    ;  // written by the restriction that produced b
+  const bool two = l == 0 && nswp > 1 && fine_sweep_forms_diagonal();  // in one launch
+  if (zero_done || two)
+    ;  // written by the restriction that produced b; not formed
   else if (l == 0 && fine_sweep_forms_diagonal())
     launch_fine_jacobi_zero<T, T>(*g, b, young_t<T>(), (T)kOmega, cur);
   else
     launch_jacobi_zero<T, T>(*g, l, b, invd<T>(l), (T)kOmega, cur);
   const bool rec = l == 0 && nswp > 1 && sweep_timing_begin();
   for (int s = 1; s < nswp; s++) {
-    op<T>(l, 1, cur, oth, b);
+    if (two && s == 1)
+      launch_fine_first_sweeps<T>(*g, young_t<T>(), (const T *)rs0, b, (T)kOmega, oth, bcsym);
+    else
+      op<T>(l, 1, cur, oth, b);
     std::swap(cur, oth);
   }
   sweep_timing_end(rec, nswp - 1);

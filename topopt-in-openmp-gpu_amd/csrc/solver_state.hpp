@@ -20,6 +20,7 @@ struct SolverState {
   // Young's moduli of the fine elements
   double *E64 = nullptr;
   float *E32 = nullptr;
+  void *rs0 = nullptr;  // 1 / (sum of the moduli) per fine node, in the V-cycle's type
   // their per-level-1-element transform for the level-1 sweeps, in the
   // precision of the last set-up's V-cycle (launch_level1_moduli; sized for
   // FP64)
