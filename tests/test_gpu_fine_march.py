@@ -80,3 +80,47 @@ def test_vectors_beyond_the_cache():
     check_operator(g, o, 5, sweeps=False)
     g.close()
     o.close()
+
+
+# One CG iteration from zero leaves u = alpha z, z the V-cycle of the load:
+# checks the V-cycle's own launches, the first two sweeps in one and (mixed)
+# the sweep that adds the coarse correction.
+def vcycle_of_load(g, seed):
+    x = g.density(np.random.default_rng(seed).uniform(0.1, 1.0, g.nelx * g.nely * g.nelz))
+    F, U = g.load(), g.zeros(0)
+    g.set_max_iter(1)
+    g.solve(x, F, U, allow_no_converge=True)
+    return x.cpu().numpy(), F.cpu().numpy(), U.cpu().numpy()
+
+
+# FP64: 1e-10; the FP32 V-cycle: 2^-24 for each of 24 products and 32 sweeps,
+# ten times that for what the coarse correction amplifies, 1e-3
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-10), ("mixed", 1e-3)])
+@pytest.mark.parametrize("shape", [(16, 24, 8), (12, 20, 44), (8, 88, 36)])
+def test_vcycle(shape, precision, tol):
+    print(f"[gpu fine march] v-cycle {shape} {precision}", flush=True)
+    g = top3d_amd.Grid(*shape, 3, precision=precision)
+    o = pyoracle.Grid(*shape, 3)
+    x, r, got = vcycle_of_load(g, shape[1])
+    assert o.setup(x) == 0
+    z = o.vcycle(x, r)
+    assert relerr(got, (r @ z) / (z @ o.matvec0(x, z)) * z) <= tol
+    g.close()
+    o.close()
+
+
+# Every tile shape forms a node from the same operands in the same order: only
+# the order of the sums for alpha changes, 1e-12
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("shape,tile", [((140, 36, 28), "17,12,65"), ((140, 36, 28), "20,11,7"),
+                                        ((140, 36, 28), "23,9,131"), ((12, 20, 44), "2,2,3"),
+                                        ((16, 24, 8), "5,3,1")])
+def test_vcycle_tiles(shape, tile, precision, monkeypatch):
+    print(f"[gpu fine march] v-cycle {shape} {tile} {precision}", flush=True)
+    g = top3d_amd.Grid(*shape, 3, precision=precision)
+    _, _, ref = vcycle_of_load(g, shape[1])
+    monkeypatch.setenv("TOP3D_TILE_L0", tile)
+    monkeypatch.setenv("TOP3D_TILE_L0_F64", tile)
+    _, _, got = vcycle_of_load(g, shape[1])
+    assert relerr(got, ref) <= 1e-12
+    g.close()

@@ -325,23 +325,23 @@ static DevGrid *build_dev_grid(struct gridContext *gc, int nl) {
     g->KE2 = (double *)dalloc(sizeof(double) * cnt);
     T3D_HIP(hipMemcpyAsync(g->KE2, gc->precomputedKE[2], sizeof(double) * cnt,
                            hipMemcpyHostToDevice, stream()));
-    T3D_HIP(hipStreamSynchronize(stream()));
-  }
-  if (nl >= 4) {  // KE_2 as node-pair blocks for the level-2 smoother's stencil
-    std::vector<double> kb(64 * (size_t)kKeBlocks, 0.0);
+    // as node-pair blocks for the level-2 smoother's stencil
+    std::vector<double> kb(nl >= 4 ? 64 * (size_t)kKeBlocks : 0, 0.0);
     auto node = [](int r) {  // element node at (x, z, y) = the bits of r
       const int x = r >> 2, z = (r >> 1) & 1, y = r & 1;
       return 4 * z + (y ? (x ? 1 : 0) : (x ? 2 : 3));
     };
-    for (int f = 0; f < 64; f++)
+    for (int f = 0; f < (nl >= 4 ? 64 : 0); f++)
       for (int a = 0; a < 8; a++)
         for (int b = a; b < 8; b++)
           for (int q = 0; q < 9; q++)
             kb[(size_t)kKeBlocks * f + 9 * ke_block(a, b) + q] =
                 gc->precomputedKE[2][576 * f + 24 * (3 * node(a) + q / 3) + 3 * node(b) + q % 3];
-    g->KE2b = (double *)dalloc(sizeof(double) * kb.size());
-    T3D_HIP(hipMemcpyAsync(g->KE2b, kb.data(), sizeof(double) * kb.size(), hipMemcpyHostToDevice,
-                           stream()));
+    if (nl >= 4) {
+      g->KE2b = (double *)dalloc(sizeof(double) * kb.size());
+      T3D_HIP(hipMemcpyAsync(g->KE2b, kb.data(), sizeof(double) * kb.size(),
+                             hipMemcpyHostToDevice, stream()));
+    }
     T3D_HIP(hipStreamSynchronize(stream()));
   }
   if (nl >= 4) {  // level-3 sub-cell matrices: level-3 element matrices as one GEMM

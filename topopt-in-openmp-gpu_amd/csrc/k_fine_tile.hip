@@ -38,7 +38,16 @@ namespace t3d {
 // the element moduli it already reads (fine level, solver only)
 // kModeFirst: two sweeps from zero in one, in and b being the right-hand side
 // and invD the reciprocal of the moduli's sum at each node (k_recip_moduli)
-enum { kModeApply = 0, kModeJacobi = 1, kModeResidual = 2, kModeJacobiDiag = 3, kModeFirst = 4 };
+// kModeProlong: a sweep of in + P aux, aux the next level's vector, with invD as
+// in kModeFirst
+enum {
+  kModeApply = 0,
+  kModeJacobi = 1,
+  kModeResidual = 2,
+  kModeJacobiDiag = 3,
+  kModeFirst = 4,
+  kModeProlong = 5
+};
 
 // position bits (x, y, z) of the reference's local node n (stencil_utility.h:19-26)
 static constexpr int kPos[8][3] = {{0, 1, 0}, {1, 1, 0}, {1, 0, 0}, {0, 0, 0},
@@ -391,6 +400,8 @@ struct TileArgs {
   int stream_out;        // store the output past the caches
   uint32_t out_bytes;    // size of the level's vectors (below 2^32 - 32)
   uint32_t e_bytes;      // size of the moduli (below 2^32)
+  int c_wx, c_wy, c_wz;  // kModeProlong: nodes of the next level's vector
+  uint32_t c_bytes;      // and its size
 };
 
 // The tile of a workgroup of the (slabs, tiles) grid.  The device deals
@@ -804,8 +815,9 @@ __device__ __forceinline__ void fine_march_body(
     TileArgs a, Blocks<T> B, const T *__restrict__ E, const T *__restrict__ in,
     T *__restrict__ out, const T *__restrict__ b, const T *__restrict__ invD, T omega,
     const uint8_t *__restrict__ fix, const int *__restrict__ fixplane,
-    double *__restrict__ dotp, float *__restrict__ out32) {
+    double *__restrict__ dotp, void *__restrict__ aux) {
   constexpr bool kDiag = MODE == kModeJacobiDiag, kFirst = MODE == kModeFirst;
+  constexpr bool kProl = MODE == kModeProlong;
   constexpr int N = march_threads<T>(), XV = kDiag ? 10 : 9;
   extern __shared__ unsigned char smem_raw[];
   T *xch = reinterpret_cast<T *>(smem_raw);  // [2][XV][N]; slot N-1: zeros
@@ -845,8 +857,8 @@ __device__ __forceinline__ void fine_march_body(
   const __amdgpu_buffer_rsrc_t rin = rsrc(in, a.out_bytes), re = rsrc(E, a.e_bytes);
   const __amdgpu_buffer_rsrc_t rfix = rsrc(fix, a.out_bytes / (3u * (uint32_t)sizeof(T)));
   const __amdgpu_buffer_rsrc_t rb = rsrc(MODE == kModeApply || kFirst ? in : b, a.out_bytes);
-  const __amdgpu_buffer_rsrc_t rd = rsrc(MODE == kModeJacobi || kFirst ? invD : in,
-                                         kFirst ? a.out_bytes / 3u : a.out_bytes);
+  const __amdgpu_buffer_rsrc_t rd = rsrc(MODE == kModeJacobi || kFirst || kProl ? invD : in,
+                                         kFirst || kProl ? a.out_bytes / 3u : a.out_bytes);
   // the planes from plane fbase on with a fixed DOF
   int fbase = i0 - 1;
   auto fixed_planes = [&]() {
@@ -904,7 +916,43 @@ __device__ __forceinline__ void fine_march_body(
     if (kFirst) return;  // (all carried with the planes)
     if (MODE != kModeApply) load3<T>(rb, vnode, (uint32_t)i * sv, s.bb);
     if (MODE == kModeJacobi) load3<T>(rd, vnode, (uint32_t)i * sv, s.di);
+    if (kProl) s.di[0] = load1<T>(rd, vnode / 3u, (uint32_t)i * (sx * (uint32_t)sizeof(T)));
     s.m = load_mask(i, s.fixed);
+  };
+  // kProl: the nodes of the coarse plane over the tile, in LDS one at a time, a
+  // thread each; Cm, the plane's interpolation in y and z at the thread's node.
+  // The march starts at an odd plane, so that step 0 of a turn puts a plane
+  // between two coarse ones and step 1 a plane on one.
+  T *ctile = nodes + 2 * 3 * N;  // [ncn][3]
+  const int cj0 = (w.by * (a.TY - 1) + 1) >> 1, ck0 = (w.bz * (a.TZ - 1) + 1) >> 1;
+  const int ncy = ((w.by * (a.TY - 1) + a.TY) >> 1) + 2 - cj0;
+  const int ncn = ncy * (((w.bz * (a.TZ - 1) + a.TZ) >> 1) + 2 - ck0);
+  const int c11 = active ? (((k + 1) >> 1) - ck0) * ncy + ((j + 1) >> 1) - cj0 : 0;
+  const int c12 = c11 + (active && (j & 1) == 0);
+  const int c21 = c11 + (active && (k & 1) == 0 ? ncy : 0), c22 = c21 + c12 - c11;
+  const __amdgpu_buffer_rsrc_t rc = rsrc(kProl ? aux : in, kProl ? a.c_bytes : 0u);
+  const uint32_t vc =
+      t < ncn ? 3u * (uint32_t)sizeof(T) *
+                    ((uint32_t)min(ck0 + t / ncy, a.c_wz - 1) * (uint32_t)a.c_wy +
+                     (uint32_t)min(cj0 + t % ncy, a.c_wy - 1))
+              : 0u;
+  T cz[3] = {0, 0, 0}, Cm[3] = {0, 0, 0};
+  auto load_coarse = [&](int ic, T (&v)[3]) {
+    load3<T>(rc, vc, (uint32_t)min(ic, a.c_wx - 1) * (3u * (uint32_t)sizeof(T)) *
+                         ((uint32_t)a.c_wy * (uint32_t)a.c_wz), v);
+  };
+  auto put_coarse = [&](const T (&v)[3]) {
+    if (t < ncn) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) ctile[3 * t + c] = v[c];
+    }
+  };
+  auto get_coarse = [&](T (&C)[3]) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const T *q = ctile + c;
+      C[c] = T(0.25) * ((q[3 * c11] + q[3 * c12]) + (q[3 * c21] + q[3 * c22]));
+    }
   };
   // plane i into LDS buffer P; n: the node as carried; BCSYM: the fixed DOFs
   // are handed on, and read back, as zeros
@@ -924,14 +972,32 @@ __device__ __forceinline__ void fine_march_body(
           if ((n.m >> c) & 1) v[c] = 0;
       }
     } else {
+      if constexpr (kProl) {
+        if (P == 0) {
+          T Cn[3];
+          get_coarse(Cn);
+#pragma unroll
+          for (int c = 0; c < 3; c++) {
+            n.u[c] += T(0.5) * (Cm[c] + Cn[c]);
+            Cm[c] = Cn[c];
+          }
+        } else {
+#pragma unroll
+          for (int c = 0; c < 3; c++) n.u[c] += Cm[c];
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 3; c++) v[c] = n.u[c];
       if (BCSYM && fixplane[min(i, i1 + 1)] != 0) {
         const uint8_t m = fix[(uint32_t)min(i, i1 + 1) * sx + node];
 #pragma unroll
         for (int c = 0; c < 3; c++)
-          if ((m >> c) & 1) n.u[c] = 0;
+          if ((m >> c) & 1) v[c] = 0;
       }
+      if constexpr (BCSYM && !kProl) {
 #pragma unroll
-      for (int c = 0; c < 3; c++) v[c] = n.u[c];
+        for (int c = 0; c < 3; c++) n.u[c] = v[c];
+      }
     }
     T *nb = nodes + P * 3 * N + t;
 #pragma unroll
@@ -946,7 +1012,7 @@ __device__ __forceinline__ void fine_march_body(
       v[0][0][c] = nb[c * N + f00];
       v[1][0][c] = nb[c * N + f00 + 1];
       v[0][1][c] = nb[c * N + f01];
-      v[1][1][c] = kFirst ? nb[c * N + t] : n.u[c];
+      v[1][1][c] = kFirst || kProl ? nb[c * N + t] : n.u[c];
     }
     face_wht<T>(v, F);
   };
@@ -1003,6 +1069,10 @@ __device__ __forceinline__ void fine_march_body(
     }
     put_plane(i + 2, P, s.p, u2);
     load_plane(i + 3, s.p);
+    if constexpr (kProl && P == 1) {
+      put_coarse(cz);
+      load_coarse((i + 2 + 3) / 2 + 1, cz);
+    }
     lds_barrier();
     // the owned node's row, in every lane: stored where own_ok and emit
     T kin[3] = {tot[1][1][0], tot[1][1][1], tot[1][1][2]}, o[3], uo[3], dd[3];
@@ -1035,11 +1105,15 @@ __device__ __forceinline__ void fine_march_body(
 #pragma unroll
       for (int c = 0; c < 3; c++) dd[c] = rs * B.ikd[c];
     }
+    if constexpr (kProl) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) dd[c] = s.di[0] * B.ikd[c];
+    }
     uint32_t m = s.m;
     if constexpr (!kFirst)
       pin(m);  // (used in the branch only, its copies for the next step would wait for the load)
     if (!kFirst && s.fixed) {
-      if (BCSYM && m != 0) {  // u0 holds zeros there
+      if (BCSYM && !kProl && m != 0) {  // u0 holds zeros there
         const T *pu = at32(in, 3u * ((uint32_t)i * sx + node));
 #pragma unroll
         for (int c = 0; c < 3; c++) uo[c] = pu[c];
@@ -1048,16 +1122,16 @@ __device__ __forceinline__ void fine_march_body(
       for (int c = 0; c < 3; c++)
         if ((m >> c) & 1) {  // identity row
           kin[c] = uo[c];
-          if constexpr (kDiag) dd[c] = T(1);
+          if constexpr (kDiag || kProl) dd[c] = T(1);
         }
     }
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       if (MODE == kModeApply) o[c] = kin[c];
-      else if (MODE == kModeJacobi || kDiag || kFirst) o[c] = uo[c] + omega * dd[c] * (s.bb[c] - kin[c]);
+      else if (MODE == kModeJacobi || kDiag || kFirst || kProl) o[c] = uo[c] + omega * dd[c] * (s.bb[c] - kin[c]);
       else o[c] = s.bb[c] - kin[c];
     }
-    if (MODE != kModeResidual && !kFirst && dotp) {
+    if (MODE != kModeResidual && !kFirst && !kProl && dotp) {
       double d = dacc;
 #pragma unroll
       for (int c = 0; c < 3; c++)
@@ -1068,9 +1142,9 @@ __device__ __forceinline__ void fine_march_body(
     const __amdgpu_buffer_rsrc_t ro = rsrc(out, emit ? a.out_bytes : 0u);
     if (a.stream_out) store_node<kNt>(ro, vout, o, (uint32_t)i * sv);
     else store_node(ro, vout, o, (uint32_t)i * sv);
-    if (MODE == kModeResidual && sizeof(T) == 8 && out32) {  // the FP32 copy too
+    if (MODE == kModeResidual && sizeof(T) == 8 && aux) {  // the FP32 copy too
       const float o32[3] = {(float)o[0], (float)o[1], (float)o[2]};
-      store_node(rsrc(out32, emit ? a.out_bytes / 2 : 0u), vout / 2, o32, (uint32_t)i * sv / 2);
+      store_node(rsrc(aux, emit ? a.out_bytes / 2 : 0u), vout / 2, o32, (uint32_t)i * sv / 2);
     }
     load_node(i + 1);
   };
@@ -1084,8 +1158,27 @@ __device__ __forceinline__ void fine_march_body(
   s.e = load_modulus(i0 - 1);
   load_node(i0 - 1);
   if (t < 2 * XV) xch[t * N + N - 1] = 0;
-  put_plane(i0 - 1, 0, pa, ua);
-  put_plane(i0, 1, pb, ub);
+  if constexpr (kProl) {  // the coarse planes at and beside plane i0
+    const int ic = i0 / 2;
+    T ca[3], cb[3], cc[3];
+    load_coarse(ic, ca);
+    load_coarse(ic + 1, cb);
+    load_coarse(ic + 2, cc);
+    load_coarse(ic + 3, cz);
+    put_coarse(ca);
+    __syncthreads();
+    get_coarse(Cm);
+    __syncthreads();
+    put_coarse(cb);
+    __syncthreads();
+    put_plane(i0 - 1, 0, pa, ua);
+    put_plane(i0, 1, pb, ub);
+    __syncthreads();
+    put_coarse(cc);
+  } else {
+    put_plane(i0 - 1, 0, pa, ua);
+    put_plane(i0, 1, pb, ub);
+  }
   __syncthreads();
   get_face(0, Fa, ua);
 #pragma unroll
@@ -1093,7 +1186,9 @@ __device__ __forceinline__ void fine_march_body(
     pin(s.p.u[c]);
     if (MODE != kModeApply && !kFirst) pin(s.bb[c]);
     if (MODE == kModeJacobi) pin(s.di[c]);
+    if (kProl) pin(cz[c]);
   }
+  if (kProl) pin(s.di[0]);
   if constexpr (kFirst) {
     pin(s.p.rs);
     pin(s.p.m);
@@ -1111,7 +1206,7 @@ __device__ __forceinline__ void fine_march_body(
     ub = ua;
     ua = uz;
   }
-  if (MODE != kModeResidual && !kFirst && dotp) {  // one partial per workgroup, fixed order
+  if (MODE != kModeResidual && !kFirst && !kProl && dotp) {  // one partial per workgroup, fixed order
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) dacc += __shfl_down(dacc, off, 64);
     __syncthreads();
@@ -1132,9 +1227,8 @@ __global__ __launch_bounds__(march_threads<T>())
     TileArgs a, Blocks<T> B, const T *__restrict__ E, const T *__restrict__ in,
     T *__restrict__ out, const T *__restrict__ b, const T *__restrict__ invD, T omega,
     const uint8_t *__restrict__ fix, const int *__restrict__ fixplane,
-    double *__restrict__ dotp, float *__restrict__ out32) {
-  fine_march_body<T, MODE, BCSYM>(a, B, E, in, out, b, invD, omega, fix, fixplane, dotp,
-                                  out32);
+    double *__restrict__ dotp, void *__restrict__ aux) {
+  fine_march_body<T, MODE, BCSYM>(a, B, E, in, out, b, invD, omega, fix, fixplane, dotp, aux);
 }
 
 template <typename T, int MODE, bool BCSYM>
@@ -1409,7 +1503,7 @@ static void tile_args_shape(const TileShape &s, TileArgs &a) {
 template <typename T>
 static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out, const T *b,
                        const T *invD, T omega, int bcsym, double *dotp = nullptr,
-                       int dot_cap = 0, float *out32 = nullptr) {
+                       int dot_cap = 0, void *aux = nullptr) {
   init_coef();
   const Level &L = g.lv[0];
   TileArgs a;
@@ -1421,6 +1515,7 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
   if (mode == kModeJacobiDiag && !g_coef.diag0) mode = kModeJacobi;
   const bool diag = mode == kModeJacobiDiag;
   const size_t shm = sizeof(T) * march_lds_values(diag) * (size_t)march_threads<T>();
+  size_t coarse_lds = 0;  // the coarse plane of kModeProlong
   // workgroups per CU, [0] sweeps reading invD, [1] forming the diagonal
   static int per_cu[2] = {0, 0};
   if (!per_cu[diag])
@@ -1431,6 +1526,16 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
   int nx_fixed = 0;
   TileShape s = march_shape(L, slots, sizeof(T) == 8, nx_fixed);
   tile_x(s, L, nx_fixed, slots);
+  if (mode == kModeProlong) {  // (marches that start at odd planes)
+    s.NX += s.NX & 1;
+    s.ntx = (L.nx + s.NX - 1) / s.NX;
+    const Level &C = g.lv[1];
+    a.c_wx = C.wx;
+    a.c_wy = C.wy;
+    a.c_wz = C.wz;
+    a.c_bytes = (uint32_t)(sizeof(T) * 3 * C.nodes());
+    coarse_lds = sizeof(T) * 3 * (size_t)(s.TY / 2 + 3) * (s.TZ / 2 + 3);
+  }
   tile_args_shape(s, a);
   // Past the caches where the launch reads no more than the memory-side cache
   // holds (256 MB) and with its output exceeds it: the output would push out
@@ -1442,6 +1547,7 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
   // us per FP32 sweep of 256x128x128 (171 MB in all).
   const int64_t cache = int64_t(256) << 20;
   const int64_t reads = (mode == kModeFirst   ? 4
+                         : mode == kModeProlong ? 7
                          : mode == kModeApply ? 3
                          : mode == kModeJacobi ? 9
                                                : 6) *
@@ -1454,20 +1560,22 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
   if (dotp && nwg > dot_cap) dotp = nullptr;
   const auto B = fine_values<T>();
 #define T3D_LAUNCH(M, S)                                                                  \
-  hipLaunchKernelGGL((k_fine_march<T, M, S>), grid, dim3(bs), shm, stream(), a, B, E, in, \
-                     out, b, invD, omega, g.fixmask[0], g.fixplane[0], dotp, out32)
+  hipLaunchKernelGGL((k_fine_march<T, M, S>), grid, dim3(bs), shm + coarse_lds, stream(), a, B, \
+                     E, in, out, b, invD, omega, g.fixmask[0], g.fixplane[0], dotp, aux)
   if (bcsym) {
     if (mode == kModeApply) T3D_LAUNCH(kModeApply, true);
     else if (mode == kModeJacobi) T3D_LAUNCH(kModeJacobi, true);
     else if (mode == kModeResidual) T3D_LAUNCH(kModeResidual, true);
     else if (mode == kModeFirst) T3D_LAUNCH(kModeFirst, true);
-    else T3D_LAUNCH(kModeJacobiDiag, true);
+    else if (mode == kModeJacobiDiag) T3D_LAUNCH(kModeJacobiDiag, true);
+    else if constexpr (sizeof(T) == 4) T3D_LAUNCH(kModeProlong, true);
   } else {
     if (mode == kModeApply) T3D_LAUNCH(kModeApply, false);
     else if (mode == kModeJacobi) T3D_LAUNCH(kModeJacobi, false);
     else if (mode == kModeResidual) T3D_LAUNCH(kModeResidual, false);
     else if (mode == kModeFirst) T3D_LAUNCH(kModeFirst, false);
-    else T3D_LAUNCH(kModeJacobiDiag, false);
+    else if (mode == kModeJacobiDiag) T3D_LAUNCH(kModeJacobiDiag, false);
+    else if constexpr (sizeof(T) == 4) T3D_LAUNCH(kModeProlong, false);
   }
 #undef T3D_LAUNCH
   return dotp ? nwg : 0;
@@ -1698,6 +1806,19 @@ template void launch_fine_first_sweeps<float>(const DevGrid &, const float *, co
                                               const float *, float, float *, int);
 template void launch_fine_first_sweeps<double>(const DevGrid &, const double *, const double *,
                                                const double *, double, double *, int);
+
+// out = a Jacobi sweep of z + P zc, zc the level-1 vector: the correction of the
+// V-cycle is added as the nodes are loaded, the coarse planes interpolated from
+// LDS.  In the V-cycle at 256x128x128 48.6 us against 25.6 + 40 for prolongation
+// and sweep, at 512x256x256 346 against 189 + 302.  FP32 only: in FP64 it takes
+// more than the 168 registers of three workgroups per CU (288 us against
+// 62 + 85).
+void launch_fine_prolong_sweep(const DevGrid &g, const float *E, const float *rs, const float *z,
+                               const float *zc, const float *b, float omega, float *out,
+                               int bcsym) {
+  run_fine<float>(g, kModeProlong, E, z, out, b, rs, omega, bcsym, nullptr, 0,
+                  const_cast<float *>(zc));
+}
 
 // Inverse diagonal of the fine operator from the moduli (KE_0's diagonal is
 // one value per component): 1 / (KE[c][c] sum of the node's 8 element

@@ -306,11 +306,20 @@ T *SolverState::smooth_from_zero(int l, const T *b, T *zb, T *tb, bool zero_done
 }
 
 // The last fine sweep of a preconditioner application also writes the
-// partial sums of r . z for the CG (rz_parts of them, 0 if it could not).
+// partial sums of r . z for the CG (rz_parts of them, 0 if it could not).  add:
+// the coarse correction that the first sweep is to add to cur.
 template <typename T>
-T *SolverState::smooth(int l, const T *b, T *cur, T *oth) {
+T *SolverState::smooth(int l, const T *b, T *cur, T *oth, const T *add) {
   const bool rec = l == 0 && nswp > 0 && sweep_timing_begin();
   for (int s = 0; s < nswp; s++) {
+    if constexpr (sizeof(T) == 4) {
+      if (add && s == 0) {
+        launch_fine_prolong_sweep(*g, E32, (const float *)rs0, cur, add, b, (float)kOmega, oth,
+                                  bcsym);
+        std::swap(cur, oth);
+        continue;
+      }
+    }
     if (l == 0 && s == nswp - 1)
       rz_parts = launch_fine_sweep_dot<T>(*g, young_t<T>(), cur, oth, b, invd<T>(0), (T)kOmega,
                                           bcsym, cgpart, kPartRZ);
@@ -344,8 +353,11 @@ void SolverState::vcycle(int l, bool zero_done) {
     launch_restrict<T>(*g, l, d_, vec<T>(l + 1, kR), invd<T>(l + 1), (T)kOmega, first);
     vcycle<T>(l + 1, true);
   }
-  launch_prolong_add<T>(*g, l, vec<T>(l + 1, kZ), zc);  // z += P zc
-  T *res = smooth<T>(l, r_, zc, other);
+  // z += P zc, on the FP32 fine level with the first sweep (the last one has
+  // sums to write)
+  const bool with_sweep = sizeof(T) == 4 && l == 0 && nswp > 1 && fine_sweep_forms_diagonal();
+  if (!with_sweep) launch_prolong_add<T>(*g, l, vec<T>(l + 1, kZ), zc);
+  T *res = smooth<T>(l, r_, zc, other, with_sweep ? vec<T>(l + 1, kZ) : nullptr);
   if (res != z_)
     hipMemcpyAsync(z_, res, sizeof(T) * g->lv[l].ndof, hipMemcpyDeviceToDevice, stream());
 }

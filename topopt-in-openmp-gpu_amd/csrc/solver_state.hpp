@@ -92,7 +92,7 @@ struct SolverState {
   template <typename T> void vcycle(int l, bool zero_done = false);
   template <typename T> T *smooth_from_zero(int l, const T *b, T *zb, T *tb,
                                             bool zero_done = false);
-  template <typename T> T *smooth(int l, const T *b, T *cur, T *oth);
+  template <typename T> T *smooth(int l, const T *b, T *cur, T *oth, const T *add);
 
   template <typename T> T *vec(int l, int which) {
     if constexpr (sizeof(T) == 8) return (T *)v64[l][which]; else return (T *)v32[l][which];

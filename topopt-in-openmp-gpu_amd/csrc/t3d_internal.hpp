@@ -136,13 +136,16 @@ bool tile_level1_available();  // the level-1 element matrices have the mirror s
 bool tile_fine_diag_available();  // the fine tile sweep can form its diagonal from E
 // launch_fine mode 3 forms the diagonal from E (no invD read)
 bool fine_sweep_forms_diagonal();
-// when they do: the reciprocal of the moduli's sum at every node, and the first
-// two Jacobi sweeps from zero with it
+// when they do: the reciprocal of the moduli's sum at every node, and with it the
+// first two Jacobi sweeps from zero, and (FP32) the sweep of z + P zc
 template <typename T>
 void launch_recip_moduli(const DevGrid &g, const T *E, T *rs);
 template <typename T>
 void launch_fine_first_sweeps(const DevGrid &g, const T *E, const T *rs, const T *b, T omega,
                               T *out, int bcsym);
+void launch_fine_prolong_sweep(const DevGrid &g, const float *E, const float *rs, const float *z,
+                               const float *zc, const float *b, float omega, float *out,
+                               int bcsym);
 // zero the padded y rows (j > nely+1) of a level-0 vector
 void launch_zero_pad_rows(const DevGrid &g, double *out);
 // level-1 matrix-free operator with fine moduli E, same modes; Eh: their
