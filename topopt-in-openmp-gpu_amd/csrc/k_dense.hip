@@ -25,7 +25,9 @@
 namespace t3d {
 
 constexpr int kNB = kTile;      // tile size
-constexpr int kLd = kNB + 1;    // LDS row stride of a 64x64 tile
+// LDS row stride of a 64x64 tile: rows 16-byte aligned, and the pairs of an MFMA
+// operand in distinct banks
+constexpr int kLd = kNB + 2;
 constexpr int kStrip = 16;      // columns per workgroup of the W = L^{-1} kernel
 constexpr int kTriBatch = 64;   // tiles per batch of loads of the triangular products
 
@@ -39,7 +41,7 @@ __device__ inline double4_t mfma4(double a, double b, double4_t c) {
 }
 
 // ---------------------------------------------------------------------------
-// Cholesky and inverse of one 64x64 SPD tile in LDS, 256 threads (4 waves),
+// Cholesky and inverse of one 64x64 SPD tile in LDS, 8 waves (6 of them at work),
 // blocked by 16.  The 64 pivots are a serial chain, and a wave alone on its
 // SIMD issues one FP64 instruction in about 8 cycles, so the chain costs the
 // instructions of one wave.  Wave 0 does nothing else: it holds a 64x16 panel
@@ -58,15 +60,33 @@ __device__ inline double4_t mfma4(double a, double b, double4_t c) {
 // X = L^{-1}.  A non-positive pivot sets *info (and is replaced by 1 so that
 // the factorization finishes).
 
+// two neighbouring values in LDS (16-byte aligned)
+__device__ __forceinline__ void pair_load(const double *p, double &a, double &b) {
+  const double2 v = *reinterpret_cast<const double2 *>(p);
+  a = v.x;
+  b = v.y;
+}
+__device__ __forceinline__ void pair_store(double *p, double a, double b) {
+  *reinterpret_cast<double2 *>(p) = double2{a, b};
+}
+
+// Workgroup barrier for LDS: the wave's LDS accesses complete (lgkmcnt 0; the
+// other counters left at their maxima), then s_barrier.  __syncthreads() also
+// waits for the wave's global loads and stores.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // 1/sqrt(x) for x > 0: the hardware estimate and two Newton steps
-// y <- y + y (1 - x y^2) / 2
+// y <- y + y (1/2 - (x / 2) y^2)
 __device__ inline double rsqrt_refined(double x) {
   double y = __builtin_amdgcn_rsq(x);
+  const double xh = 0.5 * x;
 #pragma unroll
-  for (int it = 0; it < 2; it++) {
-    const double h = fma(-x * y, y, 1.0);
-    y = fma(0.5 * y, h, y);
-  }
+  for (int it = 0; it < 2; it++) y = fma(y, fma(-xh * y, y, 0.5), y);
   return y;
 }
 
@@ -172,9 +192,9 @@ __device__ __forceinline__ void factor_panel(double *T, double *X, double *inv, 
   double u[16], v[16], ij[16];
   bool bad = false;
 #pragma unroll
-  for (int c = 0; c < 16; c++) {
-    u[c] = T[(d0 + r) * kLd + d0 + c];
-    v[c] = LAST ? 0.0 : T[vrow * kLd + d0 + c];
+  for (int c = 0; c < 16; c += 2) {
+    pair_load(T + (d0 + r) * kLd + d0 + c, u[c], u[c + 1]);
+    if constexpr (!LAST) pair_load(T + vrow * kLd + d0 + c, v[c], v[c + 1]);
   }
   panel_pivots<0, !LAST>(u, v, ij, bad);
   if (bad && lane == 0) info[0] = 1;
@@ -183,14 +203,14 @@ __device__ __forceinline__ void factor_panel(double *T, double *X, double *inv, 
   } else {
     if (g == 0) {
 #pragma unroll
-      for (int c = 0; c < 16; c++) {
-        T[(d0 + r) * kLd + d0 + c] = u[c];
-        inv[d0 + c] = ij[c];  // (16 lanes write the same value)
+      for (int c = 0; c < 16; c += 2) {
+        pair_store(T + (d0 + r) * kLd + d0 + c, u[c], u[c + 1]);
+        pair_store(inv + d0 + c, ij[c], ij[c + 1]);  // (16 lanes write the same values)
       }
     }
     if (kb + 1 + g < 4) {
 #pragma unroll
-      for (int c = 0; c < 16; c++) T[vrow * kLd + d0 + c] = v[c];
+      for (int c = 0; c < 16; c += 2) pair_store(T + vrow * kLd + d0 + c, v[c], v[c + 1]);
     }
   }
 }
@@ -200,9 +220,9 @@ __device__ __forceinline__ void invert_block_lds(const double *T, double *X, con
                                                  int b, int lane) {
   double u[16], ij[16];
 #pragma unroll
-  for (int c = 0; c < 16; c++) {
-    u[c] = T[(16 * b + (lane & 15)) * kLd + 16 * b + c];
-    ij[c] = inv[16 * b + c];
+  for (int c = 0; c < 16; c += 2) {
+    pair_load(T + (16 * b + (lane & 15)) * kLd + 16 * b + c, u[c], u[c + 1]);
+    pair_load(inv + 16 * b + c, ij[c], ij[c + 1]);
   }
   invert_block(X, b, u, ij, lane);
 }
@@ -253,12 +273,12 @@ __device__ __forceinline__ void factor_tile(double *T, double *X, double *inv, i
     if (w == 0) {
       if (kb < 3) factor_panel<false>(T, X, inv, kb, lane, info);
       else factor_panel<true>(T, X, inv, kb, lane, info);
-    } else if (kb > 0) {
+    } else if (kb > 0 && w < 6) {
       // what the panel before left: its blocks (ti, tj), kb < tj <= ti, and
       // the inverse of its diagonal block
-      if (kb == 1) trail_block(T, w == 1 ? 2 : 3, w == 3 ? 3 : 2, d0 - 16, lane);
+      if (kb == 1 && w < 4) trail_block(T, w == 1 ? 2 : 3, w == 3 ? 3 : 2, d0 - 16, lane);
       if (kb == 2 && w == 1) trail_block(T, 3, 3, d0 - 16, lane);
-      if (w == 3) invert_block_lds(T, X, inv, kb - 1, lane);
+      if (w == 5) invert_block_lds(T, X, inv, kb - 1, lane);
       if (kb == 3 && w == 1) {
         double4_t y = zero;
         inv_term(T, X, 1, 0, 0, lane, y);
@@ -266,10 +286,10 @@ __device__ __forceinline__ void factor_tile(double *T, double *X, double *inv, i
       }
       if (kb == 3 && w == 2) inv_term(T, X, 3, 0, 0, lane, y30);
     }
-    __syncthreads();
+    lds_barrier();
     if (kb < 3) {  // the next panel's columns
       if (w < 3 - kb) trail_block(T, kb + 1 + w, kb + 1, d0, lane);
-      __syncthreads();
+      lds_barrier();
     }
   }
   // the rest of X: X_10 and the diagonal blocks are there
@@ -283,11 +303,11 @@ __device__ __forceinline__ void factor_tile(double *T, double *X, double *inv, i
     inv_block(X, 2, 0, lane, y);
   } else if (w == 2) {
     inv_term(T, X, 3, 1, 0, lane, y30);
-  } else {
+  } else if (w == 3) {
     inv_term(T, X, 3, 2, 2, lane, y);
     inv_block(X, 3, 2, lane, y);
   }
-  __syncthreads();
+  lds_barrier();
   if (w == 1) {
     y = zero;
     inv_term(T, X, 3, 1, 1, lane, y);
@@ -297,34 +317,36 @@ __device__ __forceinline__ void factor_tile(double *T, double *X, double *inv, i
     inv_term(T, X, 3, 2, 0, lane, y30);
     inv_block(X, 3, 0, lane, y30);
   }
-  __syncthreads();
+  lds_barrier();
 }
 
-// Q = P D^T in place on the wave's 16 rows of a 64x64 tile P in LDS, D lower
-// triangular (the columns of block cb need k < 16 (cb + 1) only: 40 MFMA
-// instead of 64); Q also goes to the tile at `out` (row stride np) if given.
-// A wave reads and writes its own rows only.
-__device__ __forceinline__ void panel_product(double *P, const double *D, int w, int lane,
-                                              double *__restrict__ out, int np) {
+// The blocks C0 and C1 of the row block rb of Q = P D^T for 64x64 tiles in LDS, D
+// lower triangular (block cb needs k < 16 (cb + 1) only).
+template <int C0, int C1>
+__device__ __forceinline__ void panel_product(const double *P, const double *D, int rb, int lane,
+                                              double4_t (&q)[2]) {
   const int li = lane & 15, lk = lane >> 4;
-  double4_t acc[4];
+  q[0] = q[1] = double4_t{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int cb = 0; cb < 4; cb++) acc[cb] = double4_t{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int k = 0; k < kNB; k += 4) {
-    const double av = P[(16 * w + li) * kLd + k + lk];
-#pragma unroll
-    for (int cb = k / 16; cb < 4; cb++)
-      acc[cb] = mfma4(av, D[(16 * cb + li) * kLd + k + lk], acc[cb]);
+  for (int k = 0; k < 16 * (C1 + 1); k += 4) {
+    const double av = P[(16 * rb + li) * kLd + k + lk];
+    if (k < 16 * (C0 + 1)) q[0] = mfma4(av, D[(16 * C0 + li) * kLd + k + lk], q[0]);
+    q[1] = mfma4(av, D[(16 * C1 + li) * kLd + k + lk], q[1]);
   }
+}
+
+// acc_b -= (row block rb_b of X) (row block cb_b of Y)^T, b < NB
+template <int NB>
+__device__ __forceinline__ void update_blocks(const double *X, const double *Y,
+                                              const int (&rb)[2], const int (&cb)[2], int lane,
+                                              double4_t (&acc)[2]) {
+  const int li = lane & 15, lk = lane >> 4;
 #pragma unroll
-  for (int cb = 0; cb < 4; cb++)
+  for (int k = 0; k < kNB; k += 4)
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int r = 16 * w + lk + 4 * v, c = 16 * cb + li;
-      P[r * kLd + c] = acc[cb][v];
-      if (out) out[(int64_t)r * np + c] = acc[cb][v];
-    }
+    for (int b = 0; b < NB; b++)
+      acc[b] = mfma4(-X[(16 * rb[b] + li) * kLd + k + lk], Y[(16 * cb[b] + li) * kLd + k + lk],
+                     acc[b]);
 }
 
 // One task of an elimination step (one workgroup): the trailing tile (I, J),
@@ -332,23 +354,28 @@ __device__ __forceinline__ void panel_product(double *P, const double *D, int w,
 // this step,
 //   C_IJ = A_IJ - sum_K Q_IK Q_JK^T,   Q_XK = A_XK L_KK^{-T}
 // (each workgroup forms the two panel tiles it needs on MFMA).  C is loaded
-// into the accumulators: a 32x32 quadrant per wave, or for a diagonal tile,
-// of which only the 16x16 blocks on and below the diagonal are used, 2 or 3
-// of those blocks.  The task of a diagonal tile (I, I) also writes
+// into the accumulators: two 16x16 blocks per wave, or for a diagonal tile, of
+// which only the blocks on and below the diagonal are used, one or two of those.
+// Eight waves, two to a SIMD: alone on its SIMD a wave reaches half the FP64 MFMA
+// rate (a diagonal task's product and update took 13,400 cycles with four waves,
+// 9,900 with eight).  The task of a diagonal tile (I, I) also writes
 // L_IK = Q_IK.  With kTaskFactor the tile is complete after this update and
 // is factored in LDS right away (Cholesky, then the inverse of the 64x64
 // factor, which goes to Dinv); nsrc = 0 factors A_II as it is.
 // Matrices are np x np row-major, np a multiple of 64.
 // Latency bound: a launch takes as long as its longest chain of loads,
 // products and one factorization.
-__global__ __launch_bounds__(256) void k_chol_task(double *__restrict__ A, double *__restrict__ Lf,
+__global__ __launch_bounds__(512) void k_chol_task(double *__restrict__ A, double *__restrict__ Lf,
                                                    double *__restrict__ Dinv, int np,
                                                    const CholTask *__restrict__ tasks,
                                                    int *__restrict__ info) {
-  __shared__ double PI[kNB * kLd];
-  __shared__ double PJ[kNB * kLd];
-  __shared__ double DV[kNB * kLd];
-  __shared__ double inv[kNB];
+  __shared__ __align__(16) double PI[kNB * kLd];
+  __shared__ __align__(16) double PJ[kNB * kLd];
+  __shared__ __align__(16) double DV[kNB * kLd];
+  __shared__ __align__(16) double inv[kNB];
+  // the elimination is the set-up's critical path: its waves go first where they
+  // share a SIMD with those of the rows of W
+  __builtin_amdgcn_s_setprio(3);
   const CholTask tk = tasks[blockIdx.x];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int li = lane & 15, lk = lane >> 4;
@@ -356,25 +383,29 @@ __global__ __launch_bounds__(256) void k_chol_task(double *__restrict__ A, doubl
   const int64_t gi = (int64_t)tk.I * kNB, gj = (int64_t)tk.J * kNB;
   double *Cg = A + gi * np + gj;
   // the wave's blocks of the target: of a diagonal tile (row, column) blocks
-  // (0,0) (3,3) | (1,0) (1,1) | (2,0) (2,1) (2,2) | (3,0) (3,1) (3,2), else
-  // the quadrant's four
-  int rb[4], cb[4];
-  const int nb = diag ? (w < 2 ? 2 : 3) : 4;
-#pragma unroll
-  for (int b = 0; b < 4; b++) {
-    rb[b] = diag ? (w == 0 ? 3 * (b & 1) : w) : (w & 2) + (b >> 1);
-    cb[b] = diag ? (w == 0 ? 3 * (b & 1) : b) : 2 * (w & 1) + (b & 1);
+  // (0,0) (1,1) | (1,0) (2,2) | (2,0) | (2,1) | (3,0) | (3,1) | (3,2) | (3,3),
+  // else two neighbours of a row
+  int rb[2], cb[2];
+  const int nb = diag && w >= 2 ? 1 : 2;
+  if (diag) {
+    rb[0] = w < 2 ? w : w < 4 ? 2 : 3;
+    cb[0] = w < 2 ? 0 : w < 4 ? w - 2 : w - 4;
+    rb[1] = cb[1] = w + 1;
+  } else {
+    rb[0] = rb[1] = w >> 1;
+    cb[0] = 2 * (w & 1);
+    cb[1] = cb[0] + 1;
   }
   if (fac) {
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int e = tid + 256 * q;
-      PJ[(e >> 6) * kLd + (e & 63)] = 0.0;
+    for (int q = 0; q < 4; q++) {
+      const int e = 2 * tid + 1024 * q;
+      pair_store(PJ + (e >> 6) * kLd + (e & 63), 0.0, 0.0);
     }
   }
-  double4_t acc[4];
+  double4_t acc[2];
 #pragma unroll
-  for (int b = 0; b < 4; b++)
+  for (int b = 0; b < 2; b++)
     if (b < nb) {
 #pragma unroll
       for (int v = 0; v < 4; v++)
@@ -384,53 +415,51 @@ __global__ __launch_bounds__(256) void k_chol_task(double *__restrict__ A, doubl
     const int64_t gk = (int64_t)tk.K[s] * kNB;
     // stage A_IK, A_JK and L_KK^{-1}; all loads of a thread are issued before
     // its LDS stores
-    double ri[16], rj[16], rd[16];
+    double2 ri[4], rj[4], rd[4];
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int e = tid + 256 * q, r = e >> 6, c = e & 63;
-      ri[q] = A[(gi + r) * np + gk + c];
-      rj[q] = diag ? 0.0 : A[(gj + r) * np + gk + c];
-      rd[q] = Dinv[(int64_t)tk.K[s] * kNB * kNB + e];
+    for (int q = 0; q < 4; q++) {
+      const int e = 2 * tid + 1024 * q, r = e >> 6, c = e & 63;
+      ri[q] = *reinterpret_cast<const double2 *>(A + (gi + r) * np + gk + c);
+      if (!diag) rj[q] = *reinterpret_cast<const double2 *>(A + (gj + r) * np + gk + c);
+      rd[q] = *reinterpret_cast<const double2 *>(Dinv + (int64_t)tk.K[s] * kNB * kNB + e);
     }
-    __syncthreads();  // the previous source's products are done with the tiles
+    lds_barrier();  // the previous source's products are done with the tiles
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int e = tid + 256 * q, o = (e >> 6) * kLd + (e & 63);
-      PI[o] = ri[q];
-      if (!diag) PJ[o] = rj[q];
-      DV[o] = rd[q];
+    for (int q = 0; q < 4; q++) {
+      const int e = 2 * tid + 1024 * q, o = (e >> 6) * kLd + (e & 63);
+      pair_store(PI + o, ri[q].x, ri[q].y);
+      if (!diag) pair_store(PJ + o, rj[q].x, rj[q].y);
+      pair_store(DV + o, rd[q].x, rd[q].y);
     }
-    __syncthreads();
-    // Q_I = A_IK L_KK^{-T}
-    panel_product(PI, DV, w, lane, diag ? Lf + gi * np + gk : nullptr, np);
-    if (!diag) panel_product(PJ, DV, w, lane, nullptr, np);
-    __syncthreads();
-    const double *Y = diag ? PI : PJ;
-    if (diag) {
-#pragma unroll 4
-      for (int k = 0; k < kNB; k += 4)
-#pragma unroll
-        for (int b = 0; b < 3; b++)
-          if (b < nb)
-            acc[b] = mfma4(-PI[(16 * rb[b] + li) * kLd + k + lk],
-                           Y[(16 * cb[b] + li) * kLd + k + lk], acc[b]);
+    lds_barrier();
+    // Q_I = A_IK L_KK^{-T}, Q_J
+    double4_t qi[2], qj[2];
+    const int pr = w & 3, pc = w < 4 ? 0 : 1;  // blocks (pr, pc) and (pr, 3 - pc)
+    if (w < 4) {
+      panel_product<0, 3>(PI, DV, pr, lane, qi);
+      if (!diag) panel_product<0, 3>(PJ, DV, pr, lane, qj);
     } else {
-#pragma unroll 4
-      for (int k = 0; k < kNB; k += 4) {
-        double av[2], bv[2];
-#pragma unroll
-        for (int x = 0; x < 2; x++) {
-          av[x] = -PI[(16 * rb[2 * x] + li) * kLd + k + lk];
-          bv[x] = Y[(16 * cb[x] + li) * kLd + k + lk];
-        }
-#pragma unroll
-        for (int b = 0; b < 4; b++) acc[b] = mfma4(av[b >> 1], bv[b & 1], acc[b]);
-      }
+      panel_product<1, 2>(PI, DV, pr, lane, qi);
+      if (!diag) panel_product<1, 2>(PJ, DV, pr, lane, qj);
     }
-  }
-  if (fac) __syncthreads();  // L_KK^{-1} is done with, X is cleared
+    lds_barrier();  // the tiles are read: Q takes their place
 #pragma unroll
-  for (int b = 0; b < 4; b++)
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int r = 16 * pr + lk + 4 * v, c = 16 * (b ? 3 - pc : pc) + li;
+        PI[r * kLd + c] = qi[b][v];
+        if (diag) Lf[(gi + r) * np + gk + c] = qi[b][v];
+        else PJ[r * kLd + c] = qj[b][v];
+      }
+    lds_barrier();
+    const double *Y = diag ? PI : PJ;
+    if (nb == 2) update_blocks<2>(PI, Y, rb, cb, lane, acc);
+    else update_blocks<1>(PI, Y, rb, cb, lane, acc);
+  }
+  if (fac) lds_barrier();  // L_KK^{-1} is done with, X is cleared
+#pragma unroll
+  for (int b = 0; b < 2; b++)
     if (b < nb) {
 #pragma unroll
       for (int v = 0; v < 4; v++) {
@@ -440,12 +469,14 @@ __global__ __launch_bounds__(256) void k_chol_task(double *__restrict__ A, doubl
       }
     }
   if (!fac) return;
-  __syncthreads();
+  lds_barrier();
   factor_tile(DV, PJ, inv, info);
 #pragma unroll
-  for (int q = 0; q < 16; q++) {
-    const int e = tid + 256 * q;
-    Dinv[(int64_t)tk.I * kNB * kNB + e] = PJ[(e >> 6) * kLd + (e & 63)];
+  for (int q = 0; q < 4; q++) {
+    const int e = 2 * tid + 1024 * q;
+    double2 x;
+    pair_load(PJ + (e >> 6) * kLd + (e & 63), x.x, x.y);
+    *reinterpret_cast<double2 *>(Dinv + (int64_t)tk.I * kNB * kNB + e) = x;
   }
 }
 
@@ -456,8 +487,8 @@ __global__ __launch_bounds__(256) void k_chol_task(double *__restrict__ A, doubl
 // rows I of the reach of J,
 //   W_I = -L_II^{-1} sum_{K in ks(I)} L_IK W_K,
 // ks(I) the strip's earlier rows with L_IK != 0 (lists from the elimination
-// schedule).  k_linv_sums leaves the terms of the lower levels in W_I, one
-// workgroup per row and strip; k_linv_rows adds those of the row's own level
+// schedule).  k_linv_sums leaves the terms of the lower levels in W_I, level by
+// level as their rows are there; k_linv_rows adds those of the row's own level
 // (at most the tiles of a plane; all of them for a band), row by row, and
 // multiplies by L_II^{-1}.  (One launch after the factorization that walked
 // all rows of a strip took 270 us at coarse 16x8x8.)  W is always written;
@@ -506,24 +537,91 @@ __device__ __forceinline__ double4_t linv_terms(const double *__restrict__ Lf, c
   return acc0 + acc1;
 }
 
-// blockIdx.x: strip, blockIdx.y: its row within the level
-__global__ __launch_bounds__(256) void k_linv_sums(const double *__restrict__ Lf, int np,
+// The terms of level `from` in the rows of the levels above it, added to what the
+// lower levels left there: blockIdx.x, tile column J; blockIdx.z, the level;
+// blockIdx.y, the row of J in it.  A workgroup forms the 64x64 tile, a wave 16
+// rows and 32 columns of it: two waves to a SIMD, which the FP64 MFMA rate takes,
+// and W_KJ staged once per term in LDS.  (All terms of a row after the level
+// below it, by strips of 16 columns with L_IK loaded again for each, took 64 us
+// for the last level at coarse 16x8x8; its terms of the level below alone 29.)
+__global__ __launch_bounds__(512) void k_linv_sums(const double *__restrict__ Lf, int np,
                                                    const int2 *__restrict__ colinfo,
+                                                   const int *__restrict__ tile_level, int from,
                                                    const int4 *__restrict__ rows,
                                                    const int *__restrict__ klist, double *W) {
-  const int c0 = blockIdx.x * kStrip;
-  const int2 ci = colinfo[c0 / kNB];
+  constexpr int kLdB = kNB + 1;  // rows 16 apart in the other half of the banks
+  __shared__ double Bs[2][kNB * kLdB];
+  const int J = blockIdx.x;
+  const int2 ci = colinfo[(size_t)(from + 1 + blockIdx.z) * gridDim.x + J];
   if ((int)blockIdx.y >= ci.y) return;
   const int4 rw = rows[ci.x + blockIdx.y];
-  if (rw.w == 0) return;
-  const int rb = threadIdx.x >> 6, lane = threadIdx.x & 63, gc = c0 + (lane & 15);
-  const double4_t acc = linv_terms(Lf, W, np, rw.x, klist + rw.y, 0, rw.w, 1, rb, gc);
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int rb = w & 3, c0 = 32 * (w >> 2) + li;
+  // the row's terms are in the order of the levels: those of `from`
+  int t0 = 0, t1 = 0;
+  for (int q = 0; q < rw.w; q += 64) {
+    const int lev = q + lane < rw.w ? tile_level[klist[rw.y + q + lane]] : from + 1;
+    t0 += __popcll(__ballot(lev < from));
+    t1 += __popcll(__ballot(lev <= from));
+  }
+  if (t0 == t1) return;
+  const int *ks = klist + rw.y;
+  // lane l feeds k = 16 (l / 16) + q of MFMA step q: a run of 128 bytes of L_IK
+  const double *pa = Lf + ((int64_t)rw.x * kNB + 16 * rb + li) * np + 16 * lk;
+  double2 a[8], na[8], nb[4];
+  auto load = [&](int K) {
 #pragma unroll
-  for (int v = 0; v < 4; v++)
-    W[((int64_t)rw.x * kNB + 16 * rb + (lane >> 4) + 4 * v) * np + gc] = acc[v];
+    for (int q = 0; q < 8; q++)
+      na[q] = reinterpret_cast<const double2 *>(pa + (int64_t)K * kNB)[q];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int e = 2 * tid + 1024 * q;
+      nb[q] = *reinterpret_cast<const double2 *>(W + ((int64_t)K * kNB + (e >> 6)) * np +
+                                                 (int64_t)J * kNB + (e & 63));
+    }
+  };
+  double4_t acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+  load(ks[t0]);
+  double *out = W + ((int64_t)rw.x * kNB + 16 * rb + lk) * np + (int64_t)J * kNB + c0;
+  if (t0 > 0) {
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) acc[b][v] = out[(int64_t)(4 * v) * np + 16 * b];
+  }
+  for (int t = t0; t < t1; t++) {
+    double *B = Bs[t & 1];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int e = 2 * tid + 1024 * q;
+      double *b = B + (e >> 6) * kLdB + (e & 63);
+      b[0] = nb[q].x;
+      b[1] = nb[q].y;
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++) a[q] = na[q];
+    lds_barrier();  // (the buffer before last is read: every wave has passed the last barrier)
+    if (t + 1 < t1) load(ks[t + 1]);
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const double av = q & 1 ? a[q / 2].y : a[q / 2].x;
+      const double *b = B + (16 * lk + q) * kLdB + c0;
+      acc[0] = mfma4(av, b[0], acc[0]);
+      acc[1] = mfma4(av, b[16], acc[1]);
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) out[(int64_t)(4 * v) * np + 16 * b] = acc[b][v];
 }
 
 constexpr int kLinvGroups = 2;  // groups of 4 waves, which take alternate terms
+// Rows of a column in a level up to which its part of W stays in LDS (a plane's
+// tiles).  A row needs the one before it: read back from memory the four of the
+// last level took 43 us at coarse 16x8x8, 34 from LDS, with all lists loaded at
+// the start and the next row's L meanwhile.
+constexpr int kLinvOwn = 4;
 
 __global__ __launch_bounds__(256 * kLinvGroups) void k_linv_rows(
     const double *__restrict__ Lf, const double *__restrict__ Dinv, int np,
@@ -531,6 +629,7 @@ __global__ __launch_bounds__(256 * kLinvGroups) void k_linv_rows(
     const int4 *__restrict__ rows, const int *__restrict__ klist, double *W,
     double *__restrict__ WT, float *__restrict__ W32, float *__restrict__ WT32) {
   __shared__ double Bx[kLinvGroups][kNB * 17];
+  __shared__ double Own[kLinvOwn + 1][kNB * 17];  // W_JJ, then the rows
   const int tid = threadIdx.x, grp = tid >> 8, rb = (tid >> 6) & 3, lane = tid & 63;
   const int li = lane & 15, lk = lane >> 4;
   const int c0 = blockIdx.x * kStrip, J = c0 / kNB, cofs = c0 - J * kNB;
@@ -546,11 +645,97 @@ __global__ __launch_bounds__(256 * kLinvGroups) void k_linv_rows(
   if (tile_level[J] == level) {
     for (int e = tid; e < kNB * kStrip; e += 256 * kLinvGroups) {
       const int r = e >> 4, j = e & 15;
-      put((int64_t)J * kNB + r, c0 + j, Dinv[(int64_t)J * kNB * kNB + r * kNB + cofs + j]);
+      const double v = Dinv[(int64_t)J * kNB * kNB + r * kNB + cofs + j];
+      put((int64_t)J * kNB + r, c0 + j, v);
+      Own[0][r * 17 + j] = v;
     }
     __syncthreads();
   }
   const int2 ci = colinfo[J];
+  if (ci.y <= kLinvOwn) {
+    // the rows, and this group's terms of each, at most two: all lists at once
+    int4 rws[kLinvOwn];
+    int Ks[kLinvOwn][2], slots[kLinvOwn][2];
+#pragma unroll
+    for (int q = 0; q < kLinvOwn; q++) rws[q] = q < ci.y ? rows[ci.x + q] : int4{0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < kLinvOwn; q++)
+#pragma unroll
+      for (int x = 0; x < 2; x++) {
+        const int t = rws[q].w + grp + kLinvGroups * x;
+        Ks[q][x] = t < rws[q].z ? klist[rws[q].y + t] : -1;
+      }
+#pragma unroll
+    for (int q = 0; q < kLinvOwn; q++)
+#pragma unroll
+      for (int x = 0; x < 2; x++) {  // the place of W_K: 0, K = J
+        slots[q][x] = Ks[q][x] < 0 ? -1 : 0;
+#pragma unroll
+        for (int p = 0; p < q; p++)
+          if (Ks[q][x] >= 0 && rws[p].x == Ks[q][x]) slots[q][x] = p + 1;
+      }
+    double2 a[2][8];
+    double4_t sum;
+    auto load = [&](const int4 &rw, const int (&K)[2]) {
+#pragma unroll
+      for (int x = 0; x < 2; x++)
+        if (K[x] >= 0) {
+          const double2 *pa = reinterpret_cast<const double2 *>(
+              Lf + ((int64_t)rw.x * kNB + 16 * rb + li) * np + (int64_t)K[x] * kNB + 16 * lk);
+#pragma unroll
+          for (int m = 0; m < 8; m++) a[x][m] = pa[m];
+        }
+      sum = double4_t{0.0, 0.0, 0.0, 0.0};
+      if (grp == 0 && rw.w > 0) {
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          sum[v] = W[((int64_t)rw.x * kNB + 16 * rb + lk + 4 * v) * np + gc];
+      }
+    };
+    load(rws[0], Ks[0]);
+#pragma unroll
+    for (int q = 0; q < kLinvOwn; q++) {
+      if (q >= ci.y) break;
+      const int I = rws[q].x;
+      double dreg[16];
+      if (grp == 0) {
+        const double *D = Dinv + (int64_t)I * kNB * kNB;
+#pragma unroll
+        for (int t = 0; t < 16; t++)
+          dreg[t] = (4 * t < 16 * (rb + 1)) ? D[(16 * rb + li) * kNB + 4 * t + lk] : 0.0;
+      }
+      double4_t acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int x = 0; x < 2; x++)
+        if (slots[q][x] >= 0) {
+          const double *B = Own[slots[q][x]] + 16 * lk * 17 + li;
+#pragma unroll
+          for (int m = 0; m < 8; m++) {
+            acc0 = mfma4(a[x][m].x, B[34 * m], acc0);
+            acc1 = mfma4(a[x][m].y, B[34 * m + 17], acc1);
+          }
+        }
+      sum += acc0 + acc1;
+#pragma unroll
+      for (int v = 0; v < 4; v++) Bx[grp][(16 * rb + lk + 4 * v) * 17 + li] = sum[v];
+      if (q + 1 < kLinvOwn && q + 1 < ci.y) load(rws[(q + 1) % kLinvOwn], Ks[(q + 1) % kLinvOwn]);
+      lds_barrier();
+      if (grp == 0) {
+        double4_t o = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int t = 0; t < 16; t++)
+          if (4 * t < 16 * (rb + 1))
+            o = mfma4(dreg[t], Bx[0][(4 * t + lk) * 17 + li] + Bx[1][(4 * t + lk) * 17 + li], o);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          put((int64_t)I * kNB + 16 * rb + lk + 4 * v, gc, -o[v]);
+          Own[q + 1][(16 * rb + lk + 4 * v) * 17 + li] = -o[v];
+        }
+      }
+      lds_barrier();  // the row is there for the next one, Bx for its sums
+    }
+    return;
+  }
   for (int q = 0; q < ci.y; q++) {
     const int4 rw = rows[ci.x + q];
     const int I = rw.x;
@@ -778,28 +963,30 @@ void CoarseFactor::factor_async(bool f32out, hipStream_t with_w) {
   const bool f32 = f32out && W32;  // FP32 W, W^T for the mixed V-cycle, else FP64 W^T
   const int nlev = (int)level_launch.size(), nlaunch = (int)launch_first.size();
   hipStream_t sw = with_w ? with_w : s;
+  const int max_level_rows =
+      level_rows.empty() ? 0 : *std::max_element(level_rows.begin(), level_rows.end());
   auto rows_of = [&](int v) {  // level v's rows of W
     hipLaunchKernelGGL(k_linv_rows, dim3(np / kStrip), dim3(256 * kLinvGroups), 0, sw, L, Dinv, np,
                        dcolinfo + (size_t)v * nblk, dlevel, v, drows, dklist, W,
                        f32 ? nullptr : WT, f32 ? W32 : nullptr, f32 ? WT32 : nullptr);
   };
-  auto sums_of = [&](int v) {  // and their terms of the lower levels
-    if (level_rows[v] > 0)
-      hipLaunchKernelGGL(k_linv_sums, dim3(np / kStrip, level_rows[v]), dim3(256), 0, sw, L, np,
-                         dcolinfo + (size_t)v * nblk, drows, dklist, W);
+  auto sums_from = [&](int v) {  // its terms in the rows of the levels above
+    if (max_level_rows > 0)
+      hipLaunchKernelGGL(k_linv_sums, dim3(nblk, max_level_rows, nlev - 1 - v), dim3(512), 0, sw,
+                         L, np, dcolinfo, dlevel, v, drows, dklist, W);
   };
   // With a stream of its own, level v's rows of W follow the launch after the
   // level's last one (which completes L in its columns for the sums of the
   // levels above), and the last level's rows the last launch.
   int v = 0;
   for (int q = 0; q < nlaunch; q++) {
-    hipLaunchKernelGGL(k_chol_task, dim3(launch_count[q]), dim3(256), 0, s, A, L, Dinv, np,
+    hipLaunchKernelGGL(k_chol_task, dim3(launch_count[q]), dim3(512), 0, s, A, L, Dinv, np,
                        dtasks + launch_first[q], info);
     if (with_w && v + 1 < nlev && q == level_launch[v] + 1) {
       hipEventRecord(ev_level[v & 1], s);
       hipStreamWaitEvent(sw, ev_level[v & 1], 0);
       rows_of(v);
-      sums_of(++v);
+      sums_from(v++);
     }
   }
   if (with_w) {
@@ -808,7 +995,7 @@ void CoarseFactor::factor_async(bool f32out, hipStream_t with_w) {
   }
   for (; v < nlev; v++) {
     rows_of(v);
-    if (v + 1 < nlev) sums_of(v + 1);
+    if (v + 1 < nlev) sums_from(v);
   }
 }
 
