@@ -40,13 +40,16 @@ namespace t3d {
 // and invD the reciprocal of the moduli's sum at each node (k_recip_moduli)
 // kModeProlong: a sweep of in + P aux, aux the next level's vector, with invD as
 // in kModeFirst
+// kModeApplyX: apply with the densities in the place of the moduli, and zeros on
+// the padded rows of the output
 enum {
   kModeApply = 0,
   kModeJacobi = 1,
   kModeResidual = 2,
   kModeJacobiDiag = 3,
   kModeFirst = 4,
-  kModeProlong = 5
+  kModeProlong = 5,
+  kModeApplyX = 6
 };
 
 // position bits (x, y, z) of the reference's local node n (stencil_utility.h:19-26)
@@ -402,6 +405,8 @@ struct TileArgs {
   uint32_t e_bytes;      // size of the moduli (below 2^32)
   int c_wx, c_wy, c_wz;  // kModeProlong: nodes of the next level's vector
   uint32_t c_bytes;      // and its size
+  double E0, Emin;       // kModeApplyX: the moduli at densities 1 and 0
+  int wx;                // and the planes of the level
 };
 
 // The tile of a workgroup of the (slabs, tiles) grid.  The device deals
@@ -817,7 +822,8 @@ __device__ __forceinline__ void fine_march_body(
     const uint8_t *__restrict__ fix, const int *__restrict__ fixplane,
     double *__restrict__ dotp, void *__restrict__ aux) {
   constexpr bool kDiag = MODE == kModeJacobiDiag, kFirst = MODE == kModeFirst;
-  constexpr bool kProl = MODE == kModeProlong;
+  constexpr bool kProl = MODE == kModeProlong, kX = MODE == kModeApplyX;
+  constexpr bool kApply = MODE == kModeApply || kX;
   constexpr int N = march_threads<T>(), XV = kDiag ? 10 : 9;
   extern __shared__ unsigned char smem_raw[];
   T *xch = reinterpret_cast<T *>(smem_raw);  // [2][XV][N]; slot N-1: zeros
@@ -830,6 +836,7 @@ __device__ __forceinline__ void fine_march_body(
   const int i0 = 1 + w.slab * a.NX;
   const int i1 = min(i0 + a.NX - 1, a.nelx + 1);  // last output plane
   const bool elem_ok = active && ty > 0 && tz > 0 && j - 1 <= a.nely && k - 1 <= a.nelz;
+  const bool mat_ok = elem_ok && j > 1 && k > 1;  // kX: not an element of the halo
   const bool last_y = (ty == a.TY), last_z = (tz == a.TZ);
   const bool own_ok = elem_ok && (!last_y || j == a.nely + 1) && (!last_z || k == a.nelz + 1);
   // bytes of a plane of each array
@@ -856,7 +863,7 @@ __device__ __forceinline__ void fine_march_body(
   };
   const __amdgpu_buffer_rsrc_t rin = rsrc(in, a.out_bytes), re = rsrc(E, a.e_bytes);
   const __amdgpu_buffer_rsrc_t rfix = rsrc(fix, a.out_bytes / (3u * (uint32_t)sizeof(T)));
-  const __amdgpu_buffer_rsrc_t rb = rsrc(MODE == kModeApply || kFirst ? in : b, a.out_bytes);
+  const __amdgpu_buffer_rsrc_t rb = rsrc(kApply || kFirst ? in : b, a.out_bytes);
   const __amdgpu_buffer_rsrc_t rd = rsrc(MODE == kModeJacobi || kFirst || kProl ? invD : in,
                                          kFirst || kProl ? a.out_bytes / 3u : a.out_bytes);
   // the planes from plane fbase on with a fixed DOF
@@ -914,7 +921,7 @@ __device__ __forceinline__ void fine_march_body(
   auto load_node = [&](int i_) {
     const int i = min(i_, i1);
     if (kFirst) return;  // (all carried with the planes)
-    if (MODE != kModeApply) load3<T>(rb, vnode, (uint32_t)i * sv, s.bb);
+    if (!kApply) load3<T>(rb, vnode, (uint32_t)i * sv, s.bb);
     if (MODE == kModeJacobi) load3<T>(rd, vnode, (uint32_t)i * sv, s.di);
     if (kProl) s.di[0] = load1<T>(rd, vnode / 3u, (uint32_t)i * (sx * (uint32_t)sizeof(T)));
     s.m = load_mask(i, s.fixed);
@@ -1030,7 +1037,9 @@ __device__ __forceinline__ void fine_march_body(
                   const Node &u1, Node &u2) {
     constexpr int P = decltype(par)::value;
     const bool emit = i >= i0;  // uniform
-    const T Ee = copy_here(s.e);
+    T Ee = copy_here(s.e);
+    if constexpr (kX)  // (as k_young)
+      Ee = mat_ok && i >= 1 && i <= a.nelx ? T(a.Emin + (Ee * Ee * Ee) * (a.E0 - a.Emin)) : T(0);
     s.e = load_modulus(i + 1);
     get_face(1 - P, Fn, u1);
     T hh[8][3];
@@ -1127,7 +1136,7 @@ __device__ __forceinline__ void fine_march_body(
     }
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      if (MODE == kModeApply) o[c] = kin[c];
+      if (kApply) o[c] = kin[c];
       else if (MODE == kModeJacobi || kDiag || kFirst || kProl) o[c] = uo[c] + omega * dd[c] * (s.bb[c] - kin[c]);
       else o[c] = s.bb[c] - kin[c];
     }
@@ -1135,7 +1144,7 @@ __device__ __forceinline__ void fine_march_body(
       double d = dacc;
 #pragma unroll
       for (int c = 0; c < 3; c++)
-        d += (double)(MODE == kModeApply ? uo[c] : s.bb[c]) * (double)o[c];
+        d += (double)(kApply ? uo[c] : s.bb[c]) * (double)o[c];
       dacc = emit && own_ok ? d : dacc;
     }
     // (an empty resource where the plane is another workgroup's)
@@ -1184,7 +1193,7 @@ __device__ __forceinline__ void fine_march_body(
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     pin(s.p.u[c]);
-    if (MODE != kModeApply && !kFirst) pin(s.bb[c]);
+    if (!kApply && !kFirst) pin(s.bb[c]);
     if (MODE == kModeJacobi) pin(s.di[c]);
     if (kProl) pin(cz[c]);
   }
@@ -1205,6 +1214,15 @@ __device__ __forceinline__ void fine_march_body(
     const Node uz = uc;
     ub = ua;
     ua = uz;
+  }
+  if constexpr (kX) {  // the rows j > nely + 1 of every (i, k), as k_zero_pad_rows
+    const int first = a.nely + 2, npad = a.wy - first;
+    const uint32_t n = (uint32_t)a.wx * a.wz * (uint32_t)npad;
+    const uint32_t nt = gridDim.x * gridDim.y * blockDim.x;
+    for (uint32_t q = (blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + t; q < n; q += nt) {
+      T *po = at32(out, 3u * (q / npad * (uint32_t)a.wy + first + q % npad));
+      po[0] = po[1] = po[2] = 0;
+    }
   }
   if (MODE != kModeResidual && !kFirst && !kProl && dotp) {  // one partial per workgroup, fixed order
 #pragma unroll
@@ -1490,6 +1508,7 @@ static bool tile_args(const Level &L, int64_t nmod, bool available, TileArgs &a)
   a.out_bytes = (uint32_t)(sizeof(T) * 3 * L.nodes());
   a.e_bytes = (uint32_t)(sizeof(T) * nmod);
   a.stream_out = 0;
+  a.wx = L.wx;
   return true;
 }
 
@@ -1510,6 +1529,8 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
   if (!tile_args<T>(L, g.nelem, g_coef.ok0, a)) return 0;
   a.few = g.ewy;
   a.fez = g.ewz;
+  a.E0 = g.E0;
+  a.Emin = g.Emin;
   // the diagonal from the moduli needs a KE whose diagonal is one value per
   // component
   if (mode == kModeJacobiDiag && !g_coef.diag0) mode = kModeJacobi;
@@ -1548,7 +1569,7 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
   const int64_t cache = int64_t(256) << 20;
   const int64_t reads = (mode == kModeFirst   ? 4
                          : mode == kModeProlong ? 7
-                         : mode == kModeApply ? 3
+                         : mode == kModeApply || mode == kModeApplyX ? 3
                          : mode == kModeJacobi ? 9
                                                : 6) *
                             (int64_t)a.out_bytes / 3 +
@@ -1576,6 +1597,7 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
     else if (mode == kModeFirst) T3D_LAUNCH(kModeFirst, false);
     else if (mode == kModeJacobiDiag) T3D_LAUNCH(kModeJacobiDiag, false);
     else if constexpr (sizeof(T) == 4) T3D_LAUNCH(kModeProlong, false);
+    else T3D_LAUNCH(kModeApplyX, false);
   }
 #undef T3D_LAUNCH
   return dotp ? nwg : 0;
@@ -1624,6 +1646,11 @@ template <typename T>
 void launch_fine_tile(const DevGrid &g, int mode, const T *E, const T *in, T *out,
                       const T *b, const T *invD, T omega, int bcsym) {
   run_fine<T>(g, mode, E, in, out, b, invD, omega, bcsym);
+}
+
+// out = K(x) in from the densities x, zero on the padded rows
+void launch_fine_tile_apply_x(const DevGrid &g, const double *x, const double *in, double *out) {
+  run_fine<double>(g, kModeApplyX, x, in, out, nullptr, nullptr, 0.0, 0);
 }
 
 // r = b - K u and its FP32 copy when r32 is given

@@ -187,6 +187,12 @@ void launch_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
                        b, invD, omega, g.fixmask[0], bcsym);
 }
 
+bool launch_fine_apply_x(const DevGrid &g, const double *x, const double *in, double *out) {
+  if (use_node_kernel()) return false;
+  launch_fine_tile_apply_x(g, x, in, out);
+  return true;
+}
+
 void launch_fine_residual(const DevGrid &g, const double *E, const double *u, double *r,
                           float *r32, const double *b, int bcsym) {
   if (!use_node_kernel()) {

@@ -327,6 +327,10 @@ void launch_axpy_fused(int64_t n, const double *pq_part, int npart, double *scal
 // sums of b . out; returns their count (0: none written)
 void launch_fine_tile_residual(const DevGrid &g, const double *E, const double *u, double *r,
                                float *r32, const double *b, int bcsym);
+void launch_fine_tile_apply_x(const DevGrid &g, const double *x, const double *in, double *out);
+// out = K(x) in from the densities x, zero on the padded rows; false (nothing
+// done) with the node kernel
+bool launch_fine_apply_x(const DevGrid &g, const double *x, const double *in, double *out);
 // r = b - K u and its FP32 copy when r32 is given
 void launch_fine_residual(const DevGrid &g, const double *E, const double *u, double *r,
                           float *r32, const double *b, int bcsym);
