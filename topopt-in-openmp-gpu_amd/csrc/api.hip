@@ -636,12 +636,14 @@ float compute_change(DTYPE *x, DTYPE *xnew, const int nelem) {
   DevView vx, vn;
   if (!vx.open(x, sizeof(double) * nelem, true, true)) return 0;
   if (!vn.open(xnew, sizeof(double) * nelem, true, false)) return 0;
-  double *red = (double *)dalloc(sizeof(double) * (1024 + 16));
+  static_assert(kOcScratchDoubles >= 1024 + 16, "reduction scratch");
+  double *red = scratch_get();
+  if (!red) return 0;
   launch_change(nelem, (double *)vx.dev, (const double *)vn.dev, red, red + 1024);
   double h = 0;
   hipMemcpyAsync(&h, red + 1024, sizeof(double), hipMemcpyDeviceToHost, stream());
-  sync_ok();
-  dfree(red);
+  if (sync_ok()) scratch_put(red);
+  else dfree(red);
   vn.close();
   vx.close();
   return (float)h;
@@ -656,12 +658,15 @@ void update_solution(const DTYPE *x, DTYPE *xnew, const DTYPE *dv, const DTYPE *
       !vv.open(dv, sizeof(double) * nelem, true, false) ||
       !vc.open(dc, sizeof(double) * nelem, true, false))
     return;
-  double *scratch = (double *)dalloc(sizeof(double) * kOcScratchDoubles);
+  double *scratch = scratch_get();
   if (scratch) {
-    // a failure is recorded by oc_update (HIP error, or no convergence)
-    oc_update((const double *)vx.dev, (double *)vn.dev, (const double *)vv.dev,
-              (const double *)vc.dev, nelem, gval, scratch);
-    dfree(scratch);
+    // a failure is recorded by oc_update (HIP error, or no convergence); it
+    // returns a number of steps once the stream has completed its work
+    if (oc_update((const double *)vx.dev, (double *)vn.dev, (const double *)vv.dev,
+                  (const double *)vc.dev, nelem, gval, scratch) >= 0)
+      scratch_put(scratch);
+    else
+      dfree(scratch);
   }
   vc.close();
   vv.close();

@@ -223,15 +223,51 @@ bool dev_grid_quiet(const struct gridContext *gc) {
   return gc->precomputedKE && g_grids.count((const void *)gc->precomputedKE);
 }
 
+namespace {
+constexpr size_t kScratchKept = 4;
+std::vector<std::pair<int, double *>> g_scratch_free;  // (device, block), under g_gmu
+}  // namespace
+
+double *scratch_get() {
+  int dev = 0;
+  if (!hip_ok(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
+  {
+    std::lock_guard<std::mutex> lk(g_gmu);
+    for (size_t i = 0; i < g_scratch_free.size(); i++)
+      if (g_scratch_free[i].first == dev) {
+        double *p = g_scratch_free[i].second;
+        g_scratch_free.erase(g_scratch_free.begin() + i);
+        return p;
+      }
+  }
+  return (double *)dalloc_uninit(sizeof(double) * kOcScratchDoubles);
+}
+
+void scratch_put(double *p) {
+  int dev = 0;
+  if (!p) return;
+  if (hipGetDevice(&dev) == hipSuccess) {
+    std::lock_guard<std::mutex> lk(g_gmu);
+    if (!g_grids.empty() && g_scratch_free.size() < kScratchKept) {
+      g_scratch_free.push_back({dev, p});
+      return;
+    }
+  }
+  dfree(p);
+}
+
 void release_dev_grid(const struct gridContext *gc) {
   DevGrid *g = nullptr;
+  std::vector<std::pair<int, double *>> blocks;
   {
     std::lock_guard<std::mutex> lk(g_gmu);
     auto it = g_grids.find((const void *)gc->precomputedKE);
     if (it == g_grids.end()) return;
     g = it->second;
     g_grids.erase(it);
+    if (g_grids.empty()) blocks.swap(g_scratch_free);
   }
+  for (auto &b : blocks) dfree(b.second);
   hipStreamSynchronize(stream());
   for (int l = 0; l < kMaxLevels; l++) {
     dfree(g->fixmask[l]);

@@ -48,13 +48,14 @@ __device__ inline double4_t mfma4(double a, double b, double4_t c) {
 // in registers, the diagonal block's rows in each of its four rows of 16
 // lanes (so that pivot and multipliers are broadcast by DPP) and beside them
 // the rows below.  Per panel the 16 columns of the next panel are then updated
-// on MFMA by all waves, and the rest of the trailing triangle, and the
-// inverses of the finished diagonal blocks, by waves 1-3 while wave 0 factors
-// the next panel.  The off-diagonal 16x16 blocks of the inverse follow on
-// MFMA.  A tile takes 24,000 cycles (10 us), 19,000 of them the four panels;
-// with the 16x16 diagonal blocks factored on their own, each pivot column sent
-// through LDS, and panel, trailing triangle and inverses between barriers, it
-// took about twice that (a launch of one task 33 us against 23).
+// on MFMA by waves 0-2; while wave 0 factors the next panel, waves 1-3 update
+// the rest of the trailing triangle and wave 5, on another SIMD than wave 0,
+// inverts the finished diagonal block.  The off-diagonal 16x16 blocks of the
+// inverse follow on MFMA.  A tile takes 23,000 cycles (10 us), 19,000 of them
+// the four panels; with the 16x16 diagonal blocks factored on their own, each
+// pivot column sent through LDS, and panel, trailing triangle and inverses
+// between barriers, it took about twice that (a launch of one task 33 us
+// against 23, and 18 with eight waves for the products before it).
 // In: T (lower triangle, as 16x16 blocks; rows/cols beyond the matrix padded
 // with identity), X = 0.  Out: T = L (above the diagonal undefined),
 // X = L^{-1}.  A non-positive pivot sets *info (and is replaced by 1 so that

@@ -1458,8 +1458,8 @@ static TileShape march_shape(const Level &L, int64_t slots, bool f64, int &nx_fi
 // workgroups of `nthr` threads and `shm` bytes of LDS one CU holds at once.
 // A workgroup's waves are dealt over the CU's 4 SIMDs, so one SIMD holds
 // ceil(waves / 4) of them: two 9-wave workgroups need 6 wave slots on one
-// SIMD.  (Measured: the FP32 fine sweep at 91 VGPRs, 5 waves per SIMD, held
-// one 9-wave workgroup per CU and took 21% longer than at 79 VGPRs.)
+// SIMD.  (Measured: an FP32 fine sweep in 9-wave workgroups at 91 VGPRs, 5
+// waves per SIMD, held one workgroup per CU and took 21% longer than at 79.)
 static int wg_per_cu(const void *kernel, int nthr, size_t shm) {
   hipFuncAttributes at{};
   int per_simd = 4;
