@@ -603,24 +603,63 @@ void launch_jacobi_zero(const DevGrid &g, int l, const TB *b, const T *invD, T o
 // ---------------------------------------------------------------------------
 // Full-weighting restriction level l -> l+1 (stencil_methods.c:595-688):
 // weights 1, 1/2, 1/4, 1/8 by squared distance over the 3x3x3 fine patch.
+// Each lane reads 72 (FP64) of every 48 contiguous bytes of 9 rows, so a large
+// level is bound by the L1's lines (about 1,100 per wave, one per cycle), not by
+// HBM.  All 81 values are loaded before the first is used: 34.7 us from 256x128x128
+// in FP64 and 7.6 from 128x64x64 with the blocks dealt to the XCDs, against 44 and
+// 10.4 with the sums between the loads; in FP32 17.3 against 18.7.  A thread
+// marching over 4 planes, two loaded per step instead of three, took 38.5 and 19.
+// Workgroups go to the 8 XCDs in turn.  Of a grid that is a multiple of 8, XCD x
+// gets the x-th contiguous eighth, so that neighbours meet in its L2.
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nblocks) {
+  return (b & 7) * (nblocks >> 3) + (b >> 3);
+}
+
 template <typename T>
-__global__ void k_restrict(int cnx, int cny, int cnz, int cwy, int cwz, int fwy, int fwz,
-                           const T *__restrict__ fine, T *__restrict__ coarse,
-                           const T *__restrict__ invDc, T omega, T *__restrict__ zc,
-                           const int *__restrict__ pos, T *__restrict__ xs) {
+__device__ __forceinline__ void restrict_plane(const T *__restrict__ fine, int64_t node, int fwy,
+                                               T (&v)[3][9]) {
+#pragma unroll
+  for (int dz = 0; dz < 3; dz++)
+#pragma unroll
+    for (int m = 0; m < 9; m++) v[dz][m] = fine[3 * (node + (int64_t)(dz - 1) * fwy - 1) + m];
+}
+template <typename T>
+__device__ __forceinline__ void restrict_sum(const T (&v)[3][9], T w0, T (&acc)[3]) {
+#pragma unroll
+  for (int dz = 0; dz < 3; dz++)
+#pragma unroll
+    for (int dy = 0; dy < 3; dy++) {
+      const T w = w0 * (dz == 1 ? T(1) : T(0.5)) * (dy == 1 ? T(1) : T(0.5));
+#pragma unroll
+      for (int c = 0; c < 3; c++) acc[c] += w * v[dz][3 * dy + c];
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_restrict(int cnx, int cny, int cnz, int cwy, int cwz,
+                                                  int fwy, int fwz, const T *__restrict__ fine,
+                                                  T *__restrict__ coarse,
+                                                  const T *__restrict__ invDc, T omega,
+                                                  T *__restrict__ zc,
+                                                  const int *__restrict__ pos,
+                                                  T *__restrict__ xs) {
   // one thread per interior coarse node; only those are written
   // (stencil_methods.c:629-686).  With zc, also the coarse level's first
   // pre-smoothing sweep from zero, zc = omega invDc rc (as k_jacobi_zero; the
   // other nodes of zc stay zero).  With xs, also the coarse vector in the
   // storage order pos of the coarsest level's factor
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+  const int64_t t = (int64_t)blk * 256 + threadIdx.x;
   if (t >= (int64_t)cnx * cny * cnz) return;
   const int j = (int)(t % cny) + 1, k = (int)((t / cny) % cnz) + 1,
             i = (int)(t / ((int64_t)cny * cnz)) + 1;
   const int64_t cn = ((int64_t)i * cwz + k) * cwy + j;
-  const int fi = 2 * i - 1, fj = 2 * j - 1, fk = 2 * k - 1;
-  T acc[3] = {0, 0, 0}, dc[3] = {0, 0, 0};
+  const int64_t fn = ((int64_t)(2 * i - 1) * fwz + (2 * k - 1)) * fwy + (2 * j - 1);
+  const int64_t fplane = (int64_t)fwz * fwy;
+  T v[3][3][9], acc[3] = {0, 0, 0}, dc[3] = {0, 0, 0};
   int ps[3] = {0, 0, 0};
+#pragma unroll
+  for (int dx = 0; dx < 3; dx++) restrict_plane(fine, fn + (dx - 1) * fplane, fwy, v[dx]);
   // (loaded with the fine values, not after them)
   if (zc) {
 #pragma unroll
@@ -631,20 +670,9 @@ __global__ void k_restrict(int cnx, int cny, int cnz, int cwy, int cwz, int fwy,
     for (int c = 0; c < 3; c++) ps[c] = pos[3 * t + c];
   }
 #pragma unroll
-  for (int dx = -1; dx <= 1; dx++)
+  for (int dx = 0; dx < 3; dx++) restrict_sum(v[dx], dx == 1 ? T(1) : T(0.5), acc);
 #pragma unroll
-    for (int dz = -1; dz <= 1; dz++)
-#pragma unroll
-      for (int dy = -1; dy <= 1; dy++) {
-        const int d2 = dx * dx + dy * dy + dz * dz;
-        const T w = d2 == 0 ? T(1) : (d2 == 1 ? T(0.5) : (d2 == 2 ? T(0.25) : T(0.125)));
-        const int64_t fnode = ((int64_t)(fi + dx) * fwz + (fk + dz)) * fwy + (fj + dy);
-#pragma unroll
-        for (int c = 0; c < 3; c++) acc[c] += w * fine[3 * fnode + c];
-      }
-  coarse[3 * cn] = acc[0];
-  coarse[3 * cn + 1] = acc[1];
-  coarse[3 * cn + 2] = acc[2];
+  for (int c = 0; c < 3; c++) coarse[3 * cn + c] = acc[c];
   if (zc) {
 #pragma unroll
     for (int c = 0; c < 3; c++) zc[3 * cn + c] = omega * dc[c] * (acc[c] - T(0));
@@ -660,42 +688,46 @@ void launch_restrict(const DevGrid &g, int l, const T *fine, T *coarse, const T 
                      T omega, T *zc, const CoarseFactor *cf) {
   const Level &C = g.lv[l + 1], &F = g.lv[l];
   const int64_t nth = C.interior_nodes();
-  hipLaunchKernelGGL((k_restrict<T>), dim3((nth + 255) / 256), dim3(256), 0, stream(), C.nx,
-                     C.ny, C.nz, C.wy, C.wz, F.wy, F.wz, fine, coarse, invDc, omega, zc,
-                     cf ? cf->pos : nullptr, cf ? cf->cw<T>() : nullptr);
+  hipLaunchKernelGGL((k_restrict<T>), dim3((unsigned)((nth + 2047) / 2048 * 8)), dim3(256), 0,
+                     stream(), C.nx, C.ny, C.nz, C.wy, C.wz, F.wy, F.wz, fine, coarse, invDc,
+                     omega, zc, cf ? cf->pos : nullptr, cf ? cf->cw<T>() : nullptr);
 }
 
 // Trilinear prolongation level l+1 -> l (stencil_methods.c:521-590);
 // ADD = true fuses the correction z += P zc of the V-cycle.
-// A thread has the fine nodes 2J-1 and 2J of a row, 48 or 24 contiguous bytes,
-// loaded with the coarse nodes: per fine node the sum runs over the same 8
-// terms in the same order as stencil_methods.c:546-589.  Bound by memory on large
-// levels (219 MB in FP64 at 256x128x128: 62 us, 26 in FP32), by latency on small
-// ones (17x9x9 nodes: 3.7 us; 6 with a thread per coarse node, whose 8 fine nodes
-// were loaded one after the other).
+// A thread has the fine nodes 2J-1 and 2J of the rows 2K-1 and 2K, 48 or 24
+// contiguous bytes each, loaded with the 8 coarse nodes: per fine node the sum runs
+// over the same 8 terms in the same order as stencil_methods.c:546-589.  Bound by
+// memory on large levels (219 MB in FP64 at 256x128x128: 53 us; 61 with a pair of
+// one row per thread, which loads the coarse nodes twice as often), by latency on
+// small ones (17x9x9 nodes: 3.7 us; 6 with a thread per coarse node, whose 8 fine
+// nodes were loaded one after the other).
 template <typename T, bool ADD>
-__global__ __launch_bounds__(256) void k_prolong(int cny, int cwy, int cwz, int fnx, int fny,
+__global__ __launch_bounds__(256) void k_prolong(int cny, int cnz, int cwy, int cwz, int fnx, int fny,
                                                  int fnz, int fwy, int fwz,
                                                  const T *__restrict__ coarse,
                                                  T *__restrict__ fine) {
-  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t t = xcd_block(blockIdx.x, gridDim.x) * 256u + threadIdx.x;
   const uint32_t row = t / (uint32_t)cny;
-  const int J = (int)(t - row * cny) + 1, k = (int)(row % (uint32_t)fnz) + 1,
-            i = (int)(row / (uint32_t)fnz) + 1;
+  const int J = (int)(t - row * cny) + 1, K = (int)(row % (uint32_t)cnz) + 1,
+            i = (int)(row / (uint32_t)cnz) + 1;
   if (i > fnx) return;
-  T *pf = fine + 3 * (((int64_t)i * fwz + k) * fwy + 2 * J - 1);
-  const bool two = 2 * J <= fny;  // the row's last pair is one node
-  T z[2][3] = {{0, 0, 0}, {0, 0, 0}};
+  T *pf = fine + 3 * (((int64_t)i * fwz + 2 * K - 1) * fwy + 2 * J - 1);
+  // the last pair of a row, and of rows, is one
+  const bool have[2] = {true, 2 * J <= fny}, rows[2] = {true, 2 * K <= fnz};
+  T z[2][2][3] = {};
   if (ADD) {
 #pragma unroll
-    for (int c = 0; c < 3; c++) z[0][c] = pf[c];
-    if (two) {
+    for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-      for (int c = 0; c < 3; c++) z[1][c] = pf[3 + c];
-    }
+      for (int bb = 0; bb < 2; bb++)
+        if (rows[kk] && have[bb]) {
+#pragma unroll
+          for (int c = 0; c < 3; c++) z[kk][bb][c] = pf[3 * (kk * fwy + bb) + c];
+        }
   }
-  // coarse nodes (i-1)/2+1 and i/2+1, the same in z; J and J+1
-  const int ic[2] = {(i - 1) / 2 + 1, i / 2 + 1}, kc[2] = {(k - 1) / 2 + 1, k / 2 + 1};
+  // coarse nodes (i-1)/2+1 and i/2+1, K and K+1, J and J+1
+  const int ic[2] = {(i - 1) / 2 + 1, i / 2 + 1};
   T cv[2][2][2][3];  // [di][dk][dj][comp]
 #pragma unroll
   for (int di = 0; di < 2; di++)
@@ -703,36 +735,40 @@ __global__ __launch_bounds__(256) void k_prolong(int cny, int cwy, int cwz, int 
     for (int dk = 0; dk < 2; dk++)
 #pragma unroll
       for (int dj = 0; dj < 2; dj++) {
-        const T *pc = coarse + 3 * (((int64_t)ic[di] * cwz + kc[dk]) * cwy + J + dj);
+        const T *pc = coarse + 3 * (((int64_t)ic[di] * cwz + K + dk) * cwy + J + dj);
 #pragma unroll
         for (int c = 0; c < 3; c++) cv[di][dk][dj][c] = pc[c];
       }
 #pragma unroll
-  for (int bb = 0; bb < 2; bb++) {
-    const int q[8][3] = {{0, 0, bb}, {1, 0, bb}, {1, 0, 0}, {0, 0, 0},
-                         {0, 1, bb}, {1, 1, bb}, {1, 1, 0}, {0, 1, 0}};
+  for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-      T s = 0;
+    for (int bb = 0; bb < 2; bb++) {
+      const int q[8][3] = {{0, 0, bb}, {1, 0, bb}, {1, 0, 0}, {0, 0, 0},
+                           {0, kk, bb}, {1, kk, bb}, {1, kk, 0}, {0, kk, 0}};
 #pragma unroll
-      for (int m = 0; m < 8; m++) s += T(0.125) * cv[q[m][0]][q[m][1]][q[m][2]][d];
-      z[bb][d] = ADD ? z[bb][d] + s : s;
+      for (int d = 0; d < 3; d++) {
+        T s = 0;
+#pragma unroll
+        for (int m = 0; m < 8; m++) s += T(0.125) * cv[q[m][0]][q[m][1]][q[m][2]][d];
+        z[kk][bb][d] = ADD ? z[kk][bb][d] + s : s;
+      }
     }
-  }
 #pragma unroll
-  for (int c = 0; c < 3; c++) pf[c] = z[0][c];
-  if (two) {
+  for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-    for (int c = 0; c < 3; c++) pf[3 + c] = z[1][c];
-  }
+    for (int bb = 0; bb < 2; bb++)
+      if (rows[kk] && have[bb]) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) pf[3 * (kk * fwy + bb) + c] = z[kk][bb][c];
+      }
 }
 
 template <typename T, bool ADD>
 static void launch_prolong_t(const DevGrid &g, int l, const T *coarse, T *fine) {
   const Level &C = g.lv[l + 1], &F = g.lv[l];
-  const int64_t nth = (int64_t)F.nx * F.nz * C.ny;
-  hipLaunchKernelGGL((k_prolong<T, ADD>), dim3((unsigned)((nth + 255) / 256)), dim3(256), 0,
-                     stream(), C.ny, C.wy, C.wz, F.nx, F.ny, F.nz, F.wy, F.wz, coarse, fine);
+  const int64_t nth = (int64_t)F.nx * C.nz * C.ny;
+  hipLaunchKernelGGL((k_prolong<T, ADD>), dim3((unsigned)((nth + 2047) / 2048 * 8)), dim3(256), 0,
+                     stream(), C.ny, C.nz, C.wy, C.wz, F.nx, F.ny, F.nz, F.wy, F.wz, coarse, fine);
 }
 template <typename T>
 void launch_prolong_add(const DevGrid &g, int l, const T *coarse, T *fine) {
