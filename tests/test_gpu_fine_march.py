@@ -124,3 +124,28 @@ def test_vcycle_tiles(shape, tile, precision, monkeypatch):
     _, _, got = vcycle_of_load(g, shape[1])
     assert relerr(got, ref) <= 1e-12
     g.close()
+
+
+# The level-1 shapes that the rule takes (narrow tiles, 65 x 7 and its clipped
+# forms) and a wide tile for all: the same operands in the same order per node,
+# so the operator's 1e-13 holds between them with room
+@pytest.mark.parametrize("shape,nl", [((168, 72, 104), 4), ((200, 120, 88), 4), ((48, 48, 48), 4),
+                                      ((96, 96, 48), 4), ((64, 32, 32), 3), ((512, 16, 24), 3),
+                                      ((12, 132, 28), 3)])
+def test_level1_shapes(shape, nl, monkeypatch):
+    print(f"[gpu fine march] level 1 {shape}", flush=True)
+    g = top3d_amd.Grid(*shape, nl, precision="mixed")
+    rng = np.random.default_rng(shape[1])
+    x = g.density(rng.uniform(0.1, 1.0, g.nelx * g.nely * g.nelz))
+    v, b = (torch.from_numpy(rng.standard_normal(g.ndof(1))).cuda() for _ in range(2))
+    inv = g.invdiag(x, 1)
+
+    def results():
+        return (g.apply_level(1, x, v).cpu().numpy(),
+                g.apply_level_f32(1, x, v.float()).cpu().numpy(),
+                g.jacobi(x, 2, inv, v.clone(), b, l=1).cpu().numpy())
+    got = results()
+    monkeypatch.setenv("TOP3D_TILE_L1", "47,9,0")
+    for a, r, tol in zip(got, results(), (TOL64, TOL32, TOL_SWEEP)):
+        assert relerr(a, r) <= tol
+    g.close()

@@ -1366,30 +1366,18 @@ static void set_tiles(TileShape &s, const Level &L, int ty, int tz) {
   s.ntz = tiles(L.nz, s.TZ);
 }
 
-// Level 1: tile of TY x TZ element columns marching over NX node planes.  LDS
-// holds two exchange buffers of 9 values per thread (under 80 KiB).  Tuning
-// override: TOP3D_TILE_L1=TY,TZ,NX (NX = 0: from the occupancy).
-//
-// Shapes measured on MI355X at 128x64x64: 65 x 7 with the x-march length below
-// ran 15.5 us in FP32 and 23.6 us in FP64 (repeated on one buffer set; 20.6 and
-// 33.7 us with the memory-side cache flushed) against 15.8 / 27.1 us for
-// 65 x 11 (NX 4, FP32) and 65 x 6 (NX 8, FP64), and 15.8-19.3 / 24.3-30.5 us
-// for 65 x 3/5/6/11, 33 x 6/9/11/12/15/21 and 17 x 12/23.
-static TileShape level1_shape(const Level &L, int elem_bytes, int &nx_fixed) {
-  TileShape s{};
-  const int lds_threads = 80 * 1024 / (18 * elem_bytes);
-  // launch bounds: 1024 threads in FP32, 512 in FP64
-  const int max_threads = std::min(elem_bytes == 4 ? 1024 : 512, lds_threads);
-  set_tiles(s, L, 65, std::min(7, max_threads / std::max(2, std::min(L.nely + 1, 65))));
-  nx_fixed = 0;
-  const char *env = std::getenv("TOP3D_TILE_L1");
-  int oy = 0, oz = 0, ox = 0;
-  if (env && std::sscanf(env, "%d,%d,%d", &oy, &oz, &ox) == 3 && oy >= 2 && oz >= 2 && ox >= 0 &&
-      oy * oz <= max_threads) {
-    set_tiles(s, L, oy, oz);
-    nx_fixed = ox;
+static int device_cus() {
+  static int ncu[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!ncu[dev]) {
+    int v = 0;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        v <= 0)
+      v = 256;
+    ncu[dev] = v;
   }
-  return s;
+  return ncu[dev];
 }
 
 // The x-march length follows from the number of workgroups the device holds at
@@ -1420,6 +1408,86 @@ static int64_t tile_x(TileShape &s, const Level &L, int nx_fixed, int64_t slots)
   return best_cost;
 }
 
+// The last shapes that a thread's launches asked for, by the values they follow
+// from: a search takes 2-4 us, as long as a small level's launch.
+struct ShapeMemo {
+  struct Entry {
+    int nx = 0, ny = 0, nz = 0, kind = 0;
+    int64_t slots = 0;
+    TileShape s{};
+  } e[8];
+  int next = 0;
+  template <typename F>
+  const TileShape &get(const Level &L, int kind, int64_t slots, F search) {
+    for (Entry &v : e)
+      if (v.nx == L.nx && v.ny == L.ny && v.nz == L.nz && v.kind == kind && v.slots == slots)
+        return v.s;
+    Entry &v = e[next];
+    next = (next + 1) % 8;
+    v = Entry{L.nx, L.ny, L.nz, kind, slots, search()};
+    return v.s;
+  }
+};
+static thread_local ShapeMemo t_shapes;
+
+// Level 1: tile of TY x TZ element columns marching over NX node planes.  LDS
+// holds two exchange buffers of 9 values per thread (under 80 KiB).  Tuning
+// override: TOP3D_TILE_L1=TY,TZ,NX (NX = 0: from the occupancy).
+//
+// Tiles of up to 256 threads, 4 waves, so that every SIMD has the same share of
+// a workgroup, with the cheapest launch; among equals the least work, short rows
+// counting for more.  65 x 7 (clipped to the grid) where its launch is cheaper,
+// or as cheap with fewer waves on a CU.  Against 65 x 7 for every grid, us per
+// sweep of the level below: FP32 512x256x256 84 -> 76.5 (23 x 11), 256x128x128
+// 14.1 -> 13.8 (36 x 7), 168x72x104 8.9 -> 7.9 (37 x 6), 200x120x88 10.5 -> 9.3
+// (21 x 12); FP64 178 -> 166 (28 x 9), 22.4 -> 22.0, 13.4 -> 10.1 and 15.9 ->
+// 14.2; 65 x 7 stays in FP64 for 96x96x96 (9.5 us on 200 CUs; 10.1 with 28 x 9,
+// of which 44 CUs have two) and 120x40x40 (5.2 us in 3 waves; 5.5 with 21 x 12).
+static TileShape level1_search(const Level &L, int per_cu) {
+  TileShape best{};
+  const int64_t cus = device_cus();
+  auto waves = [](const TileShape &t) { return (t.TY * t.TZ + 63) / 64; };
+  // waves of the launch on the CU that has the most
+  auto cu_waves = [&](const TileShape &t) {
+    return ((int64_t)t.ntx * t.nty * t.ntz + cus - 1) / cus * waves(t);
+  };
+  int64_t best_cost = INT64_MAX, best_work = INT64_MAX;
+  for (int ty = 17; ty <= 42; ty++) {
+    TileShape s{};
+    set_tiles(s, L, ty, 256 / std::min(ty, std::max(2, L.nely + 1)));
+    const int64_t cost = tile_x(s, L, 0, per_cu * cus);
+    const int64_t work = (int64_t)s.ntx * s.nty * s.ntz * (s.TY + 6) * 1024 / s.TY;
+    if (cost < best_cost || (cost == best_cost && work <= best_work)) {
+      best_cost = cost;
+      best_work = work;
+      best = s;
+    }
+  }
+  TileShape wide{};
+  set_tiles(wide, L, 65, 7);
+  const int64_t cost = tile_x(wide, L, 0, std::max(1, per_cu / ((waves(wide) + 3) / 4)) * cus);
+  if (cost < best_cost || (cost == best_cost && cu_waves(wide) < cu_waves(best))) best = wide;
+  return best;
+}
+
+// per_cu: workgroups of 4 waves that a CU holds
+static TileShape level1_shape(const Level &L, int elem_bytes, int per_cu) {
+  const int lds_threads = 80 * 1024 / (18 * elem_bytes);
+  // launch bounds: 1024 threads in FP32, 512 in FP64
+  const int max_threads = std::min(elem_bytes == 4 ? 1024 : 512, lds_threads);
+  const char *env = std::getenv("TOP3D_TILE_L1");
+  int oy = 0, oz = 0, ox = 0;
+  if (env && std::sscanf(env, "%d,%d,%d", &oy, &oz, &ox) == 3 && oy >= 2 && oz >= 2 && ox >= 0 &&
+      oy <= max_threads && oz <= max_threads && oy * oz <= max_threads) {
+    TileShape s{};
+    set_tiles(s, L, oy, oz);
+    // waves in fours: one SIMD holds ceil(waves / 4) of a workgroup
+    tile_x(s, L, ox, std::max(1, per_cu / ((s.TY * s.TZ + 255) / 256)) * (int64_t)device_cus());
+    return s;
+  }
+  return t_shapes.get(L, 0, per_cu, [&] { return level1_search(L, per_cu); });
+}
+
 // The fine level's shape (k_fine_march): (TY + 1) x (TZ + 1) nodes within the
 // workgroup's threads, one of which holds the zeros.  At 257x129x129 nodes, in
 // FP64, 23 x 9 columns ran a sweep in 81.6 us, 24 x 9 in 83.8 us, 20 x 11 in
@@ -1431,11 +1499,10 @@ static int64_t tile_x(TileShape &s, const Level &L, int nx_fixed, int64_t slots)
 // cheapest launch, the longest among equals.  Tuning override:
 // TOP3D_TILE_L0 (FP32), TOP3D_TILE_L0_F64=TY,TZ,NX (NX = 0: the march length
 // from the occupancy).
-static TileShape march_shape(const Level &L, int64_t slots, bool f64, int &nx_fixed) {
+static TileShape march_search(const Level &L, int64_t slots, bool f64) {
   const int kNodes = (f64 ? march_threads<double>() : march_threads<float>()) - 1;
   TileShape best{};
   int64_t best_cost = INT64_MAX;
-  nx_fixed = 0;
   for (int ty = 17; ty <= (f64 ? 23 : 35); ty++) {
     TileShape s{};
     set_tiles(s, L, ty, kNodes / (std::min(ty, std::max(2, L.nely + 1)) + 1) - 1);
@@ -1445,14 +1512,21 @@ static TileShape march_shape(const Level &L, int64_t slots, bool f64, int &nx_fi
       best = s;
     }
   }
+  return best;
+}
+
+static TileShape march_shape(const Level &L, int64_t slots, bool f64) {
+  const int kNodes = (f64 ? march_threads<double>() : march_threads<float>()) - 1;
   const char *env = std::getenv(f64 ? "TOP3D_TILE_L0_F64" : "TOP3D_TILE_L0");
   int oy = 0, oz = 0, ox = 0;
   if (env && std::sscanf(env, "%d,%d,%d", &oy, &oz, &ox) == 3 && oy >= 2 && oz >= 2 && ox >= 0 &&
       oy <= kNodes && oz <= kNodes && (oy + 1) * (oz + 1) <= kNodes) {
-    set_tiles(best, L, oy, oz);
-    nx_fixed = ox;
+    TileShape s{};
+    set_tiles(s, L, oy, oz);
+    tile_x(s, L, ox, slots);
+    return s;
   }
-  return best;
+  return t_shapes.get(L, f64 ? 2 : 1, slots, [&] { return march_search(L, slots, f64); });
 }
 
 // workgroups of `nthr` threads and `shm` bytes of LDS one CU holds at once.
@@ -1469,20 +1543,6 @@ static int wg_per_cu(const void *kernel, int nthr, size_t shm) {
   const int by_waves = std::min(4 * per_simd / waves, per_simd / ((waves + 3) / 4));
   const int by_lds = (int)((160 * 1024) / std::max<size_t>(shm, 1));
   return std::max(1, std::min(by_waves, by_lds));
-}
-
-static int device_cus() {
-  static int ncu[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!ncu[dev]) {
-    int v = 0;
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        v <= 0)
-      v = 256;
-    ncu[dev] = v;
-  }
-  return ncu[dev];
 }
 
 // checks that a level's offsets fit in 32 bits (the output's byte size also
@@ -1544,9 +1604,7 @@ static int run_fine(const DevGrid &g, int mode, const T *E, const T *in, T *out,
                                   : (const void *)k_fine_march<T, kModeJacobi, false>,
                              march_threads<T>(), shm);
   const int64_t slots = (int64_t)per_cu[diag] * device_cus();
-  int nx_fixed = 0;
-  TileShape s = march_shape(L, slots, sizeof(T) == 8, nx_fixed);
-  tile_x(s, L, nx_fixed, slots);
+  TileShape s = march_shape(L, slots, sizeof(T) == 8);
   if (mode == kModeProlong) {  // (marches that start at odd planes)
     s.NX += s.NX & 1;
     s.ntx = (L.nx + s.NX - 1) / s.NX;
@@ -1613,16 +1671,13 @@ static void run_level1(const DevGrid &g, int mode, const T *Eh, const T *in, T *
   a.few = L.nely + 1;  // the slots of k_level1_moduli
   a.fez = L.nelz + 1;
   if (mode == kModeJacobiDiag) mode = kModeJacobi;
-  int nx_fixed = 0;
-  TileShape s = level1_shape(L, (int)sizeof(T), nx_fixed);
+  // workgroups of 4 waves per CU (their LDS, two buffers of 9 values per thread,
+  // leaves room for all that the registers do)
+  static const int per_cu = wg_per_cu((const void *)k_level1_sweep<T, kModeJacobi, false>, 256,
+                                      sizeof(T) * 2 * 9 * 256);
+  const TileShape s = level1_shape(L, (int)sizeof(T), per_cu);
   const int nthr = s.TY * s.TZ, bs = (nthr + 63) / 64 * 64;
   const size_t shm = sizeof(T) * 2 * 9 * (size_t)nthr;
-  static int cached_nthr = -1, cached_per_cu = 1;
-  if (cached_nthr != nthr) {
-    cached_per_cu = wg_per_cu((const void *)k_level1_sweep<T, kModeJacobi, false>, bs, shm);
-    cached_nthr = nthr;
-  }
-  tile_x(s, L, nx_fixed, (int64_t)cached_per_cu * device_cus());
   tile_args_shape(s, a);
   const dim3 grid(s.ntx, s.nty * s.ntz);
   K1Vals<T> B;
