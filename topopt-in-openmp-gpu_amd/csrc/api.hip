@@ -731,8 +731,9 @@ void applyDensityFilter(const struct gridContext gc, const DTYPE rmin, const DTY
   if (!vr.open(rho, sizeof(double) * g->nelem, true, false) ||
       !vo.open(out, sizeof(double) * g->nelem, true, true))
     return;
-  launch_filter(*g, rmin, (const double *)vr.dev, (double *)vo.dev, 0);
-  sync_ok();
+  ScratchBlock sums;
+  launch_filter(*g, rmin, (const double *)vr.dev, (double *)vo.dev, 0, sums);
+  if (sync_ok()) sums.done();
   vo.close();
   vr.close();
 }
@@ -744,12 +745,13 @@ void applyDensityFilterGradient(const struct gridContext gc, const DTYPE rmin, D
   DevView vv;
   if (!vv.open(v, sizeof(double) * g->nelem, true, true)) return;
   double *tmp = (double *)g->work(kSlotTmp, sizeof(double) * g->nelem);
-  if (tmp && launch_filter_grad(*g, rmin, (const double *)vv.dev, tmp, 0))
+  ScratchBlock sums;
+  if (tmp && launch_filter_grad(*g, rmin, (const double *)vv.dev, tmp, 0, sums))
     // interior elements take the filtered value; the halo of v is untouched
     hipLaunchKernelGGL(k_copy_interior_elems, dim3((g->nelem + 255) / 256), dim3(256), 0,
                        stream(), g->nelem, g->nelx, g->nely, g->nelz, g->ewy, g->ewz, tmp,
                        (double *)vv.dev);
-  sync_ok();
+  if (sync_ok()) sums.done();
   vv.close();
 }
 
@@ -764,9 +766,12 @@ int top3d_density_filter(const struct gridContext *gc, double rmin, int transpos
     return top3d_last_error();
   }
   bool ok = true;
-  if (transpose) ok = launch_filter_grad(*g, rmin, di, dout, halo);
-  else launch_filter(*g, rmin, di, dout, halo);
-  return sync_ok() && ok ? TOP3D_OK : top3d_last_error();
+  ScratchBlock sums;
+  if (transpose) ok = launch_filter_grad(*g, rmin, di, dout, halo, sums);
+  else launch_filter(*g, rmin, di, dout, halo, sums);
+  if (!sync_ok()) return top3d_last_error();
+  sums.done();
+  return ok ? TOP3D_OK : top3d_last_error();
 }
 
 // gpu_definitions.c:159-195: map every array the design loop uses
@@ -819,12 +824,15 @@ int top3d_compliance_backward(const struct gpuGrid *gpu_gc, double rmin,
   launch_sensitivity(*g, xPhys_dev, U_dev, dc, red, red + 1024);
   hipLaunchKernelGGL(k_scale, dim3((g->nelem + 255) / 256), dim3(256), 0, stream(), g->nelem,
                      grad_c, dc);
+  ScratchBlock sums;
   if (rmin > 0) {
-    if (!launch_filter_grad(*g, rmin, dc, grad_x_dev, 1)) return top3d_last_error();
+    if (!launch_filter_grad(*g, rmin, dc, grad_x_dev, 1, sums)) return top3d_last_error();
   } else {
     hipMemcpyAsync(grad_x_dev, dc, sizeof(double) * g->nelem, hipMemcpyDeviceToDevice, stream());
   }
-  return sync_ok() ? TOP3D_OK : TOP3D_ERR_HIP;
+  if (!sync_ok()) return TOP3D_ERR_HIP;
+  sums.done();
+  return TOP3D_OK;
 }
 
 }  // extern "C"

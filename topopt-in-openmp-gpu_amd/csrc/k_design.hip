@@ -489,7 +489,8 @@ static FilterClasses filter_classes(double rmin, int R) {
 // false where the loop over the window runs: no weight at all (rmin <= 0), a
 // tile beyond the LDS (rmin > 7), or a grid beyond the launch limits.
 template <bool TR>
-static bool filter_tiles(DevGrid &g, double rmin, const double *in, double *out, int halo) {
+static bool filter_tiles(DevGrid &g, double rmin, const double *in, double *out, int halo,
+                         ScratchBlock &sums) {
   const Level &L = g.lv[0];
   if (!(rmin > 0.0) || rmin > kFilterMaxR + 1 || L.nelz > kFTK * 65535 || L.nelx > 65535)
     return false;
@@ -509,7 +510,9 @@ static bool filter_tiles(DevGrid &g, double rmin, const double *in, double *out,
   }
   const FilterClasses W = filter_classes(rmin, R);
   const int nc = 2 * R + 1, n = nc * nc * nc;
-  double *hs = (double *)g.work(kSlotFilterSums, sizeof(double) * n);
+  static_assert((2 * kFilterMaxR + 1) * (2 * kFilterMaxR + 1) * (2 * kFilterMaxR + 1) <=
+                    kOcScratchDoubles, "sums of weights");
+  double *hs = sums.get();
   if (!hs) return true;  // (the error is recorded)
   hipLaunchKernelGGL(k_filter_sums, dim3(n), dim3(64), 0, stream(), R, L.nelx, L.nely, L.nelz, W,
                      hs);
@@ -538,14 +541,16 @@ static void filter_halo(const DevGrid &g, const double *in, double *out, int hal
     hipMemcpyAsync(out, in, sizeof(double) * g.nelem, hipMemcpyDeviceToDevice, stream());
 }
 
-void launch_filter(DevGrid &g, double rmin, const double *rho, double *out, int halo) {
-  if (filter_tiles<false>(g, rmin, rho, out, halo)) return;
+void launch_filter(DevGrid &g, double rmin, const double *rho, double *out, int halo,
+                   ScratchBlock &sums) {
+  if (filter_tiles<false>(g, rmin, rho, out, halo, sums)) return;
   filter_halo(g, rho, out, halo);
   filter_window<0>(g, rmin, rho, out);
 }
 
-bool launch_filter_grad(DevGrid &g, double rmin, const double *v, double *out, int halo) {
-  if (filter_tiles<true>(g, rmin, v, out, halo)) return true;
+bool launch_filter_grad(DevGrid &g, double rmin, const double *v, double *out, int halo,
+                        ScratchBlock &sums) {
+  if (filter_tiles<true>(g, rmin, v, out, halo, sums)) return true;
   double *tmp = (double *)g.work(kSlotFilterTmp, sizeof(double) * g.nelem);
   if (!tmp) return false;
   launch_fill<double>(g.nelem, tmp, 0.0);

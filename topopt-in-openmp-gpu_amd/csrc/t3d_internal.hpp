@@ -79,7 +79,7 @@ struct DevGrid {
   // element's nodal values (valid if wh0)
   bool wh0 = false;
   double M0[8][3][3] = {};
-  static constexpr int kScratchSlots = 11;
+  static constexpr int kScratchSlots = 10;
   void *scratch[kScratchSlots] = {};   // lazily allocated work arrays of the API
   size_t scratch_bytes[kScratchSlots] = {};
   LevelArgs args(int l) const;
@@ -129,9 +129,8 @@ int64_t level1_moduli_count(const DevGrid &g);
 // DevGrid::work slot of the transformed moduli formed by launch_level1
 // when the caller passes none
 constexpr int kSlotLevel1Moduli = 8;
-// the density filter's sums of weights, and its intermediate array at radii
-// beyond the tiles
-constexpr int kSlotFilterSums = 9, kSlotFilterTmp = 10;
+// the density filter's intermediate array at radii beyond the tiles
+constexpr int kSlotFilterTmp = 9;
 bool tile_level1_available();  // the level-1 element matrices have the mirror structure
 bool tile_fine_diag_available();  // the fine tile sweep can form its diagonal from E
 // launch_fine mode 3 forms the diagonal from E (no invD read)
@@ -351,22 +350,41 @@ void launch_copy_fixed(const DevGrid &g, int l, const double *in, double *out);
 void launch_sensitivity(const DevGrid &g, const double *x, const double *u,
                         double *dc, double *partials, double *c);
 // density filter and its transpose on the real elements; the halo elements
-// of out keep their values (0), become zero (1) or those of the input (2)
-void launch_filter(DevGrid &g, double rmin, const double *rho, double *out, int halo);
-bool launch_filter_grad(DevGrid &g, double rmin, const double *v, double *out, int halo);
+// of out keep their values (0), become zero (1) or those of the input (2).
+// sums: the call's block for the sums of weights (calls on one grid may overlap)
+struct ScratchBlock;
+void launch_filter(DevGrid &g, double rmin, const double *rho, double *out, int halo,
+                   ScratchBlock &sums);
+bool launch_filter_grad(DevGrid &g, double rmin, const double *v, double *out, int halo,
+                        ScratchBlock &sums);
 void launch_volume(const DevGrid &g, const double *x, double *partials,
                    double *result);
 void launch_change(int64_t n, double *x, const double *xnew, double *partials,
                    double *result);
 // scratch: kOcScratchDoubles doubles of device memory.
 constexpr int kOcScratchDoubles = 2 * (8 + 31 * 256);
-// Scratch of that size (contents undefined) for the entry points without a grid.
+// Scratch of that size (contents undefined) for the entry points without a grid
+// and for what two calls on a grid must not share.
 // A hipMalloc and hipFree per call cost about 18 us each time (OC update and
 // change at 256x128x128: 447 -> 411 us), so while the process has a grid up to 4
 // blocks that are not in use stay for the next call; they are freed with the last
 // grid.  scratch_put only after the work on the block has completed.
 double *scratch_get();
 void scratch_put(double *p);
+// Such a block for the length of one call.  done(): the work on it has completed;
+// without, it is freed, which waits for that work.
+struct ScratchBlock {
+  double *p = nullptr;
+  ScratchBlock() = default;
+  ScratchBlock(const ScratchBlock &) = delete;
+  ScratchBlock &operator=(const ScratchBlock &) = delete;
+  ~ScratchBlock() { dfree(p); }
+  double *get() { return p ? p : (p = scratch_get()); }
+  void done() {
+    scratch_put(p);
+    p = nullptr;
+  }
+};
 int oc_update(const double *x, double *xnew, const double *dv,
               const double *dc, int64_t nelem, double gval, double *scratch);
 
