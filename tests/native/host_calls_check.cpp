@@ -81,8 +81,55 @@ static int filter_sums() {
   return 0;
 }
 
+// Without memory for the sums of weights the filter runs as the loop over the
+// window, which needs none; its transpose, whose loop needs an array, reports the
+// error and leaves the output alone.
+static int filter_without_memory() {
+  Grid g(16, 8, 8, 3);
+  Device in(g.nelem()), out(g.nelem());
+  std::vector<std::string> launched;
+  fake::on_launch = [&](const Launch &l) { launched.push_back(l.name); };
+  auto starved = [&](auto call) {
+    launched.clear();
+    top3d_clear_error();
+    fake::fail_malloc = 1;
+    const int rc = call();
+    fake::fail_malloc = 0;
+    return rc;
+  };
+  const double r = 2.5;
+  REQUIRE(starved([&] {
+            return top3d_density_filter(&g.gc, r, 0, TOP3D_HALO_KEEP, in.p, out.p);
+          }) == TOP3D_OK);
+  REQUIRE(launched.size() == 1 && launched[0].find("k_filterILi0E") != std::string::npos);
+  REQUIRE(top3d_last_error() == TOP3D_OK && hipGetLastError() == 0);
+  REQUIRE(starved([&] {
+            applyDensityFilter(g.gc, r, in.p, out.p);
+            return top3d_last_error();
+          }) == TOP3D_OK && launched.size() == 1);
+  REQUIRE(starved([&] {
+            return top3d_density_filter(&g.gc, r, 1, TOP3D_HALO_KEEP, in.p, out.p);
+          }) == TOP3D_ERR_HIP && launched.empty());
+  // (the first two arrays of the gradient are the grid's: kept from this call)
+  REQUIRE(top3d_compliance_backward(&g.gpu, 1.5, in.p, out.p, 1.0, out.p) == TOP3D_OK);
+  REQUIRE(starved([&] {
+            return top3d_compliance_backward(&g.gpu, r, in.p, out.p, 1.0, out.p);
+          }) == TOP3D_ERR_HIP);
+  for (const std::string &n : launched) REQUIRE(n.find("k_filter") == std::string::npos);
+  // the gradient in place: with its result array, but none for the sums
+  top3d_clear_error();
+  applyDensityFilterGradient(g.gc, 1.5, in.p);
+  REQUIRE(starved([&] {
+            applyDensityFilterGradient(g.gc, r, in.p);
+            return top3d_last_error();
+          }) == TOP3D_ERR_HIP && launched.empty());
+  fake::on_launch = nullptr;
+  return 0;
+}
+
 int main(int argc, char **argv) {
-  const std::map<std::string, int (*)()> checks = {{"filter_sums", filter_sums}};
+  const std::map<std::string, int (*)()> checks = {
+      {"filter_sums", filter_sums}, {"filter_without_memory", filter_without_memory}};
   auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   const int rc = it->second();

@@ -228,7 +228,7 @@ constexpr size_t kScratchKept = 4;
 std::vector<std::pair<int, double *>> g_scratch_free;  // (device, block), under g_gmu
 }  // namespace
 
-double *scratch_get() {
+double *scratch_get(bool quiet) {
   int dev = 0;
   if (!hip_ok(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
   {
@@ -240,7 +240,15 @@ double *scratch_get() {
         return p;
       }
   }
-  return (double *)dalloc_uninit(sizeof(double) * kOcScratchDoubles);
+  const size_t bytes = sizeof(double) * kOcScratchDoubles;
+  if (!quiet) return (double *)dalloc_uninit(bytes);
+  void *p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();  // (a later check would find it)
+    return nullptr;
+  }
+  track_alloc(p, bytes);
+  return (double *)p;
 }
 
 void scratch_put(double *p) {

@@ -487,7 +487,8 @@ static FilterClasses filter_classes(double rmin, int R) {
 }
 
 // false where the loop over the window runs: no weight at all (rmin <= 0), a
-// tile beyond the LDS (rmin > 7), or a grid beyond the launch limits.
+// tile beyond the LDS (rmin > 7), a grid beyond the launch limits, or no memory
+// for the sums of weights (the loop needs none).
 template <bool TR>
 static bool filter_tiles(DevGrid &g, double rmin, const double *in, double *out, int halo,
                          ScratchBlock &sums) {
@@ -513,7 +514,7 @@ static bool filter_tiles(DevGrid &g, double rmin, const double *in, double *out,
   static_assert((2 * kFilterMaxR + 1) * (2 * kFilterMaxR + 1) * (2 * kFilterMaxR + 1) <=
                     kOcScratchDoubles, "sums of weights");
   double *hs = sums.get();
-  if (!hs) return true;  // (the error is recorded)
+  if (!hs) return false;
   hipLaunchKernelGGL(k_filter_sums, dim3(n), dim3(64), 0, stream(), R, L.nelx, L.nely, L.nelz, W,
                      hs);
   switch (R) {

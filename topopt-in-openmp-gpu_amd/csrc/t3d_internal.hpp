@@ -369,7 +369,8 @@ constexpr int kOcScratchDoubles = 2 * (8 + 31 * 256);
 // change at 256x128x128: 447 -> 411 us), so while the process has a grid up to 4
 // blocks that are not in use stay for the next call; they are freed with the last
 // grid.  scratch_put only after the work on the block has completed.
-double *scratch_get();
+// quiet: without memory for it, nothing is recorded as an error.
+double *scratch_get(bool quiet = false);
 void scratch_put(double *p);
 // Such a block for the length of one call.  done(): the work on it has completed;
 // without, it is freed, which waits for that work.
@@ -379,7 +380,7 @@ struct ScratchBlock {
   ScratchBlock(const ScratchBlock &) = delete;
   ScratchBlock &operator=(const ScratchBlock &) = delete;
   ~ScratchBlock() { dfree(p); }
-  double *get() { return p ? p : (p = scratch_get()); }
+  double *get() { return p ? p : (p = scratch_get(true)); }
   void done() {
     scratch_put(p);
     p = nullptr;
