@@ -100,6 +100,32 @@ def test_filter_tiles(shape, rmin):
     o.close()
 
 
+# Elements at x = 1 that stay there under every multiplier (a solid region with a
+# large volume weight) add nothing to the sums: the multiplier is that of the
+# others.  Every sum that the bisection
+# decides on is far above the rounding of the moving elements' terms (n 2^-53).
+@pytest.mark.parametrize("n", [4096, 262145])
+def test_oc_update_beside_heavy_elements(n):
+    print(f"[gpu oc] heavy elements, n {n}", flush=True)
+    rng = np.random.default_rng(n)
+    x, dv = rng.uniform(0.05, 0.95, n), rng.uniform(0.5, 1.5, n)
+    dc = -rng.uniform(0.5, 1.5, n) * 10.0 ** rng.integers(-2, 3, n)
+    heavy = rng.random(n) < 0.25
+    x[heavy], dv[heavy], dc[heavy] = 1.0, 1e18, -1e30
+    gval = 0.01 * n
+    light = ~heavy
+    ref = np.ones(n)
+    ref[light] = oc_reference(x[light], dv[light], dc[light], gval)
+    d = [torch.from_numpy(a).cuda() for a in (x, dv, dc)]
+    got = torch.full((n,), -1.0, dtype=torch.float64, device="cuda")
+    lib = top3d_amd.library()
+    lib.top3d_set_stream(ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    lib.update_solution(_p(d[0]), _p(got), _p(d[1]), _p(d[2]), n, gval)
+    top3d_amd.check("update_solution")
+    assert np.abs(got.cpu().numpy() - ref).max() <= 8 * 2.0 ** -53
+
+
 def test_oc_update_in_place():
     """xnew may be one of the inputs: the result of the update elsewhere."""
     n = 300_001

@@ -714,7 +714,7 @@ __device__ __forceinline__ OcState oc_walk(const OcState *__restrict__ in,
 // [cur] is read and [cur ^ 1] written (every workgroup reads the old ones).
 // first: the state is [0, 1e9] with this gval.  A: where xnew overlaps none of
 // the inputs, the first pass leaves x_e sqrt(-dc_e / dv_e) in xnew for the
-// passes after it (57 of their 181 instructions per element), which the
+// passes after it (57 of their some 180 instructions per element), which the
 // final write replaces.
 template <bool FIRST, bool A>
 __global__ __launch_bounds__(kOcBS) void k_oc_pass(int64_t n, const double *x, const double *dv,
@@ -737,7 +737,7 @@ __global__ __launch_bounds__(kOcBS) void k_oc_pass(int64_t n, const double *x, c
   __syncthreads();
   if (t < kOcCand) S[t] = 1.0 / sqrt(oc_candidate(st.l1, st.l2, t));
   __syncthreads();
-  double rl[kOcCand], s[kOcCand + 1];
+  double rl[kOcCand], s[kOcCand + 1];  // (slot kOcCand: zero)
 #pragma unroll
   for (int c = 0; c < kOcCand; c++) {
     // one value for the workgroup: kept in scalar registers
@@ -766,11 +766,13 @@ __global__ __launch_bounds__(kOcBS) void k_oc_pass(int64_t n, const double *x, c
       const double a = A && !FIRST ? ae[e] : xe[e] * sqrt(-ae[e] / ve[e]);
       if (A && FIRST && in) xnew[i + e * stride] = a;
       const double w = in ? ve[e] : 0.0;
-      const double hi = fmin(1.0, xe[e] + move), lo = fmax(0.0, xe[e] - move);
-      // slot kOcCand: the sum of dv x that every candidate's sum leaves out
+      // oc_x less x_e: the bounds less x_e, and the multiply-add rounds once.
+      // (Sums of dv xnew and dv x apart would lose an element's difference
+      // beside the large dv x of elements that do not move.)
+      const double hi = fmin(1.0, xe[e] + move) - xe[e], lo = fmax(0.0, xe[e] - move) - xe[e];
 #pragma unroll
-      for (int c = 0; c < kOcCand; c++) s[c] = fma(w, fmax(lo, fmin(hi, a * rl[c])), s[c]);
-      s[kOcCand] = fma(w, xe[e], s[kOcCand]);
+      for (int c = 0; c < kOcCand; c++)
+        s[c] = fma(w, fmax(lo, fmin(hi, fma(a, rl[c], -xe[e]))), s[c]);
     }
   }
   // Wave sums of the 32 values by halving: at each step a lane keeps half of
@@ -793,7 +795,7 @@ __global__ __launch_bounds__(kOcBS) void k_oc_pass(int64_t n, const double *x, c
   __syncthreads();
   if (t < kOcCand) {
     double v = 0.0;
-    for (int w = 0; w < kOcBS / 64; w++) v += red[w][t] - red[w][kOcCand];
+    for (int w = 0; w < kOcBS / 64; w++) v += red[w][t];
     partials[((cur ^ 1) * kOcCand) * kOcBlocks + (int64_t)t * np + blockIdx.x] = v;
   }
 }
