@@ -200,6 +200,8 @@ void solveSubspaceMatrix(const struct gridContext gc, const int l,
 /* ---- design loop kernels (gpu_definitions.h:58-86,
  *      stencil_optimization.h:5-15) ---------------------------------------- */
 DTYPE compute_volume(const struct gridContext gc, DTYPE *xPhys);
+/* max |x - xnew|, then x = xnew; INFINITY and x as it was where there is no
+ * memory for the reduction. */
 float compute_change(DTYPE *x, DTYPE *xnew, const int nelem);
 /* OC bisection (gpu_definitions.c:127-157) on the device, 31 multipliers per
  * pass over the elements; x_e sqrt(-dc_e / (dv_e lmid)) is formed

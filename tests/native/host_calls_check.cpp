@@ -127,9 +127,36 @@ static int filter_without_memory() {
   return 0;
 }
 
+// A change that could not be computed for want of memory does not read as none,
+// and leaves no staging arrays behind.
+static int change_without_memory() {
+  Grid g(8, 4, 4, 3);
+  const int n = (int)g.nelem();
+  std::vector<double> x(n, 0.5), xnew(n, 0.5);
+  const size_t before = fake::held();
+  REQUIRE(compute_change(x.data(), xnew.data(), n) == 0.0f);  // (its block is kept)
+  REQUIRE(fake::held() == before + 1);
+  bool launched = false;
+  freeGPUGrid(&g.gpu, g.nl);  // the kept block goes with the last grid
+  freeGC(&g.gc, g.nl);
+  const size_t none = fake::held();
+  // the third allocation fails, after the staging of the two host arrays
+  fake::on_launch = [&](const Launch &) { launched = true; };
+  top3d_clear_error();
+  fake::fail_malloc = 3;
+  const float change = compute_change(x.data(), xnew.data(), n);
+  fake::fail_malloc = 0;
+  fake::on_launch = nullptr;
+  REQUIRE(!launched && top3d_last_error() == TOP3D_ERR_HIP);
+  REQUIRE(fake::held() == none);
+  REQUIRE(change > 1.0f);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, int (*)()> checks = {
-      {"filter_sums", filter_sums}, {"filter_without_memory", filter_without_memory}};
+      {"filter_sums", filter_sums}, {"filter_without_memory", filter_without_memory},
+      {"change_without_memory", change_without_memory}};
   auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   const int rc = it->second();

@@ -28,7 +28,8 @@ def checker(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["filter_sums", "filter_without_memory"])
+@pytest.mark.parametrize("check", ["filter_sums", "filter_without_memory",
+                                   "change_without_memory"])
 def test_host_calls(checker, check):
     out = subprocess.run([checker, check], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0 and out.stdout.strip() == "OK", out.stdout + out.stderr

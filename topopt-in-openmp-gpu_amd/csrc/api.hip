@@ -172,6 +172,10 @@ struct DevView {
     }
     dev = nullptr;
   }
+  ~DevView() {  // a call that ends before its work: nothing to copy back
+    out = false;
+    close();
+  }
 };
 
 }  // namespace t3d
@@ -638,7 +642,7 @@ float compute_change(DTYPE *x, DTYPE *xnew, const int nelem) {
   if (!vn.open(xnew, sizeof(double) * nelem, true, false)) return 0;
   static_assert(kOcScratchDoubles >= 1024 + 16, "reduction scratch");
   double *red = scratch_get();
-  if (!red) return 0;
+  if (!red) return INFINITY;  // (0 would read as a converged design)
   launch_change(nelem, (double *)vx.dev, (const double *)vn.dev, red, red + 1024);
   double h = 0;
   hipMemcpyAsync(&h, red + 1024, sizeof(double), hipMemcpyDeviceToHost, stream());
