@@ -114,6 +114,7 @@ int hipHostGetDevicePointer(void **d, void *h, unsigned) {
   return 0;
 }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int, void *) {
+  if (!d || !s) return 1;
   std::memcpy(d, s, n);
   return 0;
 }
@@ -123,6 +124,7 @@ int hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, siz
   return 0;
 }
 int hipMemsetAsync(void *d, int v, size_t n, void *) {
+  if (!d) return 1;
   std::memset(d, v, n);
   return 0;
 }

@@ -153,10 +153,60 @@ static int change_without_memory() {
   return 0;
 }
 
+struct Held {
+  size_t blocks = fake::held();
+  int events = fake::events, streams = fake::streams;
+  bool operator==(const Held &o) const {
+    return blocks == o.blocks && events == o.events && streams == o.streams;
+  }
+};
+
+// Grids with their solvers, coarse factors and inverses give back all that they
+// allocated, also where an allocation failed half way.
+static int given_back() {
+  top3d_synchronize();  // (the library's stream is made once)
+  const Held none;
+  auto lives = [&](bool solve) {
+    Grid g(16, 8, 8, 3);
+    SolverDataBuffer data{};
+    allocateSolverData(g.gc, 3, &data);
+    if (solve && data.r) {
+      Device x(g.nelem()), F(g.ndof(0)), U(g.ndof(0));
+      int it;
+      float res;
+      solveStateMG_halo(&g.gpu, x.p, 4, 3, 1e-5, &data, &it, &res, F.p, U.p);
+    }
+    if (data.r) freeSolverData(&data, 3);
+    CSRMatrix M{};
+    allocateSubspaceMatrix(g.gc, 2, &M);
+    CoarseSolverData coarse{};
+    initializeCholmod(g.gc, 2, &coarse, M);
+    finishCholmod(g.gc, 2, &coarse, M, 0);
+    freeSubspaceMatrix(&M);
+  };
+  lives(true);
+  REQUIRE(Held() == none);
+  for (int n = 1; n < 200; n += 7) {
+    fake::fail_malloc = n;
+    lives(false);
+    fake::fail_malloc = 0;
+    if (!(Held() == none)) std::printf("allocation %d failing\n", n);
+    REQUIRE(Held() == none);
+  }
+  {
+    Device A(100 * 100);
+    const Held before;
+    top3d_dense_spd_inverse(A.p, 100, 20);
+    REQUIRE(Held() == before);
+  }
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, int (*)()> checks = {
       {"filter_sums", filter_sums}, {"filter_without_memory", filter_without_memory},
-      {"change_without_memory", change_without_memory}};
+      {"change_without_memory", change_without_memory},
+      {"given_back", given_back}};
   auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   const int rc = it->second();

@@ -911,9 +911,14 @@ void CoarseFactor::release() {
   for (void *p : {(void *)A, (void *)L, (void *)W, (void *)WT, (void *)Dinv, (void *)info,
                   (void *)cw64, (void *)W32, (void *)WT32, (void *)cw32, (void *)pos,
                   (void *)ipos, (void *)dtasks, (void *)dcolinfo, (void *)drows,
-                  (void *)dklist, (void *)dztiles})
+                  (void *)dklist, (void *)dztiles, (void *)dlevel, (void *)dwlist,
+                  (void *)dwtlist})
     if (p) dfree(p);
-  dztiles = nullptr;
+  for (hipEvent_t &e : ev_level) {
+    if (e) hipEventDestroy(e);
+    e = nullptr;
+  }
+  dztiles = dlevel = dwlist = dwtlist = nullptr;
   nztiles = 0;
   A = L = W = WT = Dinv = cw64 = nullptr;
   W32 = WT32 = cw32 = nullptr;
