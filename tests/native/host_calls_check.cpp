@@ -2,6 +2,7 @@
 // (fake_hip.hpp): what they launch, keep, free and report.
 // Usage: host_calls_check CHECK
 #include <cstdio>
+#include <thread>
 
 #include "../../include/top3d_hip.h"
 #include "fake_hip.hpp"
@@ -202,11 +203,36 @@ static int given_back() {
   return 0;
 }
 
+// A thread that goes from one device to another launches the level-1 sweep in
+// the shape of the device it is on, as a thread that has seen no other does.
+static int shapes_by_device() {
+  Grid g(128, 64, 64, 3);
+  Device x(g.nelem()), invD(g.ndof(1)), u(g.ndof(1)), b(g.ndof(1)), tmp(g.ndof(1));
+  Dim3 grid{};
+  fake::on_launch = [&](const Launch &l) {
+    if (named(l, "k_level1_sweep")) grid = l.grid;
+  };
+  auto sweep = [&](int device, int cus) {
+    fake::device = device;
+    fake::cus = cus;
+    smoothDampedJacobiSubspace_halo(g.gpu.target, x.p, 1, 1, 0.6, invD.p, u.p, b.p, tmp.p);
+    return grid;
+  };
+  const Dim3 first = sweep(0, 256), here = sweep(1, 32);
+  Dim3 fresh{};
+  std::thread([&] { fresh = sweep(1, 32); }).join();
+  fake::on_launch = nullptr;
+  fake::device = 0;
+  REQUIRE(first.x != fresh.x || first.y != fresh.y);
+  REQUIRE(here.x == fresh.x && here.y == fresh.y);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, int (*)()> checks = {
       {"filter_sums", filter_sums}, {"filter_without_memory", filter_without_memory},
       {"change_without_memory", change_without_memory},
-      {"given_back", given_back}};
+      {"given_back", given_back}, {"shapes_by_device", shapes_by_device}};
   auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   const int rc = it->second();

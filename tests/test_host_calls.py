@@ -29,7 +29,7 @@ def checker(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["filter_sums", "filter_without_memory",
-                                   "change_without_memory", "given_back"])
+                                   "change_without_memory", "given_back", "shapes_by_device"])
 def test_host_calls(checker, check):
     out = subprocess.run([checker, check], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0 and out.stdout.strip() == "OK", out.stdout + out.stderr

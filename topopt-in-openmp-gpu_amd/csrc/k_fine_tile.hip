@@ -1485,7 +1485,9 @@ static TileShape level1_shape(const Level &L, int elem_bytes, int per_cu) {
     tile_x(s, L, ox, std::max(1, per_cu / ((s.TY * s.TZ + 255) / 256)) * (int64_t)device_cus());
     return s;
   }
-  return t_shapes.get(L, 0, per_cu, [&] { return level1_search(L, per_cu); });
+  // (the search asks for the device's CUs too)
+  return t_shapes.get(L, 0, (int64_t)per_cu << 32 | device_cus(),
+                      [&] { return level1_search(L, per_cu); });
 }
 
 // The fine level's shape (k_fine_march): (TY + 1) x (TZ + 1) nodes within the
