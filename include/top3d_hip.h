@@ -417,12 +417,15 @@ int top3d_time_kernel(struct SolverDataBuffer *data, int which, int reps,
 
 /* Live timing of the fine-level damped-Jacobi sweeps inside the V-cycles of
  * the following solves: HIP events on the library stream around each run of
- * consecutive sweeps (the 3 after the first pre-sweep, the 4 post-sweeps),
- * which execute back to back.  enable = 1 clears the accumulators and starts
- * recording, 0 stops.
- * Outputs (any may be NULL): mean milliseconds per sweep so far, number of
- * sweeps timed, algorithmic bytes of one sweep (as top3d_time_kernel 0 / 1
- * for the mixed / FP64 form).                                               */
+ * consecutive plain sweeps, which execute back to back: of the 3 after the
+ * first pre-sweep the last 2 (the first shares a launch with the pre-sweep
+ * before it), of the 4 post-sweeps all, in the mixed form the last 3 (the
+ * first adds the coarse correction).  enable = 1 clears the accumulators and
+ * starts recording, 0 stops.
+ * Outputs (any may be NULL): mean milliseconds per plain sweep so far, number
+ * of sweeps of the V-cycles after their first (7 per V(4,4)-cycle, in launches
+ * of their own or not), algorithmic bytes of one plain sweep (as
+ * top3d_time_kernel 0 / 1 for the mixed / FP64 form).                       */
 int top3d_sweep_timing(struct SolverDataBuffer *data, int enable, double *avg_ms,
                        int *count, double *bytes);
 

@@ -228,11 +228,56 @@ static int shapes_by_device() {
   return 0;
 }
 
+// The events of the live sweep timing enclose launches of the plain fine sweep
+// (mode 3 of k_fine_march) only, and the mean is over those.
+static int sweep_timing() {
+  for (const int mixed : {0, 1}) {
+    Grid g(16, 8, 8, 3);
+    SolverDataBuffer data{};
+    allocateSolverData(g.gc, 3, &data);
+    top3d_set_precision(&data, mixed ? TOP3D_MIXED : TOP3D_FP64);
+    top3d_set_max_iter(&data, 1);
+    Device x(g.nelem()), F(g.ndof(0)), U(g.ndof(0));
+    std::vector<std::string> order;  // launches, "" for a recorded event
+    std::map<void *, int> at;
+    fake::on_launch = [&](const Launch &l) { order.push_back(l.name); };
+    fake::on_record = [&](void *e) {
+      at[e] = (int)order.size();
+      order.push_back("");
+    };
+    int enclosed = 0;
+    bool plain = true;
+    fake::elapsed = [&](void *a, void *b) {  // 1 ms per launch between them
+      for (int i = at[a] + 1; i < at[b]; i++) {
+        enclosed++;
+        plain = plain && order[i].find("k_fine_march") != std::string::npos &&
+                order[i].find("Li3E") != std::string::npos;
+      }
+      return (float)(at[b] - at[a] - 1);
+    };
+    int it, count = 0;
+    float res;
+    double ms = 0.0;
+    top3d_sweep_timing(&data, 1, nullptr, nullptr, nullptr);
+    solveStateMG_halo(&g.gpu, x.p, 4, 3, 1e-5, &data, &it, &res, F.p, U.p);
+    top3d_sweep_timing(&data, 0, &ms, &count, nullptr);
+    fake::on_launch = nullptr;
+    fake::on_record = nullptr;
+    fake::elapsed = nullptr;
+    freeSolverData(&data, 3);
+    REQUIRE(count == 7);                       // of one V(4,4)-cycle
+    REQUIRE(plain && enclosed == (mixed ? 5 : 6));  // one or two in launches with more work
+    REQUIRE(ms == 1.0);
+  }
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, int (*)()> checks = {
       {"filter_sums", filter_sums}, {"filter_without_memory", filter_without_memory},
       {"change_without_memory", change_without_memory},
-      {"given_back", given_back}, {"shapes_by_device", shapes_by_device}};
+      {"given_back", given_back}, {"shapes_by_device", shapes_by_device},
+      {"sweep_timing", sweep_timing}};
   auto it = argc > 1 ? checks.find(argv[1]) : checks.end();
   if (it == checks.end()) return 2;
   const int rc = it->second();

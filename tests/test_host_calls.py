@@ -29,7 +29,8 @@ def checker(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["filter_sums", "filter_without_memory",
-                                   "change_without_memory", "given_back", "shapes_by_device"])
+                                   "change_without_memory", "given_back", "shapes_by_device",
+                                   "sweep_timing"])
 def test_host_calls(checker, check):
     out = subprocess.run([checker, check], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0 and out.stdout.strip() == "OK", out.stdout + out.stderr

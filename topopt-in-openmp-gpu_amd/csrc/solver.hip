@@ -257,9 +257,11 @@ void SolverState::op(int l, int mode, const T *in, T *out, const T *b) {
     launch_stencil_half<T>(*g, l, mode, stencil_t<T>(l), in, out, b, invD, omega);
 }
 
-// Live sweep timing: an event pair brackets each run of consecutive fine
+// Live sweep timing: an event pair brackets each run of consecutive plain fine
 // sweeps, which the stream executes back to back.  (A pair around every
-// sweep delays the next launch by 4-8 us per record.)
+// sweep delays the next launch by 4-8 us per record.)  The launches that do more
+// than a sweep, from zero or with the coarse correction, stay outside: they move
+// other bytes (at 256x128x128 in FP32 46 and 48.6 us beside 34.5).
 bool SolverState::sweep_timing_begin() {
   if (!sweep_timing) return false;
   while (sw_ev.size() < sw_used + 2) {
@@ -293,15 +295,19 @@ T *SolverState::smooth_from_zero(int l, const T *b, T *zb, T *tb, bool zero_done
     launch_fine_jacobi_zero<T, T>(*g, b, young_t<T>(), (T)kOmega, cur);
   else
     launch_jacobi_zero<T, T>(*g, l, b, invd<T>(l), (T)kOmega, cur);
-  const bool rec = l == 0 && nswp > 1 && sweep_timing_begin();
-  for (int s = 1; s < nswp; s++) {
-    if (two && s == 1)
-      launch_fine_first_sweeps<T>(*g, young_t<T>(), (const T *)rs0, b, (T)kOmega, oth, bcsym);
-    else
-      op<T>(l, 1, cur, oth, b);
+  int s0 = 1;
+  if (two) {
+    launch_fine_first_sweeps<T>(*g, young_t<T>(), (const T *)rs0, b, (T)kOmega, oth, bcsym);
+    std::swap(cur, oth);
+    s0 = 2;
+  }
+  const bool rec = l == 0 && s0 < nswp && sweep_timing_begin();
+  for (int s = s0; s < nswp; s++) {
+    op<T>(l, 1, cur, oth, b);
     std::swap(cur, oth);
   }
-  sweep_timing_end(rec, nswp - 1);
+  sweep_timing_end(rec, nswp - s0);
+  if (l == 0 && sweep_timing) sw_count += nswp - 1;
   return cur;  // == zb
 }
 
@@ -310,16 +316,17 @@ T *SolverState::smooth_from_zero(int l, const T *b, T *zb, T *tb, bool zero_done
 // the coarse correction that the first sweep is to add to cur.
 template <typename T>
 T *SolverState::smooth(int l, const T *b, T *cur, T *oth, const T *add) {
-  const bool rec = l == 0 && nswp > 0 && sweep_timing_begin();
-  for (int s = 0; s < nswp; s++) {
-    if constexpr (sizeof(T) == 4) {
-      if (add && s == 0) {
-        launch_fine_prolong_sweep(*g, E32, (const float *)rs0, cur, add, b, (float)kOmega, oth,
-                                  bcsym);
-        std::swap(cur, oth);
-        continue;
-      }
+  int s0 = 0;
+  if constexpr (sizeof(T) == 4) {
+    if (add) {
+      launch_fine_prolong_sweep(*g, E32, (const float *)rs0, cur, add, b, (float)kOmega, oth,
+                                bcsym);
+      std::swap(cur, oth);
+      s0 = 1;
     }
+  }
+  const bool rec = l == 0 && s0 < nswp && sweep_timing_begin();
+  for (int s = s0; s < nswp; s++) {
     if (l == 0 && s == nswp - 1)
       rz_parts = launch_fine_sweep_dot<T>(*g, young_t<T>(), cur, oth, b, invd<T>(0), (T)kOmega,
                                           bcsym, cgpart, kPartRZ);
@@ -327,7 +334,8 @@ T *SolverState::smooth(int l, const T *b, T *cur, T *oth, const T *add) {
       op<T>(l, 1, cur, oth, b);
     std::swap(cur, oth);
   }
-  sweep_timing_end(rec, nswp);
+  sweep_timing_end(rec, nswp - s0);
+  if (l == 0 && sweep_timing) sw_count += nswp;
   return cur;
 }
 
@@ -378,7 +386,7 @@ void SolverState::collect_sweep_timing() {
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, sw_ev[k], sw_ev[k + 1]) == hipSuccess) {
       sw_ms += ms;
-      sw_count += sw_n[k / 2];
+      sw_timed += sw_n[k / 2];
     }
   }
   sw_used = 0;
@@ -578,11 +586,11 @@ int top3d_sweep_timing(struct SolverDataBuffer *data, int enable, double *avg_ms
   if (!s) return top3d_last_error();
   if (enable) {
     s->sw_ms = 0.0;
-    s->sw_count = 0;
+    s->sw_count = s->sw_timed = 0;
     s->sw_used = 0;
   }
   s->sweep_timing = enable != 0;
-  if (avg_ms) *avg_ms = s->sw_count ? s->sw_ms / s->sw_count : 0.0;
+  if (avg_ms) *avg_ms = s->sw_timed ? s->sw_ms / s->sw_timed : 0.0;
   if (count) *count = s->sw_count;
   if (bytes) {  // u, b (and invD unless formed from E) in; u out; E
     const DevGrid &g = *s->g;

@@ -68,13 +68,14 @@ struct SolverState {
   void join_coarse();
   Top3dSolveStats stats{};
   // live timing of the fine sweeps (top3d_sweep_timing): one event pair
-  // around each run of consecutive sweeps, sw_n[k] sweeps in pair k
+  // around each run of consecutive plain sweeps, sw_n[k] in pair k; sw_timed of
+  // the sw_count sweeps so far are in sw_ms (the others share a launch)
   bool sweep_timing = false;
   std::vector<hipEvent_t> sw_ev;
   std::vector<int> sw_n;
   size_t sw_used = 0;
   double sw_ms = 0.0;
-  int sw_count = 0;
+  int sw_count = 0, sw_timed = 0;
   bool sweep_timing_begin();
   void sweep_timing_end(bool rec, int nsweeps);
   void collect_sweep_timing();

@@ -488,7 +488,8 @@ class Grid:
 
     def sweep_timing(self, enable):
         """Start (enable=True) or stop live timing of the fine sweeps inside the
-        V-cycles; returns (mean ms per sweep, sweeps timed, bytes per sweep)."""
+        V-cycles; returns (mean ms per plain sweep, sweeps of the V-cycles, bytes
+        per plain sweep)."""
         ms, cnt, by = c_double(), c_int(), c_double()
         rc = self.lib.top3d_sweep_timing(ctypes.byref(self.data), int(bool(enable)),
                                          ctypes.byref(ms), ctypes.byref(cnt), ctypes.byref(by))
