@@ -387,7 +387,9 @@ int top3d_compliance_backward(const struct gpuGrid *gpu_gc, double rmin,
  * out = H (in / Hs) between two device (or mapped) element arrays, in != out;
  * the halo elements of out keep their values, become zero or take those of
  * in.  applyDensityFilter and applyDensityFilterGradient without their staging
- * and, for the latter, without the copy back into its in-place argument.     */
+ * and, for the latter, without the copy back into its in-place argument.
+ * Calls of several host threads on one grid may overlap, but for transposes at
+ * rmin > 7, which share an array of the grid.                                */
 #define TOP3D_HALO_KEEP 0
 #define TOP3D_HALO_ZERO 1
 #define TOP3D_HALO_COPY 2
